@@ -93,10 +93,10 @@ int qfe_get_tuning(int* tile_qubits, int* low_qubits, int* max_ops_per_pass);
  * orbit over 2, 4 or 8 lanes of a wave); no reference counterpart (autotuner hook). */
 int qfe_set_pass_tuning(int orbit_max_dims);
 int qfe_get_pass_tuning(int* orbit_max_dims);
-/* Largest number of determinant pairs for which a sector template stores one
- * 8-byte pair word per pair (templates above it rotate from the compact
- * string lists); applies to templates created afterwards.  Default 2^25.  No
- * reference counterpart (memory / speed trade-off of the sector engine). */
+/* Once the largest number of determinant pairs for which a sector template
+ * stored one word per pair.  Templates now keep compact list words per tile
+ * (a few MB for 20 qubits) whatever the limit, and results never depended on
+ * it; kept for callers that set it.  No reference counterpart. */
 int qfe_set_sector_word_limit(uint64_t max_pair_words);
 /* HIP events on the library stream, for timing kernels from the host
  * (no reference counterpart). */
@@ -264,15 +264,16 @@ int qfe_template_destroy(qfe_template t);
 /* Sector dimension and device bytes one request of this template occupies. */
 int qfe_template_info(qfe_template t, uint64_t* sector_dim, uint64_t* request_bytes);
 /* Host-side audit of a captured single-request sequence (no reference
- * counterpart; a diagnostic for callers and tests).  Templates whose state
- * does not fit one workgroup's LDS replay their energy (gradient = 0) and
- * gradient (gradient = 1) sequences as hipGraphs; every capture is checked
- * before it is kept: one chain of nodes, each node the expected memcpy or
- * kernel, grids non-zero, blocks of 1..1024 threads, arguments and copy
- * extents equal to the addresses the template owns.  Builds the graph if
- * needed and writes out4 = {nodes, kernel nodes, kernel nodes whose arguments
- * were compared, memcpy nodes whose parameters were compared}; all zero for
- * templates that launch without a graph. */
+ * counterpart; a diagnostic for callers and tests).  For templates whose state
+ * does not fit one workgroup's LDS the energy (gradient = 0) or gradient
+ * (gradient = 1) evaluation is captured as one launch per step and generator,
+ * and every node is checked: one chain of nodes, each node the expected
+ * memcpy or kernel, grids non-zero, blocks of 1..1024 threads, arguments and
+ * copy extents equal to the addresses the template owns.  Writes out4 =
+ * {nodes, kernel nodes, kernel nodes whose arguments were compared, memcpy
+ * nodes whose parameters were compared}; all zero for smaller templates.
+ * qfe_template_energy and _gradient launch tile passes instead (many steps
+ * each) and need no graph. */
 int qfe_template_graph_audit(qfe_template t, int gradient, uint64_t* out4);
 /* One request in one launch (no batching): E = <ref|U^dag H U|ref>. */
 int qfe_template_energy(qfe_template t, const double* params, const double* inputs, double* energy);

@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 #include <deque>
+#include <functional>
 #include <map>
 #include <tuple>
 #include <unordered_map>
@@ -61,7 +62,6 @@ struct SecEntry {  // one class of determinant pairs of a run
     double w, inv_lb;
     double2 ulo, uhi;  // A(p_lo) / w, A(p_hi) / w
     uint32_t step;
-    uint32_t w_off;  // first pair word of the entry (when the template has pair words)
 };
 
 struct SecGroup {  // Hamiltonian terms sharing an X mask, on sector pairs
@@ -75,6 +75,38 @@ struct SecGroup {  // Hamiltonian terms sharing an X mask, on sector pairs
 struct SecItem {  // groups [g0, g1) whole, or pairs [p0, p1) of group g0 when g1 == g0 + 1
     uint32_t g0, g1, p0, p1;
 };
+
+// ---- component tiles ----
+// A segment is a run of consecutive generators.  The flips of its entries
+// join alpha strings into components and beta strings likewise; a block is a
+// union of whole components, so no pair of the segment leaves the tile
+// (alpha block) x (beta block), and a workgroup applies the whole segment to
+// its tile in LDS: one load and one store of the state per segment.
+struct TileSeg {
+    uint32_t nab, nbb;      // alpha and beta blocks
+    uint32_t ablk, bblk;    // tix: first position of each block (nab + 1, nbb + 1 entries)
+    uint32_t aperm, bperm;  // tix: string ranks, block by block
+    uint32_t awb, bwb;      // tix: first word of each block (nab + 1, nbb + 1 entries)
+    uint32_t atab, btab;    // ttab: [list * nab + block], [list * nbb + block]
+};
+
+struct TileRec {  // one entry in the program of a pass
+    double w;
+    double2 ulo, uhi;
+    uint32_t entry, alist, blist, flags;
+};
+constexpr uint32_t kRecRot = 1;      // rotate (or un-rotate) the entry's pairs
+constexpr uint32_t kRecOv = 2;       // add the pairs' overlaps
+constexpr uint32_t kRecStepEnd = 4;  // the next record reads what this one wrote
+constexpr uint32_t kRecGenEnd = 8;   // the overlap of a generator is complete
+
+struct TileRun {  // one pass: the records [rec0, rec0 + nrec) over the tiles of a segment
+    uint32_t seg, rec0, nrec, part;  // part: first partial sum (reverse sweep)
+};
+
+// A list word: local position of a string and of its partner in their block,
+// and the parities of the entry's sign mask on both.
+constexpr uint32_t kWordBits = 14, kWordPos = (1u << kWordBits) - 1u;
 
 struct SecTables {  // device view of a template (lives in device memory)
     uint64_t D, ref_rank;
@@ -98,7 +130,15 @@ struct SecTables {  // device view of a template (lives in device memory)
     const uint32_t* map_idx;
     const double2* map_val;
     const uint2* hchunks;  // groups [x, y) staged together by the sigma kernel
-    const uint2* words;    // pair words of every entry, in entry order (null: use the lists)
+    const TileSeg* tsegs;
+    const TileRun* tfwd;   // ansatz passes, in order
+    const TileRun* trev;   // reverse-sweep passes, in order
+    const TileRec* trec;
+    const uint32_t* tix;   // block starts, permuted ranks and word starts of every segment
+    const uint2* ttab;     // (offset, length) of every list in every block
+    const uint32_t* twords;
+    const uint2* tsum;     // ranges (first, count) of reverse-sweep partial sums
+    const uint32_t* tsum_off;  // ranges of output k: [tsum_off[k], tsum_off[k + 1]); 0 the energy, k + 1 generator k
     uint32_t nsteps, nentries, ngroups, nterms, nitems, ngen, nhchunks;
 };
 
@@ -109,6 +149,7 @@ struct SlotDesc {
     double2* coef;  // per-request coefficients (null: t->tcoef)
     double2* cs;    // (cos, sin) per entry
     double* part;   // per work item energy partials
+    double* gpart;  // reverse-sweep partial sums (gradients only)
     double* gacc;   // per generator <sigma|K|psi> (gradients only)
     const double* params;
     const double* inputs;
@@ -119,7 +160,6 @@ struct PoolOp {  // entries [e0, e1) of one pool operator
     uint32_t e0, e1;
 };
 
-constexpr uint32_t kTableLds = 1024;  // alpha + beta string tables staged in LDS when they fit
 constexpr uint32_t kTermLds = 1024;   // Hamiltonian terms of one group staged in LDS when they fit
 constexpr int kUnroll = 4;            // independent pairs in flight per thread
 constexpr int kItemThreads = 256;
@@ -179,8 +219,7 @@ __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict
 
 // One pair (r1, r2) of an entry with old values (a, b), j1 the determinant
 // of r1: psi_1' = c a + s s(j2) uhi b, psi_2' = c b + s s(j1) ulo a.  Every
-// kernel that rotates pairs calls this, so a pair's result does not depend on
-// which kernel or launch shape applied it.
+// step-by-step kernel calls this; the tile passes apply the same formula.
 __device__ __forceinline__ void pair_rotate_signed(double2* __restrict__ psi, uint64_t r1, uint64_t r2, double2 a,
                                                    double2 b, double c, double s1, double s2, double2 ulo, double2 uhi) {
     const double2 hb = cmul(uhi, b), la = cmul(ulo, a);
@@ -192,13 +231,6 @@ __device__ __forceinline__ void pair_rotate(double2* __restrict__ psi, uint64_t 
                                             double2 uhi) {
     pair_rotate_signed(psi, r1, r2, a, b, c, s * parity_sign(j1 & z0), s * parity_sign((j1 ^ x) & z0), ulo, uhi);
 }
-
-// Pair word of a sector pair: .x = r1 | [parity of (j1 ^ x) & z0] << 31,
-// .y = r2 | [parity of j1 & z0] << 31, j1 the determinant of rank r1.  One
-// 8-byte load per pair instead of two list loads, two string-table loads and
-// a division; ranks stay below 2^31 (at most C(16, 8)^2 determinants).
-constexpr uint32_t kWordRank = 0x7fffffffu;
-__device__ __forceinline__ double word_sign(uint32_t v, double s) { return (v >> 31) ? -s : s; }
 
 // <sigma|K|psi> contribution of one pair (the entry_overlap formula), with
 // s1 = w (-1)^{|j1 & z0|} and s2 = w (-1)^{|(j1 ^ x) & z0|}.
@@ -220,172 +252,255 @@ __device__ __forceinline__ double flip_sign(double v, uint32_t neg) {
     return __hiloint2double(__double2hiint(v) ^ (int)neg, __double2loint(v));
 }
 
-// Rotate every pair of entry `en` by (c, sgn * s); pairs of one step are
-// disjoint, so kUnroll of them are in flight per thread (loads first).
-template <int THREADS>
-__device__ __forceinline__ void rotate_entry(const SecTables* __restrict__ T, const SecEntry& en, double c, double s,
-                                             double2* __restrict__ psi, const uint64_t* __restrict__ af,
-                                             const uint64_t* __restrict__ bf, uint32_t tid) {
-    const uint64_t Db = T->Db;
-    const uint32_t lb = en.lb_len, total = en.la_len * lb;
-    const uint64_t x = en.x, z0 = en.z0;
-    const double2 ulo = en.ulo, uhi = en.uhi;
-    const double inv = en.inv_lb;
-    for (uint32_t i0 = tid; i0 < total; i0 += kUnroll * THREADS) {
-        uint64_t r1[kUnroll], r2[kUnroll], j1[kUnroll];
-        double2 a[kUnroll], b[kUnroll];
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const uint32_t i = i0 + u * THREADS;
-            if (i < total) {
-                uint32_t ia, ib;
-                divmod_u(i, lb, inv, ia, ib);
-                const int2 pa = T->lists[en.la_off + ia];
-                const int2 pb = T->lists[en.lb_off + ib];
-                r1[u] = (uint64_t)pa.x * Db + (uint64_t)pb.x;
-                r2[u] = (uint64_t)pa.y * Db + (uint64_t)pb.y;
-                j1[u] = af[pa.x] | bf[pb.x];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (i0 + u * THREADS < total) {
-                a[u] = psi[r1[u]];
-                b[u] = psi[r2[u]];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (i0 + u * THREADS < total) pair_rotate(psi, r1[u], r2[u], a[u], b[u], j1[u], x, z0, c, s, ulo, uhi);
-        }
-    }
+// ---- 2. ansatz and reverse sweep: component tiles ---------------------------------------
+// A sector amplitude: double2, or double when every generator and every
+// Hamiltonian coefficient is real (then the state is real throughout).
+__device__ __forceinline__ double2 umul(double2 u, double2 v) { return cmul(u, v); }
+__device__ __forceinline__ double2 lincomb(double c, double2 a, double s, double2 h) {
+    return make_double2(c * a.x + s * h.x, c * a.y + s * h.y);
+}
+__device__ __forceinline__ double re_dot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
+template <typename S>
+__device__ __forceinline__ S real_amp(double v);
+template <>
+__device__ __forceinline__ double2 real_amp<double2>(double v) {
+    return make_double2(v, 0.0);
 }
 
-// Stage the string tables into LDS when they fit; returns the table pointers.
-__device__ __forceinline__ void stage_tables(const SecTables* __restrict__ T, uint64_t* tab, const uint64_t*& af,
-                                             const uint64_t*& bf, uint32_t tid, uint32_t nthreads) {
-    if (T->Da + T->Db <= kTableLds) {
-        for (uint32_t k = tid; k < T->Da; k += nthreads) tab[k] = T->afull[k];
-        for (uint32_t k = tid; k < T->Db; k += nthreads) tab[T->Da + k] = T->bfull[k];
-        af = tab;
-        bf = tab + T->Da;
-    } else {
-        af = T->afull;
-        bf = T->bfull;
-    }
+// v + the value CTRL lanes away (0 where there is none).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+// Sum over the 64 lanes in a fixed order, in lane 63: four row shifts and two
+// row broadcasts on the vector pipe, where __shfl_xor goes through LDS.
+__device__ __forceinline__ double wave_sum_last(double v) {
+    v = dpp_add<0x111>(v);  // row_shr:1
+    v = dpp_add<0x112>(v);  // row_shr:2
+    v = dpp_add<0x114>(v);  // row_shr:4
+    v = dpp_add<0x118>(v);  // row_shr:8
+    v = dpp_add<0x142>(v);  // row_bcast:15
+    v = dpp_add<0x143>(v);  // row_bcast:31
+    return v;
 }
 
-// ---- 2. ansatz: U|ref> by one workgroup per request ------------------------------------
-// With PSI_LDS the state lives in LDS (dynamic LDS = D * 16 bytes + string
-// tables) and is written to the request's buffer at the end.
-// Pair words of chunk [base, base + K * THREADS) of an entry with P pairs.
-template <int K, int THREADS>
-__device__ __forceinline__ void load_words(uint2 (&w)[K], const uint2* __restrict__ src, uint32_t P, uint32_t base,
-                                           uint32_t tid) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const uint32_t i = base + k * THREADS + tid;
-        w[k] = i < P ? src[i] : make_uint2(0u, 0u);
-    }
-}
+constexpr uint32_t kRecChunk = 128;        // records staged in LDS at a time
+constexpr uint32_t kTileWordsLds = 4096;   // list words of a tile staged in LDS when they fit
 
-// Position of a chunk of K * THREADS pairs: entry e, first pair base (e ==
-// ne: past the last entry).
-struct WordCursor {
-    uint32_t e, base;
+struct LdsRec {  // a record as the tile's loop reads it
+    double c, s, w, ulo_x, ulo_y, uhi_x, uhi_y;
+    uint32_t a_off, b_off, b_len, pairs, magic, flags;
 };
 
-template <int K, int THREADS>
-__device__ __forceinline__ WordCursor next_chunk(const SecEntry* __restrict__ ent, uint32_t ne, WordCursor c) {
-    if (c.e >= ne) return c;
-    c.base += K * THREADS;
-    if (c.base >= ent[c.e].la_len * ent[c.e].lb_len) {
-        ++c.e;
-        c.base = 0;
-    }
-    return c;
-}
+// i / d for i < 2^16, 0 < d < 2^16 by a multiplication: ceil(2^32 / d) (0 for d = 1).
+__host__ __device__ __forceinline__ uint32_t div_magic(uint32_t d) { return d > 1 ? (uint32_t)((0x100000000ull + d - 1) / d) : 0u; }
+__device__ __forceinline__ uint32_t div_by(uint32_t i, uint32_t magic) { return magic ? __umulhi(i, magic) : i; }
 
-template <int K, int THREADS>
-__device__ __forceinline__ void load_chunk(uint2 (&w)[K], const SecEntry* __restrict__ ent, const uint2* __restrict__ words,
-                                           uint32_t ne, WordCursor c, uint32_t tid) {
-    if (c.e < ne) load_words<K, THREADS>(w, words + ent[c.e].w_off, ent[c.e].la_len * ent[c.e].lb_len, c.base, tid);
-}
-
-// The entries in order from pair words, K pairs per thread per chunk.  The
-// words of the chunk DEPTH ahead are loaded while the current one rotates, so
-// a step's dependent chain is the amplitude loads and stores (DEPTH = 2 when
-// the state is in LDS and a step is shorter than a load from memory).
-template <int K, int THREADS, int DEPTH>
-__device__ __forceinline__ void ansatz_words(const SlotDesc& sd, const SecTables* __restrict__ T, double2* __restrict__ psi,
-                                             uint32_t tid) {
-    static_assert(DEPTH == 1 || DEPTH == 2, "prefetch depth 1 or 2");
-    const SecEntry* __restrict__ ent = T->entries;
-    const uint2* __restrict__ words = T->words;
-    const uint32_t ne = T->nentries;
-    WordCursor cur{0u, 0u};
-    WordCursor c1 = next_chunk<K, THREADS>(ent, ne, cur);
-    uint2 w[K], w1[K], w2[K];
-    load_chunk<K, THREADS>(w, ent, words, ne, cur, tid);
-    if constexpr (DEPTH == 2) load_chunk<K, THREADS>(w1, ent, words, ne, c1, tid);
-    WordCursor c2 = next_chunk<K, THREADS>(ent, ne, c1);
-    __syncthreads();
-    while (cur.e < ne) {
-        const uint32_t e = cur.e, P = ent[e].la_len * ent[e].lb_len;
-        const double2 cs = sd.cs[e], ulo = ent[e].ulo, uhi = ent[e].uhi;
-        double2 a[K], b[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            if (cur.base + k * THREADS + tid < P) {
-                a[k] = psi[w[k].x & kWordRank];
-                b[k] = psi[w[k].y & kWordRank];
-            }
-        }
-        if constexpr (DEPTH == 2)
-            load_chunk<K, THREADS>(w2, ent, words, ne, c2, tid);
-        else
-            load_chunk<K, THREADS>(w1, ent, words, ne, c1, tid);
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            if (cur.base + k * THREADS + tid < P)
-                pair_rotate_signed(psi, w[k].x & kWordRank, w[k].y & kWordRank, a[k], b[k], cs.x,
-                                   word_sign(w[k].y, cs.y), word_sign(w[k].x, cs.y), ulo, uhi);
-            w[k] = w1[k];
-            if constexpr (DEPTH == 2) w1[k] = w2[k];
-        }
-        if (cur.base + K * THREADS >= P && (e + 1 == ne || ent[e + 1].step != ent[e].step)) __syncthreads();
-        cur = c1;
-        c1 = c2;
-        c2 = next_chunk<K, THREADS>(ent, ne, c2);
-    }
-}
-
-template <bool PSI_LDS, int THREADS, int K>
-__global__ __launch_bounds__(THREADS) void k_sec_ansatz(const SlotDesc* __restrict__ slots) {
-    extern __shared__ double2 sh[];
-    const SlotDesc sd = slots[blockIdx.x];
-    const SecTables* __restrict__ T = sd.t;
+// One pass over the tiles of a segment, one workgroup of T threads per tile.
+// MODE 0: the segment's rotations on psi (q = 0 starts from the reference);
+// MODE 1: their inverses on sigma; MODE 2: the reverse sweep on psi and
+// sigma: for each generator, last first, the tile's part of
+// Re<sigma|K|psi>, then its inverse on both (q = 0 also adds Re<psi|sigma>).
+// One workgroup used to walk all generators of a request, or one launch took
+// each step of a lone large request: a step's pairs are few and its latency
+// (a barrier and an LDS or L2 round trip, or a launch) was what counted.
+// Tiles split the pairs of a step over many workgroups and keep many steps in
+// one launch.
+template <typename S, int T, int MODE>
+__global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slots, const uint32_t* __restrict__ prefix,
+                                                uint32_t nslots, uint32_t q, uint32_t start) {
+    extern __shared__ double2 tile_lds[];
     const uint32_t tid = threadIdx.x;
-    const uint64_t D = T->D;
-    double2* __restrict__ psi = PSI_LDS ? sh : sd.psi;
-    for (uint64_t r = tid; r < D; r += THREADS) psi[r] = make_double2(r == T->ref_rank ? 1.0 : 0.0, 0.0);
-    if (T->words) {
-        ansatz_words<K, THREADS, PSI_LDS ? 2 : 1>(sd, T, psi, tid);
-    } else {
-        const uint64_t *af, *bf;
-        stage_tables(T, (uint64_t*)(sh + (PSI_LDS ? D : 0)), af, bf, tid, THREADS);
-        __syncthreads();
-        for (uint32_t s = 0; s < T->nsteps; ++s) {
-            const uint32_t e0 = T->steps[s].e_first, e1 = e0 + T->steps[s].e_count;
-            for (uint32_t e = e0; e < e1; ++e) {
-                const double2 cs = sd.cs[e];
-                rotate_entry<THREADS>(T, T->entries[e], cs.x, cs.y, psi, af, bf, tid);
+    const uint32_t slot = nslots == 1 ? 0u : find_slot(prefix, nslots, blockIdx.x);
+    const uint32_t tile = nslots == 1 ? blockIdx.x : blockIdx.x - prefix[slot];
+    const SlotDesc sd = slots[slot];
+    const SecTables* __restrict__ Tb = sd.t;
+    const TileRun run = (MODE == 2 ? Tb->trev : Tb->tfwd)[q];
+    const TileSeg sg = Tb->tsegs[run.seg];
+    const uint32_t* __restrict__ tix = Tb->tix;
+    const uint32_t ab = tile / sg.nbb, bb = tile - ab * sg.nbb;
+    const uint32_t a0 = tix[sg.ablk + ab], na = tix[sg.ablk + ab + 1] - a0;
+    const uint32_t b0 = tix[sg.bblk + bb], nb = tix[sg.bblk + bb + 1] - b0;
+    const uint32_t aw0 = tix[sg.awb + ab], naw = tix[sg.awb + ab + 1] - aw0;
+    const uint32_t bw0 = tix[sg.bwb + bb], nbw = tix[sg.bwb + bb + 1] - bw0;
+    const uint32_t n = na * nb, nmag = div_magic(nb), ntiles = sg.nab * sg.nbb;
+    const uint32_t nrec = run.nrec, nchunk = nrec < kRecChunk ? nrec : kRecChunk;
+    S* X = reinterpret_cast<S*>(tile_lds);
+    S* Y = X + (MODE == 2 ? n : 0u);
+    LdsRec* recs = reinterpret_cast<LdsRec*>(tile_lds + ((n * (MODE == 2 ? 2u : 1u) * sizeof(S) + 15) >> 4));
+    uint32_t* lw = reinterpret_cast<uint32_t*>(recs + nchunk);
+    const bool wlds = naw + nbw <= kTileWordsLds;
+    S* __restrict__ gx = reinterpret_cast<S*>(MODE == 1 ? sd.sig : sd.psi);
+    S* __restrict__ gy = reinterpret_cast<S*>(sd.sig);
+    const uint64_t Db = Tb->Db;
+
+    // records [c0, c0 + cnt) in the order of this pass; returns whether this
+    // thread's records have pairs in the tile
+    auto stage = [&](uint32_t c0, uint32_t cnt) {
+        bool any = false;
+        for (uint32_t r = tid; r < cnt; r += T) {
+            const uint32_t at = MODE == 1 ? run.rec0 + nrec - 1 - (c0 + r) : run.rec0 + c0 + r;
+            const TileRec tr = Tb->trec[at];
+            const uint2 la = Tb->ttab[sg.atab + tr.alist * sg.nab + ab], lb = Tb->ttab[sg.btab + tr.blist * sg.nbb + bb];
+            const double2 cs = sd.cs[tr.entry];
+            LdsRec o;
+            o.c = cs.x;
+            o.s = MODE == 0 ? cs.y : -cs.y;
+            o.w = tr.w;
+            o.ulo_x = tr.ulo.x;
+            o.ulo_y = tr.ulo.y;
+            o.uhi_x = tr.uhi.x;
+            o.uhi_y = tr.uhi.y;
+            o.a_off = la.x;
+            o.b_off = lb.x;
+            o.b_len = lb.y;
+            o.pairs = la.y * lb.y;
+            o.magic = div_magic(lb.y);
+            o.flags = tr.flags;
+            // last step first: a step ends before the record that ends the step before it
+            if (MODE == 1) o.flags = kRecRot | (at > run.rec0 ? Tb->trec[at - 1].flags & kRecStepEnd : 0u);
+            any |= o.pairs != 0;
+            recs[r] = o;
+        }
+        return any;
+    };
+    bool any = stage(0, nchunk);
+    if (wlds) {
+        for (uint32_t i = tid; i < naw; i += T) lw[i] = Tb->twords[aw0 + i];
+        for (uint32_t i = tid; i < nbw; i += T) lw[naw + i] = Tb->twords[bw0 + i];
+    }
+    // a tile without pairs keeps its amplitudes
+    const bool idle = nrec <= kRecChunk && !__syncthreads_or(any) && !start;
+    if (idle) {
+        if (MODE == 2)
+            for (uint32_t r = 0, k = 0; r < nrec; ++r)
+                if (Tb->trec[run.rec0 + r].flags & kRecGenEnd) {
+                    if ((tid & (kWave - 1)) == 0)
+                        sd.gpart[run.part + (k * ntiles + tile) * (T / kWave) + tid / kWave] = 0.0;
+                    ++k;
+                }
+        return;
+    }
+    double dot = 0.0;
+    for (uint32_t i = tid; i < n; i += T) {
+        const uint32_t la = div_by(i, nmag), lb = i - la * nb;
+        const uint64_t r = (uint64_t)tix[sg.aperm + a0 + la] * Db + tix[sg.bperm + b0 + lb];
+        if (MODE == 0 && start) {
+            X[i] = real_amp<S>(r == Tb->ref_rank ? 1.0 : 0.0);
+        } else {
+            const S x = gx[r];
+            X[i] = x;
+            if (MODE == 2) {
+                const S y = gy[r];
+                Y[i] = y;
+                dot += re_dot(x, y);
             }
+        }
+    }
+    uint32_t part = MODE == 2 ? run.part + tile * (T / kWave) + tid / kWave : 0u;  // next partial sum of this wave
+    const uint32_t pstep = ntiles * (T / kWave);
+    if (MODE == 2 && start) {
+        const double v = wave_sum_last(dot);
+        if ((tid & (kWave - 1)) == kWave - 1) sd.gpart[part] = v;
+        part += pstep;
+    }
+    __syncthreads();
+
+    double acc = 0.0;
+    auto words = [&](const LdsRec& R, uint32_t i, uint32_t& wa, uint32_t& wb) {
+        const uint32_t ia = div_by(i, R.magic), ib = i - ia * R.b_len;
+        if (wlds) {
+            wa = lw[R.a_off + ia];
+            wb = lw[naw + R.b_off + ib];
+        } else {
+            wa = Tb->twords[aw0 + R.a_off + ia];
+            wb = Tb->twords[bw0 + R.b_off + ib];
+        }
+    };
+    auto pair = [&](const LdsRec& R, uint32_t wa, uint32_t wb) {
+        const uint32_t l1 = (wa & kWordPos) * nb + (wb & kWordPos);
+        const uint32_t l2 = ((wa >> kWordBits) & kWordPos) * nb + ((wb >> kWordBits) & kWordPos);
+        const uint32_t sw = wa ^ wb;  // bit 30: the parity on the string pair, bit 31: on its partner
+        const uint32_t n1 = (sw << 1) & 0x80000000u, n2 = sw & 0x80000000u;
+        const S a = X[l1], b = X[l2];
+        const double2 ulo = make_double2(R.ulo_x, R.ulo_y), uhi = make_double2(R.uhi_x, R.uhi_y);
+        if (MODE == 2) {
+            const S ya = Y[l1], yb = Y[l2];
+            if (R.flags & kRecOv)
+                acc += flip_sign(R.w, n2) * re_dot(ya, umul(uhi, b)) + flip_sign(R.w, n1) * re_dot(yb, umul(ulo, a));
+            if (R.flags & kRecRot) {
+                const double s1 = flip_sign(R.s, n1), s2 = flip_sign(R.s, n2);
+                X[l1] = lincomb(R.c, a, s2, umul(uhi, b));
+                X[l2] = lincomb(R.c, b, s1, umul(ulo, a));
+                Y[l1] = lincomb(R.c, ya, s2, umul(uhi, yb));
+                Y[l2] = lincomb(R.c, yb, s1, umul(ulo, ya));
+            }
+        } else {
+            X[l1] = lincomb(R.c, a, flip_sign(R.s, n2), umul(uhi, b));
+            X[l2] = lincomb(R.c, b, flip_sign(R.s, n1), umul(ulo, a));
+        }
+    };
+    for (uint32_t c0 = 0; c0 < nrec; c0 += kRecChunk) {
+        const uint32_t cnt = nrec - c0 < kRecChunk ? nrec - c0 : kRecChunk;
+        if (c0) {
+            __syncthreads();
+            stage(c0, cnt);
             __syncthreads();
         }
+        // the record and first words of the next entry are read while the
+        // current one is applied: they do not depend on its writes
+        LdsRec R = recs[0];
+        uint32_t wa = 0, wb = 0;
+        if (tid < R.pairs) words(R, tid, wa, wb);
+        for (uint32_t r = 0; r < cnt; ++r) {
+            LdsRec N = R;
+            uint32_t xa = 0, xb = 0;
+            if (r + 1 < cnt) {
+                N = recs[r + 1];
+                if (tid < N.pairs) words(N, tid, xa, xb);
+            }
+            if (tid < R.pairs) pair(R, wa, wb);
+            for (uint32_t i = tid + T; i < R.pairs; i += T) {
+                words(R, i, wa, wb);
+                pair(R, wa, wb);
+            }
+            if (MODE == 2 && (R.flags & kRecGenEnd)) {
+                const double v = wave_sum_last(acc);
+                if ((tid & (kWave - 1)) == kWave - 1) sd.gpart[part] = v;
+                part += pstep;
+                acc = 0.0;
+            }
+            if (R.flags & kRecStepEnd) __syncthreads();
+            R = N;
+            wa = xa;
+            wb = xb;
+        }
     }
-    if (PSI_LDS)
-        for (uint64_t r = tid; r < D; r += THREADS) sd.psi[r] = psi[r];
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += T) {
+        const uint32_t la = div_by(i, nmag), lb = i - la * nb;
+        const uint64_t r = (uint64_t)tix[sg.aperm + a0 + la] * Db + tix[sg.bperm + b0 + lb];
+        gx[r] = X[i];
+        if (MODE == 2) gy[r] = Y[i];
+    }
+}
+
+// Sums of the reverse sweep's partials in a fixed order, one wave each:
+// output 0 is the energy, output k + 1 generator k's overlap.
+__global__ __launch_bounds__(256) void k_sec_tile_sum(const SlotDesc* __restrict__ slots) {
+    const SlotDesc sd = slots[blockIdx.y];
+    const SecTables* __restrict__ T = sd.t;
+    const uint32_t k = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (k > T->ngen) return;
+    double acc = 0.0;
+    for (uint32_t r = T->tsum_off[k]; r < T->tsum_off[k + 1]; ++r) {
+        const uint2 range = T->tsum[r];
+        for (uint32_t i = lane; i < range.y; i += kWave) acc += sd.gpart[range.x + i];
+    }
+    const double v = wave_sum_last(acc);
+    if (lane == kWave - 1) (k ? sd.gacc[k - 1] : *sd.out) = v;
 }
 
 // ---- 3. energy work items: one workgroup per (request, item) ---------------------------
@@ -566,112 +681,6 @@ __global__ __launch_bounds__(256) void k_sec_hpsi(const SlotDesc* __restrict__ s
     }
 }
 
-// Sum over the pairs of entry en of Re(conj(sig) K psi).
-template <int THREADS>
-__device__ __forceinline__ double entry_overlap(const SecTables* __restrict__ T, const SecEntry& en,
-                                                const double2* __restrict__ sig, const double2* __restrict__ psi,
-                                                uint32_t tid) {
-    const uint64_t Db = T->Db;
-    const uint32_t lb = en.lb_len, total = en.la_len * lb;
-    double acc = 0.0;
-    for (uint32_t i = tid; i < total; i += THREADS) {
-        uint32_t ia, ib;
-        divmod_u(i, lb, en.inv_lb, ia, ib);
-        const int2 pa = T->lists[en.la_off + ia];
-        const int2 pb = T->lists[en.lb_off + ib];
-        const uint64_t r1 = (uint64_t)pa.x * Db + (uint64_t)pb.x, r2 = (uint64_t)pa.y * Db + (uint64_t)pb.y;
-        const uint64_t j1 = T->afull[pa.x] | T->bfull[pb.x];
-        const double s1 = en.w * parity_sign(j1 & en.z0), s2 = en.w * parity_sign((j1 ^ en.x) & en.z0);
-        // (K psi)_1 = s(j2) w uhi psi_2, (K psi)_2 = s(j1) w ulo psi_1
-        const double2 k1 = cmul(en.uhi, psi[r2]), k2 = cmul(en.ulo, psi[r1]);
-        const double2 a = sig[r1], b = sig[r2];
-        acc += s2 * (a.x * k1.x + a.y * k1.y) + s1 * (b.x * k2.x + b.y * k2.y);
-    }
-    return acc;
-}
-
-// Reverse sweep (one workgroup per request): E = Re<psi|sigma>, then for
-// k = M-1 .. 0: <sigma_k|K_k|psi_k>, and un-apply generator k on psi and sigma.
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void k_sec_reverse(const SlotDesc* __restrict__ slots) {
-    __shared__ double2 red[16];
-    const SlotDesc sd = slots[blockIdx.x];
-    const SecTables* __restrict__ T = sd.t;
-    const uint32_t tid = threadIdx.x;
-    double2* __restrict__ psi = sd.psi;
-    double2* __restrict__ sig = sd.sig;
-    double e = 0.0;
-    for (uint64_t r = tid; r < T->D; r += THREADS) e += psi[r].x * sig[r].x + psi[r].y * sig[r].y;
-    const double2 et = block_sum(make_double2(e, 0.0), red);
-    if (tid == 0) *sd.out = et.x;
-    for (uint32_t k = T->ngen; k-- > 0;) {
-        const uint32_t s0 = T->gen_step[k], s1 = T->gen_step[k + 1];
-        double acc = 0.0;
-        if (s1 == s0 + 1 && T->words) {
-            // one step from pair words: each pair's four old values give its
-            // overlap term and its un-rotated psi and sigma pair in one pass
-            for (uint32_t en = T->steps[s0].e_first; en < T->steps[s0].e_first + T->steps[s0].e_count; ++en) {
-                const SecEntry& E = T->entries[en];
-                const double2 cs = sd.cs[en];
-                const uint2* __restrict__ wp = T->words + E.w_off;
-                const uint32_t total = E.la_len * E.lb_len;
-                for (uint32_t i = tid; i < total; i += THREADS) {
-                    const uint2 w = wp[i];
-                    const uint64_t r1 = w.x & kWordRank, r2 = w.y & kWordRank;
-                    const double2 p1 = psi[r1], p2 = psi[r2], g1 = sig[r1], g2 = sig[r2];
-                    acc += pair_overlap_signed(E, word_sign(w.y, E.w), word_sign(w.x, E.w), p1, p2, g1, g2);
-                    const double n1 = word_sign(w.y, -cs.y), n2 = word_sign(w.x, -cs.y);
-                    pair_rotate_signed(psi, r1, r2, p1, p2, cs.x, n1, n2, E.ulo, E.uhi);
-                    pair_rotate_signed(sig, r1, r2, g1, g2, cs.x, n1, n2, E.ulo, E.uhi);
-                }
-            }
-            const double2 tot = block_sum(make_double2(acc, 0.0), red);  // its barriers order the writes above
-            if (tid == 0) sd.gacc[k] = tot.x;
-            continue;
-        }
-        if (s1 == s0 + 1) {
-            // one step: each pair's four old values give its overlap term and its
-            // un-rotated psi and sigma pair in one pass (pairs of a step are disjoint)
-            const uint64_t Db = T->Db;
-            for (uint32_t en = T->steps[s0].e_first; en < T->steps[s0].e_first + T->steps[s0].e_count; ++en) {
-                const SecEntry& E = T->entries[en];
-                const double2 cs = sd.cs[en];
-                const uint32_t lb = E.lb_len, total = E.la_len * lb;
-                for (uint32_t i = tid; i < total; i += THREADS) {
-                    uint32_t ia, ib;
-                    divmod_u(i, lb, E.inv_lb, ia, ib);
-                    const int2 pa = T->lists[E.la_off + ia];
-                    const int2 pb = T->lists[E.lb_off + ib];
-                    const uint64_t r1 = (uint64_t)pa.x * Db + (uint64_t)pb.x, r2 = (uint64_t)pa.y * Db + (uint64_t)pb.y;
-                    const uint64_t j1 = T->afull[pa.x] | T->bfull[pb.x];
-                    const double2 p1 = psi[r1], p2 = psi[r2], g1 = sig[r1], g2 = sig[r2];
-                    acc += pair_overlap(E, j1, p1, p2, g1, g2);
-                    pair_rotate(psi, r1, r2, p1, p2, j1, E.x, E.z0, cs.x, -cs.y, E.ulo, E.uhi);
-                    pair_rotate(sig, r1, r2, g1, g2, j1, E.x, E.z0, cs.x, -cs.y, E.ulo, E.uhi);
-                }
-            }
-            const double2 tot = block_sum(make_double2(acc, 0.0), red);  // its barriers order the writes above
-            if (tid == 0) sd.gacc[k] = tot.x;
-            continue;
-        }
-        for (uint32_t s = s0; s < s1; ++s)
-            for (uint32_t en = T->steps[s].e_first; en < T->steps[s].e_first + T->steps[s].e_count; ++en)
-                acc += entry_overlap<THREADS>(T, T->entries[en], sig, psi, tid);
-        const double2 tot = block_sum(make_double2(acc, 0.0), red);  // its barriers end every read above
-        if (tid == 0) sd.gacc[k] = tot.x;
-        if (k == 0) break;
-        for (uint32_t s = s1; s-- > s0;) {
-            const uint32_t e0 = T->steps[s].e_first, e1 = e0 + T->steps[s].e_count;
-            for (uint32_t en = e0; en < e1; ++en) {
-                const double2 cs = sd.cs[en];
-                rotate_entry<THREADS>(T, T->entries[en], cs.x, -cs.y, psi, T->afull, T->bfull, tid);
-                rotate_entry<THREADS>(T, T->entries[en], cs.x, -cs.y, sig, T->afull, T->bfull, tid);
-            }
-            __syncthreads();
-        }
-    }
-}
-
 // Pool gradients: 2 Re<H psi|A_k psi> for the operators of one batch, one
 // workgroup per operator (entries and lists of the pool's own tables).
 __global__ __launch_bounds__(256) void k_sec_pool(const SecTables* __restrict__ T, const SecEntry* __restrict__ pe,
@@ -702,11 +711,10 @@ __global__ __launch_bounds__(256) void k_sec_pool(const SecTables* __restrict__ 
     if (threadIdx.x == 0) out[blockIdx.x] = 2.0 * tot.x;
 }
 
-// ---- grid-wide single-request kernels (large sectors) ------------------------------------
-// A lone request of a large sector would run its ansatz and reverse sweep in
-// one workgroup.  These kernels spread one step (or one generator) over the
-// whole grid instead; the host launches one per step, in order, so kernel
-// boundaries order the steps.  Pair t of a step is taken in entry order.
+// ---- one launch per step (captured for the audit) -----------------------------------------
+// The evaluation as a chain of kernels, one step (or generator) each over the
+// whole grid: what qfe_template_graph_audit captures and checks node by node.
+// Pair t of a step is taken in entry order.
 constexpr int kWideTPB = 256;
 
 __device__ __forceinline__ bool step_pair(const SecTables* __restrict__ T, uint32_t e, uint32_t e_end, uint32_t t,
@@ -845,33 +853,13 @@ __global__ void k_sector_scatter(const double2* __restrict__ psi, uint64_t D, ui
     out[afull[r / Db] | bfull[r % Db]] = psi[r];
 }
 
-// Ansatz launch shapes by size tier: 0 = state in LDS, 256 threads; 1 = state
-// in LDS, 512 threads; 2 = state in device memory, 1024 threads.
+// Serving lanes by size tier: a sector state of up to 40 KiB with its string
+// tables, one that fits a workgroup's LDS, a larger one.
 constexpr size_t kTier0Lds = 40 << 10;
-constexpr int kTier2Threads = 1024;
+constexpr uint32_t kTableLds = 1024;
 
-int launch_ansatz(int tier, unsigned nblocks, size_t lds, hipStream_t st, const SlotDesc* d) {
-    if (tier == 0)
-        hipLaunchKernelGGL((k_sec_ansatz<true, 256, 4>), dim3(nblocks), dim3(256), lds, st, d);
-    else if (tier == 1)
-        hipLaunchKernelGGL((k_sec_ansatz<true, 512, 4>), dim3(nblocks), dim3(512), lds, st, d);
-    else
-        hipLaunchKernelGGL((k_sec_ansatz<false, kTier2Threads, 5>), dim3(nblocks), dim3(kTier2Threads), lds, st, d);
-    QFE_HIP(hipGetLastError());
-    return QFE_OK;
-}
-
-// Reverse sweep launch shape follows the ansatz tier (256 / 512 / 1024 threads).
-int launch_reverse(int tier, unsigned nblocks, hipStream_t st, const SlotDesc* d) {
-    if (tier == 0)
-        hipLaunchKernelGGL((k_sec_reverse<256>), dim3(nblocks), dim3(256), 0, st, d);
-    else if (tier == 1)
-        hipLaunchKernelGGL((k_sec_reverse<512>), dim3(nblocks), dim3(512), 0, st, d);
-    else
-        hipLaunchKernelGGL((k_sec_reverse<1024>), dim3(nblocks), dim3(1024), 0, st, d);
-    QFE_HIP(hipGetLastError());
-    return QFE_OK;
-}
+constexpr int kTileThreads = 64;
+constexpr uint64_t kTileAmps = 1024;  // amplitudes of a tile
 
 // ---- host-side construction -------------------------------------------------------------
 
@@ -1020,6 +1008,325 @@ int build_runs(const Space& sp, ListPool& lp, int norb, uint64_t lim, const qfe_
     return QFE_OK;
 }
 
+struct TileLaunch {  // host view of a pass: its grid and dynamic LDS
+    uint32_t tiles, lds;
+};
+
+// Union-find over the strings of one spin.
+struct Components {
+    std::vector<uint32_t> parent, size;
+    uint32_t largest = 1;
+    explicit Components(uint32_t n) : parent(n), size(n, 1) {
+        for (uint32_t i = 0; i < n; ++i) parent[i] = i;
+    }
+    uint32_t find(uint32_t v) {
+        while (parent[v] != v) v = parent[v] = parent[parent[v]];
+        return v;
+    }
+    void join(uint32_t a, uint32_t b) {
+        a = find(a);
+        b = find(b);
+        if (a == b) return;
+        if (size[a] < size[b]) std::swap(a, b);
+        parent[b] = a;
+        size[a] += size[b];
+        largest = std::max(largest, size[a]);
+    }
+};
+
+// Builds the component tiles of a template (see TileSeg).
+struct TileBuilder {
+    const Space& sp;
+    const ListPool& lp;
+    const std::vector<SecStep>& steps;
+    const std::vector<SecEntry>& entries;
+    std::vector<TileSeg> segs;
+    std::vector<TileRun> fwd, rev;
+    std::vector<TileLaunch> lfwd, lrev;
+    std::vector<TileRec> recs;
+    std::vector<uint32_t> tix, words;
+    std::vector<uint2> tab, sum;
+    std::vector<std::vector<uint2>> ranges;  // partial sums of the energy and of every generator
+    uint32_t parts = 0;
+    int norb;
+    size_t amp;  // bytes of an amplitude
+
+    TileBuilder(const Space& s, const ListPool& l, const std::vector<SecStep>& st, const std::vector<SecEntry>& en, size_t ngen,
+                int norb_, size_t amp_)
+        : sp(s), lp(l), steps(st), entries(en), ranges(ngen + 1), norb(norb_), amp(amp_) {}
+
+    void join_step(uint32_t s, Components& a, Components& b) const {
+        for (uint32_t e = steps[s].e_first; e < steps[s].e_first + steps[s].e_count; ++e) {
+            for (uint32_t i = 0; i < entries[e].la_len; ++i) {
+                const int2 v = lp.pool[entries[e].la_off + i];
+                a.join((uint32_t)v.x, (uint32_t)v.y);
+            }
+            for (uint32_t i = 0; i < entries[e].lb_len; ++i) {
+                const int2 v = lp.pool[entries[e].lb_off + i];
+                b.join((uint32_t)v.x, (uint32_t)v.y);
+            }
+        }
+    }
+
+    // Whole components into blocks of at most `most` strings, largest
+    // components first; ranks ascending within a block.
+    static std::vector<std::vector<uint32_t>> pack(Components& c, uint32_t most) {
+        const uint32_t n = (uint32_t)c.parent.size();
+        std::vector<std::vector<uint32_t>> comp(n), blocks;
+        for (uint32_t i = 0; i < n; ++i) comp[c.find(i)].push_back(i);
+        std::vector<uint32_t> order;
+        for (uint32_t i = 0; i < n; ++i)
+            if (!comp[i].empty()) order.push_back(i);
+        std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+            return comp[x].size() != comp[y].size() ? comp[x].size() > comp[y].size() : comp[x][0] < comp[y][0];
+        });
+        std::vector<size_t> open;  // blocks with room
+        for (uint32_t k : order) {
+            size_t at = blocks.size();
+            for (size_t i = 0; i < open.size(); ++i)
+                if (blocks[open[i]].size() + comp[k].size() <= most) {
+                    at = open[i];
+                    break;
+                }
+            if (at == blocks.size()) {
+                blocks.emplace_back();
+                open.push_back(at);
+                if (open.size() > 8) open.erase(open.begin());
+            }
+            blocks[at].insert(blocks[at].end(), comp[k].begin(), comp[k].end());
+        }
+        for (auto& b : blocks) std::sort(b.begin(), b.end());
+        return blocks;
+    }
+
+    // One spin of a segment: blocks, permuted ranks and list words.
+    struct Side {
+        uint32_t nblk = 0, blk = 0, perm = 0, wb = 0, tab = 0;
+        std::vector<uint32_t> len, nword;                     // strings and words of each block
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> id;  // (list offset, sign mask) -> list
+    };
+    Side build_side(int s, Components& c, uint32_t most, uint32_t s0, uint32_t s1) {
+        Side d;
+        const auto blocks = pack(c, most);
+        d.nblk = (uint32_t)blocks.size();
+        std::vector<uint32_t> where(c.parent.size()), local(c.parent.size());
+        d.blk = (uint32_t)tix.size();
+        uint32_t at = 0;
+        for (const auto& b : blocks) {
+            tix.push_back(at);
+            at += (uint32_t)b.size();
+            d.len.push_back((uint32_t)b.size());
+        }
+        tix.push_back(at);
+        d.perm = (uint32_t)tix.size();
+        for (uint32_t k = 0; k < d.nblk; ++k)
+            for (uint32_t i = 0; i < blocks[k].size(); ++i) {
+                tix.push_back(blocks[k][i]);
+                where[blocks[k][i]] = k;
+                local[blocks[k][i]] = i;
+            }
+        struct List {
+            uint32_t off, len, z;
+        };
+        std::vector<List> lists;
+        for (uint32_t e = steps_begin(s0); e < steps_begin(s1); ++e) {
+            const SecEntry& en = entries[e];
+            const uint32_t off = s ? en.lb_off : en.la_off, len = s ? en.lb_len : en.la_len;
+            const uint32_t z = compress(en.z0, s, norb);
+            if (d.id.emplace(std::make_pair(off, z), (uint32_t)lists.size()).second) lists.push_back({off, len, z});
+        }
+        std::vector<std::vector<uint32_t>> bw(d.nblk);
+        d.tab = (uint32_t)tab.size();
+        tab.resize(tab.size() + lists.size() * d.nblk, make_uint2(0, 0));
+        for (size_t l = 0; l < lists.size(); ++l) {
+            uint2* row = tab.data() + d.tab + l * d.nblk;
+            for (uint32_t k = 0; k < d.nblk; ++k) row[k].x = (uint32_t)bw[k].size();
+            for (uint32_t i = 0; i < lists[l].len; ++i) {
+                const int2 v = lp.pool[lists[l].off + i];
+                const uint32_t k = where[v.x];
+                const uint32_t p1 = popc32(sp.str[s][v.x] & lists[l].z) & 1, p2 = popc32(sp.str[s][v.y] & lists[l].z) & 1;
+                bw[k].push_back(local[v.x] | (local[v.y] << kWordBits) | (p1 << 30) | (p2 << 31));
+                ++row[k].y;
+            }
+        }
+        d.wb = (uint32_t)tix.size();
+        for (uint32_t k = 0; k < d.nblk; ++k) {
+            tix.push_back((uint32_t)words.size());
+            words.insert(words.end(), bw[k].begin(), bw[k].end());
+            d.nword.push_back((uint32_t)bw[k].size());
+        }
+        tix.push_back((uint32_t)words.size());
+        return d;
+    }
+    uint32_t steps_begin(uint32_t s) const { return s < steps.size() ? steps[s].e_first : (uint32_t)entries.size(); }
+
+    void add_run(std::vector<TileRun>& runs, std::vector<TileLaunch>& launches, const Side& a, const Side& b, uint32_t seg,
+                 uint32_t rec0, int states) {
+        TileRun r{seg, rec0, (uint32_t)recs.size() - rec0, parts};
+        uint32_t lds = 0;
+        const uint32_t chunk = std::min(r.nrec, kRecChunk) * (uint32_t)sizeof(LdsRec);
+        for (uint32_t i = 0; i < a.nblk; ++i)
+            for (uint32_t j = 0; j < b.nblk; ++j) {
+                const uint32_t w = a.nword[i] + b.nword[j];
+                const uint32_t amps = (uint32_t)(((size_t)a.len[i] * b.len[j] * states * amp + 15) & ~(size_t)15);
+                lds = std::max(lds, amps + chunk + (w <= kTileWordsLds ? 4 * w : 0u));
+            }
+        runs.push_back(r);
+        launches.push_back(TileLaunch{a.nblk * b.nblk, lds});
+    }
+
+    // Steps [s0, s1) as one segment.  gens: (first step, last step) of its
+    // generators, last generator first, for the reverse sweep.
+    void add_segment(uint32_t s0, uint32_t s1, Components& ca, Components& cb) {
+        uint32_t la = ca.largest, lb = cb.largest;
+        const uint32_t Da = (uint32_t)ca.parent.size(), Db = (uint32_t)cb.parent.size();
+        for (;;) {  // fill the tile: beta first, whose ranks are contiguous in memory
+            if (lb < Db && (uint64_t)la * lb * 2 <= kTileAmps)
+                lb = std::min(lb * 2, Db);
+            else if (la < Da && (uint64_t)la * lb * 2 <= kTileAmps)
+                la = std::min(la * 2, Da);
+            else
+                break;
+        }
+        side[0].push_back(build_side(0, ca, la, s0, s1));
+        side[1].push_back(build_side(1, cb, lb, s0, s1));
+        const Side &a = side[0].back(), &b = side[1].back();
+        segs.push_back(TileSeg{a.nblk, b.nblk, a.blk, b.blk, a.perm, b.perm, a.wb, b.wb, a.tab, b.tab});
+        seg_steps.push_back({s0, s1});
+        const uint32_t rec0 = (uint32_t)recs.size();
+        for (uint32_t s = s0; s < s1; ++s) add_step(segs.size() - 1, s, kRecRot);
+        add_run(fwd, lfwd, a, b, (uint32_t)segs.size() - 1, rec0, 1);
+    }
+    std::vector<Side> side[2];
+    std::vector<std::pair<uint32_t, uint32_t>> seg_steps;
+
+    void add_step(size_t seg, uint32_t s, uint32_t flags) {
+        for (uint32_t e = steps[s].e_first; e < steps[s].e_first + steps[s].e_count; ++e) {
+            const SecEntry& en = entries[e];
+            TileRec r{};
+            r.w = en.w;
+            r.ulo = en.ulo;
+            r.uhi = en.uhi;
+            r.entry = e;
+            r.alist = side[0][seg].id.at({en.la_off, compress(en.z0, 0, norb)});
+            r.blist = side[1][seg].id.at({en.lb_off, compress(en.z0, 1, norb)});
+            r.flags = flags | (e + 1 == steps[s].e_first + steps[s].e_count ? kRecStepEnd : 0u);
+            recs.push_back(r);
+        }
+    }
+
+    // One reverse-sweep pass over a segment: its records are recs[rec0..]; the
+    // outputs it completes are `outs` in order.
+    void add_reverse(uint32_t seg, uint32_t rec0, const std::vector<uint32_t>& outs) {
+        add_run(rev, lrev, side[0][seg], side[1][seg], seg, rec0, 2);
+        const uint32_t per = lrev.back().tiles * (kTileThreads / 64);
+        if (rev.size() == 1) {
+            ranges[0].push_back(make_uint2(parts, per));
+            parts += per;
+        }
+        for (uint32_t g : outs) {
+            ranges[g + 1].push_back(make_uint2(parts, per));
+            parts += per;
+        }
+    }
+
+    void build(const std::vector<uint32_t>& gen_step) {
+        const uint32_t ngen = (uint32_t)gen_step.size() - 1;
+        const uint32_t Da = (uint32_t)sp.str[0].size(), Db = (uint32_t)sp.str[1].size();
+        struct Part {  // generators [g0, g1) in one segment, or a generator too wide for one
+            uint32_t g0, g1, seg0, seg1;
+        };
+        std::vector<Part> plan;
+        // grow segments by generators (by steps inside a generator that is too wide)
+        auto grow = [&](uint32_t u0, uint32_t u1, auto first_step) {
+            uint32_t u = u0;
+            while (u < u1) {
+                Components ca(Da), cb(Db);
+                uint32_t v = u;
+                while (v < u1) {
+                    Components ta = ca, tb = cb;
+                    for (uint32_t s = first_step(v); s < first_step(v + 1); ++s) join_step(s, ta, tb);
+                    if (v > u && (uint64_t)ta.largest * tb.largest > kTileAmps) break;
+                    const bool wide = (uint64_t)ta.largest * tb.largest > kTileAmps;
+                    ca = std::move(ta);
+                    cb = std::move(tb);
+                    ++v;
+                    if (wide) break;
+                }
+                if ((uint64_t)ca.largest * cb.largest > kTileAmps) return std::make_pair(u, v);
+                add_segment(first_step(u), first_step(v), ca, cb);
+                u = v;
+                if (on_segment) on_segment(v);
+            }
+            return std::make_pair(u1, u1);
+        };
+        uint32_t g = 0;
+        while (g < ngen) {
+            uint32_t start = g;
+            on_segment = [&](uint32_t v) {
+                plan.push_back({start, v, (uint32_t)segs.size() - 1, (uint32_t)segs.size()});
+                start = v;
+            };
+            const auto stop = grow(g, ngen, [&](uint32_t k) { return gen_step[k]; });
+            on_segment = nullptr;
+            g = stop.first;
+            if (g >= ngen) break;
+            const uint32_t seg0 = (uint32_t)segs.size();  // generator g alone is too wide: segments of its steps
+            grow(gen_step[g], gen_step[g + 1], [](uint32_t k) { return k; });
+            plan.push_back({g, g + 1, seg0, (uint32_t)segs.size()});
+            ++g;
+        }
+        if (segs.empty()) {  // no generator: one pass still writes the reference and one adds up the energy
+            Components ca(Da), cb(Db);
+            add_segment((uint32_t)steps.size(), (uint32_t)steps.size(), ca, cb);
+            plan.push_back({0, 0, 0, 1});
+        }
+        for (size_t i = plan.size(); i-- > 0;) {
+            const Part& p = plan[i];
+            if (p.seg1 == p.seg0 + 1) {
+                const uint32_t rec0 = (uint32_t)recs.size();
+                std::vector<uint32_t> outs;
+                for (uint32_t k = p.g1; k-- > p.g0;) {
+                    const uint32_t s0 = gen_step[k], s1 = gen_step[k + 1];
+                    if (s0 == s1) continue;
+                    outs.push_back(k);
+                    if (s1 == s0 + 1) {  // one step: a pair's four old values give its overlap and both un-rotated pairs
+                        add_step(p.seg0, s0, kRecRot | kRecOv);
+                        recs.back().flags |= kRecGenEnd;
+                        continue;
+                    }
+                    const size_t first = recs.size();
+                    for (uint32_t s = s0; s < s1; ++s) add_step(p.seg0, s, kRecOv);
+                    for (size_t r = first; r < recs.size(); ++r) recs[r].flags &= ~kRecStepEnd;
+                    recs.back().flags |= kRecGenEnd | kRecStepEnd;
+                    for (uint32_t s = s1; s-- > s0;) add_step(p.seg0, s, kRecRot);
+                }
+                add_reverse(p.seg0, rec0, outs);
+                continue;
+            }
+            // a generator over several segments: its whole overlap before any un-rotation
+            for (uint32_t sgm = p.seg0; sgm < p.seg1; ++sgm) {
+                const uint32_t rec0 = (uint32_t)recs.size();
+                for (uint32_t s = seg_steps[sgm].first; s < seg_steps[sgm].second; ++s) add_step(sgm, s, kRecOv);
+                recs.back().flags |= kRecGenEnd;
+                add_reverse(sgm, rec0, {p.g0});
+            }
+            for (uint32_t sgm = p.seg1; sgm-- > p.seg0;) {
+                const uint32_t rec0 = (uint32_t)recs.size();
+                for (uint32_t s = seg_steps[sgm].second; s-- > seg_steps[sgm].first;) add_step(sgm, s, kRecRot);
+                add_reverse(sgm, rec0, {});
+            }
+        }
+        for (auto& r : ranges) {
+            sum_off.push_back((uint32_t)sum.size());
+            sum.insert(sum.end(), r.begin(), r.end());
+        }
+        sum_off.push_back((uint32_t)sum.size());
+    }
+    std::function<void(uint32_t)> on_segment;
+    std::vector<uint32_t> sum_off;
+};
+
 // Packs host arrays into one device allocation at 256-byte offsets.
 struct Packer {
     struct Piece {
@@ -1057,18 +1364,18 @@ struct qfe_template_s {
     bool has_map = false;
     uint64_t cost = 0;     // work estimate for ordering slots in a launch
     int tier = 2;          // ansatz launch shape
-    size_t lds_bytes = 0;  // dynamic LDS of the ansatz kernel
+    std::vector<TileLaunch> fwd, rev;  // tile passes of the ansatz and of the reverse sweep
     Space sp;              // host copy of the string space (pool operators)
     void* dev = nullptr;   // all tables
     SecTables* dt = nullptr;
     const uint64_t* afull = nullptr;
     const uint64_t* bfull = nullptr;
     // per-request device bytes: psi, coef, cs, part (energy); + sig, gacc (gradient)
-    size_t off_psi = 0, off_coef = 0, off_cs = 0, off_part = 0, off_sig = 0, off_gacc = 0;
+    size_t off_psi = 0, off_coef = 0, off_cs = 0, off_part = 0, off_sig = 0, off_gacc = 0, off_gpart = 0;
     size_t work_bytes = 0, grad_bytes = 0, io_count = 0, request_bytes = 0, grad_request_bytes = 0;
     void* arena = nullptr;  // single-request arena: [desc][out][io][prefix][work incl. gradient parts]
-    // grid-wide single-request path (large sectors): host step structure and
-    // device [segments (uint2 x (ngen + 1))][block partials]
+    // step-by-step sequence (large sectors): host step structure and device
+    // [segments (uint2 x (ngen + 1))][block partials]
     std::vector<uint32_t> h_gen_step, step_pairs;
     std::vector<uint2> wide_seg;  // (first partial, count): the energy, then generator k
     uint32_t wide_parts = 0;
@@ -1248,50 +1555,22 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     for (const auto& gr : groups) cost += (uint64_t)gr.la_len * gr.lb_len * (2 + gr.t_count);
     t->cost = cost;
 
-    {  // ansatz tier: the state in LDS when it fits a workgroup's share
+    {  // serving tier
         int dev = 0, max_lds = 0;
         (void)hipGetDevice(&dev);
         if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) max_lds = 65536;
         const size_t tab = ((uint64_t)t->Da + t->Db) <= kTableLds ? ((uint64_t)t->Da + t->Db) * 8 : 0;
         const size_t with_psi = t->D * sizeof(double2) + tab;
-        if (with_psi <= kTier0Lds) {
-            t->tier = 0;
-            t->lds_bytes = with_psi;
-        } else if (with_psi + 1024 <= (size_t)max_lds) {
-            t->tier = 1;
-            t->lds_bytes = with_psi;
-        } else {
-            t->tier = 2;
-            t->lds_bytes = tab;
-        }
+        t->tier = with_psi <= kTier0Lds ? 0 : (with_psi + 1024 <= (size_t)max_lds ? 1 : 2);
     }
 
     std::vector<uint64_t> af(t->Da), bf(t->Db);
     for (uint32_t a = 0; a < t->Da; ++a) af[a] = spread(sp.str[0][a], 0, norb);
     for (uint32_t b2 = 0; b2 < t->Db; ++b2) bf[b2] = spread(sp.str[1][b2], 1, norb);
-    // pair words of every entry, in entry order, when they fit the cap
-    std::vector<uint2> words;
-    {
-        uint64_t total = 0;
-        for (const auto& en : entries) total += (uint64_t)en.la_len * en.lb_len;
-        if (total <= ctx().tuning.sector_words) {
-            words.reserve(total);
-            for (auto& en : entries) {
-                en.w_off = (uint32_t)words.size();
-                for (uint32_t ia = 0; ia < en.la_len; ++ia) {
-                    const int2 pa = lp.pool[en.la_off + ia];
-                    for (uint32_t ib = 0; ib < en.lb_len; ++ib) {
-                        const int2 pb = lp.pool[en.lb_off + ib];
-                        const uint64_t j1 = af[pa.x] | bf[pb.x];
-                        const uint32_t r1 = (uint32_t)((uint64_t)pa.x * t->Db + pb.x);
-                        const uint32_t r2 = (uint32_t)((uint64_t)pa.y * t->Db + pb.y);
-                        const uint32_t g1 = popc64(j1 & en.z0) & 1, g2 = popc64((j1 ^ en.x) & en.z0) & 1;
-                        words.push_back(make_uint2(r1 | (g2 << 31), r2 | (g1 << 31)));
-                    }
-                }
-            }
-        }
-    }
+    TileBuilder tb(sp, lp, steps, entries, ngen, norb, sizeof(double2));
+    tb.build(gen_step);
+    t->fwd = tb.lfwd;
+    t->rev = tb.lrev;
     Packer pk(sizeof(SecTables));
     const size_t i_af = pk.add(af.data(), af.size() * 8), i_bf = pk.add(bf.data(), bf.size() * 8);
     const size_t i_as = pk.add(sp.str[0].data(), sp.str[0].size() * 4), i_bs = pk.add(sp.str[1].data(), sp.str[1].size() * 4);
@@ -1309,7 +1588,15 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     const size_t i_mi = pk.add(midx.data(), midx.size() * 4);
     const size_t i_mv = pk.add(mval.data(), mval.size() * sizeof(double2));
     const size_t i_hc = pk.add(hchunks.data(), hchunks.size() * sizeof(uint2));
-    const size_t i_w = pk.add(words.data(), words.size() * sizeof(uint2));
+    const size_t i_ts = pk.add(tb.segs.data(), tb.segs.size() * sizeof(TileSeg));
+    const size_t i_tf = pk.add(tb.fwd.data(), tb.fwd.size() * sizeof(TileRun));
+    const size_t i_tr = pk.add(tb.rev.data(), tb.rev.size() * sizeof(TileRun));
+    const size_t i_tc2 = pk.add(tb.recs.data(), tb.recs.size() * sizeof(TileRec));
+    const size_t i_tx = pk.add(tb.tix.data(), tb.tix.size() * 4);
+    const size_t i_tt = pk.add(tb.tab.data(), tb.tab.size() * sizeof(uint2));
+    const size_t i_tw = pk.add(tb.words.data(), tb.words.size() * 4);
+    const size_t i_tu = pk.add(tb.sum.data(), tb.sum.size() * sizeof(uint2));
+    const size_t i_to = pk.add(tb.sum_off.data(), tb.sum_off.size() * 4);
     QFE_HIP(hipMalloc(&t->dev, pk.total));
     char* base = (char*)t->dev;
     auto at = [&](size_t i) { return base + pk.pieces[i].off; };
@@ -1338,7 +1625,15 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     h.map_val = (const double2*)at(i_mv);
     h.hchunks = (const uint2*)at(i_hc);
     h.nhchunks = (uint32_t)hchunks.size();
-    h.words = entries.empty() || words.empty() ? nullptr : (const uint2*)at(i_w);
+    h.tsegs = (const TileSeg*)at(i_ts);
+    h.tfwd = (const TileRun*)at(i_tf);
+    h.trev = (const TileRun*)at(i_tr);
+    h.trec = (const TileRec*)at(i_tc2);
+    h.tix = (const uint32_t*)at(i_tx);
+    h.ttab = (const uint2*)at(i_tt);
+    h.twords = (const uint32_t*)at(i_tw);
+    h.tsum = (const uint2*)at(i_tu);
+    h.tsum_off = (const uint32_t*)at(i_to);
     h.nsteps = (uint32_t)steps.size();
     h.nentries = (uint32_t)entries.size();
     h.ngroups = (uint32_t)groups.size();
@@ -1368,6 +1663,8 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     o += align256(t->D * sizeof(double2));
     t->off_gacc = o;
     o += align256(ngen * 8 + 8);
+    t->off_gpart = o;
+    o += align256((size_t)tb.parts * 8 + 8);
     t->grad_bytes = o;
     t->io_count = nparam + ninputs;
     t->request_bytes = t->work_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + 16;
@@ -1399,19 +1696,61 @@ SlotDesc make_slot(qfe_template t, char* work, const double* io, double* out, bo
     d.part = (double*)(work + t->off_part);
     d.sig = grad ? (double2*)(work + t->off_sig) : nullptr;
     d.gacc = grad ? (double*)(work + t->off_gacc) : nullptr;
+    d.gpart = grad ? (double*)(work + t->off_gpart) : nullptr;
     d.params = io;
     d.inputs = io + t->nparam;
     d.out = out;
     return d;
 }
 
-// Energy of k requests of one tier: prologue, ansatz, items, sums.
-int launch_energy(const std::vector<qfe_template>& ts, int tier, size_t lds, const SlotDesc* ddesc, const uint32_t* dprefix,
+// The passes of one direction over k requests: launch q runs pass q of every
+// request that has one.  prefix: tile prefix of every launch (k + 1 entries
+// each, from pass_prefix); null for a single request.
+template <int MODE>
+int launch_tiles(const std::vector<qfe_template>& ts, const SlotDesc* d, const uint32_t* prefix, hipStream_t st) {
+    const uint32_t k = (uint32_t)ts.size();
+    size_t npass = 0;
+    for (const auto& t : ts) npass = std::max(npass, (MODE == 2 ? t->rev : t->fwd).size());
+    for (size_t i = 0; i < npass; ++i) {
+        const size_t q = MODE == 1 ? npass - 1 - i : i;
+        uint64_t tiles = 0;
+        uint32_t lds = 0;
+        for (const auto& t : ts) {
+            const auto& runs = MODE == 2 ? t->rev : t->fwd;
+            if (q >= runs.size()) continue;
+            tiles += runs[q].tiles;
+            lds = std::max(lds, runs[q].lds);
+        }
+        if (tiles >= (1ull << 31)) return fail(QFE_ERR_ARG, "qfe_template: too many tiles in one launch");
+        hipLaunchKernelGGL((k_sec_tile<double2, kTileThreads, MODE>), dim3((unsigned)tiles), dim3(kTileThreads), lds, st, d,
+                           prefix ? prefix + q * (k + 1) : nullptr, k, (uint32_t)q, (uint32_t)(MODE != 1 && q == 0));
+        QFE_HIP(hipGetLastError());
+    }
+    return QFE_OK;
+}
+
+// Tile prefixes of every pass of one direction over k requests.
+void pass_prefix(const std::vector<qfe_template>& ts, bool rev, std::vector<uint32_t>& out) {
+    size_t npass = 0;
+    for (const auto& t : ts) npass = std::max(npass, (rev ? t->rev : t->fwd).size());
+    for (size_t q = 0; q < npass; ++q) {
+        uint32_t at = 0;
+        for (const auto& t : ts) {
+            const auto& runs = rev ? t->rev : t->fwd;
+            out.push_back(at);
+            if (q < runs.size()) at += runs[q].tiles;
+        }
+        out.push_back(at);
+    }
+}
+
+// Energy of k requests: prologue, ansatz, items, sums.
+int launch_energy(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* dprefix, const uint32_t* tprefix,
                   uint32_t total_items, hipStream_t st) {
     const unsigned k = (unsigned)ts.size();
     hipLaunchKernelGGL(k_sec_prologue, dim3(k), dim3(256), 0, st, ddesc, 1);
     QFE_HIP(hipGetLastError());
-    int rc = launch_ansatz(tier, k, lds, st, ddesc);
+    int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
     if (rc) return rc;
     if (total_items) {
         hipLaunchKernelGGL(k_sec_energy, dim3(total_items), dim3(kItemThreads), 0, st, ddesc, dprefix, (uint32_t)k);
@@ -1422,22 +1761,37 @@ int launch_energy(const std::vector<qfe_template>& ts, int tier, size_t lds, con
     return QFE_OK;
 }
 
-// Energy and adjoint gradient of k requests of one tier: prologue, ansatz,
-// sigma = H psi (grid y = request), reverse sweep.
-int launch_gradient(const std::vector<qfe_template>& ts, int tier, size_t lds, const SlotDesc* ddesc, hipStream_t st) {
+// psi = U|ref> and sigma = H psi of k requests: prologue, ansatz, sigma (grid y = request).
+int launch_psi_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* tprefix, hipStream_t st) {
     const unsigned k = (unsigned)ts.size();
-    uint64_t chunks = 1;
-    for (const auto& t : ts) chunks = std::max<uint64_t>(chunks, (t->D + 1023) / 1024);
+    uint64_t D = 1;
+    for (const auto& t : ts) D = std::max(D, t->D);
     hipLaunchKernelGGL(k_sec_prologue, dim3(k), dim3(256), 0, st, ddesc, 1);
     QFE_HIP(hipGetLastError());
-    int rc = launch_ansatz(tier, k, lds, st, ddesc);
+    int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_sec_hpsi<4>, dim3((unsigned)chunks, k), dim3(256), 0, st, ddesc);
+    if (k == 1)
+        hipLaunchKernelGGL(k_sec_hpsi<1>, dim3((unsigned)((D + 255) / 256), k), dim3(256), 0, st, ddesc);
+    else
+        hipLaunchKernelGGL(k_sec_hpsi<4>, dim3((unsigned)((D + 1023) / 1024), k), dim3(256), 0, st, ddesc);
     QFE_HIP(hipGetLastError());
-    return launch_reverse(tier, k, st, ddesc);
+    return QFE_OK;
 }
 
-// ---- grid-wide single-request sequences (tier 2) -----------------------------------------
+// Energy and adjoint gradient of k requests; rprefix: tile prefixes of the reverse sweep.
+int launch_gradient(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* tprefix, const uint32_t* rprefix,
+                    hipStream_t st) {
+    int rc = launch_psi_sigma(ts, ddesc, tprefix, st);
+    if (!rc) rc = launch_tiles<2>(ts, ddesc, rprefix, st);
+    if (rc) return rc;
+    uint64_t ngen = 0;
+    for (const auto& t : ts) ngen = std::max(ngen, t->ngen);
+    hipLaunchKernelGGL(k_sec_tile_sum, dim3((unsigned)(ngen / 4 + 1), (unsigned)ts.size()), dim3(256), 0, st, ddesc);
+    QFE_HIP(hipGetLastError());
+    return QFE_OK;
+}
+
+// ---- step-by-step sequences (tier 2, captured for the audit) ------------------------------
 uint32_t wide_blocks(uint64_t items) { return (uint32_t)((items + kWideTPB - 1) / kWideTPB); }
 
 // U|ref>: the reference determinant, then one launch per step.
@@ -1560,24 +1914,13 @@ void gradient_from_overlaps(qfe_template t, const double* acc, double* grad) {
 // psi = U|ref> and sigma = H psi for one request (pool gradients).
 int single_psi_sigma(qfe_template t, const double* params, const double* inputs, Single& S) {
     int rc = single_setup(t, params, inputs, true, S);
-    if (rc) return rc;
-    hipStream_t st = ctx().stream;
-    if (t->tier == 2) return wide_psi_sigma(t, S.ddesc, st);
-    hipLaunchKernelGGL(k_sec_prologue, dim3(1), dim3(256), 0, st, S.ddesc, 1);
-    QFE_HIP(hipGetLastError());
-    rc = launch_ansatz(t->tier, 1, t->lds_bytes, st, S.ddesc);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_sec_hpsi<1>, dim3((unsigned)((t->D + 255) / 256), 1), dim3(256), 0, st, S.ddesc);
-    QFE_HIP(hipGetLastError());
-    return QFE_OK;
+    return rc ? rc : launch_psi_sigma({t}, S.ddesc, nullptr, ctx().stream);
 }
 
 // ---- captured single-request sequences (large sectors) ----------------------------------
-// The grid-wide sequences launch one kernel per step and per generator; as a
-// hipGraph per template they replay without per-launch host work.  The first
-// node uploads the whole request head (descriptor, prefix, amplitudes,
-// inputs) from the template's pinned block, so a replay does not depend on
-// what other calls left in the arena; the last nodes copy the energy (and the
+// The step-by-step sequence as one hipGraph per template.  The first node
+// uploads the whole request head (descriptor, prefix, amplitudes, inputs) from
+// the template's pinned block; the last nodes copy the energy (and the
 // generator overlaps) back into the same block.
 size_t single_head(qfe_template t) { return 768 + align256(t->io_count * 8 + 8); }
 
@@ -1818,25 +2161,6 @@ int graph_build(qfe_template t, int grad) {
     return QFE_OK;
 }
 
-// Replay: energy into *energy, and with grad the ngen generator overlaps into acc.
-int graph_run(qfe_template t, int grad, const double* params, const double* inputs, double* energy, double* acc) {
-    if (!t->gexec[grad]) {
-        int rc = graph_build(t, grad);
-        if (rc) return rc;
-    }
-    char* pin = (char*)t->gpin;
-    const size_t head = single_head(t);
-    // every call synchronizes before returning, so no replay is reading the block
-    if (t->nparam) std::memcpy(pin + 768, params, t->nparam * 8);
-    if (t->ninputs) std::memcpy(pin + 768 + t->nparam * 8, inputs, t->ninputs * 8);
-    hipStream_t st = ctx().stream;
-    QFE_HIP(hipGraphLaunch(t->gexec[grad], st));
-    QFE_HIP(hipStreamSynchronize(st));
-    std::memcpy(energy, pin + head, 8);
-    if (grad && t->ngen) std::memcpy(acc, pin + head + 8, t->ngen * 8);
-    return QFE_OK;
-}
-
 }  // namespace
 }  // namespace qfe
 
@@ -1981,14 +2305,13 @@ int lane_launch(qfe_batch b, Lane& L) {
     // heaviest requests first, so their workgroups start first
     std::stable_sort(take.begin(), take.end(), [](const Request& x, const Request& y) { return x.t->cost > y.t->cost; });
     const size_t k = take.size();
-    size_t io_total = 0, work_total = 0, lds = 0, gtotal = 0;
+    size_t io_total = 0, work_total = 0, gtotal = 0;
     uint64_t items = 0;
     std::vector<qfe_template> ts(k);
     for (size_t i = 0; i < k; ++i) {
         ts[i] = take[i].t;
         io_total += ts[i]->io_count;
         work_total += grad ? ts[i]->grad_bytes : ts[i]->work_bytes;
-        lds = std::max(lds, ts[i]->lds_bytes);
         items += ts[i]->nitems;
         if (grad) gtotal += ts[i]->ngen;
     }
@@ -1997,7 +2320,12 @@ int lane_launch(qfe_batch b, Lane& L) {
     const size_t nres = k + gtotal;
     const size_t o_out = align256(k * sizeof(SlotDesc));
     const size_t o_pre = o_out + align256(nres * 8);
-    const size_t o_io = o_pre + align256((k + 1) * 4);
+    std::vector<uint32_t> tpre;  // tile prefixes: the ansatz passes, then the reverse sweep's
+    pass_prefix(ts, false, tpre);
+    const size_t nfwd = tpre.size();
+    if (grad) pass_prefix(ts, true, tpre);
+    const size_t o_tpre = o_pre + align256((k + 1) * 4);
+    const size_t o_io = o_tpre + align256(tpre.size() * 4);
     const size_t head = o_io + align256(io_total * 8 + 8);
     const size_t need = head + work_total;
     int rc = grow_device<char>(L.dev, L.dev_cap, need);
@@ -2038,11 +2366,13 @@ int lane_launch(qfe_batch b, Lane& L) {
         L.ids.push_back(take[i].id);
     }
     hpre[k] = acc_items;
+    std::memcpy(up + o_tpre, tpre.data(), tpre.size() * 4);
+    const uint32_t* dtpre = (const uint32_t*)(dev + o_tpre);
     QFE_HIP(hipMemcpyAsync(dev, up, head, hipMemcpyHostToDevice, L.stream));
     if (grad)
-        rc = launch_gradient(ts, L.tier, lds, (const SlotDesc*)dev, L.stream);
+        rc = launch_gradient(ts, (const SlotDesc*)dev, dtpre, dtpre + nfwd, L.stream);
     else
-        rc = launch_energy(ts, L.tier, lds, (const SlotDesc*)dev, (const uint32_t*)(dev + o_pre), acc_items, L.stream);
+        rc = launch_energy(ts, (const SlotDesc*)dev, (const uint32_t*)(dev + o_pre), dtpre, acc_items, L.stream);
     if (rc) return rc;
     QFE_HIP(hipMemcpyAsync(L.out, dout, nres * 8, hipMemcpyDeviceToHost, L.stream));
     QFE_HIP(hipEventRecord(L.done, L.stream));
@@ -2188,11 +2518,10 @@ int qfe_template_graph_audit(qfe_template t, int gradient, uint64_t* out4) {
 int qfe_template_energy(qfe_template t, const double* params, const double* inputs, double* energy) {
     if (!t || !energy || (t->nparam && !params) || (t->ninputs && !inputs))
         return fail(QFE_ERR_ARG, "qfe_template_energy: null argument");
-    if (t->tier == 2) return graph_run(t, 0, params, inputs, energy, nullptr);
     Single S;
     int rc = single_setup(t, params, inputs, false, S);
     if (rc) return rc;
-    rc = launch_energy({t}, t->tier, t->lds_bytes, S.ddesc, S.dprefix, t->nitems, ctx().stream);
+    rc = launch_energy({t}, S.ddesc, S.dprefix, nullptr, t->nitems, ctx().stream);
     if (rc) return rc;
     return fetch_doubles(S.dout, 1, energy);
 }
@@ -2207,7 +2536,7 @@ int qfe_template_prepare(qfe_template t, const double* params, qfe_state out) {
     hipStream_t st = ctx().stream;
     hipLaunchKernelGGL(k_sec_prologue, dim3(1), dim3(256), 0, st, S.ddesc, 0);
     QFE_HIP(hipGetLastError());
-    rc = t->tier == 2 ? wide_ansatz(t, S.ddesc, st) : launch_ansatz(t->tier, 1, t->lds_bytes, st, S.ddesc);
+    rc = launch_tiles<0>({t}, S.ddesc, nullptr, st);
     if (!rc) rc = launch_zero(out->d, out->N, st);
     if (rc) return rc;
     hipLaunchKernelGGL(k_sector_scatter, dim3((unsigned)((t->D + 255) / 256)), dim3(256), 0, st,
@@ -2220,16 +2549,9 @@ int qfe_template_gradient(qfe_template t, const double* params, const double* in
     if (!t || !grad || (t->nparam && !params) || (t->ninputs && !inputs))
         return fail(QFE_ERR_ARG, "qfe_template_gradient: null argument");
     std::vector<double> acc(t->ngen + 1);
-    if (t->tier == 2) {
-        int rc = graph_run(t, 1, params, inputs, &acc[t->ngen], acc.data());
-        if (rc) return rc;
-        gradient_from_overlaps(t, acc.data(), grad);
-        if (energy) *energy = acc[t->ngen];
-        return QFE_OK;
-    }
     Single S;
     int rc = single_setup(t, params, inputs, true, S);
-    if (!rc) rc = launch_gradient({t}, t->tier, t->lds_bytes, S.ddesc, ctx().stream);
+    if (!rc) rc = launch_gradient({t}, S.ddesc, nullptr, nullptr, ctx().stream);
     if (rc) return rc;
     rc = fetch_doubles((const double*)(S.work + t->off_gacc), t->ngen, acc.data());
     if (!rc) rc = fetch_doubles(S.dout, 1, &acc[t->ngen]);
@@ -2251,17 +2573,13 @@ int qfe_template_residuals(qfe_template t, const double* params, const double* i
         if (ra < 0 || rb < 0) return fail(QFE_ERR_ARG, "qfe_template_residuals: basis index outside the sector");
         rank[i] = (uint64_t)ra * t->Db + (uint64_t)rb;
     }
-    // sigma = H U|ref>, then U^dag on sigma: every step inverted, last step
-    // first (psi is carried back to |ref> alongside)
+    // sigma = H U|ref>, then U^dag on sigma: every step inverted, last step first
     Single S;
     int rc = single_psi_sigma(t, params, inputs, S);
     if (rc) return rc;
     hipStream_t st = ctx().stream;
-    for (uint32_t sdx = (uint32_t)t->step_pairs.size(); sdx-- > 0;) {
-        if (!t->step_pairs[sdx]) continue;
-        hipLaunchKernelGGL(k_sec_step, dim3(wide_blocks(t->step_pairs[sdx])), dim3(kWideTPB), 0, st, S.ddesc, sdx, 1, 1);
-        QFE_HIP(hipGetLastError());
-    }
+    rc = launch_tiles<1>({t}, S.ddesc, nullptr, st);
+    if (rc) return rc;
     if (!count) return QFE_OK;
     void* scratch = nullptr;
     const size_t o_out = align256(count * 8);
