@@ -125,7 +125,7 @@ struct SecTables {  // device view of a template (lives in device memory)
     const uint32_t* gen_step;  // steps of generator k: [gen_step[k], gen_step[k+1])
     const uint64_t* tz;
     const double2* tph;    // phase of each term
-    const double2* tcoef;  // phase * coeff (fixed Hamiltonian)
+    const void* tcoef;     // phase * coeff (fixed Hamiltonian), in the template's scalar type
     const uint64_t* map_off;
     const uint32_t* map_idx;
     const double2* map_val;
@@ -144,9 +144,9 @@ struct SecTables {  // device view of a template (lives in device memory)
 
 struct SlotDesc {
     const SecTables* t;
-    double2* psi;
-    double2* sig;   // H psi (gradients only)
-    double2* coef;  // per-request coefficients (null: t->tcoef)
+    void* psi;      // amplitudes: double2, or double for a real template
+    void* sig;      // H psi (gradients only)
+    void* coef;     // per-request coefficients, same scalar type (null: t->tcoef)
     double2* cs;    // (cos, sin) per entry
     double* part;   // per work item energy partials
     double* gpart;  // reverse-sweep partial sums (gradients only)
@@ -191,7 +191,33 @@ __device__ __forceinline__ uint32_t find_slot(const uint32_t* __restrict__ prefi
     return lo;
 }
 
+// The scalar type S of a template: double when every generator and every
+// Hamiltonian coefficient is real (the state is then real throughout, as for
+// every UCC ansatz over real orbitals), else double2.  Real templates move
+// and multiply half as much; dropping exact zeros changes no bit of a result.
+__device__ __forceinline__ double2 umul(double2 u, double2 v) { return cmul(u, v); }
+__device__ __forceinline__ double umul(double2 u, double v) { return u.x * v; }
+__device__ __forceinline__ double2 lincomb(double c, double2 a, double s, double2 h) {
+    return make_double2(c * a.x + s * h.x, c * a.y + s * h.y);
+}
+__device__ __forceinline__ double lincomb(double c, double a, double s, double h) { return c * a + s * h; }
+__device__ __forceinline__ double re_dot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
+__device__ __forceinline__ double re_dot(double a, double b) { return a * b; }
+template <typename S>
+__device__ __forceinline__ S real_amp(double v);
+template <>
+__device__ __forceinline__ double2 real_amp<double2>(double v) {
+    return make_double2(v, 0.0);
+}
+template <>
+__device__ __forceinline__ double real_amp<double>(double v) {
+    return v;
+}
+__device__ __forceinline__ double2 to_complex(double2 v) { return v; }
+__device__ __forceinline__ double2 to_complex(double v) { return make_double2(v, 0.0); }
+
 // ---- 1. prologue: per-request Hamiltonian coefficients and rotation angles --------------
+template <typename S>
 __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict__ slots, int need_coef) {
     const SlotDesc sd = slots[blockIdx.x];
     const SecTables* __restrict__ T = sd.t;
@@ -205,7 +231,10 @@ __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict
                 cr += f.x * v;
                 ci += f.y * v;
             }
-            sd.coef[k] = cmul(T->tph[k], make_double2(cr, ci));
+            if constexpr (sizeof(S) == sizeof(double))
+                static_cast<double*>(sd.coef)[k] = T->tph[k].x * cr;
+            else
+                static_cast<double2*>(sd.coef)[k] = cmul(T->tph[k], make_double2(cr, ci));
         }
     }
     for (uint32_t e = threadIdx.x; e < T->nentries; e += blockDim.x) {
@@ -220,30 +249,26 @@ __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict
 // One pair (r1, r2) of an entry with old values (a, b), j1 the determinant
 // of r1: psi_1' = c a + s s(j2) uhi b, psi_2' = c b + s s(j1) ulo a.  Every
 // step-by-step kernel calls this; the tile passes apply the same formula.
-__device__ __forceinline__ void pair_rotate_signed(double2* __restrict__ psi, uint64_t r1, uint64_t r2, double2 a,
-                                                   double2 b, double c, double s1, double s2, double2 ulo, double2 uhi) {
-    const double2 hb = cmul(uhi, b), la = cmul(ulo, a);
-    psi[r1] = make_double2(c * a.x + s2 * hb.x, c * a.y + s2 * hb.y);
-    psi[r2] = make_double2(c * b.x + s1 * la.x, c * b.y + s1 * la.y);
-}
-__device__ __forceinline__ void pair_rotate(double2* __restrict__ psi, uint64_t r1, uint64_t r2, double2 a, double2 b,
-                                            uint64_t j1, uint64_t x, uint64_t z0, double c, double s, double2 ulo,
-                                            double2 uhi) {
-    pair_rotate_signed(psi, r1, r2, a, b, c, s * parity_sign(j1 & z0), s * parity_sign((j1 ^ x) & z0), ulo, uhi);
+template <typename S>
+__device__ __forceinline__ void pair_rotate(S* __restrict__ psi, uint64_t r1, uint64_t r2, S a, S b, uint64_t j1, uint64_t x,
+                                            uint64_t z0, double c, double s, double2 ulo, double2 uhi) {
+    const double s1 = s * parity_sign(j1 & z0), s2 = s * parity_sign((j1 ^ x) & z0);
+    psi[r1] = lincomb(c, a, s2, umul(uhi, b));
+    psi[r2] = lincomb(c, b, s1, umul(ulo, a));
 }
 
-// <sigma|K|psi> contribution of one pair (the entry_overlap formula), with
-// s1 = w (-1)^{|j1 & z0|} and s2 = w (-1)^{|(j1 ^ x) & z0|}.
-__device__ __forceinline__ double pair_overlap_signed(const SecEntry& en, double s1, double s2, double2 pa, double2 pb,
-                                                      double2 sa, double2 sb) {
-    const double2 k1 = cmul(en.uhi, pb), k2 = cmul(en.ulo, pa);
-    return s2 * (sa.x * k1.x + sa.y * k1.y) + s1 * (sb.x * k2.x + sb.y * k2.y);
+// <sigma|K|psi> contribution of one pair: (K psi)_1 = s(j2) w uhi psi_2,
+// (K psi)_2 = s(j1) w ulo psi_1.
+template <typename S>
+__device__ __forceinline__ double pair_overlap(const SecEntry& en, uint64_t j1, S pa, S pb, S sa, S sb) {
+    const double s1 = en.w * parity_sign(j1 & en.z0), s2 = en.w * parity_sign((j1 ^ en.x) & en.z0);
+    return s2 * re_dot(sa, umul(en.uhi, pb)) + s1 * re_dot(sb, umul(en.ulo, pa));
 }
-__device__ __forceinline__ double pair_overlap(const SecEntry& en, uint64_t j1, double2 pa, double2 pb, double2 sa,
-                                               double2 sb) {
-    return pair_overlap_signed(en, en.w * parity_sign(j1 & en.z0), en.w * parity_sign((j1 ^ en.x) & en.z0), pa, pb, sa,
-                               sb);
-}
+
+__device__ __forceinline__ double2 conj_mul(double2 a, double2 b) { return cconjmul(a, b); }
+__device__ __forceinline__ double conj_mul(double a, double b) { return a * b; }
+__device__ __forceinline__ double re_mul(double2 a, double2 b) { return a.x * b.x - a.y * b.y; }
+__device__ __forceinline__ double re_mul(double a, double b) { return a * b; }
 
 // v with its sign bit flipped when neg = 1u << 31: adding flip_sign(c, neg) is
 // bit-identical to fma(+-1.0, c, acc), with one integer op for the sign.
@@ -251,22 +276,19 @@ __device__ __forceinline__ double pair_overlap(const SecEntry& en, uint64_t j1, 
 __device__ __forceinline__ double flip_sign(double v, uint32_t neg) {
     return __hiloint2double(__double2hiint(v) ^ (int)neg, __double2loint(v));
 }
+__device__ __forceinline__ void add_flipped(double2& t, double2 c, uint32_t neg) {
+    t.x += flip_sign(c.x, neg);
+    t.y += flip_sign(c.y, neg);
+}
+__device__ __forceinline__ void add_flipped(double& t, double c, uint32_t neg) { t += flip_sign(c, neg); }
+// t += a b
+__device__ __forceinline__ void add_mul(double2& t, double2 a, double2 b) {
+    t.x += a.x * b.x - a.y * b.y;
+    t.y += a.x * b.y + a.y * b.x;
+}
+__device__ __forceinline__ void add_mul(double& t, double a, double b) { t += a * b; }
 
 // ---- 2. ansatz and reverse sweep: component tiles ---------------------------------------
-// A sector amplitude: double2, or double when every generator and every
-// Hamiltonian coefficient is real (then the state is real throughout).
-__device__ __forceinline__ double2 umul(double2 u, double2 v) { return cmul(u, v); }
-__device__ __forceinline__ double2 lincomb(double c, double2 a, double s, double2 h) {
-    return make_double2(c * a.x + s * h.x, c * a.y + s * h.y);
-}
-__device__ __forceinline__ double re_dot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
-template <typename S>
-__device__ __forceinline__ S real_amp(double v);
-template <>
-__device__ __forceinline__ double2 real_amp<double2>(double v) {
-    return make_double2(v, 0.0);
-}
-
 // v + the value CTRL lanes away (0 where there is none).
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
@@ -289,9 +311,60 @@ __device__ __forceinline__ double wave_sum_last(double v) {
 constexpr uint32_t kRecChunk = 128;        // records staged in LDS at a time
 constexpr uint32_t kTileWordsLds = 4096;   // list words of a tile staged in LDS when they fit
 
-struct LdsRec {  // a record as the tile's loop reads it
-    double c, s, w, ulo_x, ulo_y, uhi_x, uhi_y;
+// A record as the tile's loop reads it: which pairs, and the factors of their
+// rotation and overlap.
+struct RecHead {
     uint32_t a_off, b_off, b_len, pairs, magic, flags;
+    __device__ __forceinline__ RecHead uniform() const {  // every lane reads the same record
+        auto u = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+        return RecHead{u(a_off), u(b_off), u(b_len), u(pairs), u(magic), u(flags)};
+    }
+};
+template <typename S>
+struct RecFactors {
+    double c, s, w, ulo_x, ulo_y, uhi_x, uhi_y;
+    __device__ void set(double c_, double s_, double w_, double2 ulo, double2 uhi) {
+        c = c_;
+        s = s_;
+        w = w_;
+        ulo_x = ulo.x;
+        ulo_y = ulo.y;
+        uhi_x = uhi.x;
+        uhi_y = uhi.y;
+    }
+    // rotated pair from the old values; n1, n2: sign bits of the two directions
+    __device__ __forceinline__ void rotate(S a, S b, uint32_t n1, uint32_t n2, S& ra, S& rb) const {
+        ra = lincomb(c, a, flip_sign(s, n2), umul(make_double2(uhi_x, uhi_y), b));
+        rb = lincomb(c, b, flip_sign(s, n1), umul(make_double2(ulo_x, ulo_y), a));
+    }
+    __device__ __forceinline__ double overlap(S a, S b, S ya, S yb, uint32_t n1, uint32_t n2) const {
+        return flip_sign(w, n2) * re_dot(ya, umul(make_double2(uhi_x, uhi_y), b)) +
+               flip_sign(w, n1) * re_dot(yb, umul(make_double2(ulo_x, ulo_y), a));
+    }
+};
+// Real factors are +-1 and folded into sine and weight.
+template <>
+struct RecFactors<double> {
+    double c, slo, shi, wlo, whi;
+    __device__ void set(double c_, double s_, double w_, double2 ulo, double2 uhi) {
+        c = c_;
+        slo = s_ * ulo.x;
+        shi = s_ * uhi.x;
+        wlo = w_ * ulo.x;
+        whi = w_ * uhi.x;
+    }
+    __device__ __forceinline__ void rotate(double a, double b, uint32_t n1, uint32_t n2, double& ra, double& rb) const {
+        ra = lincomb(c, a, flip_sign(shi, n2), b);
+        rb = lincomb(c, b, flip_sign(slo, n1), a);
+    }
+    __device__ __forceinline__ double overlap(double a, double b, double ya, double yb, uint32_t n1, uint32_t n2) const {
+        return flip_sign(whi, n2) * (ya * b) + flip_sign(wlo, n1) * (yb * a);
+    }
+};
+template <typename S>
+struct LdsRec {
+    RecFactors<S> f;
+    RecHead head;
 };
 
 // i / d for i < 2^16, 0 < d < 2^16 by a multiplication: ceil(2^32 / d) (0 for d = 1).
@@ -329,7 +402,8 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
     const uint32_t nrec = run.nrec, nchunk = nrec < kRecChunk ? nrec : kRecChunk;
     S* X = reinterpret_cast<S*>(tile_lds);
     S* Y = X + (MODE == 2 ? n : 0u);
-    LdsRec* recs = reinterpret_cast<LdsRec*>(tile_lds + ((n * (MODE == 2 ? 2u : 1u) * sizeof(S) + 15) >> 4));
+    using Factors = RecFactors<S>;
+    LdsRec<S>* recs = reinterpret_cast<LdsRec<S>*>(tile_lds + ((n * (MODE == 2 ? 2u : 1u) * sizeof(S) + 15) >> 4));
     uint32_t* lw = reinterpret_cast<uint32_t*>(recs + nchunk);
     const bool wlds = naw + nbw <= kTileWordsLds;
     S* __restrict__ gx = reinterpret_cast<S*>(MODE == 1 ? sd.sig : sd.psi);
@@ -345,23 +419,17 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
             const TileRec tr = Tb->trec[at];
             const uint2 la = Tb->ttab[sg.atab + tr.alist * sg.nab + ab], lb = Tb->ttab[sg.btab + tr.blist * sg.nbb + bb];
             const double2 cs = sd.cs[tr.entry];
-            LdsRec o;
-            o.c = cs.x;
-            o.s = MODE == 0 ? cs.y : -cs.y;
-            o.w = tr.w;
-            o.ulo_x = tr.ulo.x;
-            o.ulo_y = tr.ulo.y;
-            o.uhi_x = tr.uhi.x;
-            o.uhi_y = tr.uhi.y;
-            o.a_off = la.x;
-            o.b_off = lb.x;
-            o.b_len = lb.y;
-            o.pairs = la.y * lb.y;
-            o.magic = div_magic(lb.y);
-            o.flags = tr.flags;
+            LdsRec<S> o;
+            o.f.set(cs.x, MODE == 0 ? cs.y : -cs.y, tr.w, tr.ulo, tr.uhi);
+            o.head.a_off = la.x;
+            o.head.b_off = lb.x;
+            o.head.b_len = lb.y;
+            o.head.pairs = la.y * lb.y;
+            o.head.magic = div_magic(lb.y);
+            o.head.flags = tr.flags;
             // last step first: a step ends before the record that ends the step before it
-            if (MODE == 1) o.flags = kRecRot | (at > run.rec0 ? Tb->trec[at - 1].flags & kRecStepEnd : 0u);
-            any |= o.pairs != 0;
+            if (MODE == 1) o.head.flags = kRecRot | (at > run.rec0 ? Tb->trec[at - 1].flags & kRecStepEnd : 0u);
+            any |= o.head.pairs != 0;
             recs[r] = o;
         }
         return any;
@@ -409,7 +477,7 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
     __syncthreads();
 
     double acc = 0.0;
-    auto words = [&](const LdsRec& R, uint32_t i, uint32_t& wa, uint32_t& wb) {
+    auto words = [&](const RecHead& R, uint32_t i, uint32_t& wa, uint32_t& wb) {
         const uint32_t ia = div_by(i, R.magic), ib = i - ia * R.b_len;
         if (wlds) {
             wa = lw[R.a_off + ia];
@@ -419,27 +487,28 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
             wb = Tb->twords[bw0 + R.b_off + ib];
         }
     };
-    auto pair = [&](const LdsRec& R, uint32_t wa, uint32_t wb) {
+    auto pair = [&](const Factors& F, uint32_t flags, uint32_t wa, uint32_t wb) {
         const uint32_t l1 = (wa & kWordPos) * nb + (wb & kWordPos);
         const uint32_t l2 = ((wa >> kWordBits) & kWordPos) * nb + ((wb >> kWordBits) & kWordPos);
         const uint32_t sw = wa ^ wb;  // bit 30: the parity on the string pair, bit 31: on its partner
         const uint32_t n1 = (sw << 1) & 0x80000000u, n2 = sw & 0x80000000u;
         const S a = X[l1], b = X[l2];
-        const double2 ulo = make_double2(R.ulo_x, R.ulo_y), uhi = make_double2(R.uhi_x, R.uhi_y);
+        S ra, rb;
         if (MODE == 2) {
             const S ya = Y[l1], yb = Y[l2];
-            if (R.flags & kRecOv)
-                acc += flip_sign(R.w, n2) * re_dot(ya, umul(uhi, b)) + flip_sign(R.w, n1) * re_dot(yb, umul(ulo, a));
-            if (R.flags & kRecRot) {
-                const double s1 = flip_sign(R.s, n1), s2 = flip_sign(R.s, n2);
-                X[l1] = lincomb(R.c, a, s2, umul(uhi, b));
-                X[l2] = lincomb(R.c, b, s1, umul(ulo, a));
-                Y[l1] = lincomb(R.c, ya, s2, umul(uhi, yb));
-                Y[l2] = lincomb(R.c, yb, s1, umul(ulo, ya));
+            if (flags & kRecOv) acc += F.overlap(a, b, ya, yb, n1, n2);
+            if (flags & kRecRot) {
+                F.rotate(a, b, n1, n2, ra, rb);
+                X[l1] = ra;
+                X[l2] = rb;
+                F.rotate(ya, yb, n1, n2, ra, rb);
+                Y[l1] = ra;
+                Y[l2] = rb;
             }
         } else {
-            X[l1] = lincomb(R.c, a, flip_sign(R.s, n2), umul(uhi, b));
-            X[l2] = lincomb(R.c, b, flip_sign(R.s, n1), umul(ulo, a));
+            F.rotate(a, b, n1, n2, ra, rb);
+            X[l1] = ra;
+            X[l2] = rb;
         }
     };
     for (uint32_t c0 = 0; c0 < nrec; c0 += kRecChunk) {
@@ -451,20 +520,20 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
         }
         // the record and first words of the next entry are read while the
         // current one is applied: they do not depend on its writes
-        LdsRec R = recs[0];
+        RecHead R = recs[0].head.uniform();
+        Factors F = recs[0].f;
         uint32_t wa = 0, wb = 0;
         if (tid < R.pairs) words(R, tid, wa, wb);
         for (uint32_t r = 0; r < cnt; ++r) {
-            LdsRec N = R;
+            const uint32_t nx = r + 1 < cnt ? r + 1 : r;
+            const RecHead N = recs[nx].head.uniform();
+            const Factors NF = recs[nx].f;
             uint32_t xa = 0, xb = 0;
-            if (r + 1 < cnt) {
-                N = recs[r + 1];
-                if (tid < N.pairs) words(N, tid, xa, xb);
-            }
-            if (tid < R.pairs) pair(R, wa, wb);
+            if (tid < N.pairs) words(N, tid, xa, xb);
+            if (tid < R.pairs) pair(F, R.flags, wa, wb);
             for (uint32_t i = tid + T; i < R.pairs; i += T) {
                 words(R, i, wa, wb);
-                pair(R, wa, wb);
+                pair(F, R.flags, wa, wb);
             }
             if (MODE == 2 && (R.flags & kRecGenEnd)) {
                 const double v = wave_sum_last(acc);
@@ -474,6 +543,7 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
             }
             if (R.flags & kRecStepEnd) __syncthreads();
             R = N;
+            F = NF;
             wa = xa;
             wb = xb;
         }
@@ -504,17 +574,18 @@ __global__ __launch_bounds__(256) void k_sec_tile_sum(const SlotDesc* __restrict
 }
 
 // ---- 3. energy work items: one workgroup per (request, item) ---------------------------
+template <typename S>
 __global__ __launch_bounds__(kItemThreads) void k_sec_energy(const SlotDesc* __restrict__ slots,
                                                              const uint32_t* __restrict__ prefix, uint32_t nslots) {
     __shared__ uint32_t tz_s[kTermLds];
-    __shared__ double2 c_s[kTermLds];
+    __shared__ S c_s[kTermLds];
     __shared__ double2 red[16];
     const uint32_t slot = find_slot(prefix, nslots, blockIdx.x);
     const SlotDesc sd = slots[slot];
     const SecTables* __restrict__ T = sd.t;
     const SecItem it = T->items[blockIdx.x - prefix[slot]];
-    const double2* __restrict__ coef = sd.coef ? sd.coef : T->tcoef;
-    const double2* __restrict__ psi = sd.psi;
+    const S* __restrict__ coef = static_cast<const S*>(sd.coef ? sd.coef : T->tcoef);
+    const S* __restrict__ psi = static_cast<const S*>(sd.psi);
     const uint32_t tid = threadIdx.x;
     const uint64_t Db = T->Db;
     const bool whole = it.g1 != it.g0 + 1;
@@ -537,36 +608,35 @@ __global__ __launch_bounds__(kItemThreads) void k_sec_energy(const SlotDesc* __r
         double gacc = 0.0;
         for (uint32_t i0 = p0 + tid; i0 < p1; i0 += kUnroll * kItemThreads) {
             uint32_t j2[kUnroll];
-            double2 v[kUnroll];
+            S v[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const uint32_t i = i0 + u * kItemThreads;
                 j2[u] = 0;
-                v[u] = make_double2(0.0, 0.0);
+                v[u] = real_amp<S>(0.0);
                 if (i < p1) {
                     uint32_t ia, ib;
                     divmod_u(i, lb, gr.inv_lb, ia, ib);
                     const int2 pa = T->lists[gr.la_off + ia];
                     const int2 pb = T->lists[gr.lb_off + ib];
                     j2[u] = (uint32_t)(T->afull[pa.x] | T->bfull[pb.x]) ^ x;
-                    v[u] = cconjmul(psi[(uint64_t)pa.x * Db + (uint64_t)pb.x], psi[(uint64_t)pa.y * Db + (uint64_t)pb.y]);
+                    v[u] = conj_mul(psi[(uint64_t)pa.x * Db + (uint64_t)pb.x], psi[(uint64_t)pa.y * Db + (uint64_t)pb.y]);
                 }
             }
-            double tr[kUnroll], ti[kUnroll];
+            S tr[kUnroll];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) tr[u] = ti[u] = 0.0;
+            for (int u = 0; u < kUnroll; ++u) tr[u] = real_amp<S>(0.0);
             for (uint32_t t = 0; t < nt; ++t) {
                 const uint32_t z = lds ? tz_s[t] : (uint32_t)T->tz[t0 + t];
-                const double2 c = lds ? c_s[t] : coef[t0 + t];
+                const S c = lds ? c_s[t] : coef[t0 + t];
 #pragma unroll
                 for (int u = 0; u < kUnroll; ++u) {
                     const uint32_t neg = (uint32_t)__popc(j2[u] & z) << 31;
-                    tr[u] += flip_sign(c.x, neg);
-                    ti[u] += flip_sign(c.y, neg);
+                    add_flipped(tr[u], c, neg);
                 }
             }
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) gacc += v[u].x * tr[u] - v[u].y * ti[u];
+            for (int u = 0; u < kUnroll; ++u) gacc += re_mul(v[u], tr[u]);
         }
         acc += gr.weight * gacc;
     }
@@ -593,21 +663,21 @@ constexpr uint32_t kHpsiTerms = 1024;  // terms staged per chunk (larger chunks 
 
 // PER determinants per thread: each staged term is read once for all of them
 // (batched launches use 4; a single request keeps 1 so it fills the chip).
-template <int PER>
+template <typename S, int PER>
 __global__ __launch_bounds__(256) void k_sec_hpsi(const SlotDesc* __restrict__ slots) {
     constexpr int kHpsiPer = PER;
     constexpr uint32_t kHpsiSpan = 256 * PER;  // determinants per block
     __shared__ uint4 hdr[kHpsiGroups];  // xa, xb, first term, term count
     __shared__ uint32_t gx[kHpsiGroups];
     __shared__ uint32_t tzs[kHpsiTerms];
-    __shared__ double2 cfs[kHpsiTerms];
+    __shared__ S cfs[kHpsiTerms];
     const SlotDesc sd = slots[blockIdx.y];
     const SecTables* __restrict__ T = sd.t;
     if ((uint64_t)blockIdx.x * kHpsiSpan >= T->D) return;  // the whole block: a smaller request of the launch
     uint32_t sa[kHpsiPer], sb[kHpsiPer];
     uint32_t j[kHpsiPer];
     bool live[kHpsiPer];
-    double sr[kHpsiPer], si[kHpsiPer];
+    S sr[kHpsiPer];
 #pragma unroll
     for (int q = 0; q < kHpsiPer; ++q) {
         const uint64_t r = (uint64_t)blockIdx.x * kHpsiSpan + (uint64_t)q * 256 + threadIdx.x;
@@ -616,9 +686,9 @@ __global__ __launch_bounds__(256) void k_sec_hpsi(const SlotDesc* __restrict__ s
         sa[q] = T->astr[ra];
         sb[q] = T->bstr[rb];
         j[q] = (uint32_t)(T->afull[ra] | T->bfull[rb]);
-        sr[q] = si[q] = 0.0;
+        sr[q] = real_amp<S>(0.0);
     }
-    const double2* __restrict__ coef = sd.coef ? sd.coef : T->tcoef;
+    const S* __restrict__ coef = static_cast<const S*>(sd.coef ? sd.coef : T->tcoef);
     for (uint32_t c = 0; c < T->nhchunks; ++c) {
         const uint2 ch = T->hchunks[c];
         const uint32_t t0 = T->groups[ch.x].t_first;
@@ -648,44 +718,42 @@ __global__ __launch_bounds__(256) void k_sec_hpsi(const SlotDesc* __restrict__ s
             }
             if (!any) continue;
             uint32_t j2[kHpsiPer];
-            double tr[kHpsiPer], ti[kHpsiPer];
+            S tr[kHpsiPer];
 #pragma unroll
             for (int q = 0; q < kHpsiPer; ++q) {
                 j2[q] = j[q] ^ gx[g];
-                tr[q] = ti[q] = 0.0;
+                tr[q] = real_amp<S>(0.0);
             }
             for (uint32_t t = h.z; t < h.z + h.w; ++t) {
                 const uint32_t z = tl ? tzs[t - t0] : (uint32_t)T->tz[t];
-                const double2 cf = tl ? cfs[t - t0] : coef[t];
+                const S cf = tl ? cfs[t - t0] : coef[t];
 #pragma unroll
                 for (int q = 0; q < kHpsiPer; ++q) {
                     const uint32_t neg = (uint32_t)__popc(j2[q] & z) << 31;
-                    tr[q] += flip_sign(cf.x, neg);
-                    ti[q] += flip_sign(cf.y, neg);
+                    add_flipped(tr[q], cf, neg);
                 }
             }
 #pragma unroll
             for (int q = 0; q < kHpsiPer; ++q) {
                 if (!on[q]) continue;
                 const uint64_t r2 = (uint64_t)T->arank[sa[q] ^ h.x] * T->Db + (uint64_t)T->brank[sb[q] ^ h.y];
-                const double2 p = sd.psi[r2];
-                sr[q] += tr[q] * p.x - ti[q] * p.y;
-                si[q] += tr[q] * p.y + ti[q] * p.x;
+                add_mul(sr[q], tr[q], static_cast<const S*>(sd.psi)[r2]);
             }
         }
     }
 #pragma unroll
     for (int q = 0; q < kHpsiPer; ++q) {
         const uint64_t r = (uint64_t)blockIdx.x * kHpsiSpan + (uint64_t)q * 256 + threadIdx.x;
-        if (live[q]) sd.sig[r] = make_double2(sr[q], si[q]);
+        if (live[q]) static_cast<S*>(sd.sig)[r] = sr[q];
     }
 }
 
 // Pool gradients: 2 Re<H psi|A_k psi> for the operators of one batch, one
 // workgroup per operator (entries and lists of the pool's own tables).
+template <typename S>
 __global__ __launch_bounds__(256) void k_sec_pool(const SecTables* __restrict__ T, const SecEntry* __restrict__ pe,
                                                   const int2* __restrict__ plists, const PoolOp* __restrict__ ops,
-                                                  const double2* __restrict__ sig, const double2* __restrict__ psi,
+                                                  const S* __restrict__ sig, const S* __restrict__ psi,
                                                   double* __restrict__ out) {
     __shared__ double2 red[16];
     const PoolOp op = ops[blockIdx.x];
@@ -701,10 +769,7 @@ __global__ __launch_bounds__(256) void k_sec_pool(const SecTables* __restrict__ 
             const int2 pb = plists[en.lb_off + ib];
             const uint64_t r1 = (uint64_t)pa.x * Db + (uint64_t)pb.x, r2 = (uint64_t)pa.y * Db + (uint64_t)pb.y;
             const uint64_t j1 = T->afull[pa.x] | T->bfull[pb.x];
-            const double s1 = en.w * parity_sign(j1 & en.z0), s2 = en.w * parity_sign((j1 ^ en.x) & en.z0);
-            const double2 k1 = cmul(en.uhi, psi[r2]), k2 = cmul(en.ulo, psi[r1]);
-            const double2 a = sig[r1], b = sig[r2];
-            acc += s2 * (a.x * k1.x + a.y * k1.y) + s1 * (b.x * k2.x + b.y * k2.y);
+            acc += pair_overlap(en, j1, psi[r1], psi[r2], sig[r1], sig[r2]);
         }
     }
     const double2 tot = block_sum(make_double2(acc, 0.0), red);
@@ -743,6 +808,7 @@ __device__ __forceinline__ void pair_of(const SecTables* __restrict__ T, const S
 }
 
 // Rotate the pairs of step `step` by (c, s) (inverse: (c, -s)); `both` also rotates sigma.
+template <typename S>
 __global__ __launch_bounds__(kWideTPB) void k_sec_step(const SlotDesc* __restrict__ slots, uint32_t step, int inverse,
                                                        int both) {
     const SlotDesc sd = slots[0];
@@ -755,14 +821,16 @@ __global__ __launch_bounds__(kWideTPB) void k_sec_step(const SlotDesc* __restric
     const double sn = inverse ? -cs.y : cs.y;
     uint64_t r1, r2, j1;
     pair_of(T, en, i, r1, r2, j1);
-    pair_rotate(sd.psi, r1, r2, sd.psi[r1], sd.psi[r2], j1, en.x, en.z0, cs.x, sn, en.ulo, en.uhi);
-    if (both) pair_rotate(sd.sig, r1, r2, sd.sig[r1], sd.sig[r2], j1, en.x, en.z0, cs.x, sn, en.ulo, en.uhi);
+    S *psi = static_cast<S*>(sd.psi), *sig = static_cast<S*>(sd.sig);
+    pair_rotate(psi, r1, r2, psi[r1], psi[r2], j1, en.x, en.z0, cs.x, sn, en.ulo, en.uhi);
+    if (both) pair_rotate(sig, r1, r2, sig[r1], sig[r2], j1, en.x, en.z0, cs.x, sn, en.ulo, en.uhi);
 }
 
 
 // Generator with one step: its overlap and its un-rotation of psi and sigma
 // read the same four old values of each pair, so one pass does both.
 // partial[blockIdx.x] receives the block's overlap sum.
+template <typename S>
 __global__ __launch_bounds__(kWideTPB) void k_sec_genrev(const SlotDesc* __restrict__ slots, uint32_t step,
                                                          double* __restrict__ partial) {
     __shared__ double2 red[16];
@@ -776,10 +844,11 @@ __global__ __launch_bounds__(kWideTPB) void k_sec_genrev(const SlotDesc* __restr
         const double2 cs = sd.cs[e];
         uint64_t r1, r2, j1;
         pair_of(T, en, i, r1, r2, j1);
-        const double2 pa = sd.psi[r1], pb = sd.psi[r2], sa = sd.sig[r1], sb = sd.sig[r2];
+        S *psi = static_cast<S*>(sd.psi), *sig = static_cast<S*>(sd.sig);
+        const S pa = psi[r1], pb = psi[r2], sa = sig[r1], sb = sig[r2];
         acc = pair_overlap(en, j1, pa, pb, sa, sb);
-        pair_rotate(sd.psi, r1, r2, pa, pb, j1, en.x, en.z0, cs.x, -cs.y, en.ulo, en.uhi);
-        pair_rotate(sd.sig, r1, r2, sa, sb, j1, en.x, en.z0, cs.x, -cs.y, en.ulo, en.uhi);
+        pair_rotate(psi, r1, r2, pa, pb, j1, en.x, en.z0, cs.x, -cs.y, en.ulo, en.uhi);
+        pair_rotate(sig, r1, r2, sa, sb, j1, en.x, en.z0, cs.x, -cs.y, en.ulo, en.uhi);
     }
     const double2 tot = block_sum(make_double2(acc, 0.0), red);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot.x;
@@ -787,6 +856,7 @@ __global__ __launch_bounds__(kWideTPB) void k_sec_genrev(const SlotDesc* __restr
 
 // Generator with several steps: the overlap over all of its entries first
 // (steps [s0, s1), their entries contiguous), un-rotation by k_sec_step after.
+template <typename S>
 __global__ __launch_bounds__(kWideTPB) void k_sec_genov(const SlotDesc* __restrict__ slots, uint32_t s0, uint32_t s1,
                                                         double* __restrict__ partial) {
     __shared__ double2 red[16];
@@ -799,20 +869,22 @@ __global__ __launch_bounds__(kWideTPB) void k_sec_genov(const SlotDesc* __restri
         const SecEntry& en = T->entries[e];
         uint64_t r1, r2, j1;
         pair_of(T, en, i, r1, r2, j1);
-        acc = pair_overlap(en, j1, sd.psi[r1], sd.psi[r2], sd.sig[r1], sd.sig[r2]);
+        const S *psi = static_cast<const S*>(sd.psi), *sig = static_cast<const S*>(sd.sig);
+        acc = pair_overlap(en, j1, psi[r1], psi[r2], sig[r1], sig[r2]);
     }
     const double2 tot = block_sum(make_double2(acc, 0.0), red);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot.x;
 }
 
 // Re<psi|sigma> block partials (the energy of the gradient path).
+template <typename S>
 __global__ __launch_bounds__(kWideTPB) void k_sec_edot(const SlotDesc* __restrict__ slots, double* __restrict__ partial) {
     __shared__ double2 red[16];
     const SlotDesc sd = slots[0];
     const uint64_t D = sd.t->D;
     const uint64_t r = (uint64_t)blockIdx.x * kWideTPB + threadIdx.x;
     double e = 0.0;
-    if (r < D) e = sd.psi[r].x * sd.sig[r].x + sd.psi[r].y * sd.sig[r].y;
+    if (r < D) e = re_dot(static_cast<const S*>(sd.psi)[r], static_cast<const S*>(sd.sig)[r]);
     const double2 tot = block_sum(make_double2(e, 0.0), red);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot.x;
 }
@@ -832,25 +904,28 @@ __global__ __launch_bounds__(kWideTPB) void k_sec_wsum(const SlotDesc* __restric
 }
 
 // The reference determinant (grid over the sector).
+template <typename S>
 __global__ __launch_bounds__(kWideTPB) void k_sec_ref(const SlotDesc* __restrict__ slots) {
     const SlotDesc sd = slots[0];
     const uint64_t r = (uint64_t)blockIdx.x * kWideTPB + threadIdx.x;
-    if (r < sd.t->D) sd.psi[r] = make_double2(r == sd.t->ref_rank ? 1.0 : 0.0, 0.0);
+    if (r < sd.t->D) static_cast<S*>(sd.psi)[r] = real_amp<S>(r == sd.t->ref_rank ? 1.0 : 0.0);
 }
 
 // out[i] = sigma[rank[i]] (PQE residual amplitudes).
+template <typename S>
 __global__ void k_sec_gather(const SlotDesc* __restrict__ slots, const uint64_t* __restrict__ rank, uint64_t count,
                              double2* __restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) out[i] = slots[0].sig[rank[i]];
+    if (i < count) out[i] = to_complex(static_cast<const S*>(slots[0].sig)[rank[i]]);
 }
 
 // Scatter a sector state into a zeroed full state.
-__global__ void k_sector_scatter(const double2* __restrict__ psi, uint64_t D, uint32_t Db, const uint64_t* __restrict__ afull,
+template <typename S>
+__global__ void k_sector_scatter(const S* __restrict__ psi, uint64_t D, uint32_t Db, const uint64_t* __restrict__ afull,
                                  const uint64_t* __restrict__ bfull, double2* __restrict__ out) {
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= D) return;
-    out[afull[r / Db] | bfull[r % Db]] = psi[r];
+    out[afull[r / Db] | bfull[r % Db]] = to_complex(psi[r]);
 }
 
 // Serving lanes by size tier: a sector state of up to 40 KiB with its string
@@ -858,7 +933,13 @@ __global__ void k_sector_scatter(const double2* __restrict__ psi, uint64_t D, ui
 constexpr size_t kTier0Lds = 40 << 10;
 constexpr uint32_t kTableLds = 1024;
 
-constexpr int kTileThreads = 64;
+// Tile shape.  Larger tiles take fewer passes but longer chains of steps per
+// workgroup.  20-qubit residuals / 16-qubit gradient / 512 mixed energies / 128
+// mixed gradients (us): 64 threads and 512 amplitudes 3709 / 1526 / 16480 /
+// 18470, 64 and 1024 3590 / 1538 / 15680 / 17870, 128 and 1024 3475 / 1458 /
+// 15560 / 17610, 128 and 2048 3510 / 1514 / 15390 / 17330, 128 and 4096 3975 /
+// 1762 / 15990 / 18090, 256 and 4096 3518 / 1542 / 15020 / 17020.
+constexpr int kTileThreads = 128;
 constexpr uint64_t kTileAmps = 1024;  // amplitudes of a tile
 
 // ---- host-side construction -------------------------------------------------------------
@@ -1049,11 +1130,11 @@ struct TileBuilder {
     std::vector<std::vector<uint2>> ranges;  // partial sums of the energy and of every generator
     uint32_t parts = 0;
     int norb;
-    size_t amp;  // bytes of an amplitude
+    bool real;  // amplitudes are doubles
 
     TileBuilder(const Space& s, const ListPool& l, const std::vector<SecStep>& st, const std::vector<SecEntry>& en, size_t ngen,
-                int norb_, size_t amp_)
-        : sp(s), lp(l), steps(st), entries(en), ranges(ngen + 1), norb(norb_), amp(amp_) {}
+                int norb_, bool real_)
+        : sp(s), lp(l), steps(st), entries(en), ranges(ngen + 1), norb(norb_), real(real_) {}
 
     void join_step(uint32_t s, Components& a, Components& b) const {
         for (uint32_t e = steps[s].e_first; e < steps[s].e_first + steps[s].e_count; ++e) {
@@ -1164,7 +1245,8 @@ struct TileBuilder {
                  uint32_t rec0, int states) {
         TileRun r{seg, rec0, (uint32_t)recs.size() - rec0, parts};
         uint32_t lds = 0;
-        const uint32_t chunk = std::min(r.nrec, kRecChunk) * (uint32_t)sizeof(LdsRec);
+        const size_t amp = real ? sizeof(double) : sizeof(double2);
+        const uint32_t chunk = std::min(r.nrec, kRecChunk) * (uint32_t)(real ? sizeof(LdsRec<double>) : sizeof(LdsRec<double2>));
         for (uint32_t i = 0; i < a.nblk; ++i)
             for (uint32_t j = 0; j < b.nblk; ++j) {
                 const uint32_t w = a.nword[i] + b.nword[j];
@@ -1362,6 +1444,8 @@ struct qfe_template_s {
     std::vector<double> gscale;
     uint32_t nterms = 0, nentries = 0, nitems = 0;
     bool has_map = false;
+    bool real = false;     // scalar type of the state and the coefficients (see umul)
+    size_t amp() const { return real ? sizeof(double) : sizeof(double2); }
     uint64_t cost = 0;     // work estimate for ordering slots in a launch
     int tier = 2;          // ansatz launch shape
     std::vector<TileLaunch> fwd, rev;  // tile passes of the ansatz and of the reverse sweep
@@ -1567,7 +1651,15 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     std::vector<uint64_t> af(t->Da), bf(t->Db);
     for (uint32_t a = 0; a < t->Da; ++a) af[a] = spread(sp.str[0][a], 0, norb);
     for (uint32_t b2 = 0; b2 < t->Db; ++b2) bf[b2] = spread(sp.str[1][b2], 1, norb);
-    TileBuilder tb(sp, lp, steps, entries, ngen, norb, sizeof(double2));
+    t->real = true;
+    for (const auto& en : entries) t->real = t->real && en.ulo.y == 0.0 && en.uhi.y == 0.0;
+    for (const auto& v : tph) t->real = t->real && (!t->has_map || v.y == 0.0);
+    for (const auto& v : mval) t->real = t->real && v.y == 0.0;
+    for (const auto& v : tcoef) t->real = t->real && (t->has_map || v.y == 0.0);
+    std::vector<double> tcoef_real;
+    if (t->real)
+        for (const auto& v : tcoef) tcoef_real.push_back(v.x);
+    TileBuilder tb(sp, lp, steps, entries, ngen, norb, t->real);
     tb.build(gen_step);
     t->fwd = tb.lfwd;
     t->rev = tb.lrev;
@@ -1583,7 +1675,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     const size_t i_gs = pk.add(gen_step.data(), gen_step.size() * 4);
     const size_t i_tz = pk.add(tz.data(), tz.size() * 8);
     const size_t i_tph = pk.add(tph.data(), tph.size() * sizeof(double2));
-    const size_t i_tc = pk.add(tcoef.data(), tcoef.size() * sizeof(double2));
+    const size_t i_tc = t->real ? pk.add(tcoef_real.data(), tcoef_real.size() * 8) : pk.add(tcoef.data(), tcoef.size() * sizeof(double2));
     const size_t i_mo = pk.add(moff.data(), moff.size() * 8);
     const size_t i_mi = pk.add(midx.data(), midx.size() * 4);
     const size_t i_mv = pk.add(mval.data(), mval.size() * sizeof(double2));
@@ -1619,7 +1711,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     h.gen_step = (const uint32_t*)at(i_gs);
     h.tz = (const uint64_t*)at(i_tz);
     h.tph = (const double2*)at(i_tph);
-    h.tcoef = (const double2*)at(i_tc);
+    h.tcoef = at(i_tc);
     h.map_off = t->has_map ? (const uint64_t*)at(i_mo) : nullptr;
     h.map_idx = (const uint32_t*)at(i_mi);
     h.map_val = (const double2*)at(i_mv);
@@ -1651,16 +1743,16 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     // per-request layout: energy parts first, gradient parts after
     size_t o = 0;
     t->off_psi = o;
-    o += align256(t->D * sizeof(double2));
+    o += align256(t->D * t->amp());
     t->off_coef = o;
-    if (t->has_map) o += align256((size_t)t->nterms * sizeof(double2));
+    if (t->has_map) o += align256((size_t)t->nterms * t->amp());
     t->off_cs = o;
     o += align256((size_t)t->nentries * sizeof(double2) + 16);
     t->off_part = o;
     o += align256((size_t)t->nitems * 8 + 8);
     t->work_bytes = o;
     t->off_sig = o;
-    o += align256(t->D * sizeof(double2));
+    o += align256(t->D * t->amp());
     t->off_gacc = o;
     o += align256(ngen * 8 + 8);
     t->off_gpart = o;
@@ -1690,11 +1782,11 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
 SlotDesc make_slot(qfe_template t, char* work, const double* io, double* out, bool grad) {
     SlotDesc d{};
     d.t = t->dt;
-    d.psi = (double2*)(work + t->off_psi);
-    d.coef = t->has_map ? (double2*)(work + t->off_coef) : nullptr;
+    d.psi = work + t->off_psi;
+    d.coef = t->has_map ? work + t->off_coef : nullptr;
     d.cs = (double2*)(work + t->off_cs);
     d.part = (double*)(work + t->off_part);
-    d.sig = grad ? (double2*)(work + t->off_sig) : nullptr;
+    d.sig = grad ? work + t->off_sig : nullptr;
     d.gacc = grad ? (double*)(work + t->off_gacc) : nullptr;
     d.gpart = grad ? (double*)(work + t->off_gpart) : nullptr;
     d.params = io;
@@ -1703,7 +1795,13 @@ SlotDesc make_slot(qfe_template t, char* work, const double* io, double* out, bo
     return d;
 }
 
-// The passes of one direction over k requests: launch q runs pass q of every
+// f(S{}) with the scalar type of a template.
+template <typename F>
+auto with_scalar(const qfe_template_s* t, F&& f) {
+    return t->real ? f(double{}) : f(double2{});
+}
+
+// The passes of one direction over k requests of one scalar type: launch q runs pass q of every
 // request that has one.  prefix: tile prefix of every launch (k + 1 entries
 // each, from pass_prefix); null for a single request.
 template <int MODE>
@@ -1722,8 +1820,10 @@ int launch_tiles(const std::vector<qfe_template>& ts, const SlotDesc* d, const u
             lds = std::max(lds, runs[q].lds);
         }
         if (tiles >= (1ull << 31)) return fail(QFE_ERR_ARG, "qfe_template: too many tiles in one launch");
-        hipLaunchKernelGGL((k_sec_tile<double2, kTileThreads, MODE>), dim3((unsigned)tiles), dim3(kTileThreads), lds, st, d,
-                           prefix ? prefix + q * (k + 1) : nullptr, k, (uint32_t)q, (uint32_t)(MODE != 1 && q == 0));
+        with_scalar(ts[0], [&](auto z) {
+            hipLaunchKernelGGL((k_sec_tile<decltype(z), kTileThreads, MODE>), dim3((unsigned)tiles), dim3(kTileThreads), lds, st,
+                               d, prefix ? prefix + q * (k + 1) : nullptr, k, (uint32_t)q, (uint32_t)(MODE != 1 && q == 0));
+        });
         QFE_HIP(hipGetLastError());
     }
     return QFE_OK;
@@ -1748,12 +1848,14 @@ void pass_prefix(const std::vector<qfe_template>& ts, bool rev, std::vector<uint
 int launch_energy(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* dprefix, const uint32_t* tprefix,
                   uint32_t total_items, hipStream_t st) {
     const unsigned k = (unsigned)ts.size();
-    hipLaunchKernelGGL(k_sec_prologue, dim3(k), dim3(256), 0, st, ddesc, 1);
+    with_scalar(ts[0], [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(k), dim3(256), 0, st, ddesc, 1); });
     QFE_HIP(hipGetLastError());
     int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
     if (rc) return rc;
     if (total_items) {
-        hipLaunchKernelGGL(k_sec_energy, dim3(total_items), dim3(kItemThreads), 0, st, ddesc, dprefix, (uint32_t)k);
+        with_scalar(ts[0], [&](auto z) {
+            hipLaunchKernelGGL(k_sec_energy<decltype(z)>, dim3(total_items), dim3(kItemThreads), 0, st, ddesc, dprefix, (uint32_t)k);
+        });
         QFE_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(k_sec_sum, dim3(k), dim3(256), 0, st, ddesc);
@@ -1766,14 +1868,17 @@ int launch_psi_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc,
     const unsigned k = (unsigned)ts.size();
     uint64_t D = 1;
     for (const auto& t : ts) D = std::max(D, t->D);
-    hipLaunchKernelGGL(k_sec_prologue, dim3(k), dim3(256), 0, st, ddesc, 1);
+    with_scalar(ts[0], [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(k), dim3(256), 0, st, ddesc, 1); });
     QFE_HIP(hipGetLastError());
     int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
     if (rc) return rc;
-    if (k == 1)
-        hipLaunchKernelGGL(k_sec_hpsi<1>, dim3((unsigned)((D + 255) / 256), k), dim3(256), 0, st, ddesc);
-    else
-        hipLaunchKernelGGL(k_sec_hpsi<4>, dim3((unsigned)((D + 1023) / 1024), k), dim3(256), 0, st, ddesc);
+    with_scalar(ts[0], [&](auto z) {
+        using S = decltype(z);
+        if (k == 1)
+            hipLaunchKernelGGL((k_sec_hpsi<S, 1>), dim3((unsigned)((D + 255) / 256), k), dim3(256), 0, st, ddesc);
+        else
+            hipLaunchKernelGGL((k_sec_hpsi<S, 4>), dim3((unsigned)((D + 1023) / 1024), k), dim3(256), 0, st, ddesc);
+    });
     QFE_HIP(hipGetLastError());
     return QFE_OK;
 }
@@ -1795,25 +1900,27 @@ int launch_gradient(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, 
 uint32_t wide_blocks(uint64_t items) { return (uint32_t)((items + kWideTPB - 1) / kWideTPB); }
 
 // U|ref>: the reference determinant, then one launch per step.
+template <typename S>
 int wide_ansatz(qfe_template t, const SlotDesc* d, hipStream_t st) {
-    hipLaunchKernelGGL(k_sec_ref, dim3(wide_blocks(t->D)), dim3(kWideTPB), 0, st, d);
+    hipLaunchKernelGGL(k_sec_ref<S>, dim3(wide_blocks(t->D)), dim3(kWideTPB), 0, st, d);
     QFE_HIP(hipGetLastError());
     for (uint32_t k = 0; k < (uint32_t)t->step_pairs.size(); ++k) {
         if (!t->step_pairs[k]) continue;
-        hipLaunchKernelGGL(k_sec_step, dim3(wide_blocks(t->step_pairs[k])), dim3(kWideTPB), 0, st, d, k, 0, 0);
+        hipLaunchKernelGGL(k_sec_step<S>, dim3(wide_blocks(t->step_pairs[k])), dim3(kWideTPB), 0, st, d, k, 0, 0);
         QFE_HIP(hipGetLastError());
     }
     return QFE_OK;
 }
 
 // Energy: prologue, ansatz, work items, sum (the items and sum kernels of the batched path).
+template <typename S>
 int wide_energy(qfe_template t, const SlotDesc* d, const uint32_t* dprefix, hipStream_t st) {
-    hipLaunchKernelGGL(k_sec_prologue, dim3(1), dim3(256), 0, st, d, 1);
+    hipLaunchKernelGGL(k_sec_prologue<S>, dim3(1), dim3(256), 0, st, d, 1);
     QFE_HIP(hipGetLastError());
-    int rc = wide_ansatz(t, d, st);
+    int rc = wide_ansatz<S>(t, d, st);
     if (rc) return rc;
     if (t->nitems) {
-        hipLaunchKernelGGL(k_sec_energy, dim3(t->nitems), dim3(kItemThreads), 0, st, d, dprefix, 1u);
+        hipLaunchKernelGGL(k_sec_energy<S>, dim3(t->nitems), dim3(kItemThreads), 0, st, d, dprefix, 1u);
         QFE_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(k_sec_sum, dim3(1), dim3(256), 0, st, d);
@@ -1822,39 +1929,41 @@ int wide_energy(qfe_template t, const SlotDesc* d, const uint32_t* dprefix, hipS
 }
 
 // psi and sigma = H psi (pool gradients and the gradient below).
+template <typename S>
 int wide_psi_sigma(qfe_template t, const SlotDesc* d, hipStream_t st) {
-    hipLaunchKernelGGL(k_sec_prologue, dim3(1), dim3(256), 0, st, d, 1);
+    hipLaunchKernelGGL(k_sec_prologue<S>, dim3(1), dim3(256), 0, st, d, 1);
     QFE_HIP(hipGetLastError());
-    int rc = wide_ansatz(t, d, st);
+    int rc = wide_ansatz<S>(t, d, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_sec_hpsi<1>, dim3((unsigned)((t->D + 255) / 256), 1), dim3(256), 0, st, d);
+    hipLaunchKernelGGL((k_sec_hpsi<S, 1>), dim3((unsigned)((t->D + 255) / 256), 1), dim3(256), 0, st, d);
     QFE_HIP(hipGetLastError());
     return QFE_OK;
 }
 
 // Energy and generator overlaps: E = Re<psi|sigma>, then for k = M-1 .. 0 the
 // overlap of generator k and its un-rotation on psi and sigma; fixed-order sums.
+template <typename S>
 int wide_gradient(qfe_template t, const SlotDesc* d, hipStream_t st) {
-    int rc = wide_psi_sigma(t, d, st);
+    int rc = wide_psi_sigma<S>(t, d, st);
     if (rc) return rc;
     const size_t seg_bytes = align256(t->wide_seg.size() * sizeof(uint2));
     double* part = (double*)((char*)t->wide + seg_bytes);
-    hipLaunchKernelGGL(k_sec_edot, dim3(t->wide_seg[0].y), dim3(kWideTPB), 0, st, d, part + t->wide_seg[0].x);
+    hipLaunchKernelGGL(k_sec_edot<S>, dim3(t->wide_seg[0].y), dim3(kWideTPB), 0, st, d, part + t->wide_seg[0].x);
     QFE_HIP(hipGetLastError());
     for (uint32_t k = (uint32_t)t->ngen; k-- > 0;) {
         const uint2 sg = t->wide_seg[k + 1];
         if (!sg.y) continue;
         const uint32_t s0 = t->h_gen_step[k], s1 = t->h_gen_step[k + 1];
         if (s1 == s0 + 1) {
-            hipLaunchKernelGGL(k_sec_genrev, dim3(sg.y), dim3(kWideTPB), 0, st, d, s0, part + sg.x);
+            hipLaunchKernelGGL(k_sec_genrev<S>, dim3(sg.y), dim3(kWideTPB), 0, st, d, s0, part + sg.x);
             QFE_HIP(hipGetLastError());
             continue;
         }
-        hipLaunchKernelGGL(k_sec_genov, dim3(sg.y), dim3(kWideTPB), 0, st, d, s0, s1, part + sg.x);
+        hipLaunchKernelGGL(k_sec_genov<S>, dim3(sg.y), dim3(kWideTPB), 0, st, d, s0, s1, part + sg.x);
         QFE_HIP(hipGetLastError());
         for (uint32_t sdx = s1; sdx-- > s0;) {
             if (!t->step_pairs[sdx]) continue;
-            hipLaunchKernelGGL(k_sec_step, dim3(wide_blocks(t->step_pairs[sdx])), dim3(kWideTPB), 0, st, d, sdx, 1, 1);
+            hipLaunchKernelGGL(k_sec_step<S>, dim3(wide_blocks(t->step_pairs[sdx])), dim3(kWideTPB), 0, st, d, sdx, 1, 1);
             QFE_HIP(hipGetLastError());
         }
     }
@@ -1968,6 +2077,7 @@ NodeExpect expect_copy(const void* dst, const void* src, size_t bytes) {
     return e;
 }
 
+template <typename S>
 void expected_nodes(qfe_template t, int grad, std::vector<NodeExpect>& out) {
     const size_t head = single_head(t);
     char* dev = (char*)t->arena;
@@ -1976,34 +2086,34 @@ void expected_nodes(qfe_template t, int grad, std::vector<NodeExpect>& out) {
     const auto KB = [](uint64_t items) { return (items + kWideTPB - 1) / kWideTPB; };
     out.clear();
     out.push_back(expect_copy(dev, pin, head));
-    out.push_back(expect_kernel((const void*)&k_sec_prologue, 1, 256, d, (int)1));
-    out.push_back(expect_kernel((const void*)&k_sec_ref, KB(t->D), kWideTPB, d));
+    out.push_back(expect_kernel((const void*)&k_sec_prologue<S>, 1, 256, d, (int)1));
+    out.push_back(expect_kernel((const void*)&k_sec_ref<S>, KB(t->D), kWideTPB, d));
     for (uint32_t k = 0; k < (uint32_t)t->step_pairs.size(); ++k)
         if (t->step_pairs[k])
-            out.push_back(expect_kernel((const void*)&k_sec_step, KB(t->step_pairs[k]), kWideTPB, d, k, (int)0, (int)0));
+            out.push_back(expect_kernel((const void*)&k_sec_step<S>, KB(t->step_pairs[k]), kWideTPB, d, k, (int)0, (int)0));
     if (!grad) {
         if (t->nitems)
-            out.push_back(expect_kernel((const void*)&k_sec_energy, t->nitems, kItemThreads, d,
+            out.push_back(expect_kernel((const void*)&k_sec_energy<S>, t->nitems, kItemThreads, d,
                                         (const uint32_t*)(dev + 512), (uint32_t)1));
         out.push_back(expect_kernel((const void*)&k_sec_sum, 1, 256, d));
         out.push_back(expect_copy(pin + head, dev + 256, 8));
         return;
     }
-    out.push_back(expect_kernel((const void*)&k_sec_hpsi<1>, (t->D + 255) / 256, 256, d));
+    out.push_back(expect_kernel((const void*)&k_sec_hpsi<S, 1>, (t->D + 255) / 256, 256, d));
     double* part = (double*)((char*)t->wide + align256(t->wide_seg.size() * sizeof(uint2)));
-    out.push_back(expect_kernel((const void*)&k_sec_edot, t->wide_seg[0].y, kWideTPB, d, part + t->wide_seg[0].x));
+    out.push_back(expect_kernel((const void*)&k_sec_edot<S>, t->wide_seg[0].y, kWideTPB, d, part + t->wide_seg[0].x));
     for (uint32_t k = (uint32_t)t->ngen; k-- > 0;) {
         const uint2 sg = t->wide_seg[k + 1];
         if (!sg.y) continue;
         const uint32_t s0 = t->h_gen_step[k], s1 = t->h_gen_step[k + 1];
         if (s1 == s0 + 1) {
-            out.push_back(expect_kernel((const void*)&k_sec_genrev, sg.y, kWideTPB, d, s0, part + sg.x));
+            out.push_back(expect_kernel((const void*)&k_sec_genrev<S>, sg.y, kWideTPB, d, s0, part + sg.x));
             continue;
         }
-        out.push_back(expect_kernel((const void*)&k_sec_genov, sg.y, kWideTPB, d, s0, s1, part + sg.x));
+        out.push_back(expect_kernel((const void*)&k_sec_genov<S>, sg.y, kWideTPB, d, s0, s1, part + sg.x));
         for (uint32_t sdx = s1; sdx-- > s0;)
             if (t->step_pairs[sdx])
-                out.push_back(expect_kernel((const void*)&k_sec_step, KB(t->step_pairs[sdx]), kWideTPB, d, sdx, (int)1, (int)1));
+                out.push_back(expect_kernel((const void*)&k_sec_step<S>, KB(t->step_pairs[sdx]), kWideTPB, d, sdx, (int)1, (int)1));
     }
     const uint32_t nseg = (uint32_t)t->wide_seg.size();
     out.push_back(expect_kernel((const void*)&k_sec_wsum, KB(nseg), kWideTPB, d, (const double*)part,
@@ -2031,14 +2141,14 @@ int audit_graph(qfe_template t, hipGraph_t g, int grad, GraphAudit& A) {
     std::memcpy(&d, t->gpin, sizeof(d));
     const char* work = dev + head;
     auto in_work = [&](const void* p, size_t bytes) { return p && inside(p, bytes, work, t->grad_bytes); };
-    if (d.t != t->dt || d.out != (double*)(dev + 256) || !in_work(d.psi, t->D * sizeof(double2)) ||
-        !in_work(d.sig, t->D * sizeof(double2)) || !in_work(d.cs, (size_t)t->nentries * sizeof(double2)) ||
+    if (d.t != t->dt || d.out != (double*)(dev + 256) || !in_work(d.psi, t->D * t->amp()) ||
+        !in_work(d.sig, t->D * t->amp()) || !in_work(d.cs, (size_t)t->nentries * sizeof(double2)) ||
         !in_work(d.part, (size_t)t->nitems * 8) || !in_work(d.gacc, t->ngen * 8) ||
-        (t->has_map && !in_work(d.coef, (size_t)t->nterms * sizeof(double2))) ||
+        (t->has_map && !in_work(d.coef, (size_t)t->nterms * t->amp())) ||
         !inside(d.params, t->io_count * 8, dev + 768, head - 768))
         return audit_fail(grad, 0, "descriptor pointer outside the arena");
     std::vector<NodeExpect> want;
-    expected_nodes(t, grad, want);
+    with_scalar(t, [&](auto z) { expected_nodes<decltype(z)>(t, grad, want); });
     size_t nroot = 0;
     QFE_HIP(hipGraphGetRootNodes(g, nullptr, &nroot));
     if (nroot != 1) return audit_fail(grad, 0, std::to_string(nroot) + " root nodes (expected one chain)");
@@ -2126,7 +2236,10 @@ int graph_build(qfe_template t, int grad) {
     QFE_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
     auto record = [&]() -> int {
         QFE_HIP(hipMemcpyAsync(dev, pin, head, hipMemcpyHostToDevice, st));
-        int r = grad ? wide_gradient(t, ddesc, st) : wide_energy(t, ddesc, (const uint32_t*)(dev + 512), st);
+        int r = with_scalar(t, [&](auto z) {
+            using S = decltype(z);
+            return grad ? wide_gradient<S>(t, ddesc, st) : wide_energy<S>(t, ddesc, (const uint32_t*)(dev + 512), st);
+        });
         if (r) return r;
         QFE_HIP(hipMemcpyAsync(pin + head, dout, 8, hipMemcpyDeviceToHost, st));
         if (grad && t->ngen)
@@ -2284,12 +2397,13 @@ int lane_launch(qfe_batch b, Lane& L) {
     const uint64_t share = std::min<uint64_t>(b->budget / kLanes, kLaunchFootprint);
     const bool one_dim = L.tier == 2;
     const uint64_t dim0 = queue.front().t->D;
+    const bool real0 = queue.front().t->real;  // a launch holds one scalar type
     std::vector<Request> take;
     std::vector<Request> skipped;
     uint64_t foot = 0;
     while (!queue.empty() && (int64_t)(b->active + take.size()) < b->max_active &&
            (!grad || take.size() < kMaxGradLaunch)) {
-        if (one_dim && queue.front().t->D != dim0) {
+        if ((one_dim && queue.front().t->D != dim0) || queue.front().t->real != real0) {
             skipped.push_back(std::move(queue.front()));
             queue.pop_front();
             continue;
@@ -2534,13 +2648,16 @@ int qfe_template_prepare(qfe_template t, const double* params, qfe_state out) {
     int rc = single_setup(t, params, zeros.data(), false, S);
     if (rc) return rc;
     hipStream_t st = ctx().stream;
-    hipLaunchKernelGGL(k_sec_prologue, dim3(1), dim3(256), 0, st, S.ddesc, 0);
+    with_scalar(t, [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(1), dim3(256), 0, st, S.ddesc, 0); });
     QFE_HIP(hipGetLastError());
     rc = launch_tiles<0>({t}, S.ddesc, nullptr, st);
     if (!rc) rc = launch_zero(out->d, out->N, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_sector_scatter, dim3((unsigned)((t->D + 255) / 256)), dim3(256), 0, st,
-                       (const double2*)(S.work + t->off_psi), t->D, t->Db, t->afull, t->bfull, out->d);
+    with_scalar(t, [&](auto z) {
+        using A = decltype(z);
+        hipLaunchKernelGGL(k_sector_scatter<A>, dim3((unsigned)((t->D + 255) / 256)), dim3(256), 0, st,
+                           (const A*)(S.work + t->off_psi), t->D, t->Db, t->afull, t->bfull, out->d);
+    });
     QFE_HIP(hipGetLastError());
     return QFE_OK;
 }
@@ -2587,8 +2704,10 @@ int qfe_template_residuals(qfe_template t, const double* params, const double* i
     if (rc) return rc;
     QFE_HIP(hipMemcpyAsync(scratch, rank.data(), count * 8, hipMemcpyHostToDevice, st));
     double2* dres = (double2*)((char*)scratch + o_out);
-    hipLaunchKernelGGL(k_sec_gather, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, S.ddesc,
-                       (const uint64_t*)scratch, count, dres);
+    with_scalar(t, [&](auto z) {
+        hipLaunchKernelGGL(k_sec_gather<decltype(z)>, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, S.ddesc,
+                           (const uint64_t*)scratch, count, dres);
+    });
     QFE_HIP(hipGetLastError());
     QFE_HIP(hipMemcpyAsync(out, dres, count * sizeof(double2), hipMemcpyDeviceToHost, st));
     QFE_HIP(hipStreamSynchronize(st));
@@ -2633,14 +2752,16 @@ int qfe_template_pool_gradients(qfe_template t, const double* params, const doub
         return hip_fail(e, "qfe_template_pool_gradients: upload");
     }
     char* base = (char*)dev;
-    const double2* psi = (const double2*)(S.work + t->off_psi);
-    const double2* sig = (const double2*)(S.work + t->off_sig);
     // batches of `batch` operators per launch
     for (uint64_t b0 = 0; b0 < nops; b0 += batch) {
         const uint64_t b1 = std::min(nops, b0 + batch);
-        hipLaunchKernelGGL(k_sec_pool, dim3((unsigned)(b1 - b0)), dim3(256), 0, ctx().stream, t->dt,
-                           (const SecEntry*)(base + pk.pieces[i_e].off), (const int2*)(base + pk.pieces[i_l].off),
-                           (const PoolOp*)(base + pk.pieces[i_o].off) + b0, sig, psi, (double*)(base + o_out) + b0);
+        with_scalar(t, [&](auto z) {
+            using A = decltype(z);
+            hipLaunchKernelGGL(k_sec_pool<A>, dim3((unsigned)(b1 - b0)), dim3(256), 0, ctx().stream, t->dt,
+                               (const SecEntry*)(base + pk.pieces[i_e].off), (const int2*)(base + pk.pieces[i_l].off),
+                               (const PoolOp*)(base + pk.pieces[i_o].off) + b0, (const A*)(S.work + t->off_sig),
+                               (const A*)(S.work + t->off_psi), (double*)(base + o_out) + b0);
+        });
         e = hipGetLastError();
         if (e != hipSuccess) break;
     }

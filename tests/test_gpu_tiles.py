@@ -77,3 +77,44 @@ def _sd(qf):
     pool.set_orb_spaces([1, 1, 1, 1, 0, 0, 0, 0])
     pool.fill_pool("SD")
     return pool
+
+
+def test_complex_generators_on_the_sector(qf):
+    """Imaginary hopping, i (a+_p a_q + a+_q a_p), makes the state complex:
+    the template keeps complex amplitudes, beside a real template in one
+    serving queue."""
+    n, ref = 8, [1, 1, 1, 1, 0, 0, 0, 0]
+    gens = []
+    for p, q in ((0, 4), (1, 5), (2, 6), (0, 2)):
+        string = " ".join(f"Z_{k}" for k in range(p + 1, q))
+        op = qf.QubitOperator()
+        op.add(0.5j, qf.build_circuit(f"X_{p} {string} X_{q}"))
+        op.add(0.5j, qf.build_circuit(f"Y_{p} {string} Y_{q}"))
+        gens.append(op)
+    hmap = qf.HamiltonianMap(4)
+    h, g = qf.synthetic_integrals(4, 12)
+    inputs = hmap.pack(0.2, h, g)
+    ridx = qf.ref_to_basis_idx(ref)
+    args = (n, ridx, gens, [0, 1, 2, 3], [1.0] * 4, 4)
+    prog = qf.UCCProgram(*args, hmap.operator(inputs))
+    tpl = qf.SectorTemplate(*args, hmap)
+    t = [0.3, -0.2, 0.4, 0.25]
+    e, gr = tpl.gradient(t, inputs)
+    e_p, gr_p = prog.gradient(t)
+    assert abs(e - e_p) < 1e-10 and abs(tpl.energy(t, inputs) - e_p) < 1e-10
+    assert np.max(np.abs(np.array(gr) - np.array(gr_p))) < 1e-10
+    a, b = qf.Computer(n), qf.Computer(n)
+    prog.prepare(t, a)
+    tpl.prepare(t, b)
+    amps = np.asarray(a.get_coeff_vec())
+    assert np.abs(amps.imag).max() > 1e-2
+    assert np.max(np.abs(amps - np.asarray(b.get_coeff_vec()))) < 1e-12
+    sel = [int(i) for i in np.argsort(-np.abs(amps))[:6]]
+    assert np.max(np.abs(np.asarray(tpl.residuals(t, sel, inputs)) - np.asarray(prog.residuals(t, sel)))) < 1e-11
+    real = qf.compile_ucc_template(n, ref, hmap, _sd(qf), list(range(26)))
+    eng = qf.ServingEngine(hbm_budget_bytes=1 << 30, max_active=64)
+    ids = [eng.submit(x, y, inputs, gradient=True) for x, y in ((tpl, t), (real, [0.05] * 26), (tpl, t), (real, [0.05] * 26))]
+    eng.drain()
+    assert abs(eng.results[ids[0]] - e) < 1e-12 and eng.results[ids[0]] == eng.results[ids[2]]
+    assert np.max(np.abs(np.array(eng.gradients[ids[2]]) - np.array(gr))) < 1e-12
+    assert abs(eng.results[ids[3]] - real.energy([0.05] * 26, inputs)) < 1e-12
