@@ -39,6 +39,7 @@
 #include <deque>
 #include <functional>
 #include <map>
+#include <set>
 #include <tuple>
 #include <unordered_map>
 #include <vector>
@@ -108,6 +109,61 @@ struct TileRun {  // one pass: the records [rec0, rec0 + nrec) over the tiles of
 // and the parities of the entry's sign mask on both.
 constexpr uint32_t kWordBits = 14, kWordPos = (1u << kWordBits) - 1u;
 
+// ---- Hamiltonian rows: one workgroup per alpha string ---------------------------------
+// H of a real template on one row of the sector (alpha string a, all beta
+// strings, one per lane).  With a fixed, every coefficient that depends on a
+// alone is one number for the whole row, and lists per string replace the scan
+// over X masks:
+//   alpha flips (and the diagonal): the terms of a flip merge by their beta Z
+//     mask into cells, T(b) = sum_cells C_cell (-1)^{b & mu}, times a
+//     coalesced row of psi;
+//   beta flips: per pattern of the flipped bits the terms merge by the
+//     remaining beta Z mask, times the row itself from LDS;
+//   alpha and beta flips together: one number G[alpha flip][beta flip] per
+//     pattern pair; rows of psi come through LDS four at a time, with every
+//     sign folded into the staged row, the staged numbers or the lane's word.
+// The merged numbers (M) are linear in the request's inputs and come from the
+// prologue.  A 20-qubit row has 625 + 2 x 126 connected determinants; the term
+// loops it replaces took 8 sign evaluations for each and tested all 2536 X
+// masks per determinant: sigma of a 20-qubit request 2318 -> 133 us, of a
+// 16-qubit one 2035 -> 64, energy items of an 8-qubit one 118 -> 15 (one
+// request alone; latency and LDS gathers bound it).  Groups that do not fit
+// this form (RowBuilder::fits) and complex templates stay with the term loops
+// below.
+struct RowFlip {  // an alpha flip of a row: partner rank and its cells
+    uint32_t partner, cell0, ncell, pos;
+};
+struct RowPair {  // an alpha flip of a row that goes with beta flips
+    uint32_t partner, fa, neg, pad;
+};
+struct RowTables {
+    const uint32_t* chunk_off;  // chunks of row a: [chunk_off[a], chunk_off[a + 1])
+    const uint4* chunks;        // (first flip, flips, first position, positions)
+    const RowFlip* flips;       // padded to whole groups of kRowUnroll per chunk
+    const uint32_t* pos_cell;   // cell of every position
+    const uint32_t* amu;        // beta mask of every alpha cell
+    const uint32_t* am;         // merged numbers of every alpha cell: [am[c], am[c + 1])
+    const uint32_t* bmu;        // the same for beta cells
+    const uint32_t* bm;
+    const uint32_t* mmask;      // alpha sign mask of every merged number
+    const uint32_t* b1;         // [k][Db] beta flips with one cell: partner | cell << 14 | sign << 31
+    const uint2* b2;            // [k][Db] others: (partner, first cell | cells << 20)
+    const uint32_t* pair_off;   // pair flips of row a, padded to whole groups of 4
+    const RowPair* pairs;
+    const uint32_t* words;      // [k][Db] beta flips of pairs: partner | flip << 14 | sign << 31
+    const uint32_t* fb_mask;    // alpha sign mask of every beta flip
+    const uint32_t* fa_mask;    // beta sign mask of every alpha flip
+    const double* m;            // merged numbers of a fixed Hamiltonian
+    const uint32_t *moff, *midx;  // or their inputs
+    const double* mval;
+    uint32_t nm, nbcell, nb1, nb2, nwords, nfb, gbase;
+};
+constexpr uint32_t kRowThreads = 256;
+constexpr uint32_t kRowNone = 0xffffffffu;
+constexpr uint32_t kRowCells = 512;   // alpha cells of a chunk
+constexpr uint32_t kRowUnroll = 8;    // rows of psi in flight
+constexpr uint32_t kRowCellBits = 17; // beta cells and flips per word
+
 struct SecTables {  // device view of a template (lives in device memory)
     uint64_t D, ref_rank;
     uint32_t Da, Db;
@@ -139,13 +195,17 @@ struct SecTables {  // device view of a template (lives in device memory)
     const uint32_t* twords;
     const uint2* tsum;     // ranges (first, count) of reverse-sweep partial sums
     const uint32_t* tsum_off;  // ranges of output k: [tsum_off[k], tsum_off[k + 1]); 0 the energy, k + 1 generator k
+    RowTables rows;
     uint32_t nsteps, nentries, ngroups, nterms, nitems, ngen, nhchunks;
+    uint32_t nparts;  // energy partials: the work items', then one per row workgroup
+    uint32_t nrows;   // row workgroups (0: every group is in the work items)
 };
 
 struct SlotDesc {
     const SecTables* t;
     void* psi;      // amplitudes: double2, or double for a real template
     void* sig;      // H psi (gradients only)
+    double* hm;     // per-request merged numbers of the rows (null: t->rows.m)
     void* coef;     // per-request coefficients, same scalar type (null: t->tcoef)
     double2* cs;    // (cos, sin) per entry
     double* part;   // per work item energy partials
@@ -217,12 +277,14 @@ __device__ __forceinline__ double2 to_complex(double2 v) { return v; }
 __device__ __forceinline__ double2 to_complex(double v) { return make_double2(v, 0.0); }
 
 // ---- 1. prologue: per-request Hamiltonian coefficients and rotation angles --------------
+// Grid (blocks, requests): a request's numbers are independent of each other.
 template <typename S>
 __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict__ slots, int need_coef) {
-    const SlotDesc sd = slots[blockIdx.x];
+    const SlotDesc sd = slots[blockIdx.y];
     const SecTables* __restrict__ T = sd.t;
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
     if (need_coef && sd.coef) {
-        for (uint32_t k = threadIdx.x; k < T->nterms; k += blockDim.x) {
+        for (uint32_t k = i0; k < T->nterms; k += step) {
             double cr = 0.0, ci = 0.0;
             const uint64_t e1 = T->map_off[k + 1];
             for (uint64_t e = T->map_off[k]; e < e1; ++e) {
@@ -237,7 +299,16 @@ __global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict
                 static_cast<double2*>(sd.coef)[k] = cmul(T->tph[k], make_double2(cr, ci));
         }
     }
-    for (uint32_t e = threadIdx.x; e < T->nentries; e += blockDim.x) {
+    if (need_coef && sd.hm) {
+        const RowTables& R = T->rows;
+        for (uint32_t k = i0; k < R.nm; k += step) {
+            double v = 0.0;
+            const uint32_t e1 = R.moff[k + 1];
+            for (uint32_t e = R.moff[k]; e < e1; ++e) v += R.mval[e] * sd.inputs[R.midx[e]];
+            sd.hm[k] = v;
+        }
+    }
+    for (uint32_t e = i0; e < T->nentries; e += step) {
         const SecEntry& en = T->entries[e];
         const SecStep& st = T->steps[en.step];
         double s, c;
@@ -573,7 +644,131 @@ __global__ __launch_bounds__(256) void k_sec_tile_sum(const SlotDesc* __restrict
     if (lane == kWave - 1) (k ? sd.gacc[k - 1] : *sd.out) = v;
 }
 
-// ---- 3. energy work items: one workgroup per (request, item) ---------------------------
+// ---- 3. Hamiltonian rows (see RowTables) -------------------------------------------------
+__device__ __forceinline__ uint32_t odd_sign(uint32_t v) { return (uint32_t)__popc(v) << 31; }
+
+// ENERGY: partial sums psi . (H psi) into part[]; else sigma = H psi.
+template <bool ENERGY>
+__global__ __launch_bounds__(kRowThreads) void k_sec_rows(const SlotDesc* __restrict__ slots,
+                                                          const uint32_t* __restrict__ prefix, uint32_t nslots) {
+    extern __shared__ double2 row_lds[];
+    __shared__ double2 red[16];
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    const uint32_t slot = nslots == 1 ? 0u : find_slot(prefix, nslots, blockIdx.x);
+    const uint32_t at = nslots == 1 ? blockIdx.x : blockIdx.x - prefix[slot];
+    const SlotDesc sd = slots[slot];
+    const SecTables* __restrict__ T = sd.t;
+    const RowTables& R = T->rows;
+    const uint32_t Db = T->Db, ncol = (Db + nt - 1) / nt;
+    const uint32_t ra = at / ncol, rb = (at - ra * ncol) * nt + tid;
+    const bool live = rb < Db;
+    const uint32_t rbs = live ? rb : 0u;
+    const double* __restrict__ psi = static_cast<const double*>(sd.psi);
+    const double* __restrict__ M = sd.hm ? sd.hm : R.m;
+    const uint32_t sa = T->astr[ra], sb = T->bstr[rbs];
+    // LDS: own row, beta cells, then alpha cells or the staged rows of a pair group
+    double* own = reinterpret_cast<double*>(row_lds);
+    double* cb = own + Db;
+    double* ca = cb + R.nbcell + 1;
+    uint32_t* cmu = reinterpret_cast<uint32_t*>(ca + kRowCells);
+    double* buf = reinterpret_cast<double*>(row_lds + ((Db + R.nbcell + 2) >> 1));
+    double* tab = buf + 4 * (size_t)Db;
+
+    for (uint32_t i = tid; i < Db; i += nt) own[i] = psi[(uint64_t)ra * Db + i];
+    auto merged = [&](uint32_t m0, uint32_t m1) {
+        double v = 0.0;
+        for (uint32_t m = m0; m < m1; ++m) v += flip_sign(M[m], odd_sign(sa & R.mmask[m]));
+        return v;
+    };
+    for (uint32_t c = tid; c < R.nbcell; c += nt) cb[c] = merged(R.bm[c], R.bm[c + 1]);
+    if (tid == 0) cb[R.nbcell] = 0.0;  // the cell of padding words
+    __syncthreads();
+    double acc = 0.0;
+
+    // beta flips
+    constexpr uint32_t kCell = (1u << kRowCellBits) - 1u;
+    for (uint32_t k = 0; k < R.nb1; k += kRowUnroll) {
+        uint32_t w[kRowUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kRowUnroll; ++u) w[u] = R.b1[(size_t)(k + u) * Db + rbs];
+#pragma unroll
+        for (uint32_t u = 0; u < kRowUnroll; ++u)
+            acc += flip_sign(cb[(w[u] >> 14) & kCell], w[u] & 0x80000000u) * own[w[u] & 0x3fffu];
+    }
+    if (R.nb2) {
+        uint2 w = R.b2[rbs];
+        for (uint32_t k = 1; k <= R.nb2; ++k) {
+            const uint2 next = R.b2[(size_t)(k < R.nb2 ? k : 0u) * Db + rbs];
+            const uint32_t c0 = w.y & 0xfffffu, n = w.y >> 20;
+            double t = 0.0;
+            for (uint32_t c = c0; c < c0 + n; ++c) t += flip_sign(cb[c], odd_sign(sb & R.bmu[c]));
+            acc += t * own[w.x];
+            w = next;
+        }
+    }
+
+    // alpha flips and the diagonal
+    for (uint32_t ch = R.chunk_off[ra]; ch < R.chunk_off[ra + 1]; ++ch) {
+        const uint4 cd = R.chunks[ch];
+        if (ch != R.chunk_off[ra]) __syncthreads();
+        for (uint32_t p = tid; p < cd.w; p += nt) {
+            const uint32_t c = R.pos_cell[cd.z + p];
+            ca[p] = merged(R.am[c], R.am[c + 1]);
+            cmu[p] = R.amu[c];
+        }
+        __syncthreads();
+        for (uint32_t f = 0; f < cd.y; f += kRowUnroll) {
+            double v[kRowUnroll];
+#pragma unroll
+            for (uint32_t u = 0; u < kRowUnroll; ++u) v[u] = psi[(uint64_t)R.flips[cd.x + f + u].partner * Db + rbs];
+#pragma unroll
+            for (uint32_t u = 0; u < kRowUnroll; ++u) {
+                const RowFlip fl = R.flips[cd.x + f + u];
+                double t = 0.0;
+                for (uint32_t p = fl.pos; p < fl.pos + fl.ncell; ++p) t += flip_sign(ca[p], odd_sign(sb & cmu[p]));
+                acc += t * v[u];
+            }
+        }
+    }
+
+    // alpha and beta flips together, four alpha flips at a time
+    for (uint32_t p0 = R.pair_off[ra]; p0 < R.pair_off[ra + 1]; p0 += 4) {
+        __syncthreads();
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const RowPair pr = R.pairs[p0 + q];
+            const bool on = pr.partner != kRowNone;
+            const uint32_t rm = on ? R.fa_mask[pr.fa] : 0u;
+            for (uint32_t i = tid; i < Db; i += nt)
+                buf[4 * i + q] = on ? flip_sign(psi[(uint64_t)pr.partner * Db + i], odd_sign(T->bstr[i] & rm)) : 0.0;
+            const double* __restrict__ g = M + R.gbase + (size_t)(on ? pr.fa : 0u) * R.nfb;
+            if (tid == 0) tab[4 * R.nfb + q] = 0.0;  // the flip of padding words
+            for (uint32_t i = tid; i < R.nfb; i += nt)
+                tab[4 * i + q] = on ? flip_sign(g[i], odd_sign(sa & R.fb_mask[i]) ^ pr.neg) : 0.0;
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < R.nwords; k += 4) {
+            uint32_t w[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) w[u] = R.words[(size_t)(k + u) * Db + rbs];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const double2* x = reinterpret_cast<const double2*>(buf + 4 * (w[u] & 0x3fffu));
+                const double2* g = reinterpret_cast<const double2*>(tab + 4 * ((w[u] >> 14) & kCell));
+                const double2 x0 = x[0], x1 = x[1], g0 = g[0], g1 = g[1];
+                acc += flip_sign((g0.x * x0.x + g0.y * x0.y) + (g1.x * x1.x + g1.y * x1.y), w[u] & 0x80000000u);
+            }
+        }
+    }
+    if (ENERGY) {
+        const double2 tot = block_sum(make_double2(live ? acc * own[rbs] : 0.0, 0.0), red);
+        if (tid == 0) sd.part[T->nitems + at] = tot.x;
+    } else if (live) {
+        static_cast<double*>(sd.sig)[(uint64_t)ra * Db + rb] = acc;
+    }
+}
+
+// ---- 4. energy work items: one workgroup per (request, item) ---------------------------
 template <typename S>
 __global__ __launch_bounds__(kItemThreads) void k_sec_energy(const SlotDesc* __restrict__ slots,
                                                              const uint32_t* __restrict__ prefix, uint32_t nslots) {
@@ -644,11 +839,11 @@ __global__ __launch_bounds__(kItemThreads) void k_sec_energy(const SlotDesc* __r
     if (tid == 0) sd.part[blockIdx.x - prefix[slot]] = tot.x;
 }
 
-// ---- 4. per-request sum of the item partials in a fixed order ---------------------------
+// ---- 5. per-request sum of the item partials in a fixed order ---------------------------
 __global__ __launch_bounds__(256) void k_sec_sum(const SlotDesc* __restrict__ slots) {
     __shared__ double2 red[16];
     const SlotDesc sd = slots[blockIdx.x];
-    const uint32_t n = sd.t->nitems;
+    const uint32_t n = sd.t->nparts;
     double acc = 0.0;
     for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) acc += sd.part[k];
     const double2 tot = block_sum(make_double2(acc, 0.0), red);
@@ -686,7 +881,7 @@ __global__ __launch_bounds__(256) void k_sec_hpsi(const SlotDesc* __restrict__ s
         sa[q] = T->astr[ra];
         sb[q] = T->bstr[rb];
         j[q] = (uint32_t)(T->afull[ra] | T->bfull[rb]);
-        sr[q] = real_amp<S>(0.0);
+        sr[q] = T->nrows && live[q] ? static_cast<const S*>(sd.sig)[r] : real_amp<S>(0.0);  // the rows' part
     }
     const S* __restrict__ coef = static_cast<const S*>(sd.coef ? sd.coef : T->tcoef);
     for (uint32_t c = 0; c < T->nhchunks; ++c) {
@@ -927,6 +1122,9 @@ __global__ void k_sector_scatter(const S* __restrict__ psi, uint64_t D, uint32_t
     if (r >= D) return;
     out[afull[r / Db] | bfull[r % Db]] = to_complex(psi[r]);
 }
+
+constexpr size_t kRowLdsMax = 64 << 10;   // dynamic LDS of a row workgroup
+constexpr uint64_t kRowLists = 1ull << 22;  // flips over all rows of a template
 
 // Serving lanes by size tier: a sector state of up to 40 KiB with its string
 // tables, one that fits a workgroup's LDS, a larger one.
@@ -1409,6 +1607,214 @@ struct TileBuilder {
     std::vector<uint32_t> sum_off;
 };
 
+// Builds the row tables of a real template (see k_sec_rows).
+struct RowBuilder {
+    const Space& sp;
+    int norb;
+    std::vector<uint32_t> chunk_off{0}, pos_cell, amu, am{0}, bmu, bm{0}, mmask, b1, pair_off{0}, words, fb_mask, fa_mask;
+    std::vector<uint4> chunks;
+    std::vector<uint2> b2;
+    std::vector<RowFlip> flips;
+    std::vector<RowPair> pairs;
+    std::vector<std::vector<std::pair<uint32_t, double>>> mrow;  // terms of every merged number
+    uint32_t nb1 = 0, nb2 = 0, nwords = 0, nfa = 0, nfb = 0, gbase = 0;
+
+    struct Term {
+        uint32_t za, zb, k;
+    };
+    struct Group {
+        uint64_t x;
+        uint32_t xa, xb;
+        std::vector<Term> terms;
+    };
+    explicit RowBuilder(const Space& s, int norb_) : sp(s), norb(norb_) {}
+
+    static uint32_t parity(uint32_t v) { return (uint32_t)__builtin_popcount(v) & 1u; }
+    // Qubits strictly between the first and second, third and fourth ... set bits of x.
+    static uint64_t between(uint64_t x) {
+        uint64_t r = 0;
+        while (x) {
+            const int lo = __builtin_ctzll(x);
+            x &= x - 1;
+            if (!x) break;
+            const int hi = __builtin_ctzll(x);
+            x &= x - 1;
+            r |= ((1ull << hi) - 1ull) & ~((2ull << lo) - 1ull);
+        }
+        return r;
+    }
+    // Whether a group has the form the rows take: flips of one spin (or none)
+    // always; flips of both spins when all its terms share the sign mask
+    // outside x and it is the product of the two flips' Jordan-Wigner strings.
+    bool fits(const Group& g) const {
+        if (!g.xa && !g.xb) return cells_of(g) <= kRowCells;
+        if (!g.xa || !g.xb) return popc32(g.xa | g.xb) <= 8 && g.terms.size() <= 256;
+        if (popc32(g.xa) > 4 || popc32(g.xb) > 4) return false;
+        const uint64_t j = (between(spread(g.xa, 0, norb)) ^ between(spread(g.xb, 1, norb))) & ~g.x;
+        const uint32_t ja = compress(j, 0, norb), jb = compress(j, 1, norb);
+        for (const Term& t : g.terms)
+            if ((t.za & ~g.xa) != ja || (t.zb & ~g.xb) != jb) return false;
+        return true;
+    }
+    static size_t cells_of(const Group& g) {
+        std::map<uint32_t, int> m;
+        for (const Term& t : g.terms) m[t.zb] = 1;
+        return m.size();
+    }
+    static std::vector<uint32_t> patterns(uint32_t x) {  // half of the bits of x set
+        std::vector<uint32_t> out;
+        for (uint32_t p = x;; p = (p - 1) & x) {
+            if (2 * popc32(p) == popc32(x)) out.push_back(p);
+            if (!p) break;
+        }
+        std::sort(out.begin(), out.end());
+        return out;
+    }
+    // Cells of a group with the flipped bits of spin s in pattern p: terms
+    // merged by the beta mask, then by the alpha mask.  Returns (first cell, cells).
+    std::pair<uint32_t, uint32_t> add_cells(const Group& g, int s, uint32_t p, std::vector<uint32_t>& mu, std::vector<uint32_t>& m) {
+        std::map<uint32_t, std::map<uint32_t, std::vector<std::pair<uint32_t, double>>>> cell;
+        for (const Term& t : g.terms) {
+            const double sg = parity(p & (s ? t.zb : t.za)) ? -1.0 : 1.0;
+            cell[s ? t.zb & ~g.xb : t.zb][s ? t.za : t.za & ~g.xa].push_back({t.k, sg});
+        }
+        const uint32_t c0 = (uint32_t)mu.size();
+        for (auto& c : cell) {
+            mu.push_back(c.first);
+            for (auto& v : c.second) {
+                mmask.push_back(v.first);
+                mrow.push_back(std::move(v.second));
+            }
+            m.push_back((uint32_t)mrow.size());
+        }
+        return {c0, (uint32_t)mu.size() - c0};
+    }
+
+    // LDS of a row workgroup.
+    size_t lds() const {
+        const size_t Db = sp.str[1].size(), nb = bmu.size();
+        const size_t a = kRowCells * 12 + 16, ab = nwords ? 32 * (Db + nfb + 1) : 0;
+        return ((Db + nb + 2) / 2) * 16 + std::max(a, ab);
+    }
+
+    void build(const std::vector<Group>& groups) {
+        const auto &as = sp.str[0], &bs = sp.str[1];
+        const uint32_t Da = (uint32_t)as.size(), Db = (uint32_t)bs.size();
+        auto rank = [&](int s, uint32_t v) { return (uint32_t)sp.rank[s][v]; };
+        auto flips_in = [&](uint32_t v, uint32_t x) { return 2 * popc32(v & x) == popc32(x); };
+        // alpha flips: cells per pattern of the partner's flipped bits
+        std::map<std::pair<size_t, uint32_t>, std::pair<uint32_t, uint32_t>> acells, bcells;
+        for (size_t i = 0; i < groups.size(); ++i) {
+            if (groups[i].xb) continue;
+            for (uint32_t p : patterns(groups[i].xa)) acells[{i, p}] = add_cells(groups[i], 0, p, amu, am);
+        }
+        for (uint32_t ra = 0; ra < Da; ++ra) {
+            uint4 cd = make_uint4((uint32_t)flips.size(), 0, (uint32_t)pos_cell.size(), 0);
+            auto close = [&]() {
+                if (flips.size() == cd.x) return;
+                while ((flips.size() - cd.x) % kRowUnroll) flips.push_back(RowFlip{ra, 0, 0, 0});
+                cd.y = (uint32_t)flips.size() - cd.x;
+                chunks.push_back(cd);
+                cd = make_uint4((uint32_t)flips.size(), 0, (uint32_t)pos_cell.size(), 0);
+            };
+            for (size_t i = 0; i < groups.size(); ++i) {
+                if (groups[i].xb || !flips_in(as[ra], groups[i].xa)) continue;
+                const uint32_t to = as[ra] ^ groups[i].xa;
+                const auto c = acells.at({i, to & groups[i].xa});
+                if (cd.w + c.second > kRowCells) close();
+                flips.push_back(RowFlip{rank(0, to), c.first, c.second, cd.w});
+                for (uint32_t k = 0; k < c.second; ++k) pos_cell.push_back(c.first + k);
+                cd.w += c.second;
+            }
+            close();
+            chunk_off.push_back((uint32_t)chunks.size());
+        }
+        // beta flips
+        bm[0] = (uint32_t)mrow.size();
+        for (size_t i = 0; i < groups.size(); ++i) {
+            if (groups[i].xa || !groups[i].xb) continue;
+            for (uint32_t p : patterns(groups[i].xb)) bcells[{i, p}] = add_cells(groups[i], 1, p, bmu, bm);
+        }
+        std::vector<std::vector<uint32_t>> l1(Db);
+        std::vector<std::vector<uint2>> l2(Db);
+        for (uint32_t rb = 0; rb < Db; ++rb) {
+            for (size_t i = 0; i < groups.size(); ++i) {
+                if (groups[i].xa || !groups[i].xb || !flips_in(bs[rb], groups[i].xb)) continue;
+                const uint32_t to = bs[rb] ^ groups[i].xb;
+                const auto c = bcells.at({i, to & groups[i].xb});
+                if (c.second == 1)
+                    l1[rb].push_back(rank(1, to) | (c.first << 14) | (parity(bs[rb] & bmu[c.first]) << 31));
+                else
+                    l2[rb].push_back(make_uint2(rank(1, to), c.first | (c.second << 20)));
+            }
+            nb1 = std::max(nb1, (uint32_t)l1[rb].size());
+            nb2 = std::max(nb2, (uint32_t)l2[rb].size());
+        }
+        // padding words point at a cell (below: a flip) that is zero
+        nb1 = (nb1 + kRowUnroll - 1) / kRowUnroll * kRowUnroll;
+        b1.assign((size_t)nb1 * Db, (uint32_t)bmu.size() << 14);
+        b2.assign((size_t)nb2 * Db, make_uint2(0, 0));
+        for (uint32_t rb = 0; rb < Db; ++rb) {
+            for (size_t k = 0; k < l1[rb].size(); ++k) b1[k * Db + rb] = l1[rb][k];
+            for (size_t k = 0; k < l2[rb].size(); ++k) b2[k * Db + rb] = l2[rb][k];
+        }
+        // both: flips (mask, pattern of the partner) of each spin, and the table over them
+        std::map<uint32_t, int> xas, xbs;
+        for (const Group& g : groups)
+            if (g.xa && g.xb) xas[g.xa] = xbs[g.xb] = 1;
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> fa, fb;
+        for (auto& x : xas)
+            for (uint32_t p : patterns(x.first)) {
+                fa[{x.first, p}] = nfa++;
+                fa_mask.push_back(compress(between(spread(x.first, 0, norb)), 1, norb));
+            }
+        for (auto& x : xbs)
+            for (uint32_t p : patterns(x.first)) {
+                fb[{x.first, p}] = nfb++;
+                fb_mask.push_back(compress(between(spread(x.first, 1, norb)), 0, norb));
+            }
+        gbase = (uint32_t)mrow.size();
+        mrow.resize(mrow.size() + (size_t)nfa * nfb);
+        mmask.resize(mrow.size(), 0u);
+        for (const Group& g : groups) {
+            if (!g.xa || !g.xb) continue;
+            const uint32_t jba = compress(between(spread(g.xb, 1, norb)), 0, norb);
+            const uint32_t jab = compress(between(spread(g.xa, 0, norb)), 1, norb);
+            for (uint32_t pa : patterns(g.xa))
+                for (uint32_t pb : patterns(g.xb)) {
+                    auto& row = mrow[gbase + (size_t)fa.at({g.xa, pa}) * nfb + fb.at({g.xb, pb})];
+                    // the strings' bits on the flipped qubits of the other spin depend on the patterns alone
+                    const uint32_t c = parity((g.xa ^ pa) & jba) ^ parity(pb & jab);
+                    for (const Term& t : g.terms)
+                        row.push_back({t.k, (c ^ parity(pa & t.za) ^ parity(pb & t.zb)) ? -1.0 : 1.0});
+                }
+        }
+        for (uint32_t ra = 0; ra < Da; ++ra) {
+            for (auto& x : xas) {
+                if (!flips_in(as[ra], x.first)) continue;
+                const uint32_t to = as[ra] ^ x.first, j = compress(between(spread(x.first, 0, norb)), 0, norb);
+                pairs.push_back(RowPair{rank(0, to), fa.at({x.first, to & x.first}), parity(as[ra] & j & ~x.first) << 31, 0});
+            }
+            while ((pairs.size() - pair_off.back()) % 4) pairs.push_back(RowPair{kRowNone, 0, 0, 0});
+            pair_off.push_back((uint32_t)pairs.size());
+        }
+        std::vector<std::vector<uint32_t>> lw(Db);
+        for (uint32_t rb = 0; rb < Db; ++rb) {
+            for (auto& x : xbs) {
+                if (!flips_in(bs[rb], x.first)) continue;
+                const uint32_t to = bs[rb] ^ x.first, j = compress(between(spread(x.first, 1, norb)), 1, norb);
+                lw[rb].push_back(rank(1, to) | (fb.at({x.first, to & x.first}) << 14) | (parity(bs[rb] & j & ~x.first) << 31));
+            }
+            nwords = std::max(nwords, (uint32_t)lw[rb].size());
+        }
+        nwords = (nwords + 3) / 4 * 4;
+        words.assign((size_t)nwords * Db, nfb << 14);
+        for (uint32_t rb = 0; rb < Db; ++rb)
+            for (size_t k = 0; k < lw[rb].size(); ++k) words[k * Db + rb] = lw[rb][k];
+        if (!nwords) pair_off.assign(Da + 1, 0);
+    }
+};
+
 // Packs host arrays into one device allocation at 256-byte offsets.
 struct Packer {
     struct Piece {
@@ -1442,7 +1848,8 @@ struct qfe_template_s {
     uint64_t nparam = 0, ninputs = 0, ngen = 0;
     std::vector<int32_t> gparam;
     std::vector<double> gscale;
-    uint32_t nterms = 0, nentries = 0, nitems = 0;
+    uint32_t nterms = 0, nentries = 0, nitems = 0, nrows = 0, nm = 0;
+    size_t row_lds = 0;    // dynamic LDS of a row workgroup
     bool has_map = false;
     bool real = false;     // scalar type of the state and the coefficients (see umul)
     size_t amp() const { return real ? sizeof(double) : sizeof(double2); }
@@ -1455,7 +1862,7 @@ struct qfe_template_s {
     const uint64_t* afull = nullptr;
     const uint64_t* bfull = nullptr;
     // per-request device bytes: psi, coef, cs, part (energy); + sig, gacc (gradient)
-    size_t off_psi = 0, off_coef = 0, off_cs = 0, off_part = 0, off_sig = 0, off_gacc = 0, off_gpart = 0;
+    size_t off_psi = 0, off_coef = 0, off_cs = 0, off_part = 0, off_sig = 0, off_gacc = 0, off_gpart = 0, off_hm = 0;
     size_t work_bytes = 0, grad_bytes = 0, io_count = 0, request_bytes = 0, grad_request_bytes = 0;
     void* arena = nullptr;  // single-request arena: [desc][out][io][prefix][work incl. gradient parts]
     // step-by-step sequence (large sectors): host step structure and device
@@ -1476,6 +1883,14 @@ struct qfe_template_s {
 
 namespace qfe {
 namespace {
+
+// Row lists are worth their tables unless the sector is enormous.
+bool rows_worth(const RowBuilder& b, const std::vector<RowBuilder::Group>& groups) {
+    if (groups.empty() || b.sp.str[1].size() > (1u << 14)) return false;
+    uint64_t flips = 0;
+    for (const auto& g : groups) flips += g.xb ? 0 : b.sp.str[0].size();
+    return flips <= kRowLists;
+}
 
 int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_terms, const uint64_t* gen_off, uint64_t ngen,
                    const int32_t* gen_param, const double* gen_scale, uint64_t nparam, const qfe_pauli* ham, uint64_t nham,
@@ -1513,6 +1928,18 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
         gen_step.push_back((uint32_t)steps.size());
     }
 
+    t->has_map = map_off != nullptr;
+    t->real = true;
+    for (const auto& en : entries) t->real = t->real && en.ulo.y == 0.0 && en.uhi.y == 0.0;
+    for (uint64_t k = 0; k < nham; ++k)
+        t->real = t->real && (t->has_map ? ham[k].phase.im == 0.0
+                                         : cplx_mul(make_double2(ham[k].phase.re, ham[k].phase.im),
+                                                    make_double2(ham[k].coeff.re, ham[k].coeff.im)).y == 0.0);
+    if (t->has_map)
+        for (uint64_t e = 0; e < map_off[nham]; ++e) t->real = t->real && map_val[e].im == 0.0;
+    RowBuilder rowb(sp, norb);
+    std::set<uint64_t> in_rows;
+
     // Hamiltonian: groups by X mask (first appearance), sector pairs only
     std::vector<SecGroup> groups;
     std::vector<uint64_t> tz;
@@ -1530,7 +1957,25 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
             if (v.empty()) order.push_back(ham[k].x);
             v.push_back(k);
         }
+        // groups that the rows take, in a real template
+        std::vector<RowBuilder::Group> rgroups;
         for (uint64_t x : order) {
+            RowBuilder::Group g{x, compress(x, 0, norb), compress(x, 1, norb), {}};
+            if (!t->real || (popc32(g.xa) & 1) || (popc32(g.xb) & 1)) continue;
+            for (uint64_t k : byx[x]) g.terms.push_back({compress(ham[k].z, 0, norb), compress(ham[k].z, 1, norb), (uint32_t)k});
+            if (rowb.fits(g)) rgroups.push_back(std::move(g));
+        }
+        if (rows_worth(rowb, rgroups)) {
+            rowb.build(rgroups);
+            if (rowb.lds() <= kRowLdsMax && rowb.bmu.size() < (1u << kRowCellBits) - 1 && rowb.nfb < (1u << kRowCellBits) - 1) {
+                for (const auto& g : rgroups) in_rows.insert(g.x);
+                t->row_lds = rowb.lds();
+                t->nrows = t->Da * ((t->Db + kRowThreads - 1) / kRowThreads);
+                t->nm = (uint32_t)rowb.mrow.size();
+            }
+        }
+        for (uint64_t x : order) {
+            if (in_rows.count(x)) continue;
             const uint32_t xa = compress(x, 0, norb), xb = compress(x, 1, norb);
             if ((popc32(xa) & 1) || (popc32(xb) & 1)) continue;  // never connects two sector determinants
             SecGroup gr{};
@@ -1629,7 +2074,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
         hchunks.push_back(make_uint2(g, g1));
         g = g1;
     }
-    t->has_map = map_off != nullptr;
     t->nterms = (uint32_t)tz.size();
     t->nentries = (uint32_t)entries.size();
     t->nitems = (uint32_t)items.size();
@@ -1637,6 +2081,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     uint64_t cost = t->D;
     for (const auto& en : entries) cost += (uint64_t)en.la_len * en.lb_len * 4;
     for (const auto& gr : groups) cost += (uint64_t)gr.la_len * gr.lb_len * (2 + gr.t_count);
+    if (t->nrows) cost += t->D * (rowb.nb1 + 8 * rowb.nb2 + (rowb.flips.size() + rowb.pairs.size() * (uint64_t)rowb.nwords) / t->Da);
     t->cost = cost;
 
     {  // serving tier
@@ -1651,11 +2096,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     std::vector<uint64_t> af(t->Da), bf(t->Db);
     for (uint32_t a = 0; a < t->Da; ++a) af[a] = spread(sp.str[0][a], 0, norb);
     for (uint32_t b2 = 0; b2 < t->Db; ++b2) bf[b2] = spread(sp.str[1][b2], 1, norb);
-    t->real = true;
-    for (const auto& en : entries) t->real = t->real && en.ulo.y == 0.0 && en.uhi.y == 0.0;
-    for (const auto& v : tph) t->real = t->real && (!t->has_map || v.y == 0.0);
-    for (const auto& v : mval) t->real = t->real && v.y == 0.0;
-    for (const auto& v : tcoef) t->real = t->real && (t->has_map || v.y == 0.0);
     std::vector<double> tcoef_real;
     if (t->real)
         for (const auto& v : tcoef) tcoef_real.push_back(v.x);
@@ -1663,6 +2103,32 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     tb.build(gen_step);
     t->fwd = tb.lfwd;
     t->rev = tb.lrev;
+    // merged numbers of the rows: from the inputs, or constants
+    std::vector<double> rm, rmval;
+    std::vector<uint32_t> rmoff{0}, rmidx;
+    if (t->nrows) {
+        for (const auto& row : rowb.mrow) {
+            std::map<uint32_t, double> in;
+            double v = 0.0;
+            for (const auto& tk : row) {
+                const qfe_pauli& h = ham[tk.first];
+                if (t->has_map)
+                    for (uint64_t e = map_off[tk.first]; e < map_off[tk.first + 1]; ++e)
+                        in[map_idx[e]] += tk.second * h.phase.re * map_val[e].re;
+                else
+                    v += tk.second * (h.phase.re * h.coeff.re - h.phase.im * h.coeff.im);
+            }
+            for (const auto& e : in)
+                if (e.second != 0.0) {
+                    rmidx.push_back(e.first);
+                    rmval.push_back(e.second);
+                }
+            rmoff.push_back((uint32_t)rmidx.size());
+            if (!t->has_map) rm.push_back(v);
+        }
+    }
+    const RowBuilder none(sp, norb);
+    const RowBuilder& rows = t->nrows ? rowb : none;
     Packer pk(sizeof(SecTables));
     const size_t i_af = pk.add(af.data(), af.size() * 8), i_bf = pk.add(bf.data(), bf.size() * 8);
     const size_t i_as = pk.add(sp.str[0].data(), sp.str[0].size() * 4), i_bs = pk.add(sp.str[1].data(), sp.str[1].size() * 4);
@@ -1689,6 +2155,24 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     const size_t i_tw = pk.add(tb.words.data(), tb.words.size() * 4);
     const size_t i_tu = pk.add(tb.sum.data(), tb.sum.size() * sizeof(uint2));
     const size_t i_to = pk.add(tb.sum_off.data(), tb.sum_off.size() * 4);
+    auto add_all = [&](const auto& v) { return pk.add(v.data(), v.size() * sizeof(v[0])); };
+    const size_t r_chunk_off = add_all(rows.chunk_off);
+    const size_t r_chunks = add_all(rows.chunks);
+    const size_t r_flips = add_all(rows.flips);
+    const size_t r_pos_cell = add_all(rows.pos_cell);
+    const size_t r_amu = add_all(rows.amu);
+    const size_t r_am = add_all(rows.am);
+    const size_t r_bmu = add_all(rows.bmu);
+    const size_t r_bm = add_all(rows.bm);
+    const size_t r_mmask = add_all(rows.mmask);
+    const size_t r_b1 = add_all(rows.b1);
+    const size_t r_b2 = add_all(rows.b2);
+    const size_t r_pair_off = add_all(rows.pair_off);
+    const size_t r_pairs = add_all(rows.pairs);
+    const size_t r_words = add_all(rows.words);
+    const size_t r_fb_mask = add_all(rows.fb_mask);
+    const size_t r_fa_mask = add_all(rows.fa_mask);
+    const size_t r_m = add_all(rm), r_moff = add_all(rmoff), r_midx = add_all(rmidx), r_mval = add_all(rmval);
     QFE_HIP(hipMalloc(&t->dev, pk.total));
     char* base = (char*)t->dev;
     auto at = [&](size_t i) { return base + pk.pieces[i].off; };
@@ -1726,6 +2210,35 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     h.twords = (const uint32_t*)at(i_tw);
     h.tsum = (const uint2*)at(i_tu);
     h.tsum_off = (const uint32_t*)at(i_to);
+    h.rows.chunk_off = (const uint32_t*)at(r_chunk_off);
+    h.rows.chunks = (const uint4*)at(r_chunks);
+    h.rows.flips = (const RowFlip*)at(r_flips);
+    h.rows.pos_cell = (const uint32_t*)at(r_pos_cell);
+    h.rows.amu = (const uint32_t*)at(r_amu);
+    h.rows.am = (const uint32_t*)at(r_am);
+    h.rows.bmu = (const uint32_t*)at(r_bmu);
+    h.rows.bm = (const uint32_t*)at(r_bm);
+    h.rows.mmask = (const uint32_t*)at(r_mmask);
+    h.rows.b1 = (const uint32_t*)at(r_b1);
+    h.rows.b2 = (const uint2*)at(r_b2);
+    h.rows.pair_off = (const uint32_t*)at(r_pair_off);
+    h.rows.pairs = (const RowPair*)at(r_pairs);
+    h.rows.words = (const uint32_t*)at(r_words);
+    h.rows.fb_mask = (const uint32_t*)at(r_fb_mask);
+    h.rows.fa_mask = (const uint32_t*)at(r_fa_mask);
+    h.rows.m = (const double*)at(r_m);
+    h.rows.moff = (const uint32_t*)at(r_moff);
+    h.rows.midx = (const uint32_t*)at(r_midx);
+    h.rows.mval = (const double*)at(r_mval);
+    h.rows.nm = t->nm;
+    h.rows.nbcell = (uint32_t)rows.bmu.size();
+    h.rows.nb1 = rows.nb1;
+    h.rows.nb2 = rows.nb2;
+    h.rows.nwords = rows.nwords;
+    h.rows.nfb = rows.nfb;
+    h.rows.gbase = rows.gbase;
+    h.nrows = t->nrows;
+    h.nparts = t->nitems + t->nrows;
     h.nsteps = (uint32_t)steps.size();
     h.nentries = (uint32_t)entries.size();
     h.ngroups = (uint32_t)groups.size();
@@ -1746,10 +2259,12 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     o += align256(t->D * t->amp());
     t->off_coef = o;
     if (t->has_map) o += align256((size_t)t->nterms * t->amp());
+    t->off_hm = o;
+    if (t->has_map) o += align256((size_t)t->nm * 8);
     t->off_cs = o;
     o += align256((size_t)t->nentries * sizeof(double2) + 16);
     t->off_part = o;
-    o += align256((size_t)t->nitems * 8 + 8);
+    o += align256((size_t)(t->nitems + t->nrows) * 8 + 8);
     t->work_bytes = o;
     t->off_sig = o;
     o += align256(t->D * t->amp());
@@ -1784,6 +2299,7 @@ SlotDesc make_slot(qfe_template t, char* work, const double* io, double* out, bo
     d.t = t->dt;
     d.psi = work + t->off_psi;
     d.coef = t->has_map ? work + t->off_coef : nullptr;
+    d.hm = t->has_map && t->nrows ? (double*)(work + t->off_hm) : nullptr;
     d.cs = (double2*)(work + t->off_cs);
     d.part = (double*)(work + t->off_part);
     d.sig = grad ? work + t->off_sig : nullptr;
@@ -1844,34 +2360,48 @@ void pass_prefix(const std::vector<qfe_template>& ts, bool rev, std::vector<uint
     }
 }
 
-// Energy of k requests: prologue, ansatz, items, sums.
-int launch_energy(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* dprefix, const uint32_t* tprefix,
-                  uint32_t total_items, hipStream_t st) {
-    const unsigned k = (unsigned)ts.size();
-    with_scalar(ts[0], [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(k), dim3(256), 0, st, ddesc, 1); });
-    QFE_HIP(hipGetLastError());
-    int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
-    if (rc) return rc;
-    if (total_items) {
-        with_scalar(ts[0], [&](auto z) {
-            hipLaunchKernelGGL(k_sec_energy<decltype(z)>, dim3(total_items), dim3(kItemThreads), 0, st, ddesc, dprefix, (uint32_t)k);
-        });
-        QFE_HIP(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_sec_sum, dim3(k), dim3(256), 0, st, ddesc);
+int launch_prologue(const std::vector<qfe_template>& ts, const SlotDesc* d, int need_coef, hipStream_t st) {
+    uint32_t most = 1;
+    for (const auto& t : ts) most = std::max(most, std::max(t->nentries, need_coef ? std::max(t->nterms, t->nm) : 0u));
+    with_scalar(ts[0], [&](auto z) {
+        hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3((most + 255) / 256, (unsigned)ts.size()), dim3(256), 0, st, d, need_coef);
+    });
     QFE_HIP(hipGetLastError());
     return QFE_OK;
 }
 
-// psi = U|ref> and sigma = H psi of k requests: prologue, ansatz, sigma (grid y = request).
-int launch_psi_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* tprefix, hipStream_t st) {
+// The row workgroups of k requests (prefix: row prefix, null for one request).
+int launch_rows(const std::vector<qfe_template>& ts, const SlotDesc* d, const uint32_t* prefix, bool energy, hipStream_t st) {
+    uint64_t rows = 0;
+    uint32_t Db = 1;
+    size_t lds = 0;
+    for (const auto& t : ts) {
+        rows += t->nrows;
+        Db = std::max(Db, t->Db);
+        lds = std::max(lds, t->row_lds);
+    }
+    if (!rows) return QFE_OK;
+    if (rows >= (1ull << 31)) return fail(QFE_ERR_ARG, "qfe_template: too many rows in one launch");
+    const unsigned threads = std::min(kRowThreads, (Db + 63u) & ~63u);  // a row of at most 256 strings is one workgroup
+    if (energy)
+        hipLaunchKernelGGL(k_sec_rows<true>, dim3((unsigned)rows), dim3(threads), lds, st, d, prefix, (uint32_t)ts.size());
+    else
+        hipLaunchKernelGGL(k_sec_rows<false>, dim3((unsigned)rows), dim3(threads), lds, st, d, prefix, (uint32_t)ts.size());
+    QFE_HIP(hipGetLastError());
+    return QFE_OK;
+}
+
+// sigma = H psi: the rows, then the groups that they do not take (grid y = request).
+int launch_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* rowprefix, hipStream_t st) {
     const unsigned k = (unsigned)ts.size();
     uint64_t D = 1;
-    for (const auto& t : ts) D = std::max(D, t->D);
-    with_scalar(ts[0], [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(k), dim3(256), 0, st, ddesc, 1); });
-    QFE_HIP(hipGetLastError());
-    int rc = launch_tiles<0>(ts, ddesc, tprefix, st);
-    if (rc) return rc;
+    bool rest = false;
+    for (const auto& t : ts) {
+        D = std::max(D, t->D);
+        rest = rest || t->nitems || !t->nrows;
+    }
+    int rc = launch_rows(ts, ddesc, rowprefix, false, st);
+    if (rc || !rest) return rc;
     with_scalar(ts[0], [&](auto z) {
         using S = decltype(z);
         if (k == 1)
@@ -1883,11 +2413,41 @@ int launch_psi_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc,
     return QFE_OK;
 }
 
-// Energy and adjoint gradient of k requests; rprefix: tile prefixes of the reverse sweep.
-int launch_gradient(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const uint32_t* tprefix, const uint32_t* rprefix,
-                    hipStream_t st) {
-    int rc = launch_psi_sigma(ts, ddesc, tprefix, st);
-    if (!rc) rc = launch_tiles<2>(ts, ddesc, rprefix, st);
+// Prefixes of a launch over several requests, on the device (null for one request).
+struct Prefixes {
+    const uint32_t *items, *fwd, *rows, *rev;
+};
+
+// Energy of k requests: prologue, ansatz, rows and items, sums.
+int launch_energy(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const Prefixes& pre, uint32_t total_items,
+                  hipStream_t st) {
+    const unsigned k = (unsigned)ts.size();
+    int rc = launch_prologue(ts, ddesc, 1, st);
+    if (!rc) rc = launch_tiles<0>(ts, ddesc, pre.fwd, st);
+    if (!rc) rc = launch_rows(ts, ddesc, pre.rows, true, st);
+    if (rc) return rc;
+    if (total_items) {
+        with_scalar(ts[0], [&](auto z) {
+            hipLaunchKernelGGL(k_sec_energy<decltype(z)>, dim3(total_items), dim3(kItemThreads), 0, st, ddesc, pre.items, (uint32_t)k);
+        });
+        QFE_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_sec_sum, dim3(k), dim3(256), 0, st, ddesc);
+    QFE_HIP(hipGetLastError());
+    return QFE_OK;
+}
+
+// psi = U|ref> and sigma = H psi of k requests.
+int launch_psi_sigma(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const Prefixes& pre, hipStream_t st) {
+    int rc = launch_prologue(ts, ddesc, 1, st);
+    if (!rc) rc = launch_tiles<0>(ts, ddesc, pre.fwd, st);
+    return rc ? rc : launch_sigma(ts, ddesc, pre.rows, st);
+}
+
+// Energy and adjoint gradient of k requests.
+int launch_gradient(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, const Prefixes& pre, hipStream_t st) {
+    int rc = launch_psi_sigma(ts, ddesc, pre, st);
+    if (!rc) rc = launch_tiles<2>(ts, ddesc, pre.rev, st);
     if (rc) return rc;
     uint64_t ngen = 0;
     for (const auto& t : ts) ngen = std::max(ngen, t->ngen);
@@ -1915,9 +2475,9 @@ int wide_ansatz(qfe_template t, const SlotDesc* d, hipStream_t st) {
 // Energy: prologue, ansatz, work items, sum (the items and sum kernels of the batched path).
 template <typename S>
 int wide_energy(qfe_template t, const SlotDesc* d, const uint32_t* dprefix, hipStream_t st) {
-    hipLaunchKernelGGL(k_sec_prologue<S>, dim3(1), dim3(256), 0, st, d, 1);
-    QFE_HIP(hipGetLastError());
-    int rc = wide_ansatz<S>(t, d, st);
+    int rc = launch_prologue({t}, d, 1, st);
+    if (!rc) rc = wide_ansatz<S>(t, d, st);
+    if (!rc) rc = launch_rows({t}, d, nullptr, true, st);
     if (rc) return rc;
     if (t->nitems) {
         hipLaunchKernelGGL(k_sec_energy<S>, dim3(t->nitems), dim3(kItemThreads), 0, st, d, dprefix, 1u);
@@ -1931,13 +2491,9 @@ int wide_energy(qfe_template t, const SlotDesc* d, const uint32_t* dprefix, hipS
 // psi and sigma = H psi (pool gradients and the gradient below).
 template <typename S>
 int wide_psi_sigma(qfe_template t, const SlotDesc* d, hipStream_t st) {
-    hipLaunchKernelGGL(k_sec_prologue<S>, dim3(1), dim3(256), 0, st, d, 1);
-    QFE_HIP(hipGetLastError());
-    int rc = wide_ansatz<S>(t, d, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL((k_sec_hpsi<S, 1>), dim3((unsigned)((t->D + 255) / 256), 1), dim3(256), 0, st, d);
-    QFE_HIP(hipGetLastError());
-    return QFE_OK;
+    int rc = launch_prologue({t}, d, 1, st);
+    if (!rc) rc = wide_ansatz<S>(t, d, st);
+    return rc ? rc : launch_sigma({t}, d, nullptr, st);
 }
 
 // Energy and generator overlaps: E = Re<psi|sigma>, then for k = M-1 .. 0 the
@@ -2023,7 +2579,7 @@ void gradient_from_overlaps(qfe_template t, const double* acc, double* grad) {
 // psi = U|ref> and sigma = H psi for one request (pool gradients).
 int single_psi_sigma(qfe_template t, const double* params, const double* inputs, Single& S) {
     int rc = single_setup(t, params, inputs, true, S);
-    return rc ? rc : launch_psi_sigma({t}, S.ddesc, nullptr, ctx().stream);
+    return rc ? rc : launch_psi_sigma({t}, S.ddesc, Prefixes{}, ctx().stream);
 }
 
 // ---- captured single-request sequences (large sectors) ----------------------------------
@@ -2086,11 +2642,15 @@ void expected_nodes(qfe_template t, int grad, std::vector<NodeExpect>& out) {
     const auto KB = [](uint64_t items) { return (items + kWideTPB - 1) / kWideTPB; };
     out.clear();
     out.push_back(expect_copy(dev, pin, head));
-    out.push_back(expect_kernel((const void*)&k_sec_prologue<S>, 1, 256, d, (int)1));
+    out.push_back(expect_kernel((const void*)&k_sec_prologue<S>, KB(std::max(std::max(t->nentries, 1u), std::max(t->nterms, t->nm))), 256, d,
+                                (int)1));
     out.push_back(expect_kernel((const void*)&k_sec_ref<S>, KB(t->D), kWideTPB, d));
     for (uint32_t k = 0; k < (uint32_t)t->step_pairs.size(); ++k)
         if (t->step_pairs[k])
             out.push_back(expect_kernel((const void*)&k_sec_step<S>, KB(t->step_pairs[k]), kWideTPB, d, k, (int)0, (int)0));
+    if (t->nrows)
+        out.push_back(expect_kernel(grad ? (const void*)&k_sec_rows<false> : (const void*)&k_sec_rows<true>, t->nrows,
+                                    std::min(kRowThreads, (t->Db + 63u) & ~63u), d, (const uint32_t*)nullptr, (uint32_t)1));
     if (!grad) {
         if (t->nitems)
             out.push_back(expect_kernel((const void*)&k_sec_energy<S>, t->nitems, kItemThreads, d,
@@ -2099,7 +2659,7 @@ void expected_nodes(qfe_template t, int grad, std::vector<NodeExpect>& out) {
         out.push_back(expect_copy(pin + head, dev + 256, 8));
         return;
     }
-    out.push_back(expect_kernel((const void*)&k_sec_hpsi<S, 1>, (t->D + 255) / 256, 256, d));
+    if (t->nitems || !t->nrows) out.push_back(expect_kernel((const void*)&k_sec_hpsi<S, 1>, (t->D + 255) / 256, 256, d));
     double* part = (double*)((char*)t->wide + align256(t->wide_seg.size() * sizeof(uint2)));
     out.push_back(expect_kernel((const void*)&k_sec_edot<S>, t->wide_seg[0].y, kWideTPB, d, part + t->wide_seg[0].x));
     for (uint32_t k = (uint32_t)t->ngen; k-- > 0;) {
@@ -2143,8 +2703,8 @@ int audit_graph(qfe_template t, hipGraph_t g, int grad, GraphAudit& A) {
     auto in_work = [&](const void* p, size_t bytes) { return p && inside(p, bytes, work, t->grad_bytes); };
     if (d.t != t->dt || d.out != (double*)(dev + 256) || !in_work(d.psi, t->D * t->amp()) ||
         !in_work(d.sig, t->D * t->amp()) || !in_work(d.cs, (size_t)t->nentries * sizeof(double2)) ||
-        !in_work(d.part, (size_t)t->nitems * 8) || !in_work(d.gacc, t->ngen * 8) ||
-        (t->has_map && !in_work(d.coef, (size_t)t->nterms * t->amp())) ||
+        !in_work(d.part, (size_t)(t->nitems + t->nrows) * 8) || !in_work(d.gacc, t->ngen * 8) ||
+        (t->has_map && !in_work(d.coef, (size_t)t->nterms * t->amp())) || (d.hm && !in_work(d.hm, (size_t)t->nm * 8)) ||
         !inside(d.params, t->io_count * 8, dev + 768, head - 768))
         return audit_fail(grad, 0, "descriptor pointer outside the arena");
     std::vector<NodeExpect> want;
@@ -2437,6 +2997,12 @@ int lane_launch(qfe_batch b, Lane& L) {
     std::vector<uint32_t> tpre;  // tile prefixes: the ansatz passes, then the reverse sweep's
     pass_prefix(ts, false, tpre);
     const size_t nfwd = tpre.size();
+    uint32_t row_at = 0;  // row workgroups
+    for (size_t i = 0; i <= k; ++i) {
+        tpre.push_back(row_at);
+        if (i < k) row_at += ts[i]->nrows;
+    }
+    const size_t nrow = tpre.size();
     if (grad) pass_prefix(ts, true, tpre);
     const size_t o_tpre = o_pre + align256((k + 1) * 4);
     const size_t o_io = o_tpre + align256(tpre.size() * 4);
@@ -2482,11 +3048,12 @@ int lane_launch(qfe_batch b, Lane& L) {
     hpre[k] = acc_items;
     std::memcpy(up + o_tpre, tpre.data(), tpre.size() * 4);
     const uint32_t* dtpre = (const uint32_t*)(dev + o_tpre);
+    const Prefixes pre{(const uint32_t*)(dev + o_pre), dtpre, dtpre + nfwd, dtpre + nrow};
     QFE_HIP(hipMemcpyAsync(dev, up, head, hipMemcpyHostToDevice, L.stream));
     if (grad)
-        rc = launch_gradient(ts, (const SlotDesc*)dev, dtpre, dtpre + nfwd, L.stream);
+        rc = launch_gradient(ts, (const SlotDesc*)dev, pre, L.stream);
     else
-        rc = launch_energy(ts, (const SlotDesc*)dev, (const uint32_t*)(dev + o_pre), dtpre, acc_items, L.stream);
+        rc = launch_energy(ts, (const SlotDesc*)dev, pre, acc_items, L.stream);
     if (rc) return rc;
     QFE_HIP(hipMemcpyAsync(L.out, dout, nres * 8, hipMemcpyDeviceToHost, L.stream));
     QFE_HIP(hipEventRecord(L.done, L.stream));
@@ -2635,7 +3202,7 @@ int qfe_template_energy(qfe_template t, const double* params, const double* inpu
     Single S;
     int rc = single_setup(t, params, inputs, false, S);
     if (rc) return rc;
-    rc = launch_energy({t}, S.ddesc, S.dprefix, nullptr, t->nitems, ctx().stream);
+    rc = launch_energy({t}, S.ddesc, Prefixes{S.dprefix, nullptr, nullptr, nullptr}, t->nitems, ctx().stream);
     if (rc) return rc;
     return fetch_doubles(S.dout, 1, energy);
 }
@@ -2648,9 +3215,8 @@ int qfe_template_prepare(qfe_template t, const double* params, qfe_state out) {
     int rc = single_setup(t, params, zeros.data(), false, S);
     if (rc) return rc;
     hipStream_t st = ctx().stream;
-    with_scalar(t, [&](auto z) { hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(1), dim3(256), 0, st, S.ddesc, 0); });
-    QFE_HIP(hipGetLastError());
-    rc = launch_tiles<0>({t}, S.ddesc, nullptr, st);
+    rc = launch_prologue({t}, S.ddesc, 0, st);
+    if (!rc) rc = launch_tiles<0>({t}, S.ddesc, nullptr, st);
     if (!rc) rc = launch_zero(out->d, out->N, st);
     if (rc) return rc;
     with_scalar(t, [&](auto z) {
@@ -2668,7 +3234,7 @@ int qfe_template_gradient(qfe_template t, const double* params, const double* in
     std::vector<double> acc(t->ngen + 1);
     Single S;
     int rc = single_setup(t, params, inputs, true, S);
-    if (!rc) rc = launch_gradient({t}, S.ddesc, nullptr, nullptr, ctx().stream);
+    if (!rc) rc = launch_gradient({t}, S.ddesc, Prefixes{}, ctx().stream);
     if (rc) return rc;
     rc = fetch_doubles((const double*)(S.work + t->off_gacc), t->ngen, acc.data());
     if (!rc) rc = fetch_doubles(S.dout, 1, &acc[t->ngen]);
