@@ -206,8 +206,9 @@ int launch_apply_sum_async(const double2* in, double2* out, int n, const PauliGr
 
 // ---------------------------------------------------------------------------
 // Orbit-fused expectation passes.  Groups whose X masks span <= 4 dimensions
-// over GF(2) (5 for a plain expectation value) are evaluated together: every thread loads the 2^M amplitudes
-// of its orbit {j ^ c_i} once and accumulates, for each group g with mask
+// over GF(2) (5 for a plain expectation value) are evaluated together; a pass
+// of fewer dimensions is padded with single qubits (build_orbit_tables).
+// Every thread loads the 2^M amplitudes of its orbit {j ^ c_i} once and accumulates, for each group g with mask
 // v_g in orbit coordinates, sum_i conj(bra_i) ket_{i^v} f_g(i^v).  One read
 // pass of the state then serves up to 16 groups.
 // ---------------------------------------------------------------------------
@@ -352,15 +353,150 @@ __device__ __forceinline__ uint32_t term_sign_vector(uint32_t smask) {
 //   sum_i s_i p_i = 2 sum_{i: bit h clear} s_i Re p_i    (sigma = +1)
 //                 = 2i sum_{i: bit h clear} s_i Im p_i   (sigma = -1):
 // two products and an FMA per pair of elements instead of a complex product
-// and two FMAs per element.  A diagonal group (v = 0, the terms with no X or
-// Y; one per operator; diag is the first in the pass, ngroups if none) sums
-// s_i |a_i|^2 = H[zm], the Walsh-Hadamard transform of q_i = |a_i|^2
-// at the term's sign vector zm (bit k of zm: bit 2^k of smask, since the
-// sign pattern is linear in i): it runs after the other groups, transforms
-// q in place of the amplitudes once, and then costs each of its terms (often
-// the most numerous group) one register select instead of a sum over the
-// orbit.  Further groups with v = 0 in the same pass (one per operator of
-// qfe_expval_many) sum s_i |a_i|^2 directly.
+// and two FMAs per element.  Diagonal groups (v = 0, the terms with no X or
+// Y; one per operator) come last in a pass, from position diag on.  They sum
+// s_i |a_i|^2 = H[zm], the Walsh-Hadamard transform of q_i = |a_i|^2 at the
+// term's sign vector zm (bit k of zm: bit 2^k of smask, since the sign pattern
+// is linear in i): q is transformed once in place of the amplitudes, and then
+// each term costs one register select instead of a sum over the orbit.
+struct OrbitPass {  // device view of a pass
+    OrbitBasis ob;
+    uint32_t g0, ng, diag, pad;
+};
+
+// The groups [g0, g0 + ng) of a pass on one orbit: add(g, value).
+template <int M, typename F>
+__device__ __forceinline__ void orbit_values(double2 (&a)[1 << M], uint64_t j, const OrbitGroup* __restrict__ groups,
+                                             uint32_t ngroups, uint32_t diag, const OrbitTerm* __restrict__ terms, F&& add) {
+    for (uint32_t g = 0; g < diag; ++g) {
+        const OrbitGroup G = groups[g];
+        double2 acc = make_double2(0.0, 0.0);
+        dispatch_mask<M>(G.v, [&](auto vc) {
+            constexpr uint32_t V = decltype(vc)::value;
+            if constexpr (V != 0) {
+                for (uint32_t tt = 0; tt < G.count; ++tt) {
+                    const OrbitTerm T = terms[G.first + tt];
+                    double w = 0.0;
+                    // the empty volatile asm on each partner keeps its products
+                    // inside this branch and this term: otherwise the compiler
+                    // computes the products of every branch up front, out of the
+                    // term loop, and spills them
+                    constexpr uint32_t H = 1u << (31 - __builtin_clz(V));
+                    const bool imag = (T.smask >> V) & 1u;
+                    if (!imag) {
+#pragma unroll
+                        for (int i = 0; i < (1 << M); ++i) {
+                            if (i & H) continue;
+                            double2 q = a[i ^ V];
+                            asm volatile("" : "+v"(q.x), "+v"(q.y));
+                            const double sg = ((T.pmask >> i) & 1u) ? -1.0 : 1.0;
+                            w = fma(sg, fma(a[i].x, q.x, a[i].y * q.y), w);
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < (1 << M); ++i) {
+                            if (i & H) continue;
+                            double2 q = a[i ^ V];
+                            asm volatile("" : "+v"(q.x), "+v"(q.y));
+                            const double sg = ((T.pmask >> i) & 1u) ? -1.0 : 1.0;
+                            w = fma(sg, fma(a[i].x, q.y, -(a[i].y * q.x)), w);
+                        }
+                    }
+                    w *= 2.0;
+                    if (__popcll(j & T.z) & 1) w = -w;
+                    // c * w (sigma = +1) or c * i w (sigma = -1)
+                    if (imag)
+                        acc = make_double2(fma(-T.c.y, w, acc.x), fma(T.c.x, w, acc.y));
+                    else
+                        acc = make_double2(fma(T.c.x, w, acc.x), fma(T.c.y, w, acc.y));
+                }
+            }
+        });
+        add(g, acc);
+    }
+    if (diag == ngroups) return;
+    // q_i = |a_i|^2 over the real parts, then H[k] = sum_i (-1)^popcount(i & k) q_i in place
+#pragma unroll
+    for (int i = 0; i < (1 << M); ++i) a[i].x = fma(a[i].x, a[i].x, a[i].y * a[i].y);
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+#pragma unroll
+        for (int i = 0; i < (1 << M); ++i) {
+            if (i & (1 << k)) continue;
+            const double u = a[i].x, v = a[i | (1 << k)].x;
+            a[i].x = u + v;
+            a[i | (1 << k)].x = u - v;
+        }
+    }
+    for (uint32_t g = diag; g < ngroups; ++g) {
+        const OrbitGroup G = groups[g];
+        double2 acc = make_double2(0.0, 0.0);
+        for (uint32_t tt = 0; tt < G.count; ++tt) {
+            const OrbitTerm T = terms[G.first + tt];
+            const uint32_t zm = term_sign_vector<M>(T.smask);
+            double w = 0.0;
+            // one branch per value of zm (an empty volatile asm keeps the
+            // branches apart, so the select is never a variable index into
+            // the register array, which would move it to scratch memory)
+            dispatch_mask<M>(zm, [&](auto zc) {
+                double t = a[decltype(zc)::value].x;
+                asm volatile("" : "+v"(t));
+                w = t;
+            });
+            if (__popcll(j & T.z) & 1) w = -w;
+            acc = make_double2(fma(T.c.x, w, acc.x), fma(T.c.y, w, acc.y));
+        }
+        add(g, acc);
+    }
+}
+
+template <int M, bool NT>
+__device__ __forceinline__ uint64_t load_orbit(double2 (&a)[1 << M], const double2* __restrict__ psi, uint64_t t,
+                                               const OrbitBasis& ob) {
+    uint64_t j = t;
+#pragma unroll
+    for (int k = 0; k < M; ++k) j = ins0(j, ob.p[k]);
+#pragma unroll
+    for (int i = 0; i < (1 << M); ++i) {
+        uint64_t c = 0;
+#pragma unroll
+        for (int k = 0; k < M; ++k)
+            if ((i >> k) & 1) c ^= ob.b[k];
+        a[i] = ld_s<NT>(psi + (j ^ c));
+    }
+    return j;
+}
+
+// States that stay in the last-level cache (at most one orbit per thread): all
+// passes of an operator in one launch (grid y), each thread's values
+// summed over its wave at once.  Per-thread accumulators in LDS (64 KiB for 16
+// groups) would leave two workgroups per CU and cost as much as the values.
+template <int M>
+__global__ __launch_bounds__(kEvTPB) __attribute__((amdgpu_waves_per_eu(3))) void k_orbit_expval_once(
+    const double2* __restrict__ psi, uint64_t norbit, const OrbitPass* __restrict__ passes,
+    const OrbitGroup* __restrict__ all_groups, const OrbitTerm* __restrict__ terms, double2* __restrict__ partial, uint32_t nb) {
+    __shared__ double2 sums[kEvOrbitGroups][kEvTPB / kWave];
+    const OrbitPass& P = passes[blockIdx.y];
+    const OrbitGroup* __restrict__ groups = all_groups + P.g0;
+    const uint32_t ng = P.ng;
+    const uint64_t ch = xcd_block(), t = ch * kEvTPB + threadIdx.x;
+    const bool live = t < norbit;
+    double2 a[1 << M];
+    const uint64_t j = load_orbit<M, false>(a, psi, live ? t : 0, P.ob);
+    orbit_values<M>(a, j, groups, ng, P.diag, terms, [&](uint32_t g, double2 v) {
+        const double2 s = make_double2(wave_sum_last(live ? v.x : 0.0), wave_sum_last(live ? v.y : 0.0));
+        if ((threadIdx.x & (kWave - 1)) == kWave - 1) sums[g][threadIdx.x / kWave] = s;
+    });
+    __syncthreads();
+    if (threadIdx.x < ng) {
+        double2 s = sums[threadIdx.x][0];
+        for (int w = 1; w < kEvTPB / kWave; ++w) s = cadd(s, sums[threadIdx.x][w]);
+        partial[(uint64_t)groups[threadIdx.x].slot * nb + ch] = s;
+    }
+}
+
+// Larger states: one launch per pass, every workgroup walks a range of orbits
+// with per-thread accumulators in LDS.
 template <int M, bool NT>
 __global__ __launch_bounds__(kEvTPB) __attribute__((amdgpu_waves_per_eu(3))) void k_orbit_expval_same(
     const double2* __restrict__ psi, uint64_t norbit, OrbitBasis ob, const OrbitGroup* __restrict__ groups,
@@ -372,109 +508,11 @@ __global__ __launch_bounds__(kEvTPB) __attribute__((amdgpu_waves_per_eu(3))) voi
     const uint64_t per = ((norbit + nb - 1) / nb + kEvTPB - 1) / kEvTPB * kEvTPB;
     const uint64_t t1 = min(norbit, (ch + 1) * per);
     for (uint64_t t = ch * per + threadIdx.x; t < t1; t += kEvTPB) {
-        uint64_t j = t;
-#pragma unroll
-        for (int k = 0; k < M; ++k) j = ins0(j, ob.p[k]);
         double2 a[1 << M];
-#pragma unroll
-        for (int i = 0; i < (1 << M); ++i) {
-            uint64_t c = 0;
-#pragma unroll
-            for (int k = 0; k < M; ++k)
-                if ((i >> k) & 1) c ^= ob.b[k];
-            a[i] = ld_s<NT>(psi + (j ^ c));
-        }
-        for (uint32_t g = 0; g < ngroups; ++g) {
-            if (g == diag) continue;
-            const OrbitGroup G = groups[g];
-            double2 acc = make_double2(0.0, 0.0);
-            dispatch_mask<M>(G.v, [&](auto vc) {
-                constexpr uint32_t V = decltype(vc)::value;
-                for (uint32_t tt = 0; tt < G.count; ++tt) {
-                    const OrbitTerm T = terms[G.first + tt];
-                    double w = 0.0;
-                    bool imag = false;
-                    // the empty volatile asm on each partner keeps its products
-                    // inside this branch and this term: otherwise the compiler
-                    // computes the products of every branch up front, out of the
-                    // term loop, and spills them
-                    if constexpr (V == 0) {
-                        // a second diagonal group in one pass (one per operator
-                        // of qfe_expval_many): s_i |a_i|^2 summed directly
-#pragma unroll
-                        for (int i = 0; i < (1 << M); ++i) {
-                            double2 q = a[i];
-                            asm volatile("" : "+v"(q.x), "+v"(q.y));
-                            const double sg = ((T.pmask >> i) & 1u) ? -1.0 : 1.0;
-                            w = fma(sg, fma(q.x, q.x, q.y * q.y), w);
-                        }
-                    } else {
-                        constexpr uint32_t H = 1u << (31 - __builtin_clz(V));
-                        imag = (T.smask >> V) & 1u;
-                        if (!imag) {
-#pragma unroll
-                            for (int i = 0; i < (1 << M); ++i) {
-                                if (i & H) continue;
-                                double2 q = a[i ^ V];
-                                asm volatile("" : "+v"(q.x), "+v"(q.y));
-                                const double sg = ((T.pmask >> i) & 1u) ? -1.0 : 1.0;
-                                w = fma(sg, fma(a[i].x, q.x, a[i].y * q.y), w);
-                            }
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < (1 << M); ++i) {
-                                if (i & H) continue;
-                                double2 q = a[i ^ V];
-                                asm volatile("" : "+v"(q.x), "+v"(q.y));
-                                const double sg = ((T.pmask >> i) & 1u) ? -1.0 : 1.0;
-                                w = fma(sg, fma(a[i].x, q.y, -(a[i].y * q.x)), w);
-                            }
-                        }
-                        w *= 2.0;
-                    }
-                    if (__popcll(j & T.z) & 1) w = -w;
-                    // c * w (sigma = +1) or c * i w (sigma = -1)
-                    if (imag)
-                        acc = make_double2(fma(-T.c.y, w, acc.x), fma(T.c.x, w, acc.y));
-                    else
-                        acc = make_double2(fma(T.c.x, w, acc.x), fma(T.c.y, w, acc.y));
-                }
-            });
-            acc_s[g * kEvTPB + threadIdx.x] = cadd(acc_s[g * kEvTPB + threadIdx.x], acc);
-        }
-        if (diag < ngroups) {
-            // q_i = |a_i|^2 over the real parts, then H[k] = sum_i (-1)^popcount(i & k) q_i in place
-#pragma unroll
-            for (int i = 0; i < (1 << M); ++i) a[i].x = fma(a[i].x, a[i].x, a[i].y * a[i].y);
-#pragma unroll
-            for (int k = 0; k < M; ++k) {
-#pragma unroll
-                for (int i = 0; i < (1 << M); ++i) {
-                    if (i & (1 << k)) continue;
-                    const double u = a[i].x, v = a[i | (1 << k)].x;
-                    a[i].x = u + v;
-                    a[i | (1 << k)].x = u - v;
-                }
-            }
-            const OrbitGroup G = groups[diag];
-            double2 acc = make_double2(0.0, 0.0);
-            for (uint32_t tt = 0; tt < G.count; ++tt) {
-                const OrbitTerm T = terms[G.first + tt];
-                const uint32_t zm = term_sign_vector<M>(T.smask);
-                double w = 0.0;
-                // one branch per value of zm (an empty volatile asm keeps the
-                // branches apart, so the select is never a variable index into
-                // the register array, which would move it to scratch memory)
-                dispatch_mask<M>(zm, [&](auto zc) {
-                    double t = a[decltype(zc)::value].x;
-                    asm volatile("" : "+v"(t));
-                    w = t;
-                });
-                if (__popcll(j & T.z) & 1) w = -w;
-                acc = make_double2(fma(T.c.x, w, acc.x), fma(T.c.y, w, acc.y));
-            }
-            acc_s[diag * kEvTPB + threadIdx.x] = cadd(acc_s[diag * kEvTPB + threadIdx.x], acc);
-        }
+        const uint64_t j = load_orbit<M, NT>(a, psi, t, ob);
+        orbit_values<M>(a, j, groups, ngroups, diag, terms, [&](uint32_t g, double2 v) {
+            acc_s[g * kEvTPB + threadIdx.x] = cadd(acc_s[g * kEvTPB + threadIdx.x], v);
+        });
     }
     for (uint32_t g = 0; g < ngroups; ++g) {
         const double2 s = block_sum(acc_s[g * kEvTPB + threadIdx.x], lds);
@@ -604,43 +642,23 @@ static void cached_plan(const std::vector<PauliGroup>& groups, int maxdim, std::
     *lru = PlanEntry{maxdim, std::move(masks), passes, ++g_plan_clock};
 }
 
-template <int M>
-static void launch_orbit_expval_k(const double2* bra, const double2* ket, uint64_t norbit, const OrbitBasis& ob,
-                                  const OrbitGroup* dg, uint32_t ng, uint32_t diag, const OrbitTerm* dt,
-                                  double2* partial, uint32_t nb, bool nt, hipStream_t st) {
-    const size_t lds = (size_t)ng * kEvTPB * sizeof(double2);
-    if (bra == ket) {
-        if (nt)
-            hipLaunchKernelGGL((k_orbit_expval_same<M, true>), dim3(nb), dim3(kEvTPB), lds, st, ket, norbit, ob, dg, ng,
-                               diag, dt, partial, nb);
-        else
-            hipLaunchKernelGGL((k_orbit_expval_same<M, false>), dim3(nb), dim3(kEvTPB), lds, st, ket, norbit, ob, dg, ng,
-                               diag, dt, partial, nb);
-        return;
-    }
-    if constexpr (M <= kEvOrbitMax) {
-        const uint64_t* b = ob.b;
-        const uint32_t* piv = ob.p;
-        if (nt)
-            hipLaunchKernelGGL((k_orbit_expval<M, true>), dim3(nb), dim3(kEvTPB), lds, st, bra, ket, norbit, b[0], b[1],
-                               b[2], b[3], piv[0], piv[1], piv[2], piv[3], dg, ng, dt, partial, nb);
-        else
-            hipLaunchKernelGGL((k_orbit_expval<M, false>), dim3(nb), dim3(kEvTPB), lds, st, bra, ket, norbit, b[0], b[1],
-                               b[2], b[3], piv[0], piv[1], piv[2], piv[3], dg, ng, dt, partial, nb);
-    }
-}
-
 // One orbit expectation pass as planned on the host: its basis (pivots
 // ascending) and its run of OrbitGroup entries.
 struct OrbitLaunch {
-    int M;
     OrbitBasis ob;
     size_t g0, ng;
-    uint32_t diag;  // position of the first group with v = 0 in the pass, ng if none
+    uint32_t diag;  // position of the first group with v = 0 in the pass (they come last), ng if none
 };
 
 // Host tables of every pass: per pass its OrbitGroup run (slot = group index)
-// and OrbitTerm run, in pass order.
+// and OrbitTerm run, in pass order.  Passes of fewer than maxdim dimensions
+// (the last ones, or an operator of Z strings alone) are padded with single
+// qubits from kPadBit up: a thread of a 0-dimension pass would hold one
+// amplitude and evaluate every term for it (26.5 ms for 16 Z operators at 30
+// qubits; padded, the transform serves them all at the rate of a read of the
+// state).  From kPadBit on a wave's loads cover 64 consecutive amplitudes.
+constexpr int kPadBit = 6;
+static_assert(kEvOrbitMinQubits > kPadBit + 2 * kEvOrbitMaxSame, "enough qubits to pad with");
 static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std::vector<uint64_t>& zs,
                                const std::vector<double2>& cs, int maxdim, std::vector<OrbitGroup>& og,
                                std::vector<OrbitTerm>& ot, std::vector<OrbitLaunch>& launches) {
@@ -651,39 +669,50 @@ static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std:
     launches.clear();
     for (const EvPass& p : passes) {
         std::vector<uint64_t> b = p.basis;
+        for (int q = kPadBit; (int)b.size() < maxdim; ++q) {
+            bool pivot = false;
+            for (uint64_t v : b) pivot = pivot || 63 - __builtin_clzll(v) == q;
+            if (pivot) continue;
+            for (uint64_t& v : b) v &= ~(1ull << q);
+            b.push_back(1ull << q);
+        }
         std::sort(b.begin(), b.end(), [](uint64_t u, uint64_t v) { return __builtin_clzll(u) > __builtin_clzll(v); });
         OrbitLaunch L{};
-        L.M = (int)b.size();
-        for (int k = 0; k < L.M; ++k) {
+        const int M = maxdim;
+        for (int k = 0; k < M; ++k) {
             L.ob.b[k] = b[k];
             L.ob.p[k] = (uint32_t)(63 - __builtin_clzll(b[k]));
         }
         uint64_t coff[1 << kEvOrbitMaxSame];
-        for (int i = 0; i < (1 << L.M); ++i) {
+        for (int i = 0; i < (1 << M); ++i) {
             uint64_t c = 0;
-            for (int k = 0; k < L.M; ++k)
+            for (int k = 0; k < M; ++k)
                 if ((i >> k) & 1) c ^= b[k];
             coff[i] = c;
         }
         L.g0 = og.size();
         L.ng = p.groups.size();
-        L.diag = (uint32_t)L.ng;
-        for (uint32_t gi : p.groups) {
+        std::vector<uint32_t> order;  // diagonal groups last
+        for (uint32_t gi : p.groups)
+            if (groups[gi].x) order.push_back(gi);
+        L.diag = (uint32_t)order.size();
+        for (uint32_t gi : p.groups)
+            if (!groups[gi].x) order.push_back(gi);
+        for (uint32_t gi : order) {
             const PauliGroup& pg = groups[gi];
             OrbitGroup o{};
-            for (int k = 0; k < L.M; ++k)
+            for (int k = 0; k < M; ++k)
                 if ((pg.x >> L.ob.p[k]) & 1ull) o.v |= 1u << k;
             o.first = (uint32_t)ot.size();
             o.count = pg.count;
             o.slot = gi;
-            if (o.v == 0 && L.diag == L.ng) L.diag = (uint32_t)(og.size() - L.g0);
             og.push_back(o);
             for (uint32_t t = 0; t < pg.count; ++t) {
                 OrbitTerm T{};
                 T.z = zs[pg.first + t];
-                for (int i = 0; i < (1 << L.M); ++i)
+                for (int i = 0; i < (1 << M); ++i)
                     if (__builtin_popcountll(coff[i] & T.z) & 1) T.smask |= 1u << i;
-                for (int i = 0; i < (1 << L.M); ++i)
+                for (int i = 0; i < (1 << M); ++i)
                     if ((T.smask >> (i ^ o.v)) & 1u) T.pmask |= 1u << i;
                 T.c = cs[pg.first + t];
                 ot.push_back(T);
@@ -693,38 +722,60 @@ static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std:
     }
 }
 
-// Workgroups of an orbit expectation pass over 2^n amplitudes.
-static uint32_t orbit_expval_blocks(int n) {
-    uint64_t nb64 = (1ull << n) / 4096;
-    if (nb64 < 1) nb64 = 1;
-    if (nb64 > 2048) nb64 = 2048;
-    return (uint32_t)nb64;
+// Workgroups of an orbit expectation pass over 2^n amplitudes: one orbit per
+// thread up to kEvBlocksMax.
+constexpr uint64_t kEvBlocksMax = 2048;
+static uint32_t orbit_expval_blocks(int n, int maxdim) {
+    return (uint32_t)std::min<uint64_t>(kEvBlocksMax, std::max<uint64_t>(1, (1ull << n) >> maxdim >> 8));
 }
 
-static int launch_orbit_pass(const double2* bra, const double2* ket, int n, const OrbitLaunch& L,
-                             const OrbitGroup* dg, const OrbitTerm* dt, double2* partial, uint32_t nb) {
+// The passes [l0, l1).
+static int launch_orbit_passes(const double2* bra, const double2* ket, int n, const std::vector<OrbitLaunch>& launches,
+                               size_t l0, size_t l1, const OrbitPass* dp, const OrbitGroup* dg, const OrbitTerm* dt,
+                               double2* partial, uint32_t nb) {
     Context& cx = ctx();
     const uint64_t N = 1ull << n;
-    const uint64_t norbit = N >> L.M;
-    const OrbitGroup* g = dg + L.g0;
-    const uint32_t ng = (uint32_t)L.ng;
-    const bool nt = use_nt(n, L.M == 0 ? 63u : L.ob.p[0]);  // pivots ascending
-    if (L.M > (bra == ket ? kEvOrbitMaxSame : kEvOrbitMax))
-        return fail(QFE_ERR_STATE, "internal: expectation orbit dimension out of range");
-    switch (L.M) {
-        case 0: launch_orbit_expval_k<0>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        case 1: launch_orbit_expval_k<1>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        case 2: launch_orbit_expval_k<2>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        case 3: launch_orbit_expval_k<3>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        case 4: launch_orbit_expval_k<4>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        case 5: launch_orbit_expval_k<5>(bra, ket, norbit, L.ob, g, ng, L.diag, dt, partial, nb, nt, cx.stream); break;
-        default: return fail(QFE_ERR_STATE, "internal: expectation orbit dimension out of range");
+    const bool same = bra == ket;
+    const uint64_t norbit = N >> (same ? kEvOrbitMaxSame : kEvOrbitMax);
+    const bool once = same && n < kNtMinQubits && norbit <= (uint64_t)nb * kEvTPB && l1 - l0 <= 65535;
+    if (once && l1 > l0)
+        hipLaunchKernelGGL(k_orbit_expval_once<kEvOrbitMaxSame>, dim3(nb, (unsigned)(l1 - l0)), dim3(kEvTPB), 0, cx.stream,
+                           ket, norbit, dp + l0, dg, dt, partial, nb);
+    for (size_t l = l0; l < l1; ++l) {
+        const OrbitLaunch& L = launches[l];
+        const OrbitGroup* g = dg + L.g0;
+        const uint32_t ng = (uint32_t)L.ng;
+        const size_t lds = (size_t)ng * kEvTPB * sizeof(double2);
+        const bool nt = !once && use_nt(n, L.ob.p[0]);  // pivots ascending
+        const uint64_t* b = L.ob.b;
+        const uint32_t* piv = L.ob.p;
+        if (once) {
+        } else if (same && nt) {
+            hipLaunchKernelGGL((k_orbit_expval_same<kEvOrbitMaxSame, true>), dim3(nb), dim3(kEvTPB), lds, cx.stream, ket,
+                               norbit, L.ob, g, ng, L.diag, dt, partial, nb);
+        } else if (same) {
+            hipLaunchKernelGGL((k_orbit_expval_same<kEvOrbitMaxSame, false>), dim3(nb), dim3(kEvTPB), lds, cx.stream, ket,
+                               norbit, L.ob, g, ng, L.diag, dt, partial, nb);
+        } else if (nt) {
+            hipLaunchKernelGGL((k_orbit_expval<kEvOrbitMax, true>), dim3(nb), dim3(kEvTPB), lds, cx.stream, bra, ket, norbit,
+                               b[0], b[1], b[2], b[3], piv[0], piv[1], piv[2], piv[3], g, ng, dt, partial, nb);
+        } else {
+            hipLaunchKernelGGL((k_orbit_expval<kEvOrbitMax, false>), dim3(nb), dim3(kEvTPB), lds, cx.stream, bra, ket, norbit,
+                               b[0], b[1], b[2], b[3], piv[0], piv[1], piv[2], piv[3], g, ng, dt, partial, nb);
+        }
+        QFE_HIP(hipGetLastError());
+        cx.counters.reduce++;
+        cx.counters.nt += nt ? 1 : 0;
+        cx.counters.bytes += (same ? 16.0 : 32.0) * (double)N;
     }
-    QFE_HIP(hipGetLastError());
-    cx.counters.reduce++;
-    cx.counters.nt += nt ? 1 : 0;
-    cx.counters.bytes += (bra == ket ? 16.0 : 32.0) * (double)N;
     return QFE_OK;
+}
+
+// Device views of the passes.
+static std::vector<OrbitPass> orbit_pass_table(const std::vector<OrbitLaunch>& launches) {
+    std::vector<OrbitPass> out;
+    for (const OrbitLaunch& L : launches) out.push_back(OrbitPass{L.ob, (uint32_t)L.g0, (uint32_t)L.ng, L.diag, 0});
+    return out;
 }
 
 static int expval_groups_orbit(const double2* bra, const double2* ket, int n, const std::vector<PauliGroup>& groups,
@@ -732,34 +783,37 @@ static int expval_groups_orbit(const double2* bra, const double2* ket, int n, co
                                double2* out_per_group) {
     Context& cx = ctx();
     const size_t G = groups.size();
-    const uint32_t nb = orbit_expval_blocks(n);
+    const int maxdim = bra == ket ? kEvOrbitMaxSame : kEvOrbitMax;
+    const uint32_t nb = orbit_expval_blocks(n, maxdim);
     std::vector<OrbitGroup> og;
     std::vector<OrbitTerm> ot;
     std::vector<OrbitLaunch> launches;
-    build_orbit_tables(groups, zs, cs, bra == ket ? kEvOrbitMaxSame : kEvOrbitMax, og, ot, launches);
+    build_orbit_tables(groups, zs, cs, maxdim, og, ot, launches);
+    const std::vector<OrbitPass> op = orbit_pass_table(launches);
     const size_t b_g = align256(og.size() * sizeof(OrbitGroup));
     const size_t b_t = align256(ot.size() * sizeof(OrbitTerm));
+    const size_t b_p = align256(op.size() * sizeof(OrbitPass));
     const size_t b_part = align256(G * (size_t)nb * sizeof(double2));
     const size_t b_out = align256(G * sizeof(double2));
+    const size_t b_tab = b_g + b_t + b_p;
     void* scr = nullptr;
-    int rc = scratch_reserve(b_g + b_t + b_part + b_out, &scr);
+    int rc = scratch_reserve(b_tab + b_part + b_out, &scr);
     if (rc) return rc;
     char* base = static_cast<char*>(scr);
     char* host = nullptr;
-    rc = staging_begin(b_g + b_t, reinterpret_cast<void**>(&host));
+    rc = staging_begin(b_tab, reinterpret_cast<void**>(&host));
     if (rc) return rc;
     std::memcpy(host, og.data(), og.size() * sizeof(OrbitGroup));
     std::memcpy(host + b_g, ot.data(), ot.size() * sizeof(OrbitTerm));
-    rc = staging_commit(base, b_g + b_t);
+    std::memcpy(host + b_g + b_t, op.data(), op.size() * sizeof(OrbitPass));
+    rc = staging_commit(base, b_tab);
     if (rc) return rc;
-    const OrbitGroup* dg = reinterpret_cast<const OrbitGroup*>(base);
-    const OrbitTerm* dt = reinterpret_cast<const OrbitTerm*>(base + b_g);
-    double2* partial = reinterpret_cast<double2*>(base + b_g + b_t);
-    double2* dout = reinterpret_cast<double2*>(base + b_g + b_t + b_part);
-    for (const OrbitLaunch& L : launches) {
-        rc = launch_orbit_pass(bra, ket, n, L, dg, dt, partial, nb);
-        if (rc) return rc;
-    }
+    double2* partial = reinterpret_cast<double2*>(base + b_tab);
+    double2* dout = reinterpret_cast<double2*>(base + b_tab + b_part);
+    rc = launch_orbit_passes(bra, ket, n, launches, 0, launches.size(), reinterpret_cast<const OrbitPass*>(base + b_g + b_t),
+                             reinterpret_cast<const OrbitGroup*>(base), reinterpret_cast<const OrbitTerm*>(base + b_g),
+                             partial, nb);
+    if (rc) return rc;
     hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)G), dim3(kEvTPB), 0, cx.stream, partial, nb, dout);
     QFE_HIP(hipGetLastError());
     void* pin = nullptr;
@@ -878,18 +932,21 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
         cx.counters.bytes += (bra == ket ? 16.0 : 32.0) * (double)(1ull << n) * (double)G;
         return QFE_OK;
     }
-    const uint32_t nb = orbit_expval_blocks(n);
+    const int maxdim = bra == ket ? kEvOrbitMaxSame : kEvOrbitMax;
+    const uint32_t nb = orbit_expval_blocks(n, maxdim);
     std::vector<OrbitGroup> og;
     std::vector<OrbitTerm> ot;
     std::vector<OrbitLaunch> launches;
-    build_orbit_tables(groups, zs, cs, bra == ket ? kEvOrbitMaxSame : kEvOrbitMax, og, ot, launches);
+    build_orbit_tables(groups, zs, cs, maxdim, og, ot, launches);
+    const std::vector<OrbitPass> op = orbit_pass_table(launches);
     char* dg = A.take(og.size() * sizeof(OrbitGroup));
     char* dt = A.take(ot.size() * sizeof(OrbitTerm));
+    char* dp = A.take(op.size() * sizeof(OrbitPass));
     char* dout = A.take(G * sizeof(double2));
     const size_t row = (size_t)nb * sizeof(double2);
-    const size_t window = (A.cap - A.used) / row;  // groups whose partials fit at once
+    const size_t window = dp && dout ? (A.cap - A.used) / row : 0;  // groups whose partials fit at once
     char* part = A.take(window * row);
-    if (!dg || !dt || !dout || !part || window < (size_t)kEvOrbitGroups)
+    if (!dg || !dt || !dp || !dout || !part || window < (size_t)kEvOrbitGroups)
         return fail(QFE_ERR_ARG, "qfe_expval_noalloc: operator exceeds the fixed scratch");
     // window-local output rows: whole passes in order, slot = position in the
     // window (build_orbit_tables left the group index in slot)
@@ -907,14 +964,13 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
     win_start.push_back(launches.size());
     QFE_HIP(hipMemcpyAsync(dg, og.data(), og.size() * sizeof(OrbitGroup), hipMemcpyHostToDevice, cx.stream));
     QFE_HIP(hipMemcpyAsync(dt, ot.data(), ot.size() * sizeof(OrbitTerm), hipMemcpyHostToDevice, cx.stream));
+    QFE_HIP(hipMemcpyAsync(dp, op.data(), op.size() * sizeof(OrbitPass), hipMemcpyHostToDevice, cx.stream));
     for (size_t w = 0; w + 1 < win_start.size(); ++w) {
         const size_t l0 = win_start[w], l1 = win_start[w + 1];
         const size_t g0 = launches[l0].g0, g1 = launches[l1 - 1].g0 + launches[l1 - 1].ng;
-        for (size_t l = l0; l < l1; ++l) {
-            int rc = launch_orbit_pass(bra, ket, n, launches[l], (const OrbitGroup*)dg, (const OrbitTerm*)dt,
-                                       (double2*)part, nb);
-            if (rc) return rc;
-        }
+        int rc = launch_orbit_passes(bra, ket, n, launches, l0, l1, (const OrbitPass*)dp, (const OrbitGroup*)dg,
+                                     (const OrbitTerm*)dt, (double2*)part, nb);
+        if (rc) return rc;
         hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)(g1 - g0)), dim3(kEvTPB), 0, cx.stream, (const double2*)part,
                            nb, (double2*)dout + g0);
         QFE_HIP(hipGetLastError());

@@ -360,25 +360,6 @@ __device__ __forceinline__ void add_mul(double2& t, double2 a, double2 b) {
 __device__ __forceinline__ void add_mul(double& t, double a, double b) { t += a * b; }
 
 // ---- 2. ansatz and reverse sweep: component tiles ---------------------------------------
-// v + the value CTRL lanes away (0 where there is none).
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
-    return v + __hiloint2double(hi, lo);
-}
-// Sum over the 64 lanes in a fixed order, in lane 63: four row shifts and two
-// row broadcasts on the vector pipe, where __shfl_xor goes through LDS.
-__device__ __forceinline__ double wave_sum_last(double v) {
-    v = dpp_add<0x111>(v);  // row_shr:1
-    v = dpp_add<0x112>(v);  // row_shr:2
-    v = dpp_add<0x114>(v);  // row_shr:4
-    v = dpp_add<0x118>(v);  // row_shr:8
-    v = dpp_add<0x142>(v);  // row_bcast:15
-    v = dpp_add<0x143>(v);  // row_bcast:31
-    return v;
-}
-
 constexpr uint32_t kRecChunk = 128;        // records staged in LDS at a time
 constexpr uint32_t kTileWordsLds = 4096;   // list words of a tile staged in LDS when they fit
 
