@@ -68,6 +68,9 @@ struct Context {
     // reusable device scratch for reductions and op descriptors
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    // partial outputs of apply_pauli_sum on small states (at most 64 MiB)
+    void* slices = nullptr;
+    size_t slice_bytes = 0;
     // pinned host staging for small results
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -76,6 +79,7 @@ struct Context {
 Context& ctx();
 int ensure_init();
 int scratch_reserve(size_t bytes, void** out);
+int slice_reserve(size_t bytes, void** out);
 int pinned_reserve(size_t bytes, void** out);
 // Double-buffered pinned staging: fill *host (bytes), then commit copies it to
 // dev on the library stream without blocking the host.

@@ -58,25 +58,25 @@ void group_terms(const qfe_pauli* terms, uint64_t count, std::vector<PauliGroup>
 
 constexpr int kEvTPB = 256;
 
-// f(j) = sum_t c_t (-1)^popcount(j & z_t)
-__device__ __forceinline__ double2 group_f(uint64_t j, const uint64_t* __restrict__ zs, const double2* __restrict__ cs,
-                                           uint32_t count) {
-    double2 f = make_double2(0.0, 0.0);
-    for (uint32_t t = 0; t < count; ++t) {
-        const double2 c = cs[t];
-        if (__popcll(j & zs[t]) & 1) {
-            f.x -= c.x;
-            f.y -= c.y;
-        } else {
-            f.x += c.x;
-            f.y += c.y;
-        }
-    }
-    return f;
+// v with its sign bit flipped when bit 31 of neg is set.
+__device__ __forceinline__ double sign_flip(double v, uint32_t neg) {
+    return __hiloint2double(__double2hiint(v) ^ (int)(neg & 0x80000000u), __double2loint(v));
 }
+__device__ __forceinline__ uint32_t odd_bit(uint32_t v) { return (uint32_t)__popc(v) << 31; }
+__device__ __forceinline__ uint32_t odd_bit(uint64_t v) { return (uint32_t)__popcll(v) << 31; }
+
+constexpr uint32_t kEvTerms = 256;  // terms of a group staged in LDS at a time
+constexpr int kEvPer = 4;           // amplitudes or pairs per thread and staged term
 
 // One block = (group g, chunk ch).  Pairs of group g are split into nchunk
-// equal contiguous ranges.
+// equal contiguous ranges.  W: word that holds an index (uint32_t up to 32
+// qubits).  The group's terms come through LDS and each is read once for
+// kEvPer pairs per thread.  In one state (SAME) a term's signs on a pair
+// differ by a uniform sigma = (-1)^{|x & z|}, so with p = conj(a_ja) a_jb the
+// pair gives 2 s c Re p (sigma = +1) or -2i s c Im p (sigma = -1), s the sign
+// on ja: one sign per pair and term, where both ends and complex products were
+// evaluated before (18-qubit molecule, 9316 terms: 788 us).
+template <typename W, bool SAME>
 __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restrict__ bra,
                                                           const double2* __restrict__ ket, int n,
                                                           const PauliGroup* __restrict__ groups,
@@ -84,37 +84,94 @@ __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restr
                                                           const double2* __restrict__ cs, uint32_t nchunk,
                                                           double2* __restrict__ partial) {
     __shared__ double2 lds[16];
+    __shared__ W zt[kEvTerms];
+    __shared__ double2 ct[kEvTerms];
     const uint32_t g = blockIdx.x / nchunk;
     const uint32_t ch = blockIdx.x % nchunk;
     const PauliGroup G = groups[g];
     const uint64_t* z = zs + G.first;
     const double2* c = cs + G.first;
+    const bool diag = G.x == 0;
+    const W x = (W)G.x;
+    const uint64_t P = diag ? 1ull << n : 1ull << (n - 1);
+    const uint64_t per = (P + nchunk - 1) / nchunk;
+    const uint64_t b0 = (uint64_t)ch * per, e0 = min(P, b0 + per);
     double2 acc = make_double2(0.0, 0.0);
-    if (G.x == 0) {
-        const uint64_t N = 1ull << n;
-        const uint64_t per = (N + nchunk - 1) / nchunk;
-        const uint64_t b0 = (uint64_t)ch * per;
-        const uint64_t e0 = b0 + per < N ? b0 + per : N;
-        for (uint64_t j = b0 + threadIdx.x; j < e0; j += kEvTPB) {
-            const double2 p = cconjmul(bra[j], ket[j]);
-            acc = cadd(acc, cmul(p, group_f(j, z, c, G.count)));
+    for (uint32_t t0 = 0; t0 < G.count; t0 += kEvTerms) {
+        const uint32_t nt = min(kEvTerms, G.count - t0);
+        __syncthreads();
+        bool cplx = false;
+        for (uint32_t t = threadIdx.x; t < nt; t += kEvTPB) {
+            zt[t] = (W)z[t0 + t];
+            ct[t] = c[t0 + t];
+            cplx |= ct[t].y != 0.0;
         }
-    } else {
-        const uint64_t P = 1ull << (n - 1);
-        const uint64_t per = (P + nchunk - 1) / nchunk;
-        const uint64_t b0 = (uint64_t)ch * per;
-        const uint64_t e0 = b0 + per < P ? b0 + per : P;
-        for (uint64_t k = b0 + threadIdx.x; k < e0; k += kEvTPB) {
-            const uint64_t ja = ins0(k, G.hb);
-            const uint64_t jb = ja ^ G.x;
-            const double2 ab = cconjmul(bra[ja], ket[jb]);
-            const double2 ba = cconjmul(bra[jb], ket[ja]);
-            acc = cadd(acc, cmul(ab, group_f(jb, z, c, G.count)));
-            acc = cadd(acc, cmul(ba, group_f(ja, z, c, G.count)));
+        const bool real = !__syncthreads_or(cplx);  // real coefficients: half the sums
+        for (uint64_t k0 = b0 + threadIdx.x; k0 < e0; k0 += kEvPer * kEvTPB) {
+            W ja[kEvPer];
+            double2 p[kEvPer], q[kEvPer], f[kEvPer], h[kEvPer];
+#pragma unroll
+            for (int u = 0; u < kEvPer; ++u) {
+                const uint64_t k = k0 + (uint64_t)u * kEvTPB;
+                const uint64_t j = diag ? k : ins0(k, G.hb);
+                const bool on = k < e0;
+                ja[u] = (W)j;
+                f[u] = h[u] = make_double2(0.0, 0.0);
+                p[u] = on ? cconjmul(bra[j], ket[j ^ G.x]) : make_double2(0.0, 0.0);
+                if (!SAME) q[u] = on && !diag ? cconjmul(bra[j ^ G.x], ket[j]) : make_double2(0.0, 0.0);
+            }
+            auto sum_terms = [&](auto real_c) {
+                constexpr bool REAL = decltype(real_c)::value;
+                for (uint32_t t = 0; t < nt; ++t) {
+                    const W zz = zt[t];
+                    const double2 cc = ct[t];
+                    const uint32_t sx = odd_bit((W)(x & zz));
+                    auto add = [&](double2(&to)[kEvPer], uint32_t flip) {
+#pragma unroll
+                        for (int u = 0; u < kEvPer; ++u) {
+                            const uint32_t s = odd_bit((W)(ja[u] & zz)) ^ flip;
+                            to[u].x += sign_flip(cc.x, s);
+                            if (!REAL) to[u].y += sign_flip(cc.y, s);
+                        }
+                    };
+                    if (SAME && (sx >> 31)) {  // uniform over the block
+                        add(h, 0u);
+                    } else {
+                        add(f, 0u);
+                        if (!SAME) add(h, sx);
+                    }
+                }
+            };
+            if (real)
+                sum_terms(std::true_type{});
+            else
+                sum_terms(std::false_type{});
+#pragma unroll
+            for (int u = 0; u < kEvPer; ++u) {
+                if (!SAME) {
+                    // conj(bra_ja) ket_jb f(jb) + conj(bra_jb) ket_ja f(ja); a diagonal group has the first alone
+                    acc = cadd(acc, cadd(cmul(p[u], h[u]), cmul(q[u], f[u])));
+                } else if (diag) {
+                    acc = cadd(acc, cmul(p[u], f[u]));
+                } else {
+                    const double re = 2.0 * p[u].x, im = 2.0 * p[u].y;
+                    acc = make_double2(fma(re, f[u].x, fma(im, h[u].y, acc.x)), fma(re, f[u].y, fma(-im, h[u].x, acc.y)));
+                }
+            }
         }
     }
     acc = block_sum(acc, lds);
     if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+}
+
+static void launch_expval_kernel(const double2* bra, const double2* ket, int n, const PauliGroup* dg, uint32_t ngroups,
+                                 const uint64_t* dz, const double2* dc, uint32_t nchunk, double2* partial) {
+    const dim3 grid((unsigned)((uint64_t)ngroups * nchunk));
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kEvTPB), 0, ctx().stream, bra, ket, n, dg, dz, dc, nchunk, partial); };
+    if (n <= 32)
+        bra == ket ? go(k_expval_groups<uint32_t, true>) : go(k_expval_groups<uint32_t, false>);
+    else
+        bra == ket ? go(k_expval_groups<uint64_t, true>) : go(k_expval_groups<uint64_t, false>);
 }
 
 __global__ __launch_bounds__(kEvTPB) void k_sum_groups(const double2* __restrict__ partial, uint32_t nchunk,
@@ -127,9 +184,8 @@ __global__ __launch_bounds__(kEvTPB) void k_sum_groups(const double2* __restrict
     if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
-__global__ void k_apply_sum(const double2* __restrict__ in, double2* __restrict__ out, uint64_t N,
-                            const PauliGroup* __restrict__ groups, uint32_t ngroups, const uint64_t* __restrict__ zs,
-                            const double2* __restrict__ cs);
+static int launch_apply_sum_kernel(const double2* in, double2* out, int n, const PauliGroup* dg, uint32_t ngroups,
+                                   const uint64_t* dz, const double2* dc);
 
 // Upload groups/terms into device scratch after `reserved` bytes; returns pointers.
 struct GroupDev {
@@ -164,10 +220,12 @@ static int upload_groups(const std::vector<PauliGroup>& groups, const std::vecto
 }
 
 static uint32_t chunks_for(int n, size_t ngroups) {
-    // aim for ~4096 pairs per block, at most 1024 chunks per group, and keep
-    // the partials array bounded
+    // 4096 pairs per block, or fewer (down to one staged term's 1024) while the
+    // launch has less than four blocks per CU; at most 1024 chunks per group,
+    // and the partials array bounded
     const uint64_t P = 1ull << (n > 0 ? n - 1 : 0);
     uint64_t ch = (P + 4095) / 4096;
+    while (ch * 1024 < P && ch * ngroups < 1024) ch <<= 1;
     if (ch > 1024) ch = 1024;
     if (ch < 1) ch = 1;
     while (ch > 1 && ch * ngroups > (1ull << 22)) ch >>= 1;
@@ -181,8 +239,7 @@ int launch_expval_async(const double2* bra, const double2* ket, int n, const Pau
                         double2* dout) {
     Context& cx = ctx();
     if (ngroups == 0) return QFE_OK;
-    hipLaunchKernelGGL(k_expval_groups, dim3((unsigned)((uint64_t)ngroups * nchunk)), dim3(kEvTPB), 0, cx.stream, bra,
-                       ket, n, dgroups, dzs, dcs, nchunk, partial);
+    launch_expval_kernel(bra, ket, n, dgroups, ngroups, dzs, dcs, nchunk, partial);
     QFE_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_groups, dim3(ngroups), dim3(kEvTPB), 0, cx.stream, partial, nchunk, dout);
     QFE_HIP(hipGetLastError());
@@ -196,9 +253,8 @@ int launch_apply_sum_async(const double2* in, double2* out, int n, const PauliGr
     Context& cx = ctx();
     const uint64_t N = 1ull << n;
     if (ngroups == 0) return launch_zero(out, N, cx.stream);
-    hipLaunchKernelGGL(k_apply_sum, dim3((unsigned)((N + kEvTPB - 1) / kEvTPB)), dim3(kEvTPB), 0, cx.stream, in, out,
-                       N, dgroups, ngroups, dzs, dcs);
-    QFE_HIP(hipGetLastError());
+    int rc = launch_apply_sum_kernel(in, out, n, dgroups, ngroups, dzs, dcs);
+    if (rc) return rc;
     cx.counters.single++;
     cx.counters.bytes += 16.0 * (double)N * (double)(ngroups + 1);
     return QFE_OK;
@@ -217,12 +273,19 @@ constexpr int kEvOrbitMax = 4;
 // their products leaves them memory-bound at 5 dimensions.
 constexpr int kEvOrbitMaxSame = 5;
 static_assert((1 << kEvOrbitMaxSame) <= 32, "OrbitTerm sign masks hold 32 elements");
-// Smallest state that takes orbit passes: below it one launch over every
-// group (a read of the state per group) is faster than the chain of orbit
-// passes, whose workgroups then cover too little of the state (measured on
-// MI355X, 200 and 1000 random terms: 0.25 vs 0.50 and 0.96 vs 1.91 ms at 20
-// qubits, 1.25 vs 0.89 and 5.2 vs 3.5 ms at 22).
+// Smallest state whose cross expectation values take orbit passes: below it
+// one launch over every group (a read of the states per group) is faster than
+// the chain of passes, whose workgroups then cover too little of the state
+// (200 and 1000 random terms: 0.25 vs 0.50 and 0.96 vs 1.91 ms at 20 qubits,
+// 1.25 vs 0.89 and 5.2 vs 3.5 ms at 22).
 constexpr int kEvOrbitMinQubits = 21;
+// Smallest state whose plain expectation values take them in one launch: below
+// it the groups' own reads of the state are cheap (200 random terms, group
+// launch / passes in us per call: 60 / 63 at 12 qubits, 72 / 74 at 15, 87 / 74
+// at 16, 100 / 76 at 18, 242 / 102 at 20; at 18 qubits the 1621 masks of a
+// molecule read 6.8 GB from the caches, 522 us, against 0.9 GB in passes).
+constexpr int kEvOnceMinQubits = 16;
+static bool takes_orbits(int n, bool same) { return n >= (same ? kEvOnceMinQubits : kEvOrbitMinQubits); }
 constexpr int kEvOrbitGroups = 16;
 
 struct OrbitGroup {
@@ -600,6 +663,42 @@ void plan_expval(const std::vector<PauliGroup>& groups, int maxdim, std::vector<
     }
 }
 
+// The same for states whose passes share a launch: a pass costs a read from
+// the caches there, so the groups are taken in order, each pass looking at the
+// next kQuickWindow of them (1621 masks of an 18-qubit molecule: 221 passes;
+// 195 with no window).
+constexpr size_t kQuickWindow = 256;
+static void plan_expval_quick(const std::vector<PauliGroup>& groups, int maxdim, std::vector<EvPass>& passes) {
+    std::vector<uint32_t> rem(groups.size());
+    for (size_t g = 0; g < groups.size(); ++g) rem[g] = (uint32_t)g;
+    size_t begin = 0;  // rem[begin..] remain, in order
+    while (begin < rem.size()) {
+        EvPass p;
+        const size_t end = std::min(rem.size(), begin + kQuickWindow);
+        size_t i = begin;
+        std::vector<uint32_t> skip;
+        for (; i < end && p.groups.size() < (size_t)kEvOrbitGroups; ++i) {
+            uint64_t r = groups[rem[i]].x;
+            for (uint64_t v : p.basis)
+                if ((r >> (63 - __builtin_clzll(v))) & 1ull) r ^= v;
+            if (r && (int)p.basis.size() >= maxdim) {
+                skip.push_back(rem[i]);
+                continue;
+            }
+            if (r) {
+                const int piv = 63 - __builtin_clzll(r);
+                for (uint64_t& v : p.basis)
+                    if ((v >> piv) & 1ull) v ^= r;
+                p.basis.push_back(r);
+            }
+            p.groups.push_back(rem[i]);
+        }
+        begin = i - skip.size();  // the groups not taken move up to the rest
+        std::copy(skip.begin(), skip.end(), rem.begin() + begin);
+        passes.push_back(std::move(p));
+    }
+}
+
 // Plans of the last few operators, keyed by their X masks in group order:
 // callers that evaluate one operator many times (a variational loop, a step
 // of a benchmark) plan it once.  Planning 647 masks takes about 2 ms on the
@@ -607,6 +706,7 @@ void plan_expval(const std::vector<PauliGroup>& groups, int maxdim, std::vector<
 namespace {
 struct PlanEntry {
     int maxdim = 0;
+    bool quick = false;
     std::vector<uint64_t> masks;
     std::vector<EvPass> passes;
     uint64_t used = 0;
@@ -617,29 +717,32 @@ uint64_t g_plan_clock = 0;
 constexpr size_t kPlanCacheEntries = 8;
 }  // namespace
 
-static void cached_plan(const std::vector<PauliGroup>& groups, int maxdim, std::vector<EvPass>& passes) {
+static void cached_plan(const std::vector<PauliGroup>& groups, int maxdim, bool quick, std::vector<EvPass>& passes) {
     std::vector<uint64_t> masks(groups.size());
     for (size_t g = 0; g < groups.size(); ++g) masks[g] = groups[g].x;
     {
         std::lock_guard<std::mutex> lk(g_plan_mu);
         for (PlanEntry& e : g_plans)
-            if (e.maxdim == maxdim && e.masks == masks) {
+            if (e.maxdim == maxdim && e.quick == quick && e.masks == masks) {
                 e.used = ++g_plan_clock;
                 passes = e.passes;
                 return;
             }
     }
     passes.clear();
-    plan_expval(groups, maxdim, passes);
+    if (quick)
+        plan_expval_quick(groups, maxdim, passes);
+    else
+        plan_expval(groups, maxdim, passes);
     std::lock_guard<std::mutex> lk(g_plan_mu);
     if (g_plans.size() < kPlanCacheEntries) {
-        g_plans.push_back(PlanEntry{maxdim, std::move(masks), passes, ++g_plan_clock});
+        g_plans.push_back(PlanEntry{maxdim, quick, std::move(masks), passes, ++g_plan_clock});
         return;
     }
     PlanEntry* lru = &g_plans[0];
     for (PlanEntry& e : g_plans)
         if (e.used < lru->used) lru = &e;
-    *lru = PlanEntry{maxdim, std::move(masks), passes, ++g_plan_clock};
+    *lru = PlanEntry{maxdim, quick, std::move(masks), passes, ++g_plan_clock};
 }
 
 // One orbit expectation pass as planned on the host: its basis (pivots
@@ -658,18 +761,23 @@ struct OrbitLaunch {
 // qubits; padded, the transform serves them all at the rate of a read of the
 // state).  From kPadBit on a wave's loads cover 64 consecutive amplitudes.
 constexpr int kPadBit = 6;
-static_assert(kEvOrbitMinQubits > kPadBit + 2 * kEvOrbitMaxSame, "enough qubits to pad with");
+static_assert(kEvOnceMinQubits >= kPadBit + kEvOrbitMaxSame, "enough qubits to pad with");
 static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std::vector<uint64_t>& zs,
-                               const std::vector<double2>& cs, int maxdim, std::vector<OrbitGroup>& og,
+                               const std::vector<double2>& cs, int n, int maxdim, std::vector<OrbitGroup>& og,
                                std::vector<OrbitTerm>& ot, std::vector<OrbitLaunch>& launches) {
     std::vector<EvPass> passes;
-    cached_plan(groups, maxdim, passes);
+    uint32_t linear[1 << kEvOrbitMaxSame] = {};  // bit i of linear[m]: parity of i & m
+    const uint32_t linear_all = (uint32_t)((1ull << (1 << maxdim)) - 1ull);
+    for (uint32_t m = 0; m < (1u << maxdim); ++m)
+        for (uint32_t i = 0; i < (1u << maxdim); ++i) linear[m] |= (uint32_t)(__builtin_popcount(i & m) & 1) << i;
+    cached_plan(groups, maxdim, n < kEvOrbitMinQubits, passes);
     og.clear();
     ot.clear();
     launches.clear();
     for (const EvPass& p : passes) {
         std::vector<uint64_t> b = p.basis;
-        for (int q = kPadBit; (int)b.size() < maxdim; ++q) {
+        for (int k = 0; (int)b.size() < maxdim; ++k) {
+            const int q = (kPadBit + k) % n;
             bool pivot = false;
             for (uint64_t v : b) pivot = pivot || 63 - __builtin_clzll(v) == q;
             if (pivot) continue;
@@ -682,13 +790,6 @@ static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std:
         for (int k = 0; k < M; ++k) {
             L.ob.b[k] = b[k];
             L.ob.p[k] = (uint32_t)(63 - __builtin_clzll(b[k]));
-        }
-        uint64_t coff[1 << kEvOrbitMaxSame];
-        for (int i = 0; i < (1 << M); ++i) {
-            uint64_t c = 0;
-            for (int k = 0; k < M; ++k)
-                if ((i >> k) & 1) c ^= b[k];
-            coff[i] = c;
         }
         L.g0 = og.size();
         L.ng = p.groups.size();
@@ -710,10 +811,11 @@ static void build_orbit_tables(const std::vector<PauliGroup>& groups, const std:
             for (uint32_t t = 0; t < pg.count; ++t) {
                 OrbitTerm T{};
                 T.z = zs[pg.first + t];
-                for (int i = 0; i < (1 << M); ++i)
-                    if (__builtin_popcountll(coff[i] & T.z) & 1) T.smask |= 1u << i;
-                for (int i = 0; i < (1 << M); ++i)
-                    if ((T.smask >> (i ^ o.v)) & 1u) T.pmask |= 1u << i;
+                // signs are linear in the element index: bit k of zm is the sign of basis vector k
+                uint32_t zm = 0;
+                for (int k = 0; k < M; ++k) zm |= (uint32_t)(__builtin_popcountll(b[k] & T.z) & 1) << k;
+                T.smask = linear[zm];
+                T.pmask = T.smask ^ (__builtin_popcount(zm & o.v) & 1 ? linear_all : 0u);
                 T.c = cs[pg.first + t];
                 ot.push_back(T);
             }
@@ -788,7 +890,7 @@ static int expval_groups_orbit(const double2* bra, const double2* ket, int n, co
     std::vector<OrbitGroup> og;
     std::vector<OrbitTerm> ot;
     std::vector<OrbitLaunch> launches;
-    build_orbit_tables(groups, zs, cs, maxdim, og, ot, launches);
+    build_orbit_tables(groups, zs, cs, n, maxdim, og, ot, launches);
     const std::vector<OrbitPass> op = orbit_pass_table(launches);
     const size_t b_g = align256(og.size() * sizeof(OrbitGroup));
     const size_t b_t = align256(ot.size() * sizeof(OrbitTerm));
@@ -830,7 +932,7 @@ int expval_groups(const double2* bra, const double2* ket, int n, const std::vect
     Context& cx = ctx();
     const size_t G = groups.size();
     if (G == 0) return QFE_OK;
-    if (n >= kEvOrbitMinQubits) return expval_groups_orbit(bra, ket, n, groups, zs, cs, out_per_group);
+    if (takes_orbits(n, bra == ket)) return expval_groups_orbit(bra, ket, n, groups, zs, cs, out_per_group);
     const uint32_t nchunk = chunks_for(n, G);
     const size_t b_part = align256(G * nchunk * sizeof(double2));
     const size_t b_out = align256(G * sizeof(double2));
@@ -839,10 +941,7 @@ int expval_groups(const double2* bra, const double2* ket, int n, const std::vect
     if (rc) return rc;
     double2* partial = reinterpret_cast<double2*>(gd.tail);
     double2* dout = reinterpret_cast<double2*>(gd.tail + b_part);
-    // launch in slices to keep the grid below 2^31 blocks
-    const uint64_t total_blocks = (uint64_t)G * nchunk;
-    hipLaunchKernelGGL(k_expval_groups, dim3((unsigned)total_blocks), dim3(kEvTPB), 0, cx.stream, bra, ket, n,
-                       gd.groups, gd.zs, gd.cs, nchunk, partial);
+    launch_expval_kernel(bra, ket, n, gd.groups, (uint32_t)G, gd.zs, gd.cs, nchunk, partial);
     QFE_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)G), dim3(kEvTPB), 0, cx.stream, partial, nchunk, dout);
     QFE_HIP(hipGetLastError());
@@ -908,7 +1007,7 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
     if (G == 0) return QFE_OK;
     FixedLayout A{static_cast<char*>(dev_scratch), kNoAllocBytes};
     std::vector<double2> res(G);
-    if (n < kEvOrbitMinQubits) {
+    if (!takes_orbits(n, bra == ket)) {
         const uint32_t nchunk = chunks_for(n, G);
         char* dg = A.take(G * sizeof(PauliGroup));
         char* dz = A.take(zs.size() * sizeof(uint64_t));
@@ -919,8 +1018,8 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
         QFE_HIP(hipMemcpyAsync(dg, groups.data(), G * sizeof(PauliGroup), hipMemcpyHostToDevice, cx.stream));
         QFE_HIP(hipMemcpyAsync(dz, zs.data(), zs.size() * sizeof(uint64_t), hipMemcpyHostToDevice, cx.stream));
         QFE_HIP(hipMemcpyAsync(dc, cs.data(), cs.size() * sizeof(double2), hipMemcpyHostToDevice, cx.stream));
-        hipLaunchKernelGGL(k_expval_groups, dim3((unsigned)((uint64_t)G * nchunk)), dim3(kEvTPB), 0, cx.stream, bra, ket,
-                           n, (const PauliGroup*)dg, (const uint64_t*)dz, (const double2*)dc, nchunk, (double2*)part);
+        launch_expval_kernel(bra, ket, n, (const PauliGroup*)dg, (uint32_t)G, (const uint64_t*)dz, (const double2*)dc, nchunk,
+                             (double2*)part);
         QFE_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)G), dim3(kEvTPB), 0, cx.stream, (const double2*)part, nchunk,
                            (double2*)dout);
@@ -937,7 +1036,7 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
     std::vector<OrbitGroup> og;
     std::vector<OrbitTerm> ot;
     std::vector<OrbitLaunch> launches;
-    build_orbit_tables(groups, zs, cs, maxdim, og, ot, launches);
+    build_orbit_tables(groups, zs, cs, n, maxdim, og, ot, launches);
     const std::vector<OrbitPass> op = orbit_pass_table(launches);
     char* dg = A.take(og.size() * sizeof(OrbitGroup));
     char* dt = A.take(ot.size() * sizeof(OrbitTerm));
@@ -982,21 +1081,84 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
     return QFE_OK;
 }
 
-// out_k = sum_g ket[k ^ x_g] f_g(k ^ x_g): every thread owns output amplitudes
-// and walks the groups in order (fixed summation order per element).
-__global__ void k_apply_sum(const double2* __restrict__ in, double2* __restrict__ out, uint64_t N,
-                            const PauliGroup* __restrict__ groups, uint32_t ngroups, const uint64_t* __restrict__ zs,
-                            const double2* __restrict__ cs) {
+// out_k = sum_g in[k ^ x_g] f_g(k ^ x_g): every thread owns kEvPer output
+// amplitudes and walks the groups in order (fixed summation order per
+// element), each term read once for all of them.  Grid y = slices of the
+// groups while the amplitudes alone leave CUs idle (14 qubits, 3382 terms: 64
+// workgroups took 535 us); k_add_slices then adds the slices in order.
+template <typename W>
+__global__ __launch_bounds__(kEvTPB) void k_apply_sum(const double2* __restrict__ in, double2* __restrict__ out, uint64_t N,
+                                                      const PauliGroup* __restrict__ groups, uint32_t ngroups,
+                                                      const uint64_t* __restrict__ zs, const double2* __restrict__ cs) {
+    const uint32_t g0 = (uint32_t)((uint64_t)ngroups * blockIdx.y / gridDim.y);
+    const uint32_t g1 = (uint32_t)((uint64_t)ngroups * (blockIdx.y + 1) / gridDim.y);
+    const uint64_t k0 = (uint64_t)blockIdx.x * (kEvTPB * kEvPer) + threadIdx.x;
+    double2 acc[kEvPer];
+#pragma unroll
+    for (int u = 0; u < kEvPer; ++u) acc[u] = make_double2(0.0, 0.0);
+    for (uint32_t g = g0; g < g1; ++g) {
+        const PauliGroup G = groups[g];
+        W src[kEvPer];
+        double2 v[kEvPer], f[kEvPer];
+#pragma unroll
+        for (int u = 0; u < kEvPer; ++u) {
+            const uint64_t k = k0 + (uint64_t)u * kEvTPB;
+            src[u] = (W)(k ^ G.x);
+            v[u] = k < N ? in[k ^ G.x] : make_double2(0.0, 0.0);
+            f[u] = make_double2(0.0, 0.0);
+        }
+        for (uint32_t t = G.first; t < G.first + G.count; ++t) {
+            const W z = (W)zs[t];
+            const double2 c = cs[t];
+#pragma unroll
+            for (int u = 0; u < kEvPer; ++u) {
+                const uint32_t s = odd_bit((W)(src[u] & z));
+                f[u].x += sign_flip(c.x, s);
+                f[u].y += sign_flip(c.y, s);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kEvPer; ++u) acc[u] = cadd(acc[u], cmul(f[u], v[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < kEvPer; ++u) {
+        const uint64_t k = k0 + (uint64_t)u * kEvTPB;
+        if (k < N) out[blockIdx.y * N + k] = acc[u];
+    }
+}
+
+__global__ __launch_bounds__(kEvTPB) void k_add_slices(const double2* __restrict__ slices, double2* __restrict__ out, uint64_t N,
+                                                       uint32_t count) {
     const uint64_t k = (uint64_t)blockIdx.x * kEvTPB + threadIdx.x;
     if (k >= N) return;
-    double2 acc = make_double2(0.0, 0.0);
-    for (uint32_t g = 0; g < ngroups; ++g) {
-        const PauliGroup G = groups[g];
-        const uint64_t src = k ^ G.x;
-        const double2 f = group_f(src, zs + G.first, cs + G.first, G.count);
-        acc = cadd(acc, cmul(f, in[src]));
-    }
+    double2 acc = slices[k];
+    for (uint32_t s = 1; s < count; ++s) acc = cadd(acc, slices[s * N + k]);
     out[k] = acc;
+}
+
+static int launch_apply_sum_kernel(const double2* in, double2* out, int n, const PauliGroup* dg, uint32_t ngroups,
+                                   const uint64_t* dz, const double2* dc) {
+    const uint64_t N = 1ull << n, blocks = (N + kEvTPB * kEvPer - 1) / (kEvTPB * kEvPer);
+    // slices until there are about eight workgroups per CU, at least eight groups each
+    uint32_t slices = 1;
+    while (blocks * slices < 2048 && slices * 16 <= ngroups && slices < 256) slices <<= 1;
+    double2* to = out;
+    if (slices > 1) {
+        void* work = nullptr;
+        int rc = slice_reserve((size_t)slices * N * sizeof(double2), &work);
+        if (rc) return rc;
+        to = static_cast<double2*>(work);
+    }
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, slices), dim3(kEvTPB), 0, ctx().stream, in, to, N, dg, ngroups, dz, dc);
+    };
+    n <= 32 ? go(k_apply_sum<uint32_t>) : go(k_apply_sum<uint64_t>);
+    QFE_HIP(hipGetLastError());
+    if (slices > 1) {
+        hipLaunchKernelGGL(k_add_slices, dim3((unsigned)((N + kEvTPB - 1) / kEvTPB)), dim3(kEvTPB), 0, ctx().stream, to, out, N, slices);
+        QFE_HIP(hipGetLastError());
+    }
+    return QFE_OK;
 }
 
 int launch_apply_pauli_sum(const double2* in, double2* out, int n, const std::vector<PauliGroup>& groups,
@@ -1007,9 +1169,8 @@ int launch_apply_pauli_sum(const double2* in, double2* out, int n, const std::ve
     GroupDev gd;
     int rc = upload_groups(groups, zs, cs, 0, gd);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_apply_sum, dim3((unsigned)((N + kEvTPB - 1) / kEvTPB)), dim3(kEvTPB), 0, cx.stream, in, out,
-                       N, gd.groups, (uint32_t)groups.size(), gd.zs, gd.cs);
-    QFE_HIP(hipGetLastError());
+    rc = launch_apply_sum_kernel(in, out, n, gd.groups, (uint32_t)groups.size(), gd.zs, gd.cs);
+    if (rc) return rc;
     cx.counters.single++;
     cx.counters.bytes += 16.0 * (double)N * (double)(groups.size() + 1);
     return QFE_OK;

@@ -58,6 +58,22 @@ int scratch_reserve(size_t bytes, void** out) {
     return QFE_OK;
 }
 
+int slice_reserve(size_t bytes, void** out) {
+    Context& c = g_ctx;
+    if (c.slice_bytes < bytes) {
+        if (c.slices) {
+            QFE_HIP(hipStreamSynchronize(c.stream));
+            QFE_HIP(hipFree(c.slices));
+            c.slices = nullptr;
+            c.slice_bytes = 0;
+        }
+        QFE_HIP(hipMalloc(&c.slices, bytes));
+        c.slice_bytes = bytes;
+    }
+    *out = c.slices;
+    return QFE_OK;
+}
+
 int pinned_reserve(size_t bytes, void** out) {
     Context& c = g_ctx;
     if (c.pinned_bytes < bytes) {
