@@ -171,6 +171,8 @@ struct PauliGroup {
 void group_terms(const qfe_pauli* terms, uint64_t count, std::vector<PauliGroup>& groups,
                  std::vector<uint64_t>& zs, std::vector<double2>& cs);
 
+// Whether expectation values on n qubits (same: bra == ket) take orbit passes.
+bool takes_orbits(int n, bool same);
 int expval_groups(const double2* bra, const double2* ket, int n, const std::vector<PauliGroup>& groups,
                   const std::vector<uint64_t>& zs, const std::vector<double2>& cs, double2* out_per_group);
 

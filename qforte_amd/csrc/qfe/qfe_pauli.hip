@@ -285,7 +285,7 @@ constexpr int kEvOrbitMinQubits = 21;
 // at 16, 100 / 76 at 18, 242 / 102 at 20; at 18 qubits the 1621 masks of a
 // molecule read 6.8 GB from the caches, 522 us, against 0.9 GB in passes).
 constexpr int kEvOnceMinQubits = 16;
-static bool takes_orbits(int n, bool same) { return n >= (same ? kEvOnceMinQubits : kEvOrbitMinQubits); }
+bool takes_orbits(int n, bool same) { return n >= (same ? kEvOnceMinQubits : kEvOrbitMinQubits); }
 constexpr int kEvOrbitGroups = 16;
 
 struct OrbitGroup {
