@@ -290,7 +290,8 @@ int qfe_template_residuals(qfe_template t, const double* params, const double* i
                            uint64_t count, qfe_c64* out);
 /* ADAPT pool gradients 2 Re<H psi|A_k psi> (uccvqeabc.py:253-283) for nops
  * anti-Hermitian operators given as Pauli sums (pool_terms split by
- * op_offsets); `batch` operators per launch (0: 64). */
+ * op_offsets).  An operator needs no memory of its own on the sector, so one
+ * launch takes them all and `batch` bounds nothing. */
 int qfe_template_pool_gradients(qfe_template t, const double* params, const double* inputs, const qfe_pauli* pool_terms,
                                 const uint64_t* op_offsets, uint64_t nops, uint64_t batch, double* grads);
 

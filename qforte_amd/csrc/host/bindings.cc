@@ -16,6 +16,37 @@ namespace py = pybind11;
 using namespace pybind11::literals;
 using namespace qfa;
 
+// A sequence of floats as an argument.  Accepts what std::vector<double> does;
+// a list of floats (amplitudes and packed integrals, up to a few thousand) is
+// read directly instead of through a Python object per element.
+struct Doubles : std::vector<double> {};
+
+namespace pybind11 {
+namespace detail {
+template <>
+struct type_caster<Doubles> {
+    PYBIND11_TYPE_CASTER(Doubles, const_name("List[float]"));
+    bool load(handle src, bool convert) {
+        if (PyList_CheckExact(src.ptr())) {
+            const Py_ssize_t n = PyList_GET_SIZE(src.ptr());
+            value.resize((size_t)n);
+            Py_ssize_t i = 0;
+            for (; i < n; ++i) {
+                PyObject* o = PyList_GET_ITEM(src.ptr(), i);
+                if (!PyFloat_CheckExact(o)) break;
+                value[(size_t)i] = PyFloat_AS_DOUBLE(o);
+            }
+            if (i == n) return true;
+        }
+        list_caster<std::vector<double>, double> any;
+        if (!any.load(src, convert)) return false;
+        static_cast<std::vector<double>&>(value) = std::move(static_cast<std::vector<double>&>(any));
+        return true;
+    }
+};
+}  // namespace detail
+}  // namespace pybind11
+
 namespace {
 
 const char* kOneQubit[] = {"X", "Y", "Z", "H", "R", "Rx", "Ry", "Rz", "V", "S", "T", "I"};
@@ -53,6 +84,25 @@ void set_coeffs_from(Computer& c, py::object obj) {
     c.set_coeff_vec(arr.data(), (size_t)arr.size());
 }
 
+// Operators of a call, by reference: copying them copies every term's gates.
+using OperatorList = std::vector<std::reference_wrapper<const QubitOperator>>;
+
+// The mask forms of several operators, operator k's terms at [off[k], off[k + 1]).
+bool compile_operators(const OperatorList& ops, std::vector<qfe_pauli>& terms, std::vector<uint64_t>& off) {
+    size_t n = 0;
+    for (const QubitOperator& o : ops) n += o.terms().size();
+    terms.clear();
+    terms.reserve(n);
+    off.assign(1, 0);
+    std::vector<qfe_pauli> one;
+    for (const QubitOperator& o : ops) {
+        if (!compile_pauli_sum(o, one)) return false;
+        terms.insert(terms.end(), one.begin(), one.end());
+        off.push_back(terms.size());
+    }
+    return true;
+}
+
 // ---- compiled UCC program -----------------------------------------------------------
 class UCCProgram {
   public:
@@ -82,21 +132,21 @@ class UCCProgram {
     UCCProgram(const UCCProgram&) = delete;
     UCCProgram& operator=(const UCCProgram&) = delete;
 
-    double energy(const std::vector<double>& t) {
+    double energy(const Doubles& t) {
         need(t);
         double e = 0;
         py::gil_scoped_release rel;
         check(qfe_program_energy(p_, t.data(), &e), "UCCProgram.energy");
         return e;
     }
-    double energy_graph(const std::vector<double>& t) {
+    double energy_graph(const Doubles& t) {
         need(t);
         double e = 0;
         py::gil_scoped_release rel;
         check(qfe_program_energy_graph(p_, t.data(), &e), "UCCProgram.energy_graph");
         return e;
     }
-    std::pair<double, std::vector<double>> gradient(const std::vector<double>& t) {
+    std::pair<double, std::vector<double>> gradient(const Doubles& t) {
         need(t);
         std::vector<double> g(nparam_);
         double e = 0;
@@ -104,12 +154,12 @@ class UCCProgram {
         check(qfe_program_gradient(p_, t.data(), g.data(), &e), "UCCProgram.gradient");
         return {e, g};
     }
-    void prepare(const std::vector<double>& t, Computer& out) {
+    void prepare(const Doubles& t, Computer& out) {
         need(t);
         py::gil_scoped_release rel;
         check(qfe_program_prepare(p_, t.data(), out.handle()), "UCCProgram.prepare");
     }
-    std::vector<cplx> residuals(const std::vector<double>& t, const std::vector<uint64_t>& idx) {
+    std::vector<cplx> residuals(const Doubles& t, const std::vector<uint64_t>& idx) {
         need(t);
         std::vector<cplx> out(idx.size());
         py::gil_scoped_release rel;
@@ -117,16 +167,12 @@ class UCCProgram {
               "UCCProgram.residuals");
         return out;
     }
-    std::vector<double> pool_gradients(const std::vector<double>& t, const std::vector<QubitOperator>& ops,
+    std::vector<double> pool_gradients(const Doubles& t, const OperatorList& ops,
                                        size_t batch) {
         need(t);
-        std::vector<qfe_pauli> terms, one;
-        std::vector<uint64_t> off{0};
-        for (const auto& g : ops) {
-            if (!compile_pauli_sum(g, one)) throw std::invalid_argument("pool_gradients: operators must be Pauli sums");
-            terms.insert(terms.end(), one.begin(), one.end());
-            off.push_back(terms.size());
-        }
+        std::vector<qfe_pauli> terms;
+        std::vector<uint64_t> off;
+        if (!compile_operators(ops, terms, off)) throw std::invalid_argument("pool_gradients: operators must be Pauli sums");
         std::vector<double> out(ops.size());
         py::gil_scoped_release rel;
         check(qfe_program_pool_gradients(p_, t.data(), terms.data(), off.data(), ops.size(), batch, out.data()),
@@ -185,19 +231,19 @@ class SectorTemplate {
     SectorTemplate(const SectorTemplate&) = delete;
     SectorTemplate& operator=(const SectorTemplate&) = delete;
 
-    double energy(const std::vector<double>& t, const std::vector<double>& inputs) {
+    double energy(const Doubles& t, const Doubles& inputs) {
         need(t, inputs);
         double e = 0.0;
         py::gil_scoped_release rel;
         check(qfe_template_energy(t_, t.data(), inputs.data(), &e), "SectorTemplate.energy");
         return e;
     }
-    void prepare(const std::vector<double>& t, Computer& out) {
+    void prepare(const Doubles& t, Computer& out) {
         if (t.size() != nparam_) throw std::invalid_argument("SectorTemplate: wrong number of amplitudes");
         py::gil_scoped_release rel;
         check(qfe_template_prepare(t_, t.data(), out.handle()), "SectorTemplate.prepare");
     }
-    std::pair<double, std::vector<double>> gradient(const std::vector<double>& t, const std::vector<double>& inputs) {
+    std::pair<double, std::vector<double>> gradient(const Doubles& t, const Doubles& inputs) {
         need(t, inputs);
         std::vector<double> g(nparam_);
         double e = 0.0;
@@ -205,8 +251,7 @@ class SectorTemplate {
         check(qfe_template_gradient(t_, t.data(), inputs.data(), g.data(), &e), "SectorTemplate.gradient");
         return {e, g};
     }
-    std::vector<cplx> residuals(const std::vector<double>& t, const std::vector<uint64_t>& idx,
-                                const std::vector<double>& inputs) {
+    std::vector<cplx> residuals(const Doubles& t, const std::vector<uint64_t>& idx, const Doubles& inputs) {
         need(t, inputs);
         std::vector<cplx> out(idx.size());
         py::gil_scoped_release rel;
@@ -215,16 +260,12 @@ class SectorTemplate {
               "SectorTemplate.residuals");
         return out;
     }
-    std::vector<double> pool_gradients(const std::vector<double>& t, const std::vector<QubitOperator>& ops, size_t batch,
-                                       const std::vector<double>& inputs) {
+    std::vector<double> pool_gradients(const Doubles& t, const OperatorList& ops, size_t batch, const Doubles& inputs) {
         need(t, inputs);
-        std::vector<qfe_pauli> terms, one;
-        std::vector<uint64_t> off{0};
-        for (const auto& op : ops) {
-            if (!compile_pauli_sum(op, one)) throw std::invalid_argument("SectorTemplate.pool_gradients: operators must be Pauli sums");
-            terms.insert(terms.end(), one.begin(), one.end());
-            off.push_back(terms.size());
-        }
+        std::vector<qfe_pauli> terms;
+        std::vector<uint64_t> off;
+        if (!compile_operators(ops, terms, off))
+            throw std::invalid_argument("SectorTemplate.pool_gradients: operators must be Pauli sums");
         std::vector<double> out(ops.size());
         py::gil_scoped_release rel;
         check(qfe_template_pool_gradients(t_, t.data(), inputs.data(), terms.data(), off.data(), ops.size(), batch,
@@ -289,8 +330,7 @@ class BatchEngine {
     ~BatchEngine() {
         if (b_) qfe_batch_destroy(b_);
     }
-    uint64_t submit(std::shared_ptr<SectorTemplate> t, const std::vector<double>& amps, const std::vector<double>& inputs,
-                    bool gradient) {
+    uint64_t submit(std::shared_ptr<SectorTemplate> t, const Doubles& amps, const Doubles& inputs, bool gradient) {
         t->need(amps, inputs);
         uint64_t id = 0;
         if (gradient)
@@ -585,15 +625,11 @@ PYBIND11_MODULE(_core, m) {
         return comp;
     }, "gate"_a, "computer"_a);
     m.def("inner_product", &qfa::dot, "a"_a, "b"_a);
-    m.def("cross_expectations", [](const Computer& bra, const Computer& ket, const std::vector<QubitOperator>& ops) {
+    m.def("cross_expectations", [](const Computer& bra, const Computer& ket, const OperatorList& ops) {
         // <bra|O_k|ket> for every Pauli-sum operator O_k, one device launch
-        std::vector<qfe_pauli> terms, one;
-        std::vector<uint64_t> off{0};
-        for (const auto& o : ops) {
-            if (!compile_pauli_sum(o, one)) throw std::invalid_argument("cross_expectations: operators must be Pauli sums");
-            terms.insert(terms.end(), one.begin(), one.end());
-            off.push_back(terms.size());
-        }
+        std::vector<qfe_pauli> terms;
+        std::vector<uint64_t> off;
+        if (!compile_operators(ops, terms, off)) throw std::invalid_argument("cross_expectations: operators must be Pauli sums");
         std::vector<qfe_c64> r(ops.size());
         {
             py::gil_scoped_release rel;
@@ -666,13 +702,13 @@ PYBIND11_MODULE(_core, m) {
         .def(py::init<int, uint64_t, const std::vector<QubitOperator>&, const std::vector<int>&,
                       const std::vector<double>&, size_t, const HamiltonianMap&>(),
              "nqubit"_a, "ref_index"_a, "generators"_a, "param_index"_a, "scale"_a, "nparam"_a, "hamiltonian_map"_a)
-        .def("energy", &SectorTemplate::energy, "amplitudes"_a, "inputs"_a = std::vector<double>())
+        .def("energy", &SectorTemplate::energy, "amplitudes"_a, "inputs"_a = py::list())
         .def("prepare", &SectorTemplate::prepare)
         .def("residuals", &SectorTemplate::residuals, "amplitudes"_a, "indices"_a,
-             "inputs"_a = std::vector<double>())
-        .def("gradient", &SectorTemplate::gradient, "amplitudes"_a, "inputs"_a = std::vector<double>())
+             "inputs"_a = py::list())
+        .def("gradient", &SectorTemplate::gradient, "amplitudes"_a, "inputs"_a = py::list())
         .def("pool_gradients", &SectorTemplate::pool_gradients, "amplitudes"_a, "operators"_a, "batch"_a = 64,
-             "inputs"_a = std::vector<double>())
+             "inputs"_a = py::list())
         .def_property_readonly("dim", &SectorTemplate::dim)
         .def_property_readonly("request_bytes", &SectorTemplate::request_bytes)
         .def("graph_audit", &SectorTemplate::graph_audit, "gradient"_a = false)
@@ -682,7 +718,7 @@ PYBIND11_MODULE(_core, m) {
 
     py::class_<BatchEngine>(m, "BatchEngine")
         .def(py::init<uint64_t, int>(), "hbm_budget_bytes"_a, "max_active"_a)
-        .def("submit", &BatchEngine::submit, "template"_a, "amplitudes"_a, "inputs"_a = std::vector<double>(),
+        .def("submit", &BatchEngine::submit, "template"_a, "amplitudes"_a, "inputs"_a = py::list(),
              "gradient"_a = false)
         .def("take_gradient", &BatchEngine::take_gradient, "request_id"_a, "nparam"_a)
         .def("step", &BatchEngine::step, "cap"_a = 4096)

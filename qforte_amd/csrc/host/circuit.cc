@@ -9,7 +9,40 @@ namespace qfa {
 
 // ---- Circuit -------------------------------------------------------------------
 
+void PauliForm::apply(const Gate& g) {
+    const char l = pauli ? g.pauli_letter() : 0;
+    if (!l || g.target() >= 64) {
+        pauli = false;
+        return;
+    }
+    // left-multiply: X flips; Z gives (-1)^{(j ^ x)_q}; Y = i X Z
+    const uint64_t bit = 1ull << g.target();
+    if (l == 'Z' || l == 'Y') {
+        if (x & bit) power += 2;
+        z ^= bit;
+    }
+    if (l == 'X' || l == 'Y') x ^= bit;
+    if (l == 'Y') power += 1;
+    power &= 3;
+}
+
+void PauliForm::apply(const PauliForm& f) {
+    pauli = pauli && f.pauli;
+    if (!pauli) return;
+    power = (power + f.power + ((__builtin_popcountll(x & f.z) & 1) ? 2 : 0)) & 3;
+    x ^= f.x;
+    z ^= f.z;
+}
+
+PauliForm Circuit::pauli_form() const {
+    if (form_known_) return form_;
+    PauliForm f;
+    for (const auto& g : gates_) f.apply(g);
+    return f;
+}
+
 void Circuit::add_circuit(const Circuit& c) {
+    if (form_known_) form_.apply(c.pauli_form());
     const size_t off = gates_.size();
     gates_.insert(gates_.end(), c.gates_.begin(), c.gates_.end());
     for (ExpSegment s : c.segs_) {
@@ -22,36 +55,42 @@ void Circuit::add_circuit(const Circuit& c) {
 void Circuit::insert_gate(size_t pos, const Gate& g) {
     if (pos > gates_.size()) throw std::runtime_error("Circuit::insert_gate: position out of range");
     gates_.insert(gates_.begin() + pos, g);
+    form_known_ = false;
     segs_.clear();
 }
 
 void Circuit::remove_gate(size_t pos) {
     if (pos >= gates_.size()) throw std::runtime_error("Circuit::remove_gate: position out of range");
     gates_.erase(gates_.begin() + pos);
+    form_known_ = false;
     segs_.clear();
 }
 
 void Circuit::replace_gate(size_t pos, const Gate& g) {
     if (pos >= gates_.size()) throw std::runtime_error("Circuit::replace_gate: position out of range");
     gates_[pos] = g;
+    form_known_ = false;
     segs_.clear();
 }
 
 void Circuit::swap_gates(size_t p1, size_t p2) {
     if (p1 >= gates_.size() || p2 >= gates_.size()) throw std::runtime_error("Circuit::swap_gates: position out of range");
     std::swap(gates_[p1], gates_[p2]);
+    form_known_ = false;
     segs_.clear();
 }
 
 void Circuit::insert_circuit(size_t pos, const Circuit& c) {
     if (pos > gates_.size()) throw std::runtime_error("Circuit::insert_circuit: position out of range");
     gates_.insert(gates_.begin() + pos, c.gates_.begin(), c.gates_.end());
+    form_known_ = false;
     segs_.clear();
 }
 
 void Circuit::remove_gates(size_t p1, size_t p2) {
     if (p1 >= gates_.size() || p2 >= gates_.size()) throw std::runtime_error("Circuit::remove_gates: position out of range");
     gates_.erase(gates_.begin() + p1, gates_.begin() + p2);
+    form_known_ = false;
     segs_.clear();
 }
 
@@ -59,6 +98,7 @@ Circuit Circuit::adjoint() const {
     Circuit out;
     out.gates_.reserve(gates_.size());
     for (auto it = gates_.rbegin(); it != gates_.rend(); ++it) out.gates_.push_back(it->adjoint());
+    out.form_known_ = false;
     // exp(i a P)^dag = exp(-i a P) over the mirrored gate range
     const size_t n = gates_.size();
     for (auto it = segs_.rbegin(); it != segs_.rend(); ++it) {
@@ -72,6 +112,7 @@ Circuit Circuit::adjoint() const {
 }
 
 void Circuit::set_parameters(const std::vector<double>& params) {
+    form_known_ = false;
     size_t k = 0;
     for (auto& g : gates_) {
         if (!g.has_parameter()) continue;
@@ -87,6 +128,7 @@ void Circuit::set_parameters(const std::vector<double>& params) {
 void Circuit::set_parameter(size_t pos, double param) {
     if (pos >= gates_.size()) throw std::runtime_error("Circuit::set_parameter: position out of range");
     if (!gates_[pos].has_parameter()) throw std::runtime_error("Circuit::set_parameter: gate does not have a parameter");
+    form_known_ = false;
     gates_[pos] = make_gate(gates_[pos].gate_id(), gates_[pos].target(), gates_[pos].control(), param);
     segs_.clear();
 }
@@ -144,6 +186,9 @@ cplx Circuit::canonicalize_pauli_circuit() {
     }
     gates_ = std::move(out);
     segs_.clear();
+    form_ = PauliForm();
+    for (const auto& g : gates_) form_.apply(g);
+    form_known_ = true;
     return coeff;
 }
 
@@ -178,30 +223,12 @@ bool operator<(const Circuit& a, const Circuit& b) {
 }
 
 bool pauli_masks(const Circuit& c, uint64_t& x, uint64_t& z, cplx& phase) {
-    // Left-multiply letter by letter in application order:
-    //   X_q: flip; Z_q: sign (-1)^{(j^x)_q}; Y_q = i X Z: both, times i.
-    x = z = 0;
-    phase = 1.0;
-    const cplx i(0.0, 1.0);
-    for (const auto& g : c.gates()) {
-        const char l = g.pauli_letter();
-        if (!l) return false;
-        const size_t q = g.target();
-        if (q >= 64) return false;
-        const uint64_t bit = 1ull << q;
-        if (l == 'X') {
-            x ^= bit;
-        } else if (l == 'Z') {
-            if (x & bit) phase = -phase;
-            z ^= bit;
-        } else if (l == 'Y') {
-            phase *= i;
-            if (x & bit) phase = -phase;
-            z ^= bit;
-            x ^= bit;
-        }
-    }
-    return true;
+    static const cplx kPower[4] = {{1.0, 0.0}, {0.0, 1.0}, {-1.0, 0.0}, {0.0, -1.0}};
+    const PauliForm f = c.pauli_form();
+    x = f.x;
+    z = f.z;
+    phase = kPower[f.power];
+    return f.pauli;
 }
 
 // ---- QubitOperator ----------------------------------------------------------------

@@ -98,10 +98,24 @@ struct ExpSegment {
     double angle;
 };
 
+// The operator a run of X, Y, Z and I gates applies (first gate first), as
+// P|j> = i^power (-1)^popcount(j & z) |j ^ x>; pauli is false once a gate is
+// none of them (or acts beyond qubit 63).
+struct PauliForm {
+    uint64_t x = 0, z = 0;
+    int power = 0;
+    bool pauli = true;
+    void apply(const Gate& g);
+    void apply(const PauliForm& f);
+};
+
 class Circuit {
   public:
     Circuit() = default;
-    void add_gate(const Gate& g) { gates_.push_back(g); }
+    void add_gate(const Gate& g) {
+        gates_.push_back(g);
+        if (form_known_) form_.apply(g);
+    }
     void add_circuit(const Circuit& c);
     void insert_gate(size_t pos, const Gate& g);
     void remove_gate(size_t pos);
@@ -122,10 +136,17 @@ class Circuit {
     bool is_pauli() const;                                 // circuit.cc:222-230
     const std::vector<ExpSegment>& segments() const { return segs_; }
     void add_segment(const ExpSegment& s) { segs_.push_back(s); }
+    // The Pauli form of the whole circuit.  Appending keeps it up to date, so
+    // compiling an operator reads one form per term instead of its gates (about
+    // 330 bytes each, six per term of a molecular Hamiltonian); any other
+    // mutation leaves it to be read from the gates.
+    PauliForm pauli_form() const;
 
   private:
     std::vector<Gate> gates_;
     std::vector<ExpSegment> segs_;
+    PauliForm form_;
+    bool form_known_ = true;
 };
 
 bool operator==(const Circuit& a, const Circuit& b);

@@ -14,7 +14,6 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include "qfe_device.h"
@@ -25,34 +24,39 @@ namespace qfe {
 void group_terms(const qfe_pauli* terms, uint64_t count, std::vector<PauliGroup>& groups, std::vector<uint64_t>& zs,
                  std::vector<double2>& cs) {
     groups.clear();
-    zs.clear();
-    cs.clear();
-    std::unordered_map<uint64_t, size_t> where;
-    std::vector<std::vector<uint64_t>> members;
+    zs.resize(count);
+    cs.resize(count);
+    // group of every term (open addressing over the X masks), then each term to its place
+    size_t cap = 16;
+    while (cap < 2 * count) cap <<= 1;
+    std::vector<uint32_t> slot(cap, 0), of(count);  // slot: group + 1
     for (uint64_t i = 0; i < count; ++i) {
-        auto it = where.find(terms[i].x);
-        if (it == where.end()) {
-            where.emplace(terms[i].x, members.size());
-            members.emplace_back();
-            members.back().push_back(i);
-        } else {
-            members[it->second].push_back(i);
+        size_t h = (size_t)((terms[i].x * 0x9E3779B97F4A7C15ull) >> 20) & (cap - 1);
+        while (slot[h] && groups[slot[h] - 1].x != terms[i].x) h = (h + 1) & (cap - 1);
+        if (!slot[h]) {
+            PauliGroup g{};
+            g.x = terms[i].x;
+            g.hb = g.x ? (uint32_t)(63 - __builtin_clzll(g.x)) : 0u;
+            groups.push_back(g);
+            slot[h] = (uint32_t)groups.size();
         }
+        of[i] = slot[h] - 1;
+        groups[of[i]].count++;
     }
-    for (auto& mem : members) {
-        PauliGroup g{};
-        g.x = terms[mem[0]].x;
-        g.first = (uint32_t)zs.size();
-        g.count = (uint32_t)mem.size();
-        g.hb = g.x ? (uint32_t)(63 - __builtin_clzll(g.x)) : 0u;
-        for (uint64_t i : mem) {
-            const qfe_pauli& t = terms[i];
-            zs.push_back(t.z);
-            // fold the coefficient and the phase of the mask form
-            cs.push_back(make_double2(t.coeff.re * t.phase.re - t.coeff.im * t.phase.im,
-                                      t.coeff.re * t.phase.im + t.coeff.im * t.phase.re));
-        }
-        groups.push_back(g);
+    uint32_t at = 0;
+    for (PauliGroup& g : groups) {
+        g.first = at;
+        at += g.count;
+        g.count = 0;
+    }
+    for (uint64_t i = 0; i < count; ++i) {
+        const qfe_pauli& t = terms[i];
+        PauliGroup& g = groups[of[i]];
+        const uint32_t k = g.first + g.count++;
+        zs[k] = t.z;
+        // fold the coefficient and the phase of the mask form
+        cs[k] = make_double2(t.coeff.re * t.phase.re - t.coeff.im * t.phase.im,
+                             t.coeff.re * t.phase.im + t.coeff.im * t.phase.re);
     }
 }
 

@@ -40,7 +40,6 @@
 #include <functional>
 #include <map>
 #include <set>
-#include <tuple>
 #include <unordered_map>
 #include <vector>
 
@@ -1163,9 +1162,22 @@ struct Space {
 // (a & clear) == 0.  The partner is a ^ flip.
 struct ListPool {
     std::vector<int2> pool;
-    std::map<std::tuple<int, int, uint32_t, uint32_t, uint32_t>, std::pair<uint32_t, uint32_t>> index;
+    struct Key {
+        int s, kind;
+        uint32_t mask, pattern, flip;
+        bool operator==(const Key& o) const {
+            return s == o.s && kind == o.kind && mask == o.mask && pattern == o.pattern && flip == o.flip;
+        }
+    };
+    struct Hash {
+        size_t operator()(const Key& k) const {
+            const uint64_t a = ((uint64_t)k.mask << 32) | k.pattern, b = ((uint64_t)k.flip << 8) | (uint32_t)(k.s * 4 + k.kind);
+            return (size_t)((a * 0x9E3779B97F4A7C15ull) ^ ((b * 0xC2B2AE3D27D4EB4Full) >> 17));
+        }
+    };
+    std::unordered_map<Key, std::pair<uint32_t, uint32_t>, Hash> index;
     std::pair<uint32_t, uint32_t> get(const Space& sp, int s, int kind, uint32_t mask, uint32_t pattern, uint32_t flip) {
-        auto key = std::make_tuple(s, kind, mask, pattern, flip);
+        const Key key{s, kind, mask, pattern, flip};
         auto it = index.find(key);
         if (it != index.end()) return it->second;
         const uint32_t off = (uint32_t)pool.size();
@@ -1192,6 +1204,8 @@ struct ListPool {
 int build_runs(const Space& sp, ListPool& lp, int norb, uint64_t lim, const qfe_pauli* terms, uint64_t b, uint64_t e,
                int32_t param, double scale, uint32_t gen, std::vector<SecStep>& steps, std::vector<SecEntry>& entries,
                const char* who) {
+    std::vector<std::pair<uint64_t, double2>> A;
+    std::vector<double2> kap;
     while (b < e) {
         const uint64_t x = terms[b].x, z0 = terms[b].z;
         uint64_t r = b;
@@ -1203,23 +1217,25 @@ int build_runs(const Space& sp, ListPool& lp, int norb, uint64_t lim, const qfe_
         }
         if (popc64(m) > 20) return fail(QFE_ERR_ARG, std::string(who) + ": a run of commuting terms spans more than 20 qubits");
         double scale_abs = 0.0;
-        std::vector<double2> kap(r - b);
+        kap.assign(r - b, make_double2(0.0, 0.0));
         for (uint64_t k = b; k < r; ++k) {
             // exp(theta * coeff * P) with coeff purely imaginary, as the full-space program applies it
             kap[k - b] = cplx_mul(make_double2(0.0, terms[k].coeff.im), make_double2(terms[k].phase.re, terms[k].phase.im));
             scale_abs += cplx_abs(kap[k - b]);
         }
         const double tol = 1e-13 * (scale_abs > 0 ? scale_abs : 1.0);
-        std::map<uint64_t, double2> A;  // A(p) over the submasks of m
-        for (uint64_t p = m;; p = (p - 1) & m) {
+        // A(p) over the submasks p of m, ascending, where it is not zero
+        A.clear();
+        for (uint64_t p = 0;;) {
             double2 s = make_double2(0.0, 0.0);
             for (uint64_t k = b; k < r; ++k) {
                 const double sg = (popc64(p & (terms[k].z ^ z0)) & 1) ? -1.0 : 1.0;
                 s.x += sg * kap[k - b].x;
                 s.y += sg * kap[k - b].y;
             }
-            if (cplx_abs(s) > tol) A.emplace(p, s);
-            if (p == 0) break;
+            if (std::fabs(s.x) > tol || std::fabs(s.y) > tol || cplx_abs(s) > tol) A.emplace_back(p, s);
+            if (p == m) break;
+            p = (p - m) & m;  // the next submask
         }
         if (x == 0 && !A.empty()) return fail(QFE_ERR_ARG, std::string(who) + ": diagonal runs are not supported on the sector");
         SecStep st{};
@@ -1230,8 +1246,8 @@ int build_runs(const Space& sp, ListPool& lp, int norb, uint64_t lim, const qfe_
         const double sx = (popc64(x & z0) & 1) ? -1.0 : 1.0;
         for (const auto& kv : A) {
             const uint64_t plo = kv.first, phi = plo ^ x;
-            auto it = A.find(phi);
-            if (it == A.end()) return fail(QFE_ERR_ARG, std::string(who) + ": a run is not anti-Hermitian");
+            const auto it = std::lower_bound(A.begin(), A.end(), phi, [](const std::pair<uint64_t, double2>& u, uint64_t v) { return u.first < v; });
+            if (it == A.end() || it->first != phi) return fail(QFE_ERR_ARG, std::string(who) + ": a run is not anti-Hermitian");
             if (plo > phi) continue;
             const double2 alo = kv.second, ahi = it->second;
             const double w = cplx_abs(alo);
@@ -1810,10 +1826,9 @@ struct Packer {
         total += align256(bytes ? bytes : 1);
         return pieces.size() - 1;
     }
-    void fill(std::vector<char>& img) const {
-        img.assign(total, 0);
+    void fill(char* img) const {
         for (const auto& p : pieces)
-            if (p.bytes) std::memcpy(img.data() + p.off, p.src, p.bytes);
+            if (p.bytes) std::memcpy(img + p.off, p.src, p.bytes);
     }
 };
 
@@ -2226,8 +2241,8 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     h.nterms = (uint32_t)tz.size();
     h.nitems = (uint32_t)items.size();
     h.ngen = (uint32_t)ngen;
-    std::vector<char> img;
-    pk.fill(img);
+    std::vector<char> img(pk.total, 0);
+    pk.fill(img.data());
     std::memcpy(img.data(), &h, sizeof(h));
     QFE_HIP(hipMemcpy(t->dev, img.data(), pk.total, hipMemcpyHostToDevice));
     t->dt = (SecTables*)t->dev;
@@ -3261,11 +3276,16 @@ int qfe_template_residuals(qfe_template t, const double* params, const double* i
     return QFE_OK;
 }
 
+// Largest tables of a pool-gradient call that go through the kept scratch and
+// staging: an allocation and its release cost the 14-qubit call (0.4 MiB) more
+// than its kernel, and nothing next to tables above this.
+constexpr size_t kPoolKeep = 16u << 20;
+
 int qfe_template_pool_gradients(qfe_template t, const double* params, const double* inputs, const qfe_pauli* pool_terms,
                                 const uint64_t* op_offsets, uint64_t nops, uint64_t batch, double* grads) {
     if (!t || (nops && (!pool_terms || !op_offsets || !grads)) || (t->nparam && !params) || (t->ninputs && !inputs))
         return fail(QFE_ERR_ARG, "qfe_template_pool_gradients: null argument");
-    if (batch == 0) batch = 64;
+    (void)batch;
     // pool operators as pair rotations on the template's sector
     ListPool lp;
     std::vector<SecStep> steps;
@@ -3289,19 +3309,38 @@ int qfe_template_pool_gradients(qfe_template t, const double* params, const doub
     const size_t i_o = pk.add(ops.data(), ops.size() * sizeof(PoolOp));
     const size_t o_out = pk.total;
     const size_t total = o_out + align256(nops * 8 + 8);
+    // The tables of the call go through the context's staging and scratch; above
+    // kPoolKeep they get memory of their own, given back at the end.
     void* dev = nullptr;
-    QFE_HIP(hipMalloc(&dev, total));
+    const bool keep = total <= kPoolKeep;
     std::vector<char> img;
-    pk.fill(img);
-    hipError_t e = hipMemcpy(dev, img.data(), pk.total, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(dev);
-        return hip_fail(e, "qfe_template_pool_gradients: upload");
+    if (keep) {
+        rc = scratch_reserve(total, &dev);
+        if (rc) return rc;
+        void* host = nullptr;
+        rc = staging_begin(pk.total, &host);
+        if (rc) return rc;
+        pk.fill(static_cast<char*>(host));
+        rc = staging_commit(dev, pk.total);
+        if (rc) return rc;
+    } else {
+        QFE_HIP(hipMalloc(&dev, total));
+        img.resize(pk.total);
+        pk.fill(img.data());
+        const hipError_t e = hipMemcpy(dev, img.data(), pk.total, hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(dev);
+            return hip_fail(e, "qfe_template_pool_gradients: upload");
+        }
     }
     char* base = (char*)dev;
-    // batches of `batch` operators per launch
-    for (uint64_t b0 = 0; b0 < nops; b0 += batch) {
-        const uint64_t b1 = std::min(nops, b0 + batch);
+    // One workgroup per operator and all of them in one launch: an operator needs
+    // no memory of its own, so `batch` bounds nothing here (1638 operators at 14
+    // qubits in launches of 64 left three CUs of four idle).
+    hipError_t e = hipSuccess;
+    constexpr uint64_t kGridMax = 1u << 30;
+    for (uint64_t b0 = 0; b0 < nops && e == hipSuccess; b0 += kGridMax) {
+        const uint64_t b1 = std::min(nops, b0 + kGridMax);
         with_scalar(t, [&](auto z) {
             using A = decltype(z);
             hipLaunchKernelGGL(k_sec_pool<A>, dim3((unsigned)(b1 - b0)), dim3(256), 0, ctx().stream, t->dt,
@@ -3310,12 +3349,13 @@ int qfe_template_pool_gradients(qfe_template t, const double* params, const doub
                                (const A*)(S.work + t->off_psi), (double*)(base + o_out) + b0);
         });
         e = hipGetLastError();
-        if (e != hipSuccess) break;
     }
-    if (e == hipSuccess && nops) rc = fetch_doubles((const double*)(base + o_out), nops, grads);
-    (void)hipStreamSynchronize(ctx().stream);
-    (void)hipFree(dev);
-    if (e != hipSuccess) return hip_fail(e, "qfe_template_pool_gradients: launch");
+    rc = e != hipSuccess ? hip_fail(e, "qfe_template_pool_gradients: launch")
+                         : nops ? fetch_doubles((const double*)(base + o_out), nops, grads) : QFE_OK;
+    if (!keep) {
+        (void)hipStreamSynchronize(ctx().stream);
+        (void)hipFree(dev);
+    }
     return rc;
 }
 

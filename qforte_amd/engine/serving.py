@@ -30,7 +30,10 @@ class ServingEngine:
         self._grad_len = {}
 
     def submit(self, template, amplitudes, inputs=(), arrival_time=None, gradient=False):
-        rid = self._eng.submit(template, list(amplitudes), list(inputs), bool(gradient))
+        # the engine copies both; lists go as they are
+        amplitudes = amplitudes if type(amplitudes) is list else list(amplitudes)
+        inputs = inputs if type(inputs) is list else list(inputs)
+        rid = self._eng.submit(template, amplitudes, inputs, bool(gradient))
         self._arrival[rid] = time.perf_counter() if arrival_time is None else arrival_time
         if gradient:
             self._grad_len[rid] = template.nparam
