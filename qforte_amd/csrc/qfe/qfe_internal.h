@@ -33,10 +33,10 @@ struct Tuning {
 };
 
 // Pass shape for a state of n qubits: the explicit tuning, or by default the
-// shape measured fastest for the size on MI355X.  A small state needs small
-// tiles so that a pass has enough workgroups and each op a short per-thread
-// chain: (8, 4, 64) up to 14 qubits (500 random gates at 12 qubits: 0.59 vs
-// 0.93 ms), (10, 4, 32) at 15-20 (the 16-qubit UCCSD energy, 2688
+// shape measured fastest for the size on MI355X (gate circuits of small states
+// go elsewhere, run_rounds; these shapes serve exponentials and large states).
+// A small state needs small tiles so that a pass has enough workgroups and each
+// op a short per-thread chain: (8, 4, 64) up to 14 qubits, (10, 4, 32) at 15-20 (the 16-qubit UCCSD energy, 2688
 // exponentials: 2.73 ms, against 3.38 ms with 8-qubit tiles), (11, 4, 24)
 // from 21 on.  Register-orbit passes keep 24 ops: longer ones are bound by
 // their arithmetic while the state sits in cache (the same UCCSD energy with
@@ -140,6 +140,11 @@ int lower_pexp(const qfe_pauli& p, double angle, int n, std::vector<HostOp>& out
 
 // Execute a lowered op list on a state (plans fused passes and launches).
 int run_ops(qfe_state_s* s, std::vector<HostOp>& ops);
+
+// Gates of a small state as rounds of register orbits (qfe_rounds.hip); taken:
+// false when an op has no form there (nothing was applied then).
+constexpr int kRoundsMaxQubits = 22;
+int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken);
 
 // A planned op list kept for replay: the descriptor image (uploaded by the
 // caller to device memory it owns) and the launch sequence over it.  With

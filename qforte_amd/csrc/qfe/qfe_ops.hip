@@ -1877,8 +1877,25 @@ int plan_launch(const OpPlan* P, qfe_state_s* st, char* dev) {
 
 void plan_free(OpPlan* p) { delete p; }
 
+// Gate circuits go as rounds up to 22 qubits (the second buffer of a
+// multi-tile circuit is then at most 64 MiB), by default only: explicit tile
+// shapes are honoured.  Few gates stay on the streaming and tile passes, which
+// need no second buffer and no move back.  500 random gates, rounds against
+// tiles: 87 / 457 us at 3 qubits, 101 / 525 at 12, 152 / 641 at 18, 291 / 1846 at
+// 22; 25 gates: 43 / 61 us at 20, 69 / 126 at 22; one layer of rotations and CNOTs:
+// 33 / 38 us at 12, 48 / 52 at 17, 117 / 138 at 22; 8 gates: 25 / 25 us at 12,
+// 30 / 27 at 17, 65 / 57 at 22.
+static bool takes_rounds(const Tuning& tu, int n, size_t ops) {
+    return tu.tile_auto && n <= kRoundsMaxQubits && ops >= (n <= 12 ? 8u : 24u);
+}
+
 int run_ops(qfe_state_s* st, std::vector<HostOp>& ops) {
     if (ops.empty()) return QFE_OK;
+    if (takes_rounds(ctx().tuning, st->n, ops.size())) {
+        bool taken = false;
+        const int rc = run_rounds(st, ops, taken);
+        if (rc || taken) return rc;
+    }
     OpPlan* P = nullptr;
     std::vector<char> image;
     std::vector<AngleRef> angles;
