@@ -1172,6 +1172,176 @@ __global__ __launch_bounds__(kOrbitTPB) void k_orbit_lanes(double2* __restrict__
     }
 }
 
+// ---------------------------------------------------------------------------
+// Device: LDS passes for runs of exponentials whose flips span many dimensions
+//
+// A tile is a coset of a span of kWideTile dimensions that holds the lowest
+// index bits (2 or 3: runs of half or whole lines) and the run's flip masks, so
+// a pass takes nine independent strings where a lane orbit takes seven.  The
+// exponentials go in rounds of up to three flips b_k: a thread owns the 8
+// amplitudes j ^ span(b) and pairs them at compile-time positions; the sign of
+// an element is the parity of j & z (per thread) times a bit of the op's
+// pattern (uniform).  The first round reads global memory and the last writes
+// it; LDS only carries the tile from one round to the next.
+//
+// A pass is bound by memory as long as enough waves hide the rounds' chain:
+// four workgroups of four waves per CU.  400 random strings at 23 qubits: 44
+// passes of 54 us against 56 lane orbits of 57 us; 120 at 30 qubits: 14 of
+// 6.7 ms against 17 of 6.6 ms.  16 amplitudes per thread (half the waves): 60 us;
+// 12-dimension tiles (two workgroups per CU): 39 passes of 62.5 us and 13 of
+// 7.35 ms; the next tile's loads issued behind the rounds (256 registers, spills):
+// 74 us.
+// ---------------------------------------------------------------------------
+
+constexpr int kWideTile = 11;
+constexpr int kWideG = 3;             // flips per round
+constexpr int kWideE = 1 << kWideG;   // amplitudes per thread
+constexpr int kWideBits = kWideTile - kWideG;
+constexpr int kWideTPB = 1 << kWideBits;
+constexpr int kWideRounds = 24;       // a pass has at most this many ops
+
+struct WideOp {
+    uint32_t mode;  // axis | kind << 4 (0: P imaginary, 1: P real, 2: diagonal)
+    uint32_t pat;   // bit i: sign of the term of element i
+    uint64_t z;     // sign functional outside the tile
+    uint32_t zl;    // and on tile bits
+    uint32_t pad;
+    double c, g;    // cos, and sin times the string's sign
+};
+
+struct WideRound {
+    uint64_t off[kWideG];  // flips as global masks
+    uint32_t b[kWideG];    // and in tile bits
+    uint32_t piv[kWideG];  // ascending tile bits with a zero inserted
+    uint32_t first, count;
+};
+
+struct WideDesc {
+    uint64_t sv[kWideTile];  // global mask of every tile bit, ascending pivots
+    uint32_t rounds, pad;
+    WideRound r[kWideRounds];
+};
+
+// g with its sign flipped when bit i of the uniform pattern is set.
+__device__ __forceinline__ double flip_uniform(double g, uint32_t pat, int i) {
+    const int m = (int)((pat << (31 - i)) & 0x80000000u);
+    return __hiloint2double(__double2hiint(g) ^ m, __double2loint(g));
+}
+
+// a_i' = c a_i + (sign) g a_partner for strings with a real factor i * phase
+// (KIND 0), c a_i + (sign) i g a_partner for the others (KIND 1).
+template <int AX, int KIND>
+__device__ __forceinline__ void wide_pairs(double2 (&a)[kWideE], double c, double g, uint32_t pat) {
+#pragma unroll
+    for (int i = 0; i < kWideE; ++i) {
+        if (i & (1 << AX)) continue;
+        const int k = i | (1 << AX);
+        const double2 x = a[i], y = a[k];
+        const double gi = flip_uniform(g, pat, i), gk = flip_uniform(g, pat, k);
+        if constexpr (KIND == 0) {
+            a[i] = make_double2(fma(gi, y.x, c * x.x), fma(gi, y.y, c * x.y));
+            a[k] = make_double2(fma(gk, x.x, c * y.x), fma(gk, x.y, c * y.y));
+        } else {
+            a[i] = make_double2(fma(-gi, y.y, c * x.x), fma(gi, y.x, c * x.y));
+            a[k] = make_double2(fma(-gk, x.y, c * y.x), fma(gk, x.x, c * y.y));
+        }
+    }
+}
+
+template <bool NT>
+__global__ __launch_bounds__(kWideTPB) void k_wide(double2* __restrict__ s, const WideDesc* __restrict__ D,
+                                                   const WideOp* __restrict__ ops) {
+    extern __shared__ double2 tile[];
+    uint64_t base = xcd_block();
+    for (int i = 0; i < kWideTile; ++i) base = ins0(base, (uint32_t)(63 - __builtin_clzll(D->sv[i])));
+    double2 a[kWideE];
+    const uint32_t rounds = D->rounds;
+    for (uint32_t r = 0; r < rounds; ++r) {
+        const WideRound& R = D->r[r];
+        uint32_t j = threadIdx.x;
+#pragma unroll
+        for (int d = 0; d < kWideG; ++d) j = ins0_32(j, R.piv[d]);
+        if (r == 0) {
+            uint64_t g = base;
+#pragma unroll
+            for (int i = 0; i < kWideTile; ++i) g ^= ((j >> i) & 1u) ? D->sv[i] : 0ull;
+            uint64_t o[kWideG];
+#pragma unroll
+            for (int d = 0; d < kWideG; ++d) o[d] = R.off[d];
+#pragma unroll
+            for (int i = 0; i < kWideE; ++i) {
+                uint64_t q = g;
+#pragma unroll
+                for (int d = 0; d < kWideG; ++d)
+                    if (i & (1 << d)) q ^= o[d];
+                a[i] = ld_s<NT>(s + q);
+            }
+        } else {
+            __syncthreads();
+            uint32_t b[kWideG];
+#pragma unroll
+            for (int d = 0; d < kWideG; ++d) b[d] = R.b[d];
+#pragma unroll
+            for (int i = 0; i < kWideE; ++i) {
+                uint32_t q = j;
+#pragma unroll
+                for (int d = 0; d < kWideG; ++d)
+                    if (i & (1 << d)) q ^= b[d];
+                a[i] = tile[q];
+            }
+        }
+        for (uint32_t oi = R.first; oi < R.first + R.count; ++oi) {
+            const WideOp& op = ops[oi];
+            const uint32_t odd = ((uint32_t)__popcll(base & op.z) ^ (uint32_t)__popc(j & op.zl)) & 1u;
+            const double c = op.c, g = odd ? -op.g : op.g;
+            const uint32_t pat = op.pat;
+            switch (op.mode) {
+                case 0x00: wide_pairs<0, 0>(a, c, g, pat); break;
+                case 0x01: wide_pairs<1, 0>(a, c, g, pat); break;
+                case 0x02: wide_pairs<2, 0>(a, c, g, pat); break;
+                case 0x10: wide_pairs<0, 1>(a, c, g, pat); break;
+                case 0x11: wide_pairs<1, 1>(a, c, g, pat); break;
+                case 0x12: wide_pairs<2, 1>(a, c, g, pat); break;
+                default:  // diagonal: its own partner
+#pragma unroll
+                    for (int i = 0; i < kWideE; ++i) {
+                        const double gi = flip_uniform(g, pat, i);
+                        a[i] = make_double2(fma(-gi, a[i].y, c * a[i].x), fma(gi, a[i].x, c * a[i].y));
+                    }
+                    break;
+            }
+        }
+        if (r + 1 < rounds) {
+            uint32_t b[kWideG];
+#pragma unroll
+            for (int d = 0; d < kWideG; ++d) b[d] = R.b[d];
+#pragma unroll
+            for (int i = 0; i < kWideE; ++i) {
+                uint32_t q = j;
+#pragma unroll
+                for (int d = 0; d < kWideG; ++d)
+                    if (i & (1 << d)) q ^= b[d];
+                tile[q] = a[i];
+            }
+        } else {
+            uint64_t g = base;
+#pragma unroll
+            for (int i = 0; i < kWideTile; ++i) g ^= ((j >> i) & 1u) ? D->sv[i] : 0ull;
+            uint64_t o[kWideG];
+#pragma unroll
+            for (int d = 0; d < kWideG; ++d) o[d] = R.off[d];
+#pragma unroll
+            for (int i = 0; i < kWideE; ++i) {
+                uint64_t q = g;
+#pragma unroll
+                for (int d = 0; d < kWideG; ++d)
+                    if (i & (1 << d)) q ^= o[d];
+                st_s<NT>(s + q, a[i]);
+            }
+        }
+    }
+}
+
 // Reduced GF(2) basis with pivot = highest bit; every pivot bit appears in
 // exactly one basis vector.
 struct Span {
@@ -1181,12 +1351,11 @@ struct Span {
             if ((x >> (63 - __builtin_clzll(v))) & 1ull) x ^= v;
         return x;
     }
-    bool add(uint64_t x, int maxdim, int minpiv = 0) {
+    bool add(uint64_t x, int maxdim) {
         const uint64_t r = reduce(x);
         if (!r) return true;
         if ((int)b.size() >= maxdim) return false;
         const int p = 63 - __builtin_clzll(r);
-        if (p < minpiv) return false;
         for (uint64_t& v : b)
             if ((v >> p) & 1ull) v ^= r;
         b.push_back(r);
@@ -1194,13 +1363,13 @@ struct Span {
     }
 };
 
-enum PassKind { P_SINGLE = 0, P_TILE = 1, P_ORBIT = 2 };
+enum PassKind { P_SINGLE = 0, P_TILE = 1, P_ORBIT = 2, P_WIDE = 3 };
 
 struct Pass {
     int kind = P_SINGLE;
     uint64_t bmask = 0;
     std::vector<int> ops;  // indices into the lowered op list
-    Span span;             // P_ORBIT
+    Span span;             // P_ORBIT, P_WIDE
 };
 
 // Greedy planner.  Ops may move ahead of an earlier op only when their qubit
@@ -1208,7 +1377,7 @@ struct Pass {
 // two ways from the first pending op -- as an LDS tile (mixing qubits fit
 // 2^k amplitudes) and as a register orbit (a run of exponentials whose flip
 // masks span at most orbit_dims <= 7 dimensions) -- and the one covering more
-// ops is kept.
+// ops is kept; an orbit that ran out of dimensions may grow on as a wide pass.
 static void grow_tile(const std::vector<HostOp>& ops, const std::vector<char>& done, size_t first, int K,
                       uint64_t lowmask, uint64_t all, int max_ops, Pass& p) {
     p = Pass{};
@@ -1235,9 +1404,10 @@ static void grow_tile(const std::vector<HostOp>& ops, const std::vector<char>& d
 }
 
 static void grow_orbit(const std::vector<HostOp>& ops, const std::vector<char>& done, size_t first, uint64_t all,
-                       int max_ops, Pass& p, int kind = P_ORBIT, int maxdim = kOrbitMax, int minpiv = 0) {
+                       int max_ops, Pass& p, int kind = P_ORBIT, int maxdim = kOrbitMax, int low = 0) {
     p = Pass{};
     p.kind = kind;
+    for (int q = 0; q < low; ++q) p.span.b.push_back(1ull << q);
     uint64_t blocked = 0;
     for (size_t i = first; i < ops.size(); ++i) {
         if (done[i]) continue;
@@ -1248,7 +1418,7 @@ static void grow_orbit(const std::vector<HostOp>& ops, const std::vector<char>& 
             continue;
         }
         Span trial = p.span;
-        if (h.op.kind == K_PEXP && (int)p.ops.size() < max_ops && trial.add(h.op.x, maxdim, minpiv)) {
+        if (h.op.kind == K_PEXP && (int)p.ops.size() < max_ops && trial.add(h.op.x, maxdim)) {
             p.span = trial;
             p.ops.push_back((int)i);
         } else {
@@ -1258,6 +1428,22 @@ static void grow_orbit(const std::vector<HostOp>& ops, const std::vector<char>& 
     }
 }
 
+// Wide passes by default from here on, where a run of exponentials fills the
+// seven dimensions of a lane orbit before its op limit: 400 random strings 635 us
+// against 876 at 13 qubits, 590 / 872 at 16, 873 / 1282 at 20, 2463 / 3363 at 23,
+// 22.5 / 23.9 ms at 26.  Runs that share their masks (UCC) stay on the orbits.
+constexpr int kWideMinQubits = 13;
+// Lowest index bits kept in every wide tile: whole lines where accesses are
+// non-temporal, else one flip more per pass.
+static int wide_low(int n) { return use_nt(n, 3) ? 3 : 2; }
+
+// Every exponential's string has a factor of exactly +-1 or +-i.
+static bool exact_strings(const std::vector<HostOp>& ops) {
+    for (const HostOp& h : ops)
+        if (h.op.kind == K_PEXP && h.op.m[1].x != 0.0 && h.op.m[1].y != 0.0) return false;
+    return true;
+}
+
 static void plan(const std::vector<HostOp>& ops, int n, const Tuning& tu, std::vector<Pass>& passes,
                  bool device_angles) {
     const TileShape shape = tile_shape(tu, n);
@@ -1265,6 +1451,7 @@ static void plan(const std::vector<HostOp>& ops, int n, const Tuning& tu, std::v
     const int L = std::max(std::min(shape.low, K), K - 9);
     const uint64_t all = (n >= 64) ? ~0ull : ((1ull << n) - 1ull);
     const uint64_t lowmask = (L >= 64) ? ~0ull : ((1ull << L) - 1ull);
+    const bool wide_ok = !device_angles && tu.tile_auto && tu.orbit_dims == kLaneOrbitMax && n >= kWideMinQubits && exact_strings(ops);
     std::vector<char> done(ops.size(), 0);
     size_t first = 0;
     while (first < ops.size()) {
@@ -1273,12 +1460,14 @@ static void plan(const std::vector<HostOp>& ops, int n, const Tuning& tu, std::v
         Pass tile, orbit;
         grow_tile(ops, done, first, K, lowmask, all, shape.max_ops, tile);
         grow_orbit(ops, done, first, all, shape.orbit_ops, orbit, P_ORBIT, std::max(1, std::min(tu.orbit_dims, kLaneOrbitMax)));
-        Pass p;
+        Pass p, wide;
+        if (wide_ok && orbit.span.b.size() == (size_t)kLaneOrbitMax && orbit.ops.size() < (size_t)shape.orbit_ops)
+            grow_orbit(ops, done, first, all, shape.orbit_ops, wide, P_WIDE, kWideTile, wide_low(n));
         // an orbit pass at its op limit wins over a longer tile pass (tiles may
         // take more ops than orbits when the shape is chosen by state size)
         const size_t rival = std::min(tile.ops.size(), (size_t)shape.orbit_ops);
         if (orbit.ops.size() >= 2 && orbit.ops.size() >= rival && n > (int)orbit.span.b.size()) {
-            p = std::move(orbit);
+            p = std::move(wide.ops.size() > orbit.ops.size() ? wide : orbit);
         } else if (tile.ops.size() >= 2) {
             p = std::move(tile);
         } else if (device_angles && ops[first].op.kind == K_PEXP && n > (int)orbit.span.b.size()) {
@@ -1397,6 +1586,108 @@ static void build_orbit_lanes(const Pass& p, const std::vector<HostOp>& ops, Lan
         o.ph = g.m[1];
         out.push_back(o);
     }
+}
+
+// Rounds and op data of a wide pass (a pass has at most kWideRounds ops, so
+// rounds).
+static void build_wide(Pass& p, const std::vector<HostOp>& ops, int n, WideDesc& d, std::vector<WideOp>& out) {
+    for (int q = 0; q < n && (int)p.span.b.size() < kWideTile; ++q) (void)p.span.add(1ull << q, kWideTile);
+    std::vector<uint64_t> sv = p.span.b;
+    std::sort(sv.begin(), sv.end());
+    d = WideDesc{};
+    for (int i = 0; i < kWideTile; ++i) d.sv[i] = sv[i];
+    auto local = [&](uint64_t x) {
+        uint32_t r = 0;
+        for (int i = 0; i < kWideTile; ++i) r |= (uint32_t)((x >> (63 - __builtin_clzll(d.sv[i]))) & 1u) << i;
+        return r;
+    };
+    auto global = [&](uint32_t l) {
+        uint64_t x = 0;
+        for (; l; l &= l - 1) x ^= d.sv[__builtin_ctz(l)];
+        return x;
+    };
+    const uint32_t op0 = (uint32_t)out.size();
+    size_t at = 0;
+    while (at < p.ops.size()) {
+        WideRound& R = d.r[d.rounds++];
+        // flips of the round: in order, as long as they are single axes
+        uint32_t e[kWideG], piv[kWideG];
+        int g = 0;
+        auto reduce = [&](uint32_t v) {
+            for (int c = 0; c < g; ++c)
+                if ((v >> piv[c]) & 1u) v ^= e[c];
+            return v;
+        };
+        auto add = [&](uint32_t b, uint32_t v) {
+            const uint32_t t = (uint32_t)(31 - __builtin_clz(v));
+            for (int c = 0; c < g; ++c)
+                if ((e[c] >> t) & 1u) e[c] ^= v;
+            R.b[g] = b;
+            R.off[g] = global(b);
+            e[g] = v;
+            piv[g++] = t;
+        };
+        const size_t from = at;
+        std::vector<int> axis;
+        for (; at < p.ops.size(); ++at) {
+            const uint32_t b = local(ops[p.ops[at]].op.x);
+            int ax = -1;
+            for (int c = 0; c < g; ++c)
+                if (R.b[c] == b) ax = c;
+            if (b && ax < 0) {
+                const uint32_t v = reduce(b);
+                if (!v || g == kWideG) break;
+                ax = g;
+                add(b, v);
+            }
+            axis.push_back(ax);
+        }
+        for (int c = kWideTile; c-- > 0 && g < kWideG;) {
+            const uint32_t v = reduce(1u << c);
+            if (v) add(1u << c, v);
+        }
+        std::copy(piv, piv + kWideG, R.piv);
+        std::sort(R.piv, R.piv + kWideG);
+        R.first = (uint32_t)out.size() - op0;
+        R.count = (uint32_t)(at - from);
+        for (size_t i = from; i < at; ++i) {
+            const DevOp& g0 = ops[p.ops[i]].op;
+            WideOp o{};
+            const bool odd = __builtin_popcountll(g0.x & g0.z) & 1;
+            const int ax = axis[i - from];
+            o.mode = !g0.x ? 0x20u : ((uint32_t)ax | (odd ? 0u : 0x10u));
+            // i * phase = -phase.y (odd strings: phase imaginary) or i * phase.x
+            o.c = g0.m[0].x;
+            o.g = g0.m[0].y * (odd ? -g0.m[1].y : g0.m[1].x);
+            for (int k = 0; k < kWideTile; ++k) o.zl |= (uint32_t)(__builtin_popcountll(d.sv[k] & g0.z) & 1) << k;
+            o.z = g0.z;
+            for (int k = 0; k < kWideE; ++k) {
+                const int from_k = g0.x ? k ^ (1 << ax) : k;  // the sign belongs to the partner
+                uint32_t m = 0;
+                for (int c = 0; c < kWideG; ++c)
+                    if ((from_k >> c) & 1) m ^= R.b[c];
+                o.pat |= (uint32_t)(__builtin_popcount(m & o.zl) & 1) << k;
+            }
+            out.push_back(o);
+        }
+    }
+}
+
+static int launch_wide(qfe_state_s* st, const WideDesc* d, const WideOp* ops) {
+    Context& cx = ctx();
+    constexpr size_t lds = sizeof(double2) << kWideTile;
+    const unsigned blocks = (unsigned)(st->N >> kWideTile);
+    const bool nt = use_nt(st->n, (uint32_t)wide_low(st->n));
+    if (nt)
+        hipLaunchKernelGGL(k_wide<true>, dim3(blocks), dim3(kWideTPB), lds, cx.stream, st->d, d, ops);
+    else
+        hipLaunchKernelGGL(k_wide<false>, dim3(blocks), dim3(kWideTPB), lds, cx.stream, st->d, d, ops);
+    QFE_HIP(hipGetLastError());
+    cx.counters.fused++;
+    cx.counters.orbit++;
+    cx.counters.nt += nt ? 1 : 0;
+    cx.counters.bytes += 32.0 * (double)st->N;
+    return QFE_OK;
 }
 
 // In-lane dimensions of a lane orbit: 2^kLaneBits amplitudes per lane, the
@@ -1710,7 +2001,7 @@ struct OpPlan {
     std::vector<PassDesc> pdescs;
     std::vector<size_t> pass_pd, pass_op0, single_mat, span_d;
     std::vector<OrbitDesc> odescs;
-    size_t off_ops = 0, off_mat = 0, off_orb = 0, off_ld = 0, off_lo = 0, total = 0;
+    size_t off_ops = 0, off_mat = 0, off_orb = 0, off_ld = 0, off_lo = 0, off_wd = 0, off_wo = 0, total = 0;
 };
 
 int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** out, std::vector<char>& image,
@@ -1725,12 +2016,14 @@ int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** 
     plan(ops, n, cx.tuning, passes, device_angles);
 
     // Descriptor image layout: [PassDesc per tile pass][DevOp arrays][U2 matrices for single passes]
-    // [OrbitOp arrays][LaneDesc per lane-orbit pass][OrbitOp2 arrays]
+    // [OrbitOp arrays][LaneDesc per lane-orbit pass][OrbitOp2 arrays][WideDesc per wide pass][WideOp arrays]
     std::vector<DevOp> dops;
     std::vector<double2> mats;
     std::vector<OrbitOp> oops;
     std::vector<LaneDesc> ldescs;
     std::vector<OrbitOp2> lops;
+    std::vector<WideDesc> wdescs;
+    std::vector<WideOp> wops;
     // angle refs by region (0: DevOp, 1: OrbitOp, 2: OrbitOp2) and index, resolved to bytes below
     struct Ref {
         int region;
@@ -1748,7 +2041,7 @@ int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** 
         return fail(code, msg);
     };
     for (size_t pi = 0; pi < passes.size(); ++pi) {
-        const Pass& p = passes[pi];
+        Pass& p = passes[pi];
         if (p.kind == P_SINGLE) {
             const HostOp& h = ops[p.ops[0]];
             if (device_angles && h.op.kind == K_PEXP && h.src >= 0)
@@ -1757,6 +2050,13 @@ int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** 
                 P->single_mat[pi] = mats.size();
                 for (int i = 0; i < 16; ++i) mats.push_back(h.op.m[i]);
             }
+            continue;
+        }
+        if (p.kind == P_WIDE) {
+            P->span_d[pi] = wdescs.size();
+            P->pass_op0[pi] = wops.size();
+            wdescs.emplace_back();
+            build_wide(passes[pi], ops, n, wdescs.back(), wops);
             continue;
         }
         if (p.kind == P_ORBIT && p.span.b.size() > (size_t)kOrbitMax) {
@@ -1824,7 +2124,11 @@ int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** 
     const size_t bytes_ld = ldescs.size() * sizeof(LaneDesc);
     P->off_lo = align_up(P->off_ld + bytes_ld, 256);
     const size_t bytes_lo = lops.size() * sizeof(OrbitOp2);
-    P->total = (bytes_ops || bytes_mat || bytes_orb || bytes_ld) ? P->off_lo + bytes_lo : 0;
+    P->off_wd = align_up(P->off_lo + bytes_lo, 256);
+    const size_t bytes_wd = wdescs.size() * sizeof(WideDesc);
+    P->off_wo = align_up(P->off_wd + bytes_wd, 256);
+    const size_t bytes_wo = wops.size() * sizeof(WideOp);
+    P->total = (bytes_ops || bytes_mat || bytes_orb || bytes_ld || bytes_wd) ? P->off_wo + bytes_wo : 0;
     image.assign(P->total, 0);
     char* host = image.data();
     if (bytes_pd) std::memcpy(host, P->pdescs.data(), bytes_pd);
@@ -1833,6 +2137,8 @@ int plan_build(std::vector<HostOp>& ops_in, int n, bool device_angles, OpPlan** 
     if (bytes_orb) std::memcpy(host + P->off_orb, oops.data(), bytes_orb);
     if (bytes_ld) std::memcpy(host + P->off_ld, ldescs.data(), bytes_ld);
     if (bytes_lo) std::memcpy(host + P->off_lo, lops.data(), bytes_lo);
+    if (bytes_wd) std::memcpy(host + P->off_wd, wdescs.data(), bytes_wd);
+    if (bytes_wo) std::memcpy(host + P->off_wo, wops.data(), bytes_wo);
     angles.clear();
     for (const Ref& r : refs) {
         uint64_t off;
@@ -1856,6 +2162,9 @@ int plan_launch(const OpPlan* P, qfe_state_s* st, char* dev) {
             double2* m = P->single_mat[pi] == (size_t)-1 ? nullptr
                                                          : reinterpret_cast<double2*>(dev + P->off_mat) + P->single_mat[pi];
             rc = launch_single(st, P->ops[p.ops[0]], m);
+        } else if (p.kind == P_WIDE) {
+            rc = launch_wide(st, reinterpret_cast<const WideDesc*>(dev + P->off_wd) + P->span_d[pi],
+                             reinterpret_cast<const WideOp*>(dev + P->off_wo) + P->pass_op0[pi]);
         } else if (p.kind == P_ORBIT && p.span.b.size() > (size_t)kOrbitMax) {
             uint32_t low = 63;
             for (uint64_t v : p.span.b) low = std::min(low, (uint32_t)(63 - __builtin_clzll(v)));
