@@ -146,6 +146,21 @@ int run_ops(qfe_state_s* s, std::vector<HostOp>& ops);
 constexpr int kRoundsMaxQubits = 22;
 int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken);
 
+// One pass of rounds.  sv / wv: stored (source) and target index of tile bit i;
+// sq / wq the same for bit i of the tile's number; w0: the target's constant part.
+constexpr int kRoundTileMax = 12;    // 64 KiB of LDS
+constexpr int kLargeRoundTile = 11;  // tile bits of a pass on a state beyond kRoundsMaxQubits (at most 32 qubits)
+struct RoundsPass {
+    uint32_t k, chunks, w0, low;
+    uint32_t sv[kRoundTileMax], wv[kRoundTileMax];
+    uint32_t sq[32 - kLargeRoundTile], wq[32 - kLargeRoundTile];
+};
+// The gates `take` of a tile pass on the index bits `bits` as rounds, in place;
+// false when one has no such form (words untouched then).
+bool plan_tile_rounds(const std::vector<HostOp>& ops, const std::vector<int>& take, int n, uint32_t bits, RoundsPass& p,
+                      std::vector<uint4>& words);
+int launch_tile_rounds(qfe_state_s* st, const RoundsPass& p, const uint4* words);
+
 // A planned op list kept for replay: the descriptor image (uploaded by the
 // caller to device memory it owns) and the launch sequence over it.  With
 // device_angles every K_PEXP lands in a fused, orbit or lane-orbit pass (never

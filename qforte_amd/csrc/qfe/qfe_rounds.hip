@@ -23,6 +23,11 @@
 // at one wave per SIMD).  500 random gates on 12 qubits are 28 rounds in one
 // launch of one workgroup, 55 us (15 launches of gate-by-gate 8-qubit tiles on
 // 16 workgroups: 374 us); 800 on 17 qubits seven launches of 18 us (27 of 30 us).
+// On states beyond 22 qubits every tile pass is planned on its own and works in
+// place (a move's target lies in the tile, so its frame stays in the coset), with
+// 11-bit tiles, three flips a round and 8 amplitudes per thread: four waves per
+// SIMD hide the rounds' chain behind the other tiles' loads.  Brickwork of 4 layers at 29 qubits: four passes of 7.1 ms
+// (nine of 4.6 ms gate by gate; a bare read and write takes 3.4 ms).
 // Tiles of 11 or 13 bits (2^(k - 4) threads) were level or slower from 15 qubits
 // on: 13 bits halve the workgroups, 11 bits add passes.  64-byte runs against 128:
 // 15-20 qubits 2-10 % faster, since a pass has one more free flip.
@@ -41,10 +46,9 @@ namespace qfe {
 
 namespace {
 
-constexpr int kRoundDims = 4;                        // rotations' flips per round: 16 amplitudes per thread
-constexpr int kRoundTileMax = 12;                    // k: 64 KiB of LDS
+constexpr int kRoundDims = 4;                        // flips per round: 16 amplitudes per thread
+constexpr int kLargeDims = kLargeRoundTile - 8;      // on large states, where waves matter more: 8 amplitudes
 constexpr int kRoundLow = 2;                         // lowest index bits in every tile: runs of 64 bytes
-constexpr int kRoundOut = kRoundsMaxQubits - kRoundTileMax;  // tile numbers have at most this many bits
 constexpr int kOrbitBits = kRoundTileMax - kRoundDims;  // a full tile has 2^8 orbits of 16,
 constexpr int kRoundTPB = 1 << kOrbitBits;              // one per thread
 constexpr uint32_t kChunkWords = 2 * kRoundTPB;      // 8 KiB of the program staged in LDS at a time
@@ -52,14 +56,6 @@ constexpr uint32_t kRoundWords = 6;                  // 16-byte words of a round
 constexpr uint32_t kPhaseWords = 17, kRotWords = 2;  // of a phase table and of a further rotation
 constexpr int kPhaseBits = 4;                        // parities of one phase table (16 factors)
 constexpr int kPhasesMax = 16, kRotsMax = 16;        // gates per round: 6 + 16 * 17 + 16 * 2 words fit a chunk
-
-// One pass.  sv / wv: stored (source) and target index of tile bit i; sq / wq
-// the same for bit i of the tile's number; w0: the target's constant part.
-struct RoundsPass {
-    uint32_t k, chunks, w0;
-    uint32_t sv[kRoundTileMax], wv[kRoundTileMax];
-    uint32_t sq[kRoundOut], wq[kRoundOut];
-};
 
 __device__ __forceinline__ uint32_t parity32(uint32_t v) { return (uint32_t)__popc(v) & 1u; }
 __device__ __forceinline__ uint32_t sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
@@ -170,14 +166,16 @@ __device__ __forceinline__ void round_body(double2* tile, const uint4* buf, uint
     for (int i = 0; i < (1 << G); ++i) tile[q[i]] = a[i];
 }
 
-__global__ __launch_bounds__(kRoundTPB) void k_rounds(const double2* src, double2* dst, const RoundsPass P,
+// DIMS: most flips of a round (registers); NT: non-temporal accesses.
+template <int DIMS, bool NT>
+__global__ __launch_bounds__(kRoundTPB) __attribute__((amdgpu_waves_per_eu(DIMS > 3 ? 2 : 4))) void k_rounds(const double2* src, double2* dst, const RoundsPass P,
                                                       const uint4* __restrict__ prog) {
     extern __shared__ double2 tile[];
-    const uint32_t T = 1u << P.k, tid = threadIdx.x, number = blockIdx.x;
+    const uint32_t T = 1u << P.k, tid = threadIdx.x, number = (uint32_t)xcd_block();
     uint4* buf = reinterpret_cast<uint4*>(tile + T);
     uint32_t sb = 0, wb = P.w0;
 #pragma unroll
-    for (int u = 0; u < kRoundOut; ++u) {
+    for (int u = 0; u < 32 - kLargeRoundTile; ++u) {
         sb ^= ((number >> u) & 1u) ? P.sq[u] : 0u;
         wb ^= ((number >> u) & 1u) ? P.wq[u] : 0u;
     }
@@ -201,7 +199,7 @@ __global__ __launch_bounds__(kRoundTPB) void k_rounds(const double2* src, double
     const uint32_t rows = (T + kRoundTPB - 1) / kRoundTPB;
 #pragma unroll 8
     for (uint32_t r = 0; r < rows; ++r)
-        if (tid < T) tile[tid + r * kRoundTPB] = src[sb ^ upper(r, P.sv)];
+        if (tid < T) tile[tid + r * kRoundTPB] = ld_s<NT>(src + (sb ^ upper(r, P.sv)));
     for (uint32_t c = 0; c < P.chunks; ++c) {
         // the rounds of the chunk before have ended (their last barrier)
         buf[tid] = next0;
@@ -221,17 +219,19 @@ __global__ __launch_bounds__(kRoundTPB) void k_rounds(const double2* src, double
                 case 1: round_body<1>(tile, buf, at, h, P.k, number); break;
                 case 2: round_body<2>(tile, buf, at, h, P.k, number); break;
                 case 3: round_body<3>(tile, buf, at, h, P.k, number); break;
-                default: round_body<4>(tile, buf, at, h, P.k, number); break;
+                default:
+                    if constexpr (DIMS > 3) round_body<4>(tile, buf, at, h, P.k, number);
+                    break;
             }
             at += kRoundWords + ((h.x >> 8) & 0xFFu) * kPhaseWords + ((h.x >> 16) & 0xFFu) * kRotWords;
-            h = buf[at];  // the next header, or the word behind the chunk
+            h = buf[min(at, kChunkWords - 1u)];  // the next header, if there is one
             __syncthreads();
         }
     }
     __syncthreads();
 #pragma unroll 8
     for (uint32_t r = 0; r < rows; ++r)
-        if (tid < T) dst[wb ^ upper(r, P.wv)] = tile[tid + r * kRoundTPB];
+        if (tid < T) st_s<NT>(dst + (wb ^ upper(r, P.wv)), tile[tid + r * kRoundTPB]);
 }
 
 // ---- host: gates to rotations and phases in stored coordinates ------------------------
@@ -436,26 +436,31 @@ struct RoundPlan {
 
 class RoundPlanner {
   public:
-    RoundPlanner(const std::vector<RoundOp>& o, int n, int k, int low) : ops_(o), n_(n), k_(std::min(n, k)), low_(low) {}
-
-    void run(RoundPlan& plan) {
+    RoundPlanner(const std::vector<RoundOp>& o, int n, int k, int low, int dims)
+        : ops_(o), n_(n), k_(std::min(n, k)), low_(low), dims_(dims) {
         for (auto& w : wx_) w = 0;
         for (auto& w : conf_) w = 0;
         for (auto& w : wf_) w = 0;
         for (auto& w : wg_) w = 0;
         fill();
+    }
+
+
+    void run(RoundPlan& plan) {
         while (pending_) {
             basis_.clear();
             for (int q = 0; q < (n_ > k_ ? std::min(low_, k_) : k_); ++q) basis_.push_back(1u << q);
-            rounds_.clear();
-            out_ = 0;
-            for (;;) {
-                Round r;
-                if (!form(r)) break;
-                rounds_.push_back(std::move(r));
-            }
+            collect();
             emit(plan);
         }
+    }
+    // one pass over the given index bits; false when it does not take every op
+    bool run_on(RoundPlan& plan, uint32_t bits) {
+        for (uint32_t m = bits; m; m &= m - 1) basis_.push_back(m & (0u - m));
+        collect();
+        if (pending_) return false;
+        emit(plan);
+        return true;
     }
     // a pass without rounds
     void empty(RoundPlan& plan) {
@@ -465,6 +470,15 @@ class RoundPlanner {
     }
 
   private:
+    void collect() {
+        rounds_.clear();
+        out_ = 0;
+        for (;;) {
+            Round r;
+            if (!form(r)) break;
+            rounds_.push_back(r);
+        }
+    }
     // Slot s of the window holds op slot_[s]; a word per index bit over the
     // slots makes one op's parities against all of them a few XORs.
     void fill() {
@@ -566,7 +580,7 @@ class RoundPlanner {
                 r.rots[r.nrots++] = slot_[s];
                 return true;
             }
-        if (r.g == kRoundDims) return false;
+        if (r.g == dims_) return false;
         if (par(o.x & o.f1)) return false;
         for (int d = 0; d < r.g; ++d)
             if (par(r.b[d] & o.f0) | par(o.x & r.f[d]) | par(r.b[d] & o.f1)) return false;
@@ -610,7 +624,7 @@ class RoundPlanner {
             }
         // functional -> tile bits, then bits of the tile's number (linear: one
         // word per index bit); flip -> tile bits
-        uint32_t reads[kRoundsMaxQubits];
+        uint32_t reads[32];
         for (int q = 0; q < n_; ++q) {
             reads[q] = 0;
             for (int i = 0; i < k_; ++i) reads[q] |= ((p.sv[i] >> q) & 1u) << i;
@@ -769,7 +783,7 @@ class RoundPlanner {
     }
 
     const std::vector<RoundOp>& ops_;
-    int n_, k_, low_;
+    int n_, k_, low_, dims_;
     size_t next_ = 0;
     uint64_t pending_ = 0, out_ = 0, conf_[64];
     uint32_t slot_[64];
@@ -778,6 +792,18 @@ class RoundPlanner {
     std::vector<Round> rounds_;
     std::vector<uint4> scratch_;
 };
+
+// Let the pass store every amplitude at its logical index.
+void to_logical(const FrameLowering& fl, RoundsPass& p) {
+    auto logical = [&](uint32_t v) {
+        uint32_t l = 0;
+        for (int q = 0; q < fl.n; ++q) l |= par(fl.row[q] & v) << q;
+        return l;
+    };
+    for (uint32_t& v : p.wv) v = logical(v);
+    for (uint32_t& v : p.wq) v = logical(v);
+    p.w0 = fl.neg;
+}
 
 // Passes and program of an op list; false when an op has no such form.  The
 // stored index that the last pass leaves differs from the logical one unless
@@ -791,26 +817,56 @@ bool plan_rounds(const std::vector<HostOp>& ops, int n, RoundPlan& plan, bool& p
         if (!fl.flush(q)) return false;
     plain = fl.neg == 0;
     for (int q = 0; q < n; ++q) plain = plain && fl.col[q] == 1u << q;
-    RoundPlanner pl(fl.out, n, kRoundTileMax, kRoundLow);
+    RoundPlanner pl(fl.out, n, kRoundTileMax, kRoundLow, kRoundDims);
     pl.run(plan);
     if (plain) return true;
     // one tile moves its amplitudes by itself; more need a second buffer, so
     // the first pass stores there and the last pass comes back
     const size_t least = n > kRoundTileMax ? 2 : 1;
     while (plan.passes.size() < least) pl.empty(plan);
-    RoundsPass& last = plan.passes.back();
-    auto logical = [&](uint32_t p) {
-        uint32_t l = 0;
-        for (int q = 0; q < n; ++q) l |= par(fl.row[q] & p) << q;
-        return l;
-    };
-    for (uint32_t& v : last.wv) v = logical(v);
-    for (uint32_t& v : last.wq) v = logical(v);
-    last.w0 = fl.neg;
+    to_logical(fl, plan.passes.back());
     return true;
 }
 
+template <int DIMS, bool NT>
+int launch_rounds(qfe_state_s* st, const double2* src, double2* dst, const RoundsPass& p, const uint4* prog) {
+    Context& cx = ctx();
+    constexpr int tile = kOrbitBits + DIMS;
+    static const hipError_t big = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rounds<DIMS, NT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      (sizeof(double2) << tile) + kChunkWords * sizeof(uint4));
+    QFE_HIP(big);
+    hipLaunchKernelGGL((k_rounds<DIMS, NT>), dim3(1u << (st->n - (int)p.k)), dim3(kRoundTPB),
+                       (sizeof(double2) << p.k) + kChunkWords * sizeof(uint4), cx.stream, src, dst, p, prog);
+    QFE_HIP(hipGetLastError());
+    cx.counters.fused++;
+    cx.counters.tile++;
+    cx.counters.nt += NT ? 1 : 0;
+    cx.counters.bytes += 32.0 * (double)st->N;
+    return QFE_OK;
+}
+
 }  // namespace
+
+bool plan_tile_rounds(const std::vector<HostOp>& ops, const std::vector<int>& take, int n, uint32_t bits, RoundsPass& p,
+                      std::vector<uint4>& words) {
+    FrameLowering fl(n);
+    for (int i : take)
+        if (!fl.add(ops[i].op)) return false;
+    for (int q = 0; q < n; ++q)
+        if (!fl.flush(q)) return false;
+    RoundPlan plan;
+    RoundPlanner pl(fl.out, n, __builtin_popcount(bits), 0, kLargeDims);
+    if (!pl.run_on(plan, bits)) return false;
+    p = plan.passes[0];
+    to_logical(fl, p);
+    words.insert(words.end(), plan.words.begin(), plan.words.end());
+    return true;
+}
+
+int launch_tile_rounds(qfe_state_s* st, const RoundsPass& p, const uint4* words) {
+    return use_nt(st->n, (uint32_t)p.low) ? launch_rounds<kLargeDims, true>(st, st->d, st->d, p, words)
+                                          : launch_rounds<kLargeDims, false>(st, st->d, st->d, p, words);
+}
 
 int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken) {
     taken = false;
@@ -842,20 +898,12 @@ int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken) {
         if (rc) return rc;
         prog = static_cast<const uint4*>(dev);
     }
-    const size_t lds = (sizeof(double2) << k) + (kChunkWords + 1) * sizeof(uint4);
-    static const hipError_t big = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rounds), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                      (sizeof(double2) << kRoundTileMax) + (kChunkWords + 1) * sizeof(uint4));
-    QFE_HIP(big);
     for (size_t i = 0; i < plan.passes.size(); ++i) {
         const RoundsPass& p = plan.passes[i];
         const double2* src = i == 0 ? st->d : other;
         double2* dst = i + 1 == plan.passes.size() ? st->d : other;
-        hipLaunchKernelGGL(k_rounds, dim3(1u << (st->n - k)), dim3(kRoundTPB), lds, cx.stream, src, dst, p,
-                           p.chunks ? prog + (size_t)plan.first[i] * kChunkWords : nullptr);
-        QFE_HIP(hipGetLastError());
-        cx.counters.fused++;
-        cx.counters.tile++;
-        cx.counters.bytes += 32.0 * (double)st->N;
+        rc = launch_rounds<kRoundDims, false>(st, src, dst, p, p.chunks ? prog + (size_t)plan.first[i] * kChunkWords : nullptr);
+        if (rc) return rc;
     }
     return QFE_OK;
 }
