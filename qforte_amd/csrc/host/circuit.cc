@@ -41,10 +41,14 @@ PauliForm Circuit::pauli_form() const {
     return f;
 }
 
-void Circuit::add_circuit(const Circuit& c) {
+void Circuit::append_gates(const Circuit& c) {
     if (form_known_) form_.apply(c.pauli_form());
-    const size_t off = gates_.size();
     gates_.insert(gates_.end(), c.gates_.begin(), c.gates_.end());
+}
+
+void Circuit::add_circuit(const Circuit& c) {
+    const size_t off = gates_.size();
+    append_gates(c);
     for (ExpSegment s : c.segs_) {
         s.begin += off;
         s.end += off;
@@ -170,6 +174,7 @@ cplx Circuit::canonicalize_pauli_circuit() {
             "Circuit::canonicalize_pauli_circuit is undefined for circuits with gates other than X, Y, or Z");
     std::stable_sort(gates_.begin(), gates_.end(), [](const Gate& a, const Gate& b) { return a.target() < b.target(); });
     std::vector<Gate> out;
+    PauliForm form;
     cplx coeff = 1.0;
     size_t i = 0;
     while (i < gates_.size()) {
@@ -181,13 +186,19 @@ cplx Circuit::canonicalize_pauli_circuit() {
             coeff *= pr.first;
             acc = pr.second;
         }
-        if (acc != 'I') out.push_back(make_gate(std::string(1, acc), q, q));
+        if (acc != 'I') {
+            out.push_back(make_gate(std::string(1, acc), q, q));
+            const uint64_t bit = q < 64 ? 1ull << q : 0ull;
+            form.pauli = form.pauli && bit;
+            if (acc != 'Z') form.x |= bit;
+            if (acc != 'X') form.z |= bit;
+            form.power = (form.power + (acc == 'Y' ? 1 : 0)) & 3;
+        }
         i = j;
     }
     gates_ = std::move(out);
     segs_.clear();
-    form_ = PauliForm();
-    for (const auto& g : gates_) form_.apply(g);
+    form_ = form;
     form_known_ = true;
     return coeff;
 }
@@ -286,8 +297,9 @@ void QubitOperator::operator_product(const QubitOperator& r, bool pre_simplify, 
     for (const auto& tl : terms_)
         for (const auto& tr : r.terms_) {
             Circuit c;
-            for (const auto& g : tl.second.gates()) c.add_gate(g);
-            for (const auto& g : tr.second.gates()) c.add_gate(g);
+            c.reserve(tl.second.size() + tr.second.size());
+            c.append_gates(tl.second);
+            c.append_gates(tr.second);
             prod.emplace_back(tl.first * tr.first, std::move(c));
         }
     terms_ = std::move(prod);

@@ -117,6 +117,8 @@ class Circuit {
         if (form_known_) form_.apply(g);
     }
     void add_circuit(const Circuit& c);
+    void append_gates(const Circuit& c);  // without its segments
+    void reserve(size_t gates) { gates_.reserve(gates); }
     void insert_gate(size_t pos, const Gate& g);
     void remove_gate(size_t pos);
     void swap_gates(size_t p1, size_t p2);
