@@ -7,12 +7,14 @@ the state size, so the tuner times candidates on the caller's own circuits,
 applied to a replica state of ``probe_qubits`` qubits (the circuits must act
 only on those qubits), with HIP events on the engine stream, and keeps the
 fastest.  Orbit width is chosen on the exponential circuits, the tile shape on
-the gate circuits, each with the other knob at its current value.
+the gate circuits, each with the other knob at its current value.  The first
+tile candidate is the planner's own choice by state size, which alone runs gate
+lists as rounds and wide exponential passes; an explicit shape turns both off.
 """
 
 import json
 
-DEFAULT_TILES = ((10, 4, 16), (11, 4, 16), (11, 4, 24), (11, 4, 32), (12, 4, 32))
+DEFAULT_TILES = ((-1, -1, -1), (10, 4, 16), (11, 4, 16), (11, 4, 24), (11, 4, 32), (12, 4, 32))
 DEFAULT_ORBITS = (4, 5, 6, 7)
 
 
