@@ -29,7 +29,7 @@ struct Tuning {
     int low_qubits = 4;    // L: lowest qubits always in the tile (contiguous 2^L runs)
     int max_ops = 24;      // ops per fused pass before LDS traffic dominates
     int orbit_dims = 7;    // max dimensions of a register orbit (5, 6, 7: spread over 2, 4 or 8 lanes)
-    uint64_t sector_words = 1ull << 25;  // max pair words of one sector template (256 MB)
+    uint64_t sector_words = 1ull << 25;  // accepted and kept; templates store no pair words
 };
 
 // Pass shape for a state of n qubits: the explicit tuning, or by default the

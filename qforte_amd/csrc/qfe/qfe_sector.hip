@@ -2945,11 +2945,9 @@ int lane_launch(qfe_batch b, Lane& L) {
     std::deque<Request>& queue = grad ? qg : qe;
     // admit from the front of the queue while the footprint fits this lane's
     // share.  A tier-2 launch holds requests of one sector dimension, that of
-    // its oldest request: a tier-2 request runs its whole ansatz chain in one
-    // workgroup, and the launch ends with its longest chain (alone, 1.7 ms for
-    // an 18-qubit and 6.6 ms for a 20-qubit UCCSD energy), so shorter requests
-    // would otherwise wait for the longest; requests of other dimensions keep
-    // their place in the queue.
+    // its oldest request: a launch ends with its largest request, and the
+    // shorter ones would wait for it; requests of other dimensions keep their
+    // place in the queue.
     const uint64_t share = std::min<uint64_t>(b->budget / kLanes, kLaunchFootprint);
     const bool one_dim = L.tier == 2;
     const uint64_t dim0 = queue.front().t->D;
