@@ -276,13 +276,14 @@ struct FrameLowering {
     uint32_t col[32], row[32];
     uint32_t neg = 0;  // bit q: logical qubit q reads inverted
     double2 acc[32][4];
-    uint8_t kind[32];  // of acc: 0 identity, 1 diagonal, 2 antidiagonal, 3 dense
+    uint8_t kind[32];   // of acc: 0 identity, 1 diagonal, 2 antidiagonal, 3 dense
+    uint8_t chain[32];  // gates multiplied since the last split for length
     std::vector<RoundOp> out;
 
     explicit FrameLowering(int nq) : n(nq) {
         for (int q = 0; q < n; ++q) {
             col[q] = row[q] = 1u << q;
-            kind[q] = 0;
+            kind[q] = chain[q] = 0;
         }
     }
     void classify(int q) {
@@ -375,6 +376,7 @@ struct FrameLowering {
             std::swap(row[t], row[c]);
             std::swap(col[t], col[c]);
             std::swap(kind[t], kind[c]);
+            std::swap(chain[t], chain[c]);
             for (int i = 0; i < 4; ++i) std::swap(acc[t][i], acc[c][i]);
             const uint32_t d = ((neg >> t) ^ (neg >> c)) & 1u;
             neg ^= (d << t) | (d << c);
@@ -384,6 +386,12 @@ struct FrameLowering {
         const double2 diag[4] = {o.m[0], z, z, o.m[1]};
         const double2* m = o.kind == K_DIAG1 ? diag : o.m;
         if (!o.cmask) {
+            // a long product drifts from unitary by its roundings: split it off
+            // well before split_rotation's bound
+            if (++chain[t] > 16) {
+                if (!flush(t)) return false;
+                chain[t] = 1;
+            }
             multiply(t, m);
             return true;
         }
