@@ -2230,10 +2230,10 @@ void plan_free(OpPlan* p) { delete p; }
 // multi-tile circuit is then at most 64 MiB), by default only: explicit tile
 // shapes are honoured.  Few gates stay on the streaming and tile passes, which
 // need no second buffer and no move back.  500 random gates, rounds against
-// tiles: 87 / 457 us at 3 qubits, 101 / 525 at 12, 152 / 641 at 18, 291 / 1846 at
-// 22; 25 gates: 43 / 61 us at 20, 69 / 126 at 22; one layer of rotations and CNOTs:
-// 33 / 38 us at 12, 48 / 52 at 17, 117 / 138 at 22; 8 gates: 25 / 25 us at 12,
-// 30 / 27 at 17, 65 / 57 at 22.
+// tiles: 112 / 460 us at 3 qubits, 127 / 525 at 12, 170 / 640 at 18, 347 / 1837 at
+// 22; 25 gates: 30 / 41 us at 12, 40 / 49 at 17, 72 / 125 at 22; one layer of
+// rotations and CNOTs: 36 / 37 us at 12, 50 / 52 at 17, 73 / 71 at 20, 110 / 139 at
+// 22; 8 gates (by rounds up to 12): 25 / 25 us at 12.
 static bool takes_rounds(const Tuning& tu, int n, size_t ops) {
     return tu.tile_auto && n <= kRoundsMaxQubits && ops >= (n <= 12 ? 8u : 24u);
 }
