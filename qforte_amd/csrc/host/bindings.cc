@@ -7,6 +7,7 @@
 #include <pybind11/stl.h>
 
 #include <algorithm>
+#include <functional>
 #include <memory>
 #include <unordered_map>
 
@@ -21,8 +22,35 @@ using namespace qfa;
 // read directly instead of through a Python object per element.
 struct Doubles : std::vector<double> {};
 
+// Operators of a call as the mask forms of their terms, operator k's at
+// [off[k], off[k + 1]).  Accepts what std::vector<QubitOperator> does.  Each
+// operator is read where the caster has it in hand: copying it would copy
+// every term's gates, and the items of a generator or of a sequence made on
+// access are gone by the time of the call.
+struct OperatorTerms {
+    std::vector<qfe_pauli> terms;
+    std::vector<uint64_t> off{0};
+    bool pauli = true;  // every operator is a Pauli sum
+    void clear() {
+        terms.clear();
+        off.assign(1, 0);
+        pauli = true;
+    }
+    void reserve(size_t operators) {
+        off.reserve(operators + 1);
+        terms.reserve(8 * operators);  // strings of a double excitation
+    }
+    void push_back(const QubitOperator& o) {
+        pauli = pauli && append_pauli_sum(o, terms);
+        off.push_back(terms.size());
+    }
+    size_t size() const { return off.size() - 1; }
+};
+
 namespace pybind11 {
 namespace detail {
+template <>
+struct type_caster<OperatorTerms> : list_caster<OperatorTerms, std::reference_wrapper<const QubitOperator>> {};
 template <>
 struct type_caster<Doubles> {
     PYBIND11_TYPE_CASTER(Doubles, const_name("List[float]"));
@@ -82,25 +110,6 @@ void set_coeffs_from(Computer& c, py::object obj) {
     if (!arr) throw std::invalid_argument("set_coeff_vec: expected a sequence of complex numbers");
     py::gil_scoped_release rel;
     c.set_coeff_vec(arr.data(), (size_t)arr.size());
-}
-
-// Operators of a call, by reference: copying them copies every term's gates.
-using OperatorList = std::vector<std::reference_wrapper<const QubitOperator>>;
-
-// The mask forms of several operators, operator k's terms at [off[k], off[k + 1]).
-bool compile_operators(const OperatorList& ops, std::vector<qfe_pauli>& terms, std::vector<uint64_t>& off) {
-    size_t n = 0;
-    for (const QubitOperator& o : ops) n += o.terms().size();
-    terms.clear();
-    terms.reserve(n);
-    off.assign(1, 0);
-    std::vector<qfe_pauli> one;
-    for (const QubitOperator& o : ops) {
-        if (!compile_pauli_sum(o, one)) return false;
-        terms.insert(terms.end(), one.begin(), one.end());
-        off.push_back(terms.size());
-    }
-    return true;
 }
 
 // ---- compiled UCC program -----------------------------------------------------------
@@ -167,15 +176,12 @@ class UCCProgram {
               "UCCProgram.residuals");
         return out;
     }
-    std::vector<double> pool_gradients(const Doubles& t, const OperatorList& ops,
-                                       size_t batch) {
+    std::vector<double> pool_gradients(const Doubles& t, const OperatorTerms& ops, size_t batch) {
         need(t);
-        std::vector<qfe_pauli> terms;
-        std::vector<uint64_t> off;
-        if (!compile_operators(ops, terms, off)) throw std::invalid_argument("pool_gradients: operators must be Pauli sums");
+        if (!ops.pauli) throw std::invalid_argument("pool_gradients: operators must be Pauli sums");
         std::vector<double> out(ops.size());
         py::gil_scoped_release rel;
-        check(qfe_program_pool_gradients(p_, t.data(), terms.data(), off.data(), ops.size(), batch, out.data()),
+        check(qfe_program_pool_gradients(p_, t.data(), ops.terms.data(), ops.off.data(), ops.size(), batch, out.data()),
               "UCCProgram.pool_gradients");
         return out;
     }
@@ -260,15 +266,12 @@ class SectorTemplate {
               "SectorTemplate.residuals");
         return out;
     }
-    std::vector<double> pool_gradients(const Doubles& t, const OperatorList& ops, size_t batch, const Doubles& inputs) {
+    std::vector<double> pool_gradients(const Doubles& t, const OperatorTerms& ops, size_t batch, const Doubles& inputs) {
         need(t, inputs);
-        std::vector<qfe_pauli> terms;
-        std::vector<uint64_t> off;
-        if (!compile_operators(ops, terms, off))
-            throw std::invalid_argument("SectorTemplate.pool_gradients: operators must be Pauli sums");
+        if (!ops.pauli) throw std::invalid_argument("SectorTemplate.pool_gradients: operators must be Pauli sums");
         std::vector<double> out(ops.size());
         py::gil_scoped_release rel;
-        check(qfe_template_pool_gradients(t_, t.data(), inputs.data(), terms.data(), off.data(), ops.size(), batch,
+        check(qfe_template_pool_gradients(t_, t.data(), inputs.data(), ops.terms.data(), ops.off.data(), ops.size(), batch,
                                           out.data()),
               "SectorTemplate.pool_gradients");
         return out;
@@ -625,15 +628,13 @@ PYBIND11_MODULE(_core, m) {
         return comp;
     }, "gate"_a, "computer"_a);
     m.def("inner_product", &qfa::dot, "a"_a, "b"_a);
-    m.def("cross_expectations", [](const Computer& bra, const Computer& ket, const OperatorList& ops) {
+    m.def("cross_expectations", [](const Computer& bra, const Computer& ket, const OperatorTerms& ops) {
         // <bra|O_k|ket> for every Pauli-sum operator O_k, one device launch
-        std::vector<qfe_pauli> terms;
-        std::vector<uint64_t> off;
-        if (!compile_operators(ops, terms, off)) throw std::invalid_argument("cross_expectations: operators must be Pauli sums");
+        if (!ops.pauli) throw std::invalid_argument("cross_expectations: operators must be Pauli sums");
         std::vector<qfe_c64> r(ops.size());
         {
             py::gil_scoped_release rel;
-            check(qfe_cross_expval_many(bra.handle(), ket.handle(), terms.data(), off.data(), ops.size(), r.data()),
+            check(qfe_cross_expval_many(bra.handle(), ket.handle(), ops.terms.data(), ops.off.data(), ops.size(), r.data()),
                   "cross_expectations");
         }
         std::vector<std::complex<double>> out;

@@ -338,6 +338,10 @@ size_t QubitOperator::num_qubits() const {
 bool compile_pauli_sum(const QubitOperator& op, std::vector<qfe_pauli>& out, cplx mult) {
     out.clear();
     out.reserve(op.terms().size());
+    return append_pauli_sum(op, out, mult);
+}
+
+bool append_pauli_sum(const QubitOperator& op, std::vector<qfe_pauli>& out, cplx mult) {
     for (const auto& t : op.terms()) {
         uint64_t x, z;
         cplx ph;

@@ -329,6 +329,8 @@ void check(int rc, const char* what);
 
 // Compile a QubitOperator whose terms are all Pauli circuits; false if not.
 bool compile_pauli_sum(const QubitOperator& op, std::vector<qfe_pauli>& out, cplx mult = 1.0);
+// The same, behind what `out` holds.
+bool append_pauli_sum(const QubitOperator& op, std::vector<qfe_pauli>& out, cplx mult = 1.0);
 
 // The JW-mapped molecular Hamiltonian of norb spatial orbitals as a linear
 // map from integrals to Pauli coefficients: term k is M(x_k, z_k) with
