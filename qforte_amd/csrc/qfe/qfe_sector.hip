@@ -1925,18 +1925,52 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     }
 
     t->has_map = map_off != nullptr;
+    // Hamiltonian terms by X mask (first appearance).  A flip connects
+    // determinants of the sector when each spin has room for it: half of its
+    // bits occupied, half empty.  The other masks are read by nothing.
+    std::map<uint64_t, std::vector<uint64_t>> byx;
+    std::vector<uint64_t> order;
+    {
+        const int ne[2] = {popc32(refa), popc32(refb)};
+        auto connects = [&](uint64_t x) {
+            for (int s = 0; s < 2; ++s) {
+                const int m = popc32(compress(x, s, norb));
+                if ((m & 1) || m / 2 > ne[s] || m / 2 > norb - ne[s]) return false;
+            }
+            return true;
+        };
+        for (uint64_t k = 0; k < nham; ++k) {
+            if ((ham[k].x | ham[k].z) & ~lim)
+                return fail(QFE_ERR_ARG, "qfe_template_create: Hamiltonian term acts on a qubit out of range");
+            if (!connects(ham[k].x)) continue;
+            auto& v = byx[ham[k].x];
+            if (v.empty()) order.push_back(ham[k].x);
+            v.push_back(k);
+        }
+    }
+    // the map of every such term, before anything reads it
+    if (map_off)
+        for (uint64_t x : order)
+            for (uint64_t k : byx[x]) {
+                if (map_off[k + 1] < map_off[k]) return fail(QFE_ERR_ARG, "qfe_template_create: map offsets must not decrease");
+                for (uint64_t e = map_off[k]; e < map_off[k + 1]; ++e)
+                    if (map_idx[e] >= ninputs) return fail(QFE_ERR_ARG, "qfe_template_create: map index out of range");
+            }
     t->real = true;
     for (const auto& en : entries) t->real = t->real && en.ulo.y == 0.0 && en.uhi.y == 0.0;
-    for (uint64_t k = 0; k < nham; ++k)
-        t->real = t->real && (t->has_map ? ham[k].phase.im == 0.0
-                                         : cplx_mul(make_double2(ham[k].phase.re, ham[k].phase.im),
-                                                    make_double2(ham[k].coeff.re, ham[k].coeff.im)).y == 0.0);
-    if (t->has_map)
-        for (uint64_t e = 0; e < map_off[nham]; ++e) t->real = t->real && map_val[e].im == 0.0;
+    for (uint64_t x : order)
+        for (uint64_t k : byx[x]) {
+            if (!t->has_map) {
+                t->real = t->real && cplx_mul(make_double2(ham[k].phase.re, ham[k].phase.im),
+                                              make_double2(ham[k].coeff.re, ham[k].coeff.im)).y == 0.0;
+                continue;
+            }
+            t->real = t->real && ham[k].phase.im == 0.0;
+            for (uint64_t e = map_off[k]; e < map_off[k + 1]; ++e) t->real = t->real && map_val[e].im == 0.0;
+        }
     RowBuilder rowb(sp, norb);
     std::set<uint64_t> in_rows;
 
-    // Hamiltonian: groups by X mask (first appearance), sector pairs only
     std::vector<SecGroup> groups;
     std::vector<uint64_t> tz;
     std::vector<double2> tph, tcoef;
@@ -1944,20 +1978,11 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     std::vector<uint32_t> midx;
     std::vector<double2> mval;
     {
-        std::map<uint64_t, std::vector<uint64_t>> byx;
-        std::vector<uint64_t> order;
-        for (uint64_t k = 0; k < nham; ++k) {
-            if ((ham[k].x | ham[k].z) & ~lim)
-                return fail(QFE_ERR_ARG, "qfe_template_create: Hamiltonian term acts on a qubit out of range");
-            auto& v = byx[ham[k].x];
-            if (v.empty()) order.push_back(ham[k].x);
-            v.push_back(k);
-        }
         // groups that the rows take, in a real template
         std::vector<RowBuilder::Group> rgroups;
         for (uint64_t x : order) {
+            if (!t->real) break;
             RowBuilder::Group g{x, compress(x, 0, norb), compress(x, 1, norb), {}};
-            if (!t->real || (popc32(g.xa) & 1) || (popc32(g.xb) & 1)) continue;
             for (uint64_t k : byx[x]) g.terms.push_back({compress(ham[k].z, 0, norb), compress(ham[k].z, 1, norb), (uint32_t)k});
             if (rowb.fits(g)) rgroups.push_back(std::move(g));
         }
@@ -1973,7 +1998,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
         for (uint64_t x : order) {
             if (in_rows.count(x)) continue;
             const uint32_t xa = compress(x, 0, norb), xb = compress(x, 1, norb);
-            if ((popc32(xa) & 1) || (popc32(xb) & 1)) continue;  // never connects two sector determinants
             SecGroup gr{};
             gr.x = x;
             gr.xa = xa;
@@ -1996,7 +2020,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
                 }
                 gr.weight = 2.0;
             }
-            if (!la.second || !lb.second) continue;
             gr.la_off = la.first;
             gr.la_len = la.second;
             gr.lb_off = lb.first;
@@ -2009,9 +2032,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
                 tph.push_back(ph);
                 tcoef.push_back(cplx_mul(ph, make_double2(ham[k].coeff.re, ham[k].coeff.im)));
                 if (map_off) {
-                    if (map_off[k + 1] < map_off[k]) return fail(QFE_ERR_ARG, "qfe_template_create: map offsets must not decrease");
                     for (uint64_t e = map_off[k]; e < map_off[k + 1]; ++e) {
-                        if (map_idx[e] >= ninputs) return fail(QFE_ERR_ARG, "qfe_template_create: map index out of range");
                         midx.push_back(map_idx[e]);
                         mval.push_back(make_double2(map_val[e].re, map_val[e].im));
                     }
