@@ -276,12 +276,15 @@ __device__ __forceinline__ double2 to_complex(double2 v) { return v; }
 __device__ __forceinline__ double2 to_complex(double v) { return make_double2(v, 0.0); }
 
 // ---- 1. prologue: per-request Hamiltonian coefficients and rotation angles --------------
-// Grid (blocks, requests): a request's numbers are independent of each other.
+// `blocks` workgroups per request: a request's numbers are independent of each
+// other.  Requests share grid x, since a launch of small ones holds more of
+// them than the grid's second dimension does.
 template <typename S>
-__global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict__ slots, int need_coef) {
-    const SlotDesc sd = slots[blockIdx.y];
+__global__ __launch_bounds__(256) void k_sec_prologue(const SlotDesc* __restrict__ slots, int need_coef, uint32_t blocks) {
+    const uint32_t slot = blockIdx.x / blocks;
+    const SlotDesc sd = slots[slot];
     const SecTables* __restrict__ T = sd.t;
-    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    const uint32_t i0 = (blockIdx.x - slot * blocks) * blockDim.x + threadIdx.x, step = blocks * blockDim.x;
     if (need_coef && sd.coef) {
         for (uint32_t k = i0; k < T->nterms; k += step) {
             double cr = 0.0, ci = 0.0;
@@ -2380,8 +2383,9 @@ void pass_prefix(const std::vector<qfe_template>& ts, bool rev, std::vector<uint
 int launch_prologue(const std::vector<qfe_template>& ts, const SlotDesc* d, int need_coef, hipStream_t st) {
     uint32_t most = 1;
     for (const auto& t : ts) most = std::max(most, std::max(t->nentries, need_coef ? std::max(t->nterms, t->nm) : 0u));
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((most + 255) / 256, ((1ull << 31) - 1) / ts.size());
     with_scalar(ts[0], [&](auto z) {
-        hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3((most + 255) / 256, (unsigned)ts.size()), dim3(256), 0, st, d, need_coef);
+        hipLaunchKernelGGL(k_sec_prologue<decltype(z)>, dim3(blocks * (unsigned)ts.size()), dim3(256), 0, st, d, need_coef, blocks);
     });
     QFE_HIP(hipGetLastError());
     return QFE_OK;
@@ -2659,8 +2663,8 @@ void expected_nodes(qfe_template t, int grad, std::vector<NodeExpect>& out) {
     const auto KB = [](uint64_t items) { return (items + kWideTPB - 1) / kWideTPB; };
     out.clear();
     out.push_back(expect_copy(dev, pin, head));
-    out.push_back(expect_kernel((const void*)&k_sec_prologue<S>, KB(std::max(std::max(t->nentries, 1u), std::max(t->nterms, t->nm))), 256, d,
-                                (int)1));
+    const uint64_t pro = KB(std::max(std::max(t->nentries, 1u), std::max(t->nterms, t->nm)));
+    out.push_back(expect_kernel((const void*)&k_sec_prologue<S>, pro, 256, d, (int)1, (uint32_t)pro));
     out.push_back(expect_kernel((const void*)&k_sec_ref<S>, KB(t->D), kWideTPB, d));
     for (uint32_t k = 0; k < (uint32_t)t->step_pairs.size(); ++k)
         if (t->step_pairs[k])
