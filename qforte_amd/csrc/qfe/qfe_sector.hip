@@ -104,6 +104,16 @@ struct TileRun {  // one pass: the records [rec0, rec0 + nrec) over the tiles of
     uint32_t seg, rec0, nrec, part;  // part: first partial sum (reverse sweep)
 };
 
+// The partial sums of the reverse sweep (one per wave of a tile and output) are
+// kept for a window of consecutive passes and added up behind the last of
+// them; the next window uses the same memory (see TileBuilder::most).
+struct TileOut {  // output 0 is the energy, k + 1 generator k's overlap
+    uint32_t out, r0, r1, add;  // its ranges tsum[r0 .. r1); add: an earlier window has a part of it
+};
+struct TileWindow {
+    uint32_t pass, o0, o1, pad;  // last pass, outputs touts[o0 .. o1)
+};
+
 // A list word: local position of a string and of its partner in their block,
 // and the parities of the entry's sign mask on both.
 constexpr uint32_t kWordBits = 14, kWordPos = (1u << kWordBits) - 1u;
@@ -193,9 +203,10 @@ struct SecTables {  // device view of a template (lives in device memory)
     const uint2* ttab;     // (offset, length) of every list in every block
     const uint32_t* twords;
     const uint2* tsum;     // ranges (first, count) of reverse-sweep partial sums
-    const uint32_t* tsum_off;  // ranges of output k: [tsum_off[k], tsum_off[k + 1]); 0 the energy, k + 1 generator k
+    const TileOut* touts;
+    const TileWindow* twins;
     RowTables rows;
-    uint32_t nsteps, nentries, ngroups, nterms, nitems, ngen, nhchunks;
+    uint32_t nsteps, nentries, ngroups, nterms, nitems, ngen, nhchunks, nwins;
     uint32_t nparts;  // energy partials: the work items', then one per row workgroup
     uint32_t nrows;   // row workgroups (0: every group is in the work items)
 };
@@ -611,20 +622,33 @@ __global__ __launch_bounds__(T) void k_sec_tile(const SlotDesc* __restrict__ slo
     }
 }
 
-// Sums of the reverse sweep's partials in a fixed order, one wave each:
-// output 0 is the energy, output k + 1 generator k's overlap.
-__global__ __launch_bounds__(256) void k_sec_tile_sum(const SlotDesc* __restrict__ slots) {
+// Sums of a window's partials in a fixed order, one wave per output: the
+// window that ends with pass `pass` (a request that has none does nothing), or
+// for kLastWindow every request's last one.
+constexpr uint32_t kLastWindow = 0xffffffffu;
+__global__ __launch_bounds__(256) void k_sec_tile_sum(const SlotDesc* __restrict__ slots, uint32_t pass) {
     const SlotDesc sd = slots[blockIdx.y];
     const SecTables* __restrict__ T = sd.t;
-    const uint32_t k = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    if (k > T->ngen) return;
+    uint32_t w = T->nwins - 1;
+    if (pass != kLastWindow) {
+        w = 0;
+        while (w + 1 < T->nwins && T->twins[w].pass != pass) ++w;
+        if (w + 1 == T->nwins) return;
+    }
+    const TileWindow W = T->twins[w];
+    const uint32_t k = W.o0 + blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (k >= W.o1) return;
+    const TileOut O = T->touts[k];
     double acc = 0.0;
-    for (uint32_t r = T->tsum_off[k]; r < T->tsum_off[k + 1]; ++r) {
+    for (uint32_t r = O.r0; r < O.r1; ++r) {
         const uint2 range = T->tsum[r];
         for (uint32_t i = lane; i < range.y; i += kWave) acc += sd.gpart[range.x + i];
     }
     const double v = wave_sum_last(acc);
-    if (lane == kWave - 1) (k ? sd.gacc[k - 1] : *sd.out) = v;
+    if (lane == kWave - 1) {
+        double* to = O.out ? sd.gacc + (O.out - 1) : sd.out;
+        *to = O.add ? *to + v : v;
+    }
 }
 
 // ---- 3. Hamiltonian rows (see RowTables) -------------------------------------------------
@@ -1325,14 +1349,27 @@ struct TileBuilder {
     std::vector<TileRec> recs;
     std::vector<uint32_t> tix, words;
     std::vector<uint2> tab, sum;
-    std::vector<std::vector<uint2>> ranges;  // partial sums of the energy and of every generator
-    uint32_t parts = 0;
+    std::vector<TileOut> outs;
+    std::vector<TileWindow> wins;
     int norb;
     bool real;  // amplitudes are doubles
+    // Partial sums of a window: 2 MB, which holds a whole sweep up to about 20
+    // qubits; on larger sectors the bytes that a real request's two states save
+    // against a complex one's (a complex one takes 1/16 on top), at most 256
+    // MB.  All at once they took 15 GB at 32 qubits (8, 8) beside states of
+    // 2.6 GB, and more than 2^32 numbers from 13.4 thousand generators on.
+    const uint64_t most;
 
     TileBuilder(const Space& s, const ListPool& l, const std::vector<SecStep>& st, const std::vector<SecEntry>& en, size_t ngen,
                 int norb_, bool real_)
-        : sp(s), lp(l), steps(st), entries(en), ranges(ngen + 1), norb(norb_), real(real_) {}
+        : sp(s), lp(l), steps(st), entries(en), norb(norb_), real(real_), most(window((uint64_t)s.str[0].size() * s.str[1].size(), real_)),
+          seen(ngen + 1, 0) {}
+    static uint64_t window(uint64_t D, bool real) {
+        return std::min<uint64_t>(1u << 25, std::max<uint64_t>(1u << 18, real ? 2 * D : D / 4));
+    }
+    uint32_t parts = 0, peak = 0;            // of the open window, of all
+    std::map<uint32_t, std::vector<uint2>> ranges;  // of the open window's outputs
+    std::vector<char> seen;                  // outputs of earlier windows
 
     void join_step(uint32_t s, Components& a, Components& b) const {
         for (uint32_t e = steps[s].e_first; e < steps[s].e_first + steps[s].e_count; ++e) {
@@ -1495,19 +1532,34 @@ struct TileBuilder {
         }
     }
 
+    // Partial sums of one output of a pass over a segment.
+    uint32_t per_out(uint32_t seg) const { return side[0][seg].nblk * side[1][seg].nblk * (kTileThreads / 64); }
+
     // One reverse-sweep pass over a segment: its records are recs[rec0..]; the
-    // outputs it completes are `outs` in order.
-    void add_reverse(uint32_t seg, uint32_t rec0, const std::vector<uint32_t>& outs) {
+    // generators it completes are `gens` in order.
+    void add_reverse(uint32_t seg, uint32_t rec0, const std::vector<uint32_t>& gens) {
+        const uint32_t per = per_out(seg);
+        if (parts && parts + (uint64_t)per * gens.size() > most) close_window();
         add_run(rev, lrev, side[0][seg], side[1][seg], seg, rec0, 2);
-        const uint32_t per = lrev.back().tiles * (kTileThreads / 64);
-        if (rev.size() == 1) {
-            ranges[0].push_back(make_uint2(parts, per));
+        auto add = [&](uint32_t out) {
+            ranges[out].push_back(make_uint2(parts, per));
             parts += per;
+        };
+        if (rev.size() == 1) add(0);
+        for (uint32_t g : gens) add(g + 1);
+        peak = std::max(peak, parts);
+    }
+    void close_window() {
+        const uint32_t o0 = (uint32_t)outs.size();
+        for (const auto& r : ranges) {
+            const uint32_t r0 = (uint32_t)sum.size();
+            sum.insert(sum.end(), r.second.begin(), r.second.end());
+            outs.push_back(TileOut{r.first, r0, (uint32_t)sum.size(), (uint32_t)seen[r.first]});
+            seen[r.first] = 1;
         }
-        for (uint32_t g : outs) {
-            ranges[g + 1].push_back(make_uint2(parts, per));
-            parts += per;
-        }
+        wins.push_back(TileWindow{(uint32_t)rev.size() - 1, o0, (uint32_t)outs.size(), 0});
+        ranges.clear();
+        parts = 0;
     }
 
     void build(const std::vector<uint32_t>& gen_step) {
@@ -1564,12 +1616,18 @@ struct TileBuilder {
         for (size_t i = plan.size(); i-- > 0;) {
             const Part& p = plan[i];
             if (p.seg1 == p.seg0 + 1) {
-                const uint32_t rec0 = (uint32_t)recs.size();
-                std::vector<uint32_t> outs;
+                uint32_t rec0 = (uint32_t)recs.size();
+                std::vector<uint32_t> gens;
                 for (uint32_t k = p.g1; k-- > p.g0;) {
                     const uint32_t s0 = gen_step[k], s1 = gen_step[k + 1];
                     if (s0 == s1) continue;
-                    outs.push_back(k);
+                    // a pass's own sums (the first has the energy's too) fit a window
+                    if (!gens.empty() && (gens.size() + 1 + rev.empty()) * (uint64_t)per_out(p.seg0) > most) {
+                        add_reverse(p.seg0, rec0, gens);
+                        rec0 = (uint32_t)recs.size();
+                        gens.clear();
+                    }
+                    gens.push_back(k);
                     if (s1 == s0 + 1) {  // one step: a pair's four old values give its overlap and both un-rotated pairs
                         add_step(p.seg0, s0, kRecRot | kRecOv);
                         recs.back().flags |= kRecGenEnd;
@@ -1581,7 +1639,7 @@ struct TileBuilder {
                     recs.back().flags |= kRecGenEnd | kRecStepEnd;
                     for (uint32_t s = s1; s-- > s0;) add_step(p.seg0, s, kRecRot);
                 }
-                add_reverse(p.seg0, rec0, outs);
+                add_reverse(p.seg0, rec0, gens);
                 continue;
             }
             // a generator over several segments: its whole overlap before any un-rotation
@@ -1597,14 +1655,11 @@ struct TileBuilder {
                 add_reverse(sgm, rec0, {});
             }
         }
-        for (auto& r : ranges) {
-            sum_off.push_back((uint32_t)sum.size());
-            sum.insert(sum.end(), r.begin(), r.end());
-        }
-        sum_off.push_back((uint32_t)sum.size());
+        for (uint32_t k = 0; k < seen.size(); ++k)
+            if (!seen[k]) (void)ranges[k];  // a generator without pairs: a sum of nothing
+        close_window();
     }
     std::function<void(uint32_t)> on_segment;
-    std::vector<uint32_t> sum_off;
 };
 
 // Builds the row tables of a real template (see k_sec_rows).
@@ -1855,6 +1910,7 @@ struct qfe_template_s {
     uint64_t cost = 0;     // work estimate for ordering slots in a launch
     int tier = 2;          // ansatz launch shape
     std::vector<TileLaunch> fwd, rev;  // tile passes of the ansatz and of the reverse sweep
+    std::vector<TileWindow> wins;      // windows of the reverse sweep's partial sums
     Space sp;              // host copy of the string space (pool operators)
     void* dev = nullptr;   // all tables
     SecTables* dt = nullptr;
@@ -1863,7 +1919,9 @@ struct qfe_template_s {
     // per-request device bytes: psi, coef, cs, part (energy); + sig, gacc (gradient)
     size_t off_psi = 0, off_coef = 0, off_cs = 0, off_part = 0, off_sig = 0, off_gacc = 0, off_gpart = 0, off_hm = 0;
     size_t work_bytes = 0, grad_bytes = 0, io_count = 0, request_bytes = 0, grad_request_bytes = 0;
-    void* arena = nullptr;  // single-request arena: [desc][out][io][prefix][work incl. gradient parts]
+    size_t grad_least_bytes = 0;  // without the partial sums, which no budget is refused for
+    void* arena = nullptr;  // single-request arena: [desc][out][prefix][io][work, with gradient parts from the first call that has them]
+    size_t arena_bytes = 0;
     // step-by-step sequence (large sectors): host step structure and device
     // [segments (uint2 x (ngen + 1))][block partials]
     std::vector<uint32_t> h_gen_step, step_pairs;
@@ -2123,6 +2181,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     tb.build(gen_step);
     t->fwd = tb.lfwd;
     t->rev = tb.lrev;
+    t->wins = tb.wins;
     // merged numbers of the rows: from the inputs, or constants
     std::vector<double> rm, rmval;
     std::vector<uint32_t> rmoff{0}, rmidx;
@@ -2174,7 +2233,8 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     const size_t i_tt = pk.add(tb.tab.data(), tb.tab.size() * sizeof(uint2));
     const size_t i_tw = pk.add(tb.words.data(), tb.words.size() * 4);
     const size_t i_tu = pk.add(tb.sum.data(), tb.sum.size() * sizeof(uint2));
-    const size_t i_to = pk.add(tb.sum_off.data(), tb.sum_off.size() * 4);
+    const size_t i_to = pk.add(tb.outs.data(), tb.outs.size() * sizeof(TileOut));
+    const size_t i_tv = pk.add(tb.wins.data(), tb.wins.size() * sizeof(TileWindow));
     auto add_all = [&](const auto& v) { return pk.add(v.data(), v.size() * sizeof(v[0])); };
     const size_t r_chunk_off = add_all(rows.chunk_off);
     const size_t r_chunks = add_all(rows.chunks);
@@ -2229,7 +2289,9 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     h.ttab = (const uint2*)at(i_tt);
     h.twords = (const uint32_t*)at(i_tw);
     h.tsum = (const uint2*)at(i_tu);
-    h.tsum_off = (const uint32_t*)at(i_to);
+    h.touts = (const TileOut*)at(i_to);
+    h.twins = (const TileWindow*)at(i_tv);
+    h.nwins = (uint32_t)tb.wins.size();
     h.rows.chunk_off = (const uint32_t*)at(r_chunk_off);
     h.rows.chunks = (const uint4*)at(r_chunks);
     h.rows.flips = (const RowFlip*)at(r_flips);
@@ -2291,10 +2353,11 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     t->off_gacc = o;
     o += align256(ngen * 8 + 8);
     t->off_gpart = o;
-    o += align256((size_t)tb.parts * 8 + 8);
+    const size_t sums = align256((size_t)tb.peak * 8);
+    o += sums;
     t->grad_bytes = o;
     t->io_count = nparam + ninputs;
-    t->request_bytes = t->work_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + 16;
+    t->request_bytes = t->work_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc);
     if (t->tier == 2) {  // partial-sum segments of the grid-wide reverse sweep
         auto blocks = [](uint64_t items) { return (uint32_t)((items + kWideTPB - 1) / kWideTPB); };
         t->wide_seg.push_back(make_uint2(0, blocks(t->D)));
@@ -2310,7 +2373,8 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
         QFE_HIP(hipMalloc(&t->wide, seg_bytes + (size_t)t->wide_parts * 8 + 8));
         QFE_HIP(hipMemcpy(t->wide, t->wide_seg.data(), t->wide_seg.size() * sizeof(uint2), hipMemcpyHostToDevice));
     }
-    t->grad_request_bytes = t->grad_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + 16 + ngen * 8;
+    t->grad_request_bytes = t->grad_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + ngen * 8;
+    t->grad_least_bytes = t->grad_request_bytes - sums;
     return QFE_OK;
 }
 
@@ -2361,6 +2425,15 @@ int launch_tiles(const std::vector<qfe_template>& ts, const SlotDesc* d, const u
                                d, prefix ? prefix + q * (k + 1) : nullptr, k, (uint32_t)q, (uint32_t)(MODE != 1 && q == 0));
         });
         QFE_HIP(hipGetLastError());
+        if (MODE != 2) continue;
+        uint32_t outs = 0;  // of the windows that end here, but for every request's last
+        for (const auto& t : ts)
+            for (size_t w = 0; w + 1 < t->wins.size(); ++w)
+                if (t->wins[w].pass == q) outs = std::max(outs, t->wins[w].o1 - t->wins[w].o0);
+        if (outs) {
+            hipLaunchKernelGGL(k_sec_tile_sum, dim3((outs + 3) / 4, k), dim3(256), 0, st, d, (uint32_t)q);
+            QFE_HIP(hipGetLastError());
+        }
     }
     return QFE_OK;
 }
@@ -2470,9 +2543,9 @@ int launch_gradient(const std::vector<qfe_template>& ts, const SlotDesc* ddesc, 
     int rc = launch_psi_sigma(ts, ddesc, pre, st);
     if (!rc) rc = launch_tiles<2>(ts, ddesc, pre.rev, st);
     if (rc) return rc;
-    uint64_t ngen = 0;
-    for (const auto& t : ts) ngen = std::max(ngen, t->ngen);
-    hipLaunchKernelGGL(k_sec_tile_sum, dim3((unsigned)(ngen / 4 + 1), (unsigned)ts.size()), dim3(256), 0, st, ddesc);
+    uint32_t outs = 1;
+    for (const auto& t : ts) outs = std::max(outs, t->wins.back().o1 - t->wins.back().o0);
+    hipLaunchKernelGGL(k_sec_tile_sum, dim3((outs + 3) / 4, (unsigned)ts.size()), dim3(256), 0, st, ddesc, kLastWindow);
     QFE_HIP(hipGetLastError());
     return QFE_OK;
 }
@@ -2559,17 +2632,34 @@ struct Single {
     char* work;
 };
 
+size_t single_head(qfe_template t) { return 768 + align256(t->io_count * 8 + 8); }
+
+// The arena of single requests; it grows when the first gradient parts are asked for.
+int single_arena(qfe_template t, bool grad) {
+    const size_t need = single_head(t) + (grad ? t->grad_bytes : t->work_bytes);
+    if (t->arena_bytes >= need) return QFE_OK;
+    if (t->arena) {
+        QFE_HIP(hipStreamSynchronize(ctx().stream));
+        QFE_HIP(hipFree(t->arena));
+        t->arena = nullptr;
+        t->arena_bytes = 0;
+    }
+    QFE_HIP(hipMalloc(&t->arena, need));
+    t->arena_bytes = need;
+    return QFE_OK;
+}
+
 int single_setup(qfe_template t, const double* params, const double* inputs, bool grad, Single& S) {
-    const size_t io_bytes = align256(t->io_count * 8 + 8);
-    const size_t head = 768 + io_bytes;
-    if (!t->arena) QFE_HIP(hipMalloc(&t->arena, head + t->grad_bytes));
+    const size_t head = single_head(t);
+    int rc = single_arena(t, grad);
+    if (rc) return rc;
     char* dev = (char*)t->arena;
     S.ddesc = (SlotDesc*)dev;
     S.dout = (double*)(dev + 256);
     S.dprefix = (uint32_t*)(dev + 512);
     S.work = dev + head;
     void* host = nullptr;
-    int rc = staging_begin(head, &host);
+    rc = staging_begin(head, &host);
     if (rc) return rc;
     char* h = (char*)host;
     SlotDesc d = make_slot(t, S.work, (const double*)(dev + 768), S.dout, grad);
@@ -2608,7 +2698,6 @@ int single_psi_sigma(qfe_template t, const double* params, const double* inputs,
 // uploads the whole request head (descriptor, prefix, amplitudes, inputs) from
 // the template's pinned block; the last nodes copy the energy (and the
 // generator overlaps) back into the same block.
-size_t single_head(qfe_template t) { return 768 + align256(t->io_count * 8 + 8); }
 
 // ---- host-side audit of a captured sequence ---------------------------------------------
 // After instantiation every node of a template graph is compared with the
@@ -2801,7 +2890,8 @@ int audit_graph(qfe_template t, hipGraph_t g, int grad, GraphAudit& A) {
 
 int graph_build(qfe_template t, int grad) {
     const size_t head = single_head(t);
-    if (!t->arena) QFE_HIP(hipMalloc(&t->arena, head + t->grad_bytes));
+    int rc = single_arena(t, true);  // of its final size: the captured addresses stay valid
+    if (rc) return rc;
     if (!t->gpin) QFE_HIP(hipHostMalloc(&t->gpin, head + 8 * (t->ngen + 2), hipHostMallocDefault));
     char* dev = (char*)t->arena;
     char* pin = (char*)t->gpin;
@@ -2827,7 +2917,7 @@ int graph_build(qfe_template t, int grad) {
             QFE_HIP(hipMemcpyAsync(pin + head + 8, dev + head + t->off_gacc, t->ngen * 8, hipMemcpyDeviceToHost, st));
         return QFE_OK;
     };
-    int rc = record();
+    rc = record();
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &g);
     if (!rc && e != hipSuccess) rc = hip_fail(e, "qfe_template: end capture");
@@ -3437,7 +3527,7 @@ int qfe_batch_submit_gradient(qfe_batch b, qfe_template t, const double* params,
     if (!b || !t || !request_id) return fail(QFE_ERR_ARG, "qfe_batch_submit_gradient: invalid argument");
     if ((t->nparam && !params) || (t->ninputs && !inputs))
         return fail(QFE_ERR_ARG, "qfe_batch_submit_gradient: null parameters");
-    if (t->grad_request_bytes > b->budget / kLanes)
+    if (t->grad_least_bytes > b->budget / kLanes)
         return fail(QFE_ERR_ARG, "qfe_batch_submit_gradient: one request exceeds the per-launch share of the HBM budget");
     b->gqueue[t->tier].push_back(make_request(b, t, params, inputs));
     *request_id = b->gqueue[t->tier].back().id;
