@@ -68,7 +68,9 @@ struct Context {
     // reusable device scratch for reductions and op descriptors
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
-    // partial outputs of apply_pauli_sum on small states (at most 64 MiB)
+    // memory that only makes a call faster: partial outputs of apply_pauli_sum
+    // and the second buffer of run_rounds (at most 64 MiB), kept between calls
+    // and given back to an allocation that would fail
     void* slices = nullptr;
     size_t slice_bytes = 0;
     // pinned host staging for small results
@@ -79,7 +81,15 @@ struct Context {
 Context& ctx();
 int ensure_init();
 int scratch_reserve(size_t bytes, void** out);
-int slice_reserve(size_t bytes, void** out);
+// Null when device memory is short: the caller then takes a route without.
+// The next device_malloc may free it, so nothing is allocated before its use.
+void* slice_memory(size_t bytes);
+// hipMalloc of what a call needs.
+hipError_t device_malloc_bytes(void** p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc_bytes(reinterpret_cast<void**>(p), bytes);
+}
 int pinned_reserve(size_t bytes, void** out);
 // Double-buffered pinned staging: fill *host (bytes), then commit copies it to
 // dev on the library stream without blocking the host.

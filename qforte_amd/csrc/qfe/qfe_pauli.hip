@@ -1146,12 +1146,10 @@ static int launch_apply_sum_kernel(const double2* in, double2* out, int n, const
     // slices until there are about eight workgroups per CU, at least eight groups each
     uint32_t slices = 1;
     while (blocks * slices < 2048 && slices * 16 <= ngroups && slices < 256) slices <<= 1;
-    double2* to = out;
-    if (slices > 1) {
-        void* work = nullptr;
-        int rc = slice_reserve((size_t)slices * N * sizeof(double2), &work);
-        if (rc) return rc;
-        to = static_cast<double2*>(work);
+    double2* to = slices > 1 ? static_cast<double2*>(slice_memory((size_t)slices * N * sizeof(double2))) : out;
+    if (!to) {
+        slices = 1;
+        to = out;
     }
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, slices), dim3(kEvTPB), 0, ctx().stream, in, to, N, dg, ngroups, dz, dc);

@@ -30,9 +30,9 @@ static int table_upload(const std::vector<PauliGroup>& groups, const std::vector
                         const std::vector<double2>& cs, DevTable& t) {
     t.ngroups = (uint32_t)groups.size();
     if (groups.empty()) return QFE_OK;
-    QFE_HIP(hipMalloc(&t.g, groups.size() * sizeof(PauliGroup)));
-    QFE_HIP(hipMalloc(&t.z, zs.size() * sizeof(uint64_t)));
-    QFE_HIP(hipMalloc(&t.c, cs.size() * sizeof(double2)));
+    QFE_HIP(device_malloc(&t.g, groups.size() * sizeof(PauliGroup)));
+    QFE_HIP(device_malloc(&t.z, zs.size() * sizeof(uint64_t)));
+    QFE_HIP(device_malloc(&t.c, cs.size() * sizeof(double2)));
     QFE_HIP(hipMemcpy(t.g, groups.data(), groups.size() * sizeof(PauliGroup), hipMemcpyHostToDevice));
     QFE_HIP(hipMemcpy(t.z, zs.data(), zs.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
     QFE_HIP(hipMemcpy(t.c, cs.data(), cs.size() * sizeof(double2), hipMemcpyHostToDevice));
@@ -302,8 +302,9 @@ struct ProgTiles {
     std::vector<ProgTerm> terms;
     std::vector<uint2> ranges;  // partial sums: the energy, then generator k
     uint32_t parts = 0, dims = 0;
-    void* dev = nullptr;  // tables, (cos, sin / w) of every run, partial sums, results
-    size_t o_fwd = 0, o_rev = 0, o_fruns = 0, o_rruns = 0, o_terms = 0, o_ranges = 0, o_cs = 0, o_part = 0, o_out = 0;
+    void* dev = nullptr;  // tables, (cos, sin / w) of every run, results
+    double* part = nullptr;  // partial sums, from the first gradient on
+    size_t o_fwd = 0, o_rev = 0, o_fruns = 0, o_rruns = 0, o_terms = 0, o_ranges = 0, o_cs = 0, o_out = 0;
 
     // |alpha| over the patterns of the bits it depends on; false unless one
     // value stands out from zero.
@@ -441,6 +442,8 @@ struct ProgTiles {
         ok = !segs.empty();
     }
 
+    // Tables on the device; dev stays null when memory is short, and the caller
+    // goes one exponential at a time.
     int upload() {
         if (!ok || dev) return QFE_OK;
         size_t at = 0;
@@ -457,7 +460,6 @@ struct ProgTiles {
         o_ranges = place(ranges.size() * sizeof(uint2));
         const size_t tables = at;
         o_cs = place(runs.size() * sizeof(double2));
-        o_part = place((size_t)parts * sizeof(double));
         o_out = place(ranges.size() * sizeof(double));
         std::vector<char> img(tables);
         auto put = [&](size_t o, const void* src, size_t bytes) { std::memcpy(img.data() + o, src, bytes); };
@@ -467,9 +469,28 @@ struct ProgTiles {
         put(o_rruns, rruns.data(), rruns.size() * sizeof(ProgRun));
         put(o_terms, terms.data(), terms.size() * sizeof(ProgTerm));
         put(o_ranges, ranges.data(), ranges.size() * sizeof(uint2));
-        QFE_HIP(hipMalloc(&dev, at));
-        QFE_HIP(hipMemcpy(dev, img.data(), tables, hipMemcpyHostToDevice));
+        if (!try_malloc(&dev, at)) return QFE_OK;
+        const hipError_t e = hipMemcpy(dev, img.data(), tables, hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            release();
+            return hip_fail(e, "qfe_program: table upload");
+        }
         return QFE_OK;
+    }
+    template <typename T>
+    static bool try_malloc(T** p, size_t bytes) {
+        if (device_malloc(p, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();  // no error of the call
+        *p = nullptr;
+        return false;
+    }
+    // Whether a reverse sweep can take the tiles.
+    bool sums() { return dev && (part || try_malloc(&part, (size_t)parts * sizeof(double))); }
+    void release() {
+        if (dev) (void)hipFree(dev);
+        if (part) (void)hipFree(part);
+        dev = nullptr;
+        part = nullptr;
     }
     template <typename T>
     T* at(size_t o) const {
@@ -479,7 +500,7 @@ struct ProgTiles {
     // (cos, sin / w) of every run for these amplitudes.
     int angles(const double* params, const std::vector<int32_t>& gparam, const std::vector<double>& gscale) {
         int rc = upload();
-        if (rc) return rc;
+        if (rc || !dev) return rc;
         void* host = nullptr;
         rc = staging_begin(runs.size() * sizeof(double2), &host);
         if (rc) return rc;
@@ -501,7 +522,7 @@ struct ProgTiles {
             hipLaunchKernelGGL(k_program_tile<MODE>, dim3((unsigned)(1ull << (n - (int)dims))), dim3(kProgThreads), lds, cx.stream,
                                x, y, at<const ProgPass>(MODE == 2 ? o_rev : o_fwd), pass,
                                at<const ProgRun>(MODE == 2 ? o_rruns : o_fruns), at<const ProgTerm>(o_terms),
-                               at<const double2>(o_cs), at<double>(o_part), (uint32_t)(MODE == 2 && i == 0));
+                               at<const double2>(o_cs), part, (uint32_t)(MODE == 2 && i == 0));
             QFE_HIP(hipGetLastError());
             cx.counters.fused++;
             cx.counters.tile++;
@@ -547,7 +568,7 @@ static int ensure_partial(qfe_program p, size_t entries) {
         QFE_HIP(hipFree(p->partial));
         p->partial = nullptr;
     }
-    QFE_HIP(hipMalloc(&p->partial, entries * sizeof(double2)));
+    QFE_HIP(device_malloc(&p->partial, entries * sizeof(double2)));
     p->partial_cap = entries;
     return QFE_OK;
 }
@@ -559,7 +580,7 @@ static int ensure_gout(qfe_program p, size_t entries) {
         QFE_HIP(hipFree(p->gout));
         p->gout = nullptr;
     }
-    QFE_HIP(hipMalloc(&p->gout, entries * sizeof(double2)));
+    QFE_HIP(device_malloc(&p->gout, entries * sizeof(double2)));
     p->gout_cap = entries;
     return QFE_OK;
 }
@@ -590,7 +611,8 @@ static int prepare(qfe_program p, const double* params, qfe_state out) {
     if (rc) return rc;
     if (p->tiles.ok) {
         rc = p->tiles.angles(params, p->gparam, p->gscale);
-        return rc ? rc : p->tiles.launch<0>(p->n, out->d, nullptr);
+        if (rc) return rc;
+        if (p->tiles.dev) return p->tiles.launch<0>(p->n, out->d, nullptr);
     }
     std::vector<HostOp> ops;
     ops.reserve(p->gen_terms.size());
@@ -675,11 +697,11 @@ static int graph_build(qfe_program p) {
     const uint32_t nhg = p->ham.ngroups;
     const uint32_t nch = expval_chunks(p->n, nhg);
     auto alloc = [&]() -> int {
-        if (!image.empty()) QFE_HIP(hipMalloc(&g->image, image.size()));
-        if (!angles.empty()) QFE_HIP(hipMalloc(&g->angles, angles.size() * sizeof(DevAngle)));
-        QFE_HIP(hipMalloc(&g->dparams, (p->nparam + 1) * sizeof(double)));
-        QFE_HIP(hipMalloc(&g->partial, ((size_t)nhg * nch + 1) * sizeof(double2)));
-        QFE_HIP(hipMalloc(&g->gout, ((size_t)nhg + 1) * sizeof(double2)));
+        if (!image.empty()) QFE_HIP(device_malloc(&g->image, image.size()));
+        if (!angles.empty()) QFE_HIP(device_malloc(&g->angles, angles.size() * sizeof(DevAngle)));
+        QFE_HIP(device_malloc(&g->dparams, (p->nparam + 1) * sizeof(double)));
+        QFE_HIP(device_malloc(&g->partial, ((size_t)nhg * nch + 1) * sizeof(double2)));
+        QFE_HIP(device_malloc(&g->gout, ((size_t)nhg + 1) * sizeof(double2)));
         QFE_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->hparams), (p->nparam + 1) * sizeof(double), hipHostMallocDefault));
         QFE_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->hout), ((size_t)nhg + 1) * sizeof(double2), hipHostMallocDefault));
         if (!image.empty()) QFE_HIP(hipMemcpy(g->image, image.data(), image.size(), hipMemcpyHostToDevice));
@@ -827,7 +849,7 @@ int qfe_program_destroy(qfe_program p) {
     (void)hipStreamSynchronize(ctx().stream);
     table_free(p->ham);
     table_free(p->gens);
-    if (p->tiles.dev) (void)hipFree(p->tiles.dev);
+    p->tiles.release();
     if (p->partial) (void)hipFree(p->partial);
     if (p->gout) (void)hipFree(p->gout);
     graph_free(p->graph);
@@ -873,11 +895,11 @@ int qfe_program_gradient(qfe_program p, const double* params, double* grad, doub
     // sigma = H psi
     rc = launch_apply_sum_async(p->psi->d, p->sig->d, p->n, p->ham.g, nhg, p->ham.z, p->ham.c);
     if (rc) return rc;
-    if (p->tiles.ok) {
+    if (p->tiles.sums()) {
         ProgTiles& T = p->tiles;
         rc = T.launch<2>(p->n, p->psi->d, p->sig->d);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_program_sum, dim3((unsigned)(ngen / 4 + 1)), dim3(256), 0, ctx().stream, T.at<const double>(T.o_part),
+        hipLaunchKernelGGL(k_program_sum, dim3((unsigned)(ngen / 4 + 1)), dim3(256), 0, ctx().stream, T.part,
                            T.at<const uint2>(T.o_ranges), (uint32_t)(ngen + 1), T.at<double>(T.o_out));
         QFE_HIP(hipGetLastError());
         void* pin = nullptr;
@@ -948,7 +970,7 @@ int qfe_program_residuals(qfe_program p, const double* params, const uint64_t* i
     // sigma = H U|ref>, then U^dag: generators last to first, terms reversed
     rc = launch_apply_sum_async(p->psi->d, p->sig->d, p->n, p->ham.g, p->ham.ngroups, p->ham.z, p->ham.c);
     if (rc) return rc;
-    if (p->tiles.ok) {
+    if (p->tiles.dev) {
         rc = p->tiles.launch<1>(p->n, p->sig->d, nullptr);
     } else {
         std::vector<HostOp> ops;

@@ -914,15 +914,7 @@ int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken) {
     if (!plan_rounds(ops, st->n, plan, plain)) return QFE_OK;
     taken = true;
     if (plan.passes.empty()) return QFE_OK;
-    const int k = std::min(st->n, kRoundTileMax);
-    double2* other = st->d;
     int rc = QFE_OK;
-    if (!plain && st->n > k) {
-        void* p = nullptr;
-        rc = slice_reserve(sizeof(double2) << st->n, &p);
-        if (rc) return rc;
-        other = static_cast<double2*>(p);
-    }
     const uint4* prog = nullptr;
     if (!plan.words.empty()) {
         const size_t bytes = plan.words.size() * sizeof(uint4);
@@ -935,6 +927,14 @@ int run_rounds(qfe_state_s* st, const std::vector<HostOp>& ops, bool& taken) {
         rc = staging_commit(dev, bytes);
         if (rc) return rc;
         prog = static_cast<const uint4*>(dev);
+    }
+    double2* other = st->d;
+    if (!plain && st->n > kRoundTileMax) {
+        other = static_cast<double2*>(slice_memory(sizeof(double2) << st->n));
+        if (!other) {
+            taken = false;
+            return QFE_OK;
+        }
     }
     for (size_t i = 0; i < plan.passes.size(); ++i) {
         const RoundsPass& p = plan.passes[i];

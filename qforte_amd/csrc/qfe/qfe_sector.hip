@@ -2253,7 +2253,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     const size_t r_fb_mask = add_all(rows.fb_mask);
     const size_t r_fa_mask = add_all(rows.fa_mask);
     const size_t r_m = add_all(rm), r_moff = add_all(rmoff), r_midx = add_all(rmidx), r_mval = add_all(rmval);
-    QFE_HIP(hipMalloc(&t->dev, pk.total));
+    QFE_HIP(device_malloc(&t->dev, pk.total));
     char* base = (char*)t->dev;
     auto at = [&](size_t i) { return base + pk.pieces[i].off; };
     SecTables h{};
@@ -2370,7 +2370,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
         }
         t->wide_parts = at;
         const size_t seg_bytes = align256(t->wide_seg.size() * sizeof(uint2));
-        QFE_HIP(hipMalloc(&t->wide, seg_bytes + (size_t)t->wide_parts * 8 + 8));
+        QFE_HIP(device_malloc(&t->wide, seg_bytes + (size_t)t->wide_parts * 8 + 8));
         QFE_HIP(hipMemcpy(t->wide, t->wide_seg.data(), t->wide_seg.size() * sizeof(uint2), hipMemcpyHostToDevice));
     }
     t->grad_request_bytes = t->grad_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + ngen * 8;
@@ -2644,7 +2644,7 @@ int single_arena(qfe_template t, bool grad) {
         t->arena = nullptr;
         t->arena_bytes = 0;
     }
-    QFE_HIP(hipMalloc(&t->arena, need));
+    QFE_HIP(device_malloc(&t->arena, need));
     t->arena_bytes = need;
     return QFE_OK;
 }
@@ -3034,7 +3034,7 @@ int grow_device(void*& p, size_t& cap, size_t need) {
     if (p) QFE_HIP(hipFree(p));
     p = nullptr;
     cap = 0;
-    QFE_HIP(hipMalloc(&p, need + need / 4));
+    QFE_HIP(device_malloc(&p, need + need / 4));
     cap = need + need / 4;
     return QFE_OK;
 }
@@ -3437,7 +3437,7 @@ int qfe_template_pool_gradients(qfe_template t, const double* params, const doub
         rc = staging_commit(dev, pk.total);
         if (rc) return rc;
     } else {
-        QFE_HIP(hipMalloc(&dev, total));
+        QFE_HIP(device_malloc(&dev, total));
         img.resize(pk.total);
         pk.fill(img.data());
         const hipError_t e = hipMemcpy(dev, img.data(), pk.total, hipMemcpyHostToDevice);

@@ -51,27 +51,44 @@ int scratch_reserve(size_t bytes, void** out) {
             c.scratch_bytes = 0;
         }
         size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
-        QFE_HIP(hipMalloc(&c.scratch, want));
+        QFE_HIP(device_malloc(&c.scratch, want));
         c.scratch_bytes = want;
     }
     *out = c.scratch;
     return QFE_OK;
 }
 
-int slice_reserve(size_t bytes, void** out) {
+static void slices_free() {
+    Context& c = g_ctx;
+    if (!c.slices) return;
+    (void)hipStreamSynchronize(c.stream);
+    (void)hipFree(c.slices);
+    c.slices = nullptr;
+    c.slice_bytes = 0;
+}
+
+void* slice_memory(size_t bytes) {
     Context& c = g_ctx;
     if (c.slice_bytes < bytes) {
-        if (c.slices) {
-            QFE_HIP(hipStreamSynchronize(c.stream));
-            QFE_HIP(hipFree(c.slices));
+        slices_free();
+        if (hipMalloc(&c.slices, bytes) != hipSuccess) {
+            (void)hipGetLastError();  // no error of the call
             c.slices = nullptr;
-            c.slice_bytes = 0;
+            return nullptr;
         }
-        QFE_HIP(hipMalloc(&c.slices, bytes));
         c.slice_bytes = bytes;
     }
-    *out = c.slices;
-    return QFE_OK;
+    return c.slices;
+}
+
+hipError_t device_malloc_bytes(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && g_ctx.slices) {
+        (void)hipGetLastError();
+        slices_free();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
 }
 
 int pinned_reserve(size_t bytes, void** out) {
@@ -486,7 +503,7 @@ int qfe_state_create(int nqubit, qfe_state* out) {
     qfe_state_s* s = new qfe_state_s();
     s->n = nqubit;
     s->N = 1ull << nqubit;
-    hipError_t e = hipMalloc(&s->d, s->N * sizeof(double2));
+    hipError_t e = device_malloc(&s->d, s->N * sizeof(double2));
     if (e != hipSuccess) {
         delete s;
         return hip_fail(e, "hipMalloc(state)");
