@@ -146,6 +146,7 @@ struct HostOp {
 
 // Build HostOps from gates / op stream. Returns false + message on bad input.
 int lower_gate(const qfe_gate& g, int n, std::vector<HostOp>& out);
+const char* pexp_refusal(const qfe_pauli& p);  // why a string has no exponential, or null
 int lower_pexp(const qfe_pauli& p, double angle, int n, std::vector<HostOp>& out);
 
 // Execute a lowered op list on a state (plans fused passes and launches).

@@ -112,15 +112,20 @@ int lower_gate(const qfe_gate& g, int n, std::vector<HostOp>& out) {
     return QFE_OK;
 }
 
-int lower_pexp(const qfe_pauli& p, double angle, int n, std::vector<HostOp>& out) {
-    const uint64_t lim = (n >= 64) ? ~0ull : ((1ull << n) - 1ull);
-    if ((p.x & ~lim) || (p.z & ~lim)) return fail(QFE_ERR_ARG, "apply_pauli_exp: Pauli string acts on a qubit out of range");
+const char* pexp_refusal(const qfe_pauli& p) {
     // Hermitian P needs conj(phase) = phase * (-1)^popcount(x & z).
     const bool odd = __builtin_popcountll(p.x & p.z) & 1;
     const double er = odd ? -p.phase.re : p.phase.re, ei = odd ? -p.phase.im : p.phase.im;
     if (std::fabs(er - p.phase.re) > 1e-15 || std::fabs(-ei - p.phase.im) > 1e-15)
-        return fail(QFE_ERR_ARG, "apply_pauli_exp: the Pauli operator is not Hermitian");
-    if (std::fabs(cabs2(p.phase) - 1.0) > 1e-12) return fail(QFE_ERR_ARG, "apply_pauli_exp: phase must have modulus 1");
+        return "apply_pauli_exp: the Pauli operator is not Hermitian";
+    if (std::fabs(cabs2(p.phase) - 1.0) > 1e-12) return "apply_pauli_exp: phase must have modulus 1";
+    return nullptr;
+}
+
+int lower_pexp(const qfe_pauli& p, double angle, int n, std::vector<HostOp>& out) {
+    const uint64_t lim = (n >= 64) ? ~0ull : ((1ull << n) - 1ull);
+    if ((p.x & ~lim) || (p.z & ~lim)) return fail(QFE_ERR_ARG, "apply_pauli_exp: Pauli string acts on a qubit out of range");
+    if (const char* why = pexp_refusal(p)) return fail(QFE_ERR_ARG, why);
     if (angle == 0.0) return QFE_OK;
     HostOp h{};
     h.op.kind = K_PEXP;

@@ -833,12 +833,7 @@ int qfe_program_create(int nqubit, uint64_t ref_index, const qfe_pauli* gen_term
     }
     // strings that are not Hermitian keep the lowering, which reports them
     bool hermitian = true;
-    for (const qfe_pauli& t : p->gen_terms) {
-        // conj(phase) = phase (-1)^{x.z}, modulus 1
-        const bool odd = __builtin_popcountll(t.x & t.z) & 1;
-        hermitian = hermitian && std::fabs(odd ? t.phase.re : t.phase.im) < 1e-15 &&
-                    std::fabs(t.phase.re * t.phase.re + t.phase.im * t.phase.im - 1.0) < 1e-12;
-    }
+    for (const qfe_pauli& t : p->gen_terms) hermitian = hermitian && !pexp_refusal(t);
     if (ngen && hermitian) p->tiles.build(p->n, p->gen_terms, p->gen_off);
     *out = p;
     return QFE_OK;
