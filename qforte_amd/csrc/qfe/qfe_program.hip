@@ -306,8 +306,9 @@ struct ProgTiles {
     double* part = nullptr;  // partial sums, from the first gradient on
     size_t o_fwd = 0, o_rev = 0, o_fruns = 0, o_rruns = 0, o_terms = 0, o_ranges = 0, o_cs = 0, o_out = 0;
 
-    // |alpha| over the patterns of the bits it depends on; false unless one
-    // value stands out from zero.
+    // |alpha| over the patterns of the bits it depends on; false unless all of
+    // them are one value or zero, to the rounding of their sums: a rotation by
+    // the mean is then as close to the string's exponentials as these are.
     static bool weight(const std::vector<qfe_pauli>& t, uint64_t b, uint64_t e, double& w) {
         uint64_t m = 0;
         double total = 0.0;
@@ -317,6 +318,7 @@ struct ProgTiles {
         }
         if (__builtin_popcountll(m) > 12) return false;
         w = 0.0;
+        const double tol = 4.0 * 0x1p-52 * total;
         std::vector<double> seen;
         for (uint64_t p = m;; p = (p - 1) & m) {
             double re = 0.0, im = 0.0;
@@ -326,13 +328,13 @@ struct ProgTiles {
                 im += sg * t[k].phase.re;
             }
             const double v = std::hypot(re, im);
-            if (v > 1e-13 * total) seen.push_back(v);
+            if (v > tol) seen.push_back(v);
             if (!p) break;
         }
         if (seen.empty()) return false;
         for (double v : seen) w += v / (double)seen.size();
         for (double v : seen)
-            if (std::fabs(v - w) > 1e-14 * w) return false;
+            if (std::fabs(v - w) > tol) return false;
         return true;
     }
 
