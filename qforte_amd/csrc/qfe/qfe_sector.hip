@@ -981,6 +981,7 @@ __global__ __launch_bounds__(256) void k_sec_pool(const SecTables* __restrict__ 
 // ---- one launch per step (captured for the audit) -----------------------------------------
 // The evaluation as a chain of kernels, one step (or generator) each over the
 // whole grid: what qfe_template_graph_audit captures and checks node by node.
+// No result comes from it: every evaluation takes the tile passes above.
 // Pair t of a step is taken in entry order.
 constexpr int kWideTPB = 256;
 
@@ -1922,8 +1923,8 @@ struct qfe_template_s {
     size_t grad_least_bytes = 0;  // without the partial sums, which no budget is refused for
     void* arena = nullptr;  // single-request arena: [desc][out][prefix][io][work, with gradient parts from the first call that has them]
     size_t arena_bytes = 0;
-    // step-by-step sequence (large sectors): host step structure and device
-    // [segments (uint2 x (ngen + 1))][block partials]
+    // step-by-step sequence (large sectors, for the audit only, which allocates
+    // it): host step structure and device [segments (uint2 x (ngen + 1))][block partials]
     std::vector<uint32_t> h_gen_step, step_pairs;
     std::vector<uint2> wide_seg;  // (first partial, count): the energy, then generator k
     uint32_t wide_parts = 0;
@@ -2358,21 +2359,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     t->grad_bytes = o;
     t->io_count = nparam + ninputs;
     t->request_bytes = t->work_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc);
-    if (t->tier == 2) {  // partial-sum segments of the grid-wide reverse sweep
-        auto blocks = [](uint64_t items) { return (uint32_t)((items + kWideTPB - 1) / kWideTPB); };
-        t->wide_seg.push_back(make_uint2(0, blocks(t->D)));
-        uint32_t at = blocks(t->D);
-        for (uint64_t k = 0; k < ngen; ++k) {
-            uint64_t pairs = 0;
-            for (uint32_t sdx = gen_step[k]; sdx < gen_step[k + 1]; ++sdx) pairs += t->step_pairs[sdx];
-            t->wide_seg.push_back(make_uint2(at, blocks(pairs)));
-            at += blocks(pairs);
-        }
-        t->wide_parts = at;
-        const size_t seg_bytes = align256(t->wide_seg.size() * sizeof(uint2));
-        QFE_HIP(device_malloc(&t->wide, seg_bytes + (size_t)t->wide_parts * 8 + 8));
-        QFE_HIP(hipMemcpy(t->wide, t->wide_seg.data(), t->wide_seg.size() * sizeof(uint2), hipMemcpyHostToDevice));
-    }
     t->grad_request_bytes = t->grad_bytes + align256(t->io_count * 8 + 8) + sizeof(SlotDesc) + ngen * 8;
     t->grad_least_bytes = t->grad_request_bytes - sums;
     return QFE_OK;
@@ -2892,6 +2878,21 @@ int graph_build(qfe_template t, int grad) {
     const size_t head = single_head(t);
     int rc = single_arena(t, true);  // of its final size: the captured addresses stay valid
     if (rc) return rc;
+    if (!t->wide) {  // partial-sum segments of the step-by-step reverse sweep
+        t->wide_seg.assign(1, make_uint2(0, wide_blocks(t->D)));
+        uint64_t at = wide_blocks(t->D);
+        for (uint64_t k = 0; k < t->ngen; ++k) {
+            uint64_t pairs = 0;
+            for (uint32_t s = t->h_gen_step[k]; s < t->h_gen_step[k + 1]; ++s) pairs += t->step_pairs[s];
+            t->wide_seg.push_back(make_uint2((uint32_t)at, wide_blocks(pairs)));
+            at += wide_blocks(pairs);
+            if (at >= (1ull << 31)) return fail(QFE_ERR_ARG, "qfe_template_graph_audit: too many partial sums in one sequence");
+        }
+        t->wide_parts = (uint32_t)at;
+        const size_t seg_bytes = align256(t->wide_seg.size() * sizeof(uint2));
+        QFE_HIP(device_malloc(&t->wide, seg_bytes + at * 8 + 8));
+        QFE_HIP(hipMemcpy(t->wide, t->wide_seg.data(), t->wide_seg.size() * sizeof(uint2), hipMemcpyHostToDevice));
+    }
     if (!t->gpin) QFE_HIP(hipHostMalloc(&t->gpin, head + 8 * (t->ngen + 2), hipHostMallocDefault));
     char* dev = (char*)t->arena;
     char* pin = (char*)t->gpin;

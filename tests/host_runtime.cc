@@ -138,6 +138,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
 hipError_t hipEventCreate(hipEvent_t* e) {
     *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
     return hipSuccess;

@@ -73,6 +73,19 @@ print("ok")
     assert out.strip() == "ok"
 
 
+def test_audit_takes_its_buffers_itself(on_host):  # noqa: F811
+    out = on_host(SETUP + """
+tpl = qf.SectorTemplate(*template(9, 4, 1, None))
+tpl.gradient([0.1] * tpl.nparam, [])
+base = host.host_used()
+try: tpl.graph_audit(True)  # nothing is captured without a device
+except RuntimeError: pass
+assert host.host_used() - base >= 8 * tpl.dim // 256
+print("ok")
+""")
+    assert out.strip() == "ok"
+
+
 LONG = (9, 4, 30, None)  # 18 qubits, 16800 generators
 
 
