@@ -70,17 +70,17 @@ __device__ __forceinline__ uint32_t odd_bit(uint32_t v) { return (uint32_t)__pop
 __device__ __forceinline__ uint32_t odd_bit(uint64_t v) { return (uint32_t)__popcll(v) << 31; }
 
 constexpr uint32_t kEvTerms = 256;  // terms of a group staged in LDS at a time
-constexpr int kEvPer = 4;           // amplitudes or pairs per thread and staged term
+constexpr int kEvPer = 4;           // pairs per thread and staged term
 
 // One block = (group g, chunk ch).  Pairs of group g are split into nchunk
 // equal contiguous ranges.  W: word that holds an index (uint32_t up to 32
 // qubits).  The group's terms come through LDS and each is read once for
-// kEvPer pairs per thread.  In one state (SAME) a term's signs on a pair
+// PER pairs per thread.  In one state (SAME) a term's signs on a pair
 // differ by a uniform sigma = (-1)^{|x & z|}, so with p = conj(a_ja) a_jb the
 // pair gives 2 s c Re p (sigma = +1) or -2i s c Im p (sigma = -1), s the sign
 // on ja: one sign per pair and term, where both ends and complex products were
 // evaluated before (18-qubit molecule, 9316 terms: 788 us).
-template <typename W, bool SAME>
+template <typename W, bool SAME, int PER>
 __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restrict__ bra,
                                                           const double2* __restrict__ ket, int n,
                                                           const PauliGroup* __restrict__ groups,
@@ -111,11 +111,11 @@ __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restr
             cplx |= ct[t].y != 0.0;
         }
         const bool real = !__syncthreads_or(cplx);  // real coefficients: half the sums
-        for (uint64_t k0 = b0 + threadIdx.x; k0 < e0; k0 += kEvPer * kEvTPB) {
-            W ja[kEvPer];
-            double2 p[kEvPer], q[kEvPer], f[kEvPer], h[kEvPer];
+        for (uint64_t k0 = b0 + threadIdx.x; k0 < e0; k0 += PER * kEvTPB) {
+            W ja[PER];
+            double2 p[PER], q[PER], f[PER], h[PER];
 #pragma unroll
-            for (int u = 0; u < kEvPer; ++u) {
+            for (int u = 0; u < PER; ++u) {
                 const uint64_t k = k0 + (uint64_t)u * kEvTPB;
                 const uint64_t j = diag ? k : ins0(k, G.hb);
                 const bool on = k < e0;
@@ -130,9 +130,9 @@ __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restr
                     const W zz = zt[t];
                     const double2 cc = ct[t];
                     const uint32_t sx = odd_bit((W)(x & zz));
-                    auto add = [&](double2(&to)[kEvPer], uint32_t flip) {
+                    auto add = [&](double2(&to)[PER], uint32_t flip) {
 #pragma unroll
-                        for (int u = 0; u < kEvPer; ++u) {
+                        for (int u = 0; u < PER; ++u) {
                             const uint32_t s = odd_bit((W)(ja[u] & zz)) ^ flip;
                             to[u].x += sign_flip(cc.x, s);
                             if (!REAL) to[u].y += sign_flip(cc.y, s);
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restr
             else
                 sum_terms(std::false_type{});
 #pragma unroll
-            for (int u = 0; u < kEvPer; ++u) {
+            for (int u = 0; u < PER; ++u) {
                 if (!SAME) {
                     // conj(bra_ja) ket_jb f(jb) + conj(bra_jb) ket_ja f(ja); a diagonal group has the first alone
                     acc = cadd(acc, cadd(cmul(p[u], h[u]), cmul(q[u], f[u])));
@@ -168,14 +168,25 @@ __global__ __launch_bounds__(kEvTPB) void k_expval_groups(const double2* __restr
     if (threadIdx.x == 0) partial[blockIdx.x] = acc;
 }
 
+constexpr int kEvSingleMin = 18;
+// terms: of all groups (0: not known).
 static void launch_expval_kernel(const double2* bra, const double2* ket, int n, const PauliGroup* dg, uint32_t ngroups,
-                                 const uint64_t* dz, const double2* dc, uint32_t nchunk, double2* partial) {
+                                 const uint64_t* dz, const double2* dc, uint32_t nchunk, double2* partial, uint64_t terms) {
     const dim3 grid((unsigned)((uint64_t)ngroups * nchunk));
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kEvTPB), 0, ctx().stream, bra, ket, n, dg, dz, dc, nchunk, partial); };
-    if (n <= 32)
-        bra == ket ? go(k_expval_groups<uint32_t, true>) : go(k_expval_groups<uint32_t, false>);
+    // Between two states a group of one or two terms is a read of both, and four
+    // pairs' products leave four waves per SIMD to hide it; one pair per thread,
+    // from the size on where there are waves enough.  Random strings at 18 qubits
+    // (200 terms) / 19 (40) / 20 (10, 200) in us: 84, 61, 47, 398 by one pair, 85, 61,
+    // 48, 411 by two, 97, 68, 58, 418 by four (117, 65, 52, 447 with the complex
+    // products of both ends); 200 terms on few masks at 20: 536, 330, 228 (574).
+    const bool single = n >= kEvSingleMin && terms && terms < 2 * (uint64_t)ngroups;
+    if (bra == ket)
+        n <= 32 ? go(k_expval_groups<uint32_t, true, kEvPer>) : go(k_expval_groups<uint64_t, true, kEvPer>);
+    else if (single)
+        n <= 32 ? go(k_expval_groups<uint32_t, false, 1>) : go(k_expval_groups<uint64_t, false, 1>);
     else
-        bra == ket ? go(k_expval_groups<uint64_t, true>) : go(k_expval_groups<uint64_t, false>);
+        n <= 32 ? go(k_expval_groups<uint32_t, false, kEvPer>) : go(k_expval_groups<uint64_t, false, kEvPer>);
 }
 
 __global__ __launch_bounds__(kEvTPB) void k_sum_groups(const double2* __restrict__ partial, uint32_t nchunk,
@@ -224,7 +235,7 @@ static int upload_groups(const std::vector<PauliGroup>& groups, const std::vecto
 }
 
 static uint32_t chunks_for(int n, size_t ngroups) {
-    // 4096 pairs per block, or fewer (down to one staged term's 1024) while the
+    // 4096 pairs per block, or fewer (down to a round of a block, 1024) while the
     // launch has less than four blocks per CU; at most 1024 chunks per group,
     // and the partials array bounded
     const uint64_t P = 1ull << (n > 0 ? n - 1 : 0);
@@ -243,7 +254,7 @@ int launch_expval_async(const double2* bra, const double2* ket, int n, const Pau
                         double2* dout) {
     Context& cx = ctx();
     if (ngroups == 0) return QFE_OK;
-    launch_expval_kernel(bra, ket, n, dgroups, ngroups, dzs, dcs, nchunk, partial);
+    launch_expval_kernel(bra, ket, n, dgroups, ngroups, dzs, dcs, nchunk, partial, 0);
     QFE_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_groups, dim3(ngroups), dim3(kEvTPB), 0, cx.stream, partial, nchunk, dout);
     QFE_HIP(hipGetLastError());
@@ -945,7 +956,7 @@ int expval_groups(const double2* bra, const double2* ket, int n, const std::vect
     if (rc) return rc;
     double2* partial = reinterpret_cast<double2*>(gd.tail);
     double2* dout = reinterpret_cast<double2*>(gd.tail + b_part);
-    launch_expval_kernel(bra, ket, n, gd.groups, (uint32_t)G, gd.zs, gd.cs, nchunk, partial);
+    launch_expval_kernel(bra, ket, n, gd.groups, (uint32_t)G, gd.zs, gd.cs, nchunk, partial, zs.size());
     QFE_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)G), dim3(kEvTPB), 0, cx.stream, partial, nchunk, dout);
     QFE_HIP(hipGetLastError());
@@ -1023,7 +1034,7 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
         QFE_HIP(hipMemcpyAsync(dz, zs.data(), zs.size() * sizeof(uint64_t), hipMemcpyHostToDevice, cx.stream));
         QFE_HIP(hipMemcpyAsync(dc, cs.data(), cs.size() * sizeof(double2), hipMemcpyHostToDevice, cx.stream));
         launch_expval_kernel(bra, ket, n, (const PauliGroup*)dg, (uint32_t)G, (const uint64_t*)dz, (const double2*)dc, nchunk,
-                             (double2*)part);
+                             (double2*)part, zs.size());
         QFE_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_sum_groups, dim3((unsigned)G), dim3(kEvTPB), 0, cx.stream, (const double2*)part, nchunk,
                            (double2*)dout);
@@ -1085,7 +1096,13 @@ static int expval_groups_fixed(const double2* bra, const double2* ket, int n, co
     return QFE_OK;
 }
 
-// out_k = sum_g in[k ^ x_g] f_g(k ^ x_g): every thread owns kEvPer output
+// Output amplitudes per thread.  1 / 2 / 4 in us, one thread each with the signs
+// as branches before: 1000 terms at 2 qubits 187 / 236 / 270 (234), near-diagonal
+// ones at 14 167 / 213 / 248 (270) and at 19 277 / 230 / 263 (433), random ones at
+// 14 71 / 83 / 90 (424) and at 20 787 / 631 / 643 (1052).
+constexpr int kApplyPer = 2;
+
+// out_k = sum_g in[k ^ x_g] f_g(k ^ x_g): every thread owns kApplyPer output
 // amplitudes and walks the groups in order (fixed summation order per
 // element), each term read once for all of them.  Grid y = slices of the
 // groups while the amplitudes alone leave CUs idle (14 qubits, 3382 terms: 64
@@ -1096,16 +1113,16 @@ __global__ __launch_bounds__(kEvTPB) void k_apply_sum(const double2* __restrict_
                                                       const uint64_t* __restrict__ zs, const double2* __restrict__ cs) {
     const uint32_t g0 = (uint32_t)((uint64_t)ngroups * blockIdx.y / gridDim.y);
     const uint32_t g1 = (uint32_t)((uint64_t)ngroups * (blockIdx.y + 1) / gridDim.y);
-    const uint64_t k0 = (uint64_t)blockIdx.x * (kEvTPB * kEvPer) + threadIdx.x;
-    double2 acc[kEvPer];
+    const uint64_t k0 = (uint64_t)blockIdx.x * (kEvTPB * kApplyPer) + threadIdx.x;
+    double2 acc[kApplyPer];
 #pragma unroll
-    for (int u = 0; u < kEvPer; ++u) acc[u] = make_double2(0.0, 0.0);
+    for (int u = 0; u < kApplyPer; ++u) acc[u] = make_double2(0.0, 0.0);
     for (uint32_t g = g0; g < g1; ++g) {
         const PauliGroup G = groups[g];
-        W src[kEvPer];
-        double2 v[kEvPer], f[kEvPer];
+        W src[kApplyPer];
+        double2 v[kApplyPer], f[kApplyPer];
 #pragma unroll
-        for (int u = 0; u < kEvPer; ++u) {
+        for (int u = 0; u < kApplyPer; ++u) {
             const uint64_t k = k0 + (uint64_t)u * kEvTPB;
             src[u] = (W)(k ^ G.x);
             v[u] = k < N ? in[k ^ G.x] : make_double2(0.0, 0.0);
@@ -1115,17 +1132,17 @@ __global__ __launch_bounds__(kEvTPB) void k_apply_sum(const double2* __restrict_
             const W z = (W)zs[t];
             const double2 c = cs[t];
 #pragma unroll
-            for (int u = 0; u < kEvPer; ++u) {
+            for (int u = 0; u < kApplyPer; ++u) {
                 const uint32_t s = odd_bit((W)(src[u] & z));
                 f[u].x += sign_flip(c.x, s);
                 f[u].y += sign_flip(c.y, s);
             }
         }
 #pragma unroll
-        for (int u = 0; u < kEvPer; ++u) acc[u] = cadd(acc[u], cmul(f[u], v[u]));
+        for (int u = 0; u < kApplyPer; ++u) acc[u] = cadd(acc[u], cmul(f[u], v[u]));
     }
 #pragma unroll
-    for (int u = 0; u < kEvPer; ++u) {
+    for (int u = 0; u < kApplyPer; ++u) {
         const uint64_t k = k0 + (uint64_t)u * kEvTPB;
         if (k < N) out[blockIdx.y * N + k] = acc[u];
     }
@@ -1142,7 +1159,7 @@ __global__ __launch_bounds__(kEvTPB) void k_add_slices(const double2* __restrict
 
 static int launch_apply_sum_kernel(const double2* in, double2* out, int n, const PauliGroup* dg, uint32_t ngroups,
                                    const uint64_t* dz, const double2* dc) {
-    const uint64_t N = 1ull << n, blocks = (N + kEvTPB * kEvPer - 1) / (kEvTPB * kEvPer);
+    const uint64_t N = 1ull << n, blocks = (N + kEvTPB * kApplyPer - 1) / (kEvTPB * kApplyPer);
     // slices until there are about eight workgroups per CU, at least eight groups each
     uint32_t slices = 1;
     while (blocks * slices < 2048 && slices * 16 <= ngroups && slices < 256) slices <<= 1;
