@@ -2238,9 +2238,10 @@ void plan_free(OpPlan* p) { delete p; }
 // tiles: 112 / 460 us at 3 qubits, 127 / 525 at 12, 170 / 640 at 18, 347 / 1837 at
 // 22; 25 gates: 30 / 41 us at 12, 40 / 49 at 17, 72 / 125 at 22; one layer of
 // rotations and CNOTs: 36 / 37 us at 12, 50 / 52 at 17, 73 / 71 at 20, 110 / 139 at
-// 22; 8 gates (by rounds up to 12): 25 / 25 us at 12.
+// 22; 12 gates (by rounds up to 12 qubits): 22 / 25 us at 8, 26 / 26 at 12; 8 gates
+// 22 / 21 and 26 / 24.
 static bool takes_rounds(const Tuning& tu, int n, size_t ops) {
-    return tu.tile_auto && n <= kRoundsMaxQubits && ops >= (n <= 12 ? 8u : 24u);
+    return tu.tile_auto && n <= kRoundsMaxQubits && ops >= (n <= 12 ? 12u : 24u);
 }
 
 int run_ops(qfe_state_s* st, std::vector<HostOp>& ops) {

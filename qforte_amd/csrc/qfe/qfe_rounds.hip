@@ -287,6 +287,20 @@ bool split_rotation(const Z m[4], Z l[2], double& c, double& s, Z& r) {
     return true;
 }
 
+// Whether an op is a gate that the lowering below takes (a matrix that turns out
+// not to be unitary aside): general two-qubit matrices, exponentials and gates
+// under several conditions are not.
+bool has_form(const DevOp& o) {
+    if (o.kind == K_U2) {
+        // a swap, or a gate under "qubit c reads 0" (rows and columns 2c + t)
+        for (int r = 0; r < 4 && !o.hb; ++r)
+            for (int c = 0; c < 4; ++c)
+                if ((r > 1 || c > 1) && !zis(wide(o.m[4 * r + c]), r == c ? 1.0 : 0.0)) return false;
+        return true;
+    }
+    return (o.kind == K_U1 || o.kind == K_DIAG1) && __builtin_popcountll(o.cmask) <= 1;
+}
+
 struct FrameLowering {
     int n;
     uint32_t col[32], row[32];
@@ -385,13 +399,10 @@ struct FrameLowering {
         kind[q] = 0;
         return true;
     }
+    // o has a form
     bool add(const DevOp& o) {
         const int t = (int)o.t;
         if (o.kind == K_U2 && !o.hb) {
-            // a gate under "qubit c reads 0" (rows and columns 2c + t), else no form
-            for (int r = 0; r < 4; ++r)
-                for (int c = 0; c < 4; ++c)
-                    if ((r > 1 || c > 1) && !zis(wide(o.m[4 * r + c]), r == c ? 1.0 : 0.0)) return false;
             const Z m[4] = {wide(o.m[0]), wide(o.m[1]), wide(o.m[4]), wide(o.m[5])};
             return conditioned(t, (int)o.c, false, m);
         }
@@ -406,7 +417,6 @@ struct FrameLowering {
             neg ^= (d << t) | (d << c);
             return true;
         }
-        if (o.kind != K_U1 && o.kind != K_DIAG1) return false;
         const bool diag = o.kind == K_DIAG1;
         const Z m[4] = {wide(o.m[0]), diag ? kZero : wide(o.m[1]), diag ? kZero : wide(o.m[2]), wide(o.m[diag ? 1 : 3])};
         if (!o.cmask) {
@@ -419,7 +429,6 @@ struct FrameLowering {
             multiply(t, m);
             return true;
         }
-        if (__builtin_popcountll(o.cmask) != 1) return false;
         return conditioned(t, __builtin_ctzll(o.cmask), o.cval != 0, m);
     }
     // m on qubit t where qubit c reads cv
@@ -847,6 +856,9 @@ void to_logical(const FrameLowering& fl, RoundsPass& p) {
 // stored index that the last pass leaves differs from the logical one unless
 // `plain`.
 bool plan_rounds(const std::vector<HostOp>& ops, int n, RoundPlan& plan, bool& plain) {
+    // first of all: a list with one op that has no form is lowered for nothing
+    for (const HostOp& h : ops)
+        if (!has_form(h.op)) return false;
     FrameLowering fl(n);
     fl.out.reserve(ops.size());
     for (const HostOp& h : ops)
@@ -889,7 +901,7 @@ bool plan_tile_rounds(const std::vector<HostOp>& ops, const std::vector<int>& ta
                       std::vector<uint4>& words) {
     FrameLowering fl(n);
     for (int i : take)
-        if (!fl.add(ops[i].op)) return false;
+        if (!has_form(ops[i].op) || !fl.add(ops[i].op)) return false;
     for (int q = 0; q < n; ++q)
         if (!fl.flush(q)) return false;
     RoundPlan plan;
