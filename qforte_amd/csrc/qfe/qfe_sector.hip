@@ -39,7 +39,6 @@
 #include <deque>
 #include <functional>
 #include <map>
-#include <set>
 #include <unordered_map>
 #include <vector>
 
@@ -1150,15 +1149,21 @@ constexpr uint64_t kTileAmps = 1024;  // amplitudes of a tile
 
 // ---- host-side construction -------------------------------------------------------------
 
+// The bits of one spin (2 i + parity) together, and apart again; norb <= 16.
 inline uint32_t compress(uint64_t v, int parity, int norb) {
-    uint32_t out = 0;
-    for (int i = 0; i < norb; ++i) out |= (uint32_t)((v >> (2 * i + parity)) & 1ull) << i;
-    return out;
+    uint32_t x = (uint32_t)(v >> parity) & 0x55555555u;
+    x = (x | (x >> 1)) & 0x33333333u;
+    x = (x | (x >> 2)) & 0x0f0f0f0fu;
+    x = (x | (x >> 4)) & 0x00ff00ffu;
+    return (x | (x >> 8)) & ((1u << norb) - 1u);
 }
 inline uint64_t spread(uint32_t v, int parity, int norb) {
-    uint64_t out = 0;
-    for (int i = 0; i < norb; ++i) out |= (uint64_t)((v >> i) & 1u) << (2 * i + parity);
-    return out;
+    uint32_t x = v & ((1u << norb) - 1u);
+    x = (x | (x << 8)) & 0x00ff00ffu;
+    x = (x | (x << 4)) & 0x0f0f0f0fu;
+    x = (x | (x << 2)) & 0x33333333u;
+    x = (x | (x << 1)) & 0x55555555u;
+    return (uint64_t)x << parity;
 }
 inline int popc32(uint32_t v) { return __builtin_popcount(v); }
 inline int popc64(uint64_t v) { return __builtin_popcountll(v); }
@@ -1672,7 +1677,8 @@ struct RowBuilder {
     std::vector<uint2> b2;
     std::vector<RowFlip> flips;
     std::vector<RowPair> pairs;
-    std::vector<std::vector<std::pair<uint32_t, double>>> mrow;  // terms of every merged number
+    std::vector<uint2> mrow;                          // terms of every merged number: [x, x + y) of
+    std::vector<std::pair<uint32_t, double>> mterm;   // (term, sign)
     uint32_t nb1 = 0, nb2 = 0, nwords = 0, nfa = 0, nfb = 0, gbase = 0;
 
     struct Term {
@@ -1713,37 +1719,62 @@ struct RowBuilder {
         return true;
     }
     static size_t cells_of(const Group& g) {
-        std::map<uint32_t, int> m;
-        for (const Term& t : g.terms) m[t.zb] = 1;
-        return m.size();
+        std::vector<uint32_t> m;
+        for (const Term& t : g.terms) m.push_back(t.zb);
+        std::sort(m.begin(), m.end());
+        return (size_t)(std::unique(m.begin(), m.end()) - m.begin());
     }
-    static std::vector<uint32_t> patterns(uint32_t x) {  // half of the bits of x set
+    static std::vector<uint32_t> patterns(uint32_t x) {  // half of the bits of x set, ascending
         std::vector<uint32_t> out;
-        for (uint32_t p = x;; p = (p - 1) & x) {
+        for (uint32_t p = 0;; p = (p - x) & x) {
             if (2 * popc32(p) == popc32(x)) out.push_back(p);
-            if (!p) break;
+            if (p == x) break;
         }
-        std::sort(out.begin(), out.end());
         return out;
     }
-    // Cells of a group with the flipped bits of spin s in pattern p: terms
-    // merged by the beta mask, then by the alpha mask.  Returns (first cell, cells).
-    std::pair<uint32_t, uint32_t> add_cells(const Group& g, int s, uint32_t p, std::vector<uint32_t>& mu, std::vector<uint32_t>& m) {
-        std::map<uint32_t, std::map<uint32_t, std::vector<std::pair<uint32_t, double>>>> cell;
-        for (const Term& t : g.terms) {
-            const double sg = parity(p & (s ? t.zb : t.za)) ? -1.0 : 1.0;
-            cell[s ? t.zb & ~g.xb : t.zb][s ? t.za : t.za & ~g.xa].push_back({t.k, sg});
-        }
-        const uint32_t c0 = (uint32_t)mu.size();
-        for (auto& c : cell) {
-            mu.push_back(c.first);
-            for (auto& v : c.second) {
-                mmask.push_back(v.first);
-                mrow.push_back(std::move(v.second));
+    static bool flips_in(uint32_t v, uint32_t x) { return 2 * popc32(v & x) == popc32(x); }
+
+    // A flip of one spin by the pattern of the partner's flipped bits: what
+    // belongs to each (cells of a group, or numbers first, first + 1, ...).
+    struct Flip {
+        uint32_t x, first;
+        std::vector<uint32_t> pat;
+        std::vector<std::pair<uint32_t, uint32_t>> cells;  // (first cell, cells)
+        size_t at(uint32_t to) const { return (size_t)(std::lower_bound(pat.begin(), pat.end(), to & x) - pat.begin()); }
+    };
+
+    // Cells of a group for every pattern of the flipped bits of spin s: terms
+    // merged by the beta mask, then by the alpha mask.
+    Flip add_cells(const Group& g, int s, std::vector<uint32_t>& mu, std::vector<uint32_t>& m) {
+        Flip f{s ? g.xb : g.xa, 0, patterns(s ? g.xb : g.xa), {}};
+        // masks outside the flipped bits, which the pattern does not change
+        struct Key {
+            uint32_t b, a, t;
+        };
+        std::vector<Key> key;
+        for (uint32_t t = 0; t < g.terms.size(); ++t)
+            key.push_back(s ? Key{g.terms[t].zb & ~g.xb, g.terms[t].za, t} : Key{g.terms[t].zb, g.terms[t].za & ~g.xa, t});
+        std::sort(key.begin(), key.end(), [](const Key& u, const Key& v) { return u.b != v.b ? u.b < v.b : u.a != v.a ? u.a < v.a : u.t < v.t; });
+        for (uint32_t p : f.pat) {
+            const uint32_t c0 = (uint32_t)mu.size();
+            for (size_t i = 0; i < key.size(); ++i) {
+                const bool cell = i == 0 || key[i].b != key[i - 1].b;
+                if (cell) {
+                    if (i) m.push_back((uint32_t)mrow.size());
+                    mu.push_back(key[i].b);
+                }
+                if (cell || key[i].a != key[i - 1].a) {
+                    mmask.push_back(key[i].a);
+                    mrow.push_back(make_uint2((uint32_t)mterm.size(), 0));
+                }
+                const Term& t = g.terms[key[i].t];
+                mterm.push_back({t.k, parity(p & (s ? t.zb : t.za)) ? -1.0 : 1.0});
+                ++mrow.back().y;
             }
-            m.push_back((uint32_t)mrow.size());
+            if (!key.empty()) m.push_back((uint32_t)mrow.size());
+            f.cells.push_back({c0, (uint32_t)mu.size() - c0});
         }
-        return {c0, (uint32_t)mu.size() - c0};
+        return f;
     }
 
     // LDS of a row workgroup.
@@ -1757,13 +1788,10 @@ struct RowBuilder {
         const auto &as = sp.str[0], &bs = sp.str[1];
         const uint32_t Da = (uint32_t)as.size(), Db = (uint32_t)bs.size();
         auto rank = [&](int s, uint32_t v) { return (uint32_t)sp.rank[s][v]; };
-        auto flips_in = [&](uint32_t v, uint32_t x) { return 2 * popc32(v & x) == popc32(x); };
-        // alpha flips: cells per pattern of the partner's flipped bits
-        std::map<std::pair<size_t, uint32_t>, std::pair<uint32_t, uint32_t>> acells, bcells;
-        for (size_t i = 0; i < groups.size(); ++i) {
-            if (groups[i].xb) continue;
-            for (uint32_t p : patterns(groups[i].xa)) acells[{i, p}] = add_cells(groups[i], 0, p, amu, am);
-        }
+        // alpha flips and the diagonal
+        std::vector<Flip> af, bf;
+        for (const Group& g : groups)
+            if (!g.xb) af.push_back(add_cells(g, 0, amu, am));
         for (uint32_t ra = 0; ra < Da; ++ra) {
             uint4 cd = make_uint4((uint32_t)flips.size(), 0, (uint32_t)pos_cell.size(), 0);
             auto close = [&]() {
@@ -1773,10 +1801,10 @@ struct RowBuilder {
                 chunks.push_back(cd);
                 cd = make_uint4((uint32_t)flips.size(), 0, (uint32_t)pos_cell.size(), 0);
             };
-            for (size_t i = 0; i < groups.size(); ++i) {
-                if (groups[i].xb || !flips_in(as[ra], groups[i].xa)) continue;
-                const uint32_t to = as[ra] ^ groups[i].xa;
-                const auto c = acells.at({i, to & groups[i].xa});
+            for (const Flip& f : af) {
+                if (!flips_in(as[ra], f.x)) continue;
+                const uint32_t to = as[ra] ^ f.x;
+                const auto c = f.cells[f.at(to)];
                 if (cd.w + c.second > kRowCells) close();
                 flips.push_back(RowFlip{rank(0, to), c.first, c.second, cd.w});
                 for (uint32_t k = 0; k < c.second; ++k) pos_cell.push_back(c.first + k);
@@ -1787,17 +1815,15 @@ struct RowBuilder {
         }
         // beta flips
         bm[0] = (uint32_t)mrow.size();
-        for (size_t i = 0; i < groups.size(); ++i) {
-            if (groups[i].xa || !groups[i].xb) continue;
-            for (uint32_t p : patterns(groups[i].xb)) bcells[{i, p}] = add_cells(groups[i], 1, p, bmu, bm);
-        }
+        for (const Group& g : groups)
+            if (!g.xa && g.xb) bf.push_back(add_cells(g, 1, bmu, bm));
         std::vector<std::vector<uint32_t>> l1(Db);
         std::vector<std::vector<uint2>> l2(Db);
         for (uint32_t rb = 0; rb < Db; ++rb) {
-            for (size_t i = 0; i < groups.size(); ++i) {
-                if (groups[i].xa || !groups[i].xb || !flips_in(bs[rb], groups[i].xb)) continue;
-                const uint32_t to = bs[rb] ^ groups[i].xb;
-                const auto c = bcells.at({i, to & groups[i].xb});
+            for (const Flip& f : bf) {
+                if (!flips_in(bs[rb], f.x)) continue;
+                const uint32_t to = bs[rb] ^ f.x;
+                const auto c = f.cells[f.at(to)];
                 if (c.second == 1)
                     l1[rb].push_back(rank(1, to) | (c.first << 14) | (parity(bs[rb] & bmu[c.first]) << 31));
                 else
@@ -1815,51 +1841,59 @@ struct RowBuilder {
             for (size_t k = 0; k < l2[rb].size(); ++k) b2[k * Db + rb] = l2[rb][k];
         }
         // both: flips (mask, pattern of the partner) of each spin, and the table over them
-        std::map<uint32_t, int> xas, xbs;
-        for (const Group& g : groups)
-            if (g.xa && g.xb) xas[g.xa] = xbs[g.xb] = 1;
-        std::map<std::pair<uint32_t, uint32_t>, uint32_t> fa, fb;
-        for (auto& x : xas)
-            for (uint32_t p : patterns(x.first)) {
-                fa[{x.first, p}] = nfa++;
-                fa_mask.push_back(compress(between(spread(x.first, 0, norb)), 1, norb));
+        auto flips_of = [&](int s, uint32_t& count, std::vector<uint32_t>& mask) {
+            std::vector<uint32_t> xs;
+            for (const Group& g : groups)
+                if (g.xa && g.xb) xs.push_back(s ? g.xb : g.xa);
+            std::sort(xs.begin(), xs.end());
+            xs.erase(std::unique(xs.begin(), xs.end()), xs.end());
+            std::vector<Flip> out;
+            for (uint32_t x : xs) {
+                out.push_back(Flip{x, count, patterns(x), {}});
+                count += (uint32_t)out.back().pat.size();
+                mask.resize(count, compress(between(spread(x, s, norb)), 1 - s, norb));
             }
-        for (auto& x : xbs)
-            for (uint32_t p : patterns(x.first)) {
-                fb[{x.first, p}] = nfb++;
-                fb_mask.push_back(compress(between(spread(x.first, 1, norb)), 0, norb));
-            }
+            return out;
+        };
+        const std::vector<Flip> fa = flips_of(0, nfa, fa_mask), fb = flips_of(1, nfb, fb_mask);
+        auto find = [](const std::vector<Flip>& f, uint32_t x) -> const Flip& {
+            return *std::lower_bound(f.begin(), f.end(), x, [](const Flip& u, uint32_t v) { return u.x < v; });
+        };
         gbase = (uint32_t)mrow.size();
-        mrow.resize(mrow.size() + (size_t)nfa * nfb);
+        mrow.resize(mrow.size() + (size_t)nfa * nfb, make_uint2(0, 0));
         mmask.resize(mrow.size(), 0u);
         for (const Group& g : groups) {
             if (!g.xa || !g.xb) continue;
+            const Flip &u = find(fa, g.xa), &v = find(fb, g.xb);
             const uint32_t jba = compress(between(spread(g.xb, 1, norb)), 0, norb);
             const uint32_t jab = compress(between(spread(g.xa, 0, norb)), 1, norb);
-            for (uint32_t pa : patterns(g.xa))
-                for (uint32_t pb : patterns(g.xb)) {
-                    auto& row = mrow[gbase + (size_t)fa.at({g.xa, pa}) * nfb + fb.at({g.xb, pb})];
+            for (size_t i = 0; i < u.pat.size(); ++i)
+                for (size_t k = 0; k < v.pat.size(); ++k) {
+                    const uint32_t pa = u.pat[i], pb = v.pat[k];
                     // the strings' bits on the flipped qubits of the other spin depend on the patterns alone
                     const uint32_t c = parity((g.xa ^ pa) & jba) ^ parity(pb & jab);
-                    for (const Term& t : g.terms)
-                        row.push_back({t.k, (c ^ parity(pa & t.za) ^ parity(pb & t.zb)) ? -1.0 : 1.0});
+                    mrow[gbase + (u.first + i) * nfb + v.first + k] = make_uint2((uint32_t)mterm.size(), (uint32_t)g.terms.size());
+                    for (const Term& t : g.terms) mterm.push_back({t.k, (c ^ parity(pa & t.za) ^ parity(pb & t.zb)) ? -1.0 : 1.0});
                 }
         }
+        std::vector<uint32_t> ja, jb;  // a flip's own string
+        for (const Flip& f : fa) ja.push_back(compress(between(spread(f.x, 0, norb)), 0, norb) & ~f.x);
+        for (const Flip& f : fb) jb.push_back(compress(between(spread(f.x, 1, norb)), 1, norb) & ~f.x);
         for (uint32_t ra = 0; ra < Da; ++ra) {
-            for (auto& x : xas) {
-                if (!flips_in(as[ra], x.first)) continue;
-                const uint32_t to = as[ra] ^ x.first, j = compress(between(spread(x.first, 0, norb)), 0, norb);
-                pairs.push_back(RowPair{rank(0, to), fa.at({x.first, to & x.first}), parity(as[ra] & j & ~x.first) << 31, 0});
+            for (size_t i = 0; i < fa.size(); ++i) {
+                if (!flips_in(as[ra], fa[i].x)) continue;
+                const uint32_t to = as[ra] ^ fa[i].x;
+                pairs.push_back(RowPair{rank(0, to), fa[i].first + (uint32_t)fa[i].at(to), parity(as[ra] & ja[i]) << 31, 0});
             }
             while ((pairs.size() - pair_off.back()) % 4) pairs.push_back(RowPair{kRowNone, 0, 0, 0});
             pair_off.push_back((uint32_t)pairs.size());
         }
         std::vector<std::vector<uint32_t>> lw(Db);
         for (uint32_t rb = 0; rb < Db; ++rb) {
-            for (auto& x : xbs) {
-                if (!flips_in(bs[rb], x.first)) continue;
-                const uint32_t to = bs[rb] ^ x.first, j = compress(between(spread(x.first, 1, norb)), 1, norb);
-                lw[rb].push_back(rank(1, to) | (fb.at({x.first, to & x.first}) << 14) | (parity(bs[rb] & j & ~x.first) << 31));
+            for (size_t i = 0; i < fb.size(); ++i) {
+                if (!flips_in(bs[rb], fb[i].x)) continue;
+                const uint32_t to = bs[rb] ^ fb[i].x;
+                lw[rb].push_back(rank(1, to) | ((fb[i].first + (uint32_t)fb[i].at(to)) << 14) | (parity(bs[rb] & jb[i]) << 31));
             }
             nwords = std::max(nwords, (uint32_t)lw[rb].size());
         }
@@ -1990,8 +2024,15 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     // Hamiltonian terms by X mask (first appearance).  A flip connects
     // determinants of the sector when each spin has room for it: half of its
     // bits occupied, half empty.  The other masks are read by nothing.
-    std::map<uint64_t, std::vector<uint64_t>> byx;
-    std::vector<uint64_t> order;
+    struct Mask {
+        uint64_t x;
+        const uint64_t *first, *last;  // its terms
+        const uint64_t* begin() const { return first; }
+        const uint64_t* end() const { return last; }
+        bool in_rows;
+    };
+    std::vector<Mask> masks;
+    std::vector<uint64_t> members;
     {
         const int ne[2] = {popc32(refa), popc32(refb)};
         auto connects = [&](uint64_t x) {
@@ -2001,27 +2042,43 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
             }
             return true;
         };
+        // mask of every term (open addressing), then the terms to their places
+        size_t cap = 16;
+        while (cap < 2 * nham) cap <<= 1;
+        std::vector<uint32_t> slot(cap, 0), of(nham), count;  // slot: mask + 1
+        std::vector<uint64_t> xs;
         for (uint64_t k = 0; k < nham; ++k) {
             if ((ham[k].x | ham[k].z) & ~lim)
                 return fail(QFE_ERR_ARG, "qfe_template_create: Hamiltonian term acts on a qubit out of range");
-            if (!connects(ham[k].x)) continue;
-            auto& v = byx[ham[k].x];
-            if (v.empty()) order.push_back(ham[k].x);
-            v.push_back(k);
+            size_t h = (size_t)((ham[k].x * 0x9E3779B97F4A7C15ull) >> 20) & (cap - 1);
+            while (slot[h] && xs[slot[h] - 1] != ham[k].x) h = (h + 1) & (cap - 1);
+            if (!slot[h]) {
+                xs.push_back(ham[k].x);
+                count.push_back(0);
+                slot[h] = (uint32_t)xs.size();
+            }
+            of[k] = slot[h] - 1;
+            count[of[k]]++;
         }
+        std::vector<uint64_t> at(xs.size() + 1, 0);
+        for (size_t m = 0; m < xs.size(); ++m) at[m + 1] = at[m] + count[m];
+        members.resize(nham);
+        for (uint64_t k = nham; k-- > 0;) members[at[of[k]] + --count[of[k]]] = k;
+        for (size_t m = 0; m < xs.size(); ++m)
+            if (connects(xs[m])) masks.push_back(Mask{xs[m], members.data() + at[m], members.data() + at[m + 1], false});
     }
     // the map of every such term, before anything reads it
     if (map_off)
-        for (uint64_t x : order)
-            for (uint64_t k : byx[x]) {
+        for (const Mask& m : masks)
+            for (uint64_t k : m) {
                 if (map_off[k + 1] < map_off[k]) return fail(QFE_ERR_ARG, "qfe_template_create: map offsets must not decrease");
                 for (uint64_t e = map_off[k]; e < map_off[k + 1]; ++e)
                     if (map_idx[e] >= ninputs) return fail(QFE_ERR_ARG, "qfe_template_create: map index out of range");
             }
     t->real = true;
     for (const auto& en : entries) t->real = t->real && en.ulo.y == 0.0 && en.uhi.y == 0.0;
-    for (uint64_t x : order)
-        for (uint64_t k : byx[x]) {
+    for (const Mask& m : masks)
+        for (uint64_t k : m) {
             if (!t->has_map) {
                 t->real = t->real && cplx_mul(make_double2(ham[k].phase.re, ham[k].phase.im),
                                               make_double2(ham[k].coeff.re, ham[k].coeff.im)).y == 0.0;
@@ -2031,7 +2088,6 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
             for (uint64_t e = map_off[k]; e < map_off[k + 1]; ++e) t->real = t->real && map_val[e].im == 0.0;
         }
     RowBuilder rowb(sp, norb);
-    std::set<uint64_t> in_rows;
 
     std::vector<SecGroup> groups;
     std::vector<uint64_t> tz;
@@ -2042,23 +2098,28 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     {
         // groups that the rows take, in a real template
         std::vector<RowBuilder::Group> rgroups;
-        for (uint64_t x : order) {
-            if (!t->real) break;
+        std::vector<uint32_t> taken;  // their masks
+        for (uint32_t i = 0; t->real && i < masks.size(); ++i) {
+            const uint64_t x = masks[i].x;
             RowBuilder::Group g{x, compress(x, 0, norb), compress(x, 1, norb), {}};
-            for (uint64_t k : byx[x]) g.terms.push_back({compress(ham[k].z, 0, norb), compress(ham[k].z, 1, norb), (uint32_t)k});
-            if (rowb.fits(g)) rgroups.push_back(std::move(g));
+            g.terms.reserve((size_t)(masks[i].last - masks[i].first));
+            for (uint64_t k : masks[i]) g.terms.push_back({compress(ham[k].z, 0, norb), compress(ham[k].z, 1, norb), (uint32_t)k});
+            if (!rowb.fits(g)) continue;
+            rgroups.push_back(std::move(g));
+            taken.push_back(i);
         }
         if (rows_worth(rowb, rgroups)) {
             rowb.build(rgroups);
             if (rowb.lds() <= kRowLdsMax && rowb.bmu.size() < (1u << kRowCellBits) - 1 && rowb.nfb < (1u << kRowCellBits) - 1) {
-                for (const auto& g : rgroups) in_rows.insert(g.x);
+                for (uint32_t i : taken) masks[i].in_rows = true;
                 t->row_lds = rowb.lds();
                 t->nrows = t->Da * ((t->Db + kRowThreads - 1) / kRowThreads);
                 t->nm = (uint32_t)rowb.mrow.size();
             }
         }
-        for (uint64_t x : order) {
-            if (in_rows.count(x)) continue;
+        for (const Mask& m : masks) {
+            if (m.in_rows) continue;
+            const uint64_t x = m.x;
             const uint32_t xa = compress(x, 0, norb), xb = compress(x, 1, norb);
             SecGroup gr{};
             gr.x = x;
@@ -2088,7 +2149,7 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
             gr.lb_len = lb.second;
             gr.inv_lb = 1.0 / (double)lb.second;
             gr.t_first = (uint32_t)tz.size();
-            for (uint64_t k : byx[x]) {
+            for (uint64_t k : m) {
                 tz.push_back(ham[k].z);
                 const double2 ph = make_double2(ham[k].phase.re, ham[k].phase.im);
                 tph.push_back(ph);
@@ -2187,22 +2248,32 @@ int template_build(qfe_template t, int n, uint64_t ref, const qfe_pauli* gen_ter
     std::vector<double> rm, rmval;
     std::vector<uint32_t> rmoff{0}, rmidx;
     if (t->nrows) {
-        for (const auto& row : rowb.mrow) {
-            std::map<uint32_t, double> in;
+        struct Part {
+            uint32_t input, order;
+            double v;
+        };
+        std::vector<Part> in;
+        for (const uint2& row : rowb.mrow) {
+            in.clear();
             double v = 0.0;
-            for (const auto& tk : row) {
+            for (uint32_t i = row.x; i < row.x + row.y; ++i) {
+                const auto& tk = rowb.mterm[i];
                 const qfe_pauli& h = ham[tk.first];
                 if (t->has_map)
                     for (uint64_t e = map_off[tk.first]; e < map_off[tk.first + 1]; ++e)
-                        in[map_idx[e]] += tk.second * h.phase.re * map_val[e].re;
+                        in.push_back(Part{map_idx[e], (uint32_t)in.size(), tk.second * h.phase.re * map_val[e].re});
                 else
                     v += tk.second * (h.phase.re * h.coeff.re - h.phase.im * h.coeff.im);
             }
-            for (const auto& e : in)
-                if (e.second != 0.0) {
-                    rmidx.push_back(e.first);
-                    rmval.push_back(e.second);
-                }
+            std::sort(in.begin(), in.end(), [](const Part& a, const Part& b) { return a.input != b.input ? a.input < b.input : a.order < b.order; });
+            for (size_t i = 0; i < in.size();) {
+                const uint32_t idx = in[i].input;
+                double sum = 0.0;
+                for (; i < in.size() && in[i].input == idx; ++i) sum += in[i].v;
+                if (sum == 0.0) continue;
+                rmidx.push_back(idx);
+                rmval.push_back(sum);
+            }
             rmoff.push_back((uint32_t)rmidx.size());
             if (!t->has_map) rm.push_back(v);
         }
