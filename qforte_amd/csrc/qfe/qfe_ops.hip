@@ -2238,15 +2238,20 @@ void plan_free(OpPlan* p) { delete p; }
 // tiles: 112 / 460 us at 3 qubits, 127 / 525 at 12, 170 / 640 at 18, 347 / 1837 at
 // 22; 25 gates: 30 / 41 us at 12, 40 / 49 at 17, 72 / 125 at 22; one layer of
 // rotations and CNOTs: 36 / 37 us at 12, 50 / 52 at 17, 73 / 71 at 20, 110 / 139 at
-// 22; 12 gates (by rounds up to 12 qubits): 22 / 25 us at 8, 26 / 26 at 12; 8 gates
-// 22 / 21 and 26 / 24.
-static bool takes_rounds(const Tuning& tu, int n, size_t ops) {
-    return tu.tile_auto && n <= kRoundsMaxQubits && ops >= (n <= 12 ? 12u : 24u);
+// 22; 10 gates 22 / 23 us at 8, 23.5 / 24.5 at 10 and 27 / 25 at 12, 12 gates 26 / 26
+// at 12, 8 gates 22 / 21, 24 / 22 and 26 / 24, but 8 X gates 13 / 20 and 14 / 22.
+static bool takes_rounds(const Tuning& tu, int n, const std::vector<HostOp>& ops) {
+    if (!tu.tile_auto || n > kRoundsMaxQubits) return false;
+    if (ops.size() >= (n <= 10 ? 10u : n <= 12 ? 12u : 24u)) return true;
+    if (n > 12 || ops.size() < 8) return false;
+    for (const HostOp& h : ops)  // index moves: X under at most one condition, and swaps
+        if (!h.op.hb || !(h.op.kind == K_U2 || (h.op.kind == K_U1 && __builtin_popcountll(h.op.cmask) <= 1))) return false;
+    return true;
 }
 
 int run_ops(qfe_state_s* st, std::vector<HostOp>& ops) {
     if (ops.empty()) return QFE_OK;
-    if (takes_rounds(ctx().tuning, st->n, ops.size())) {
+    if (takes_rounds(ctx().tuning, st->n, ops)) {
         bool taken = false;
         const int rc = run_rounds(st, ops, taken);
         if (rc || taken) return rc;
