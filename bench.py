@@ -32,14 +32,16 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
-# HBM bytes per launch of the exponential-stage kernel, by (qubits, orbit
-# width), from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB per dispatch),
-# each scaled by the same counter's reading on k_scale, a plain sweep that
-# reads and writes exactly 16 GiB (FETCH 8388621-8388622 KiB: factor 2.0000;
-# WRITE 16778250-16778282 KiB: factor 0.99994).
+# HBM bytes per launch of the exponential-stage kernel, by (qubits, kernel),
+# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB per dispatch), each scaled
+# by the same counter's reading on k_scale, a plain sweep that reads and writes
+# exactly 16 GiB (FETCH 8388621-8388622 KiB: factor 2.0000; WRITE
+# 16778250-16778302 KiB: factor 0.99994).
+#   k_wide: FETCH 8401724, WRITE 17277305 -> 34079716 KiB
 #   k_orbit_lanes<4, 3>: FETCH 8388762, WRITE 16782743 -> 33559207 KiB
 #   k_orbit_lanes<4, 2>: FETCH 8388759, WRITE 16786363 -> 33562824 KiB
-TRAFFIC_PER_LAUNCH = {(30, 7): 33559207 * 1024, (30, 6): 33562824 * 1024}
+TRAFFIC_PER_LAUNCH = {(30, "k_wide"): 34079716 * 1024, (30, "k_orbit_lanes<4, 3>"): 33559207 * 1024,
+                      (30, "k_orbit_lanes<4, 2>"): 33562824 * 1024}
 METRIC = "HBM GB/s (% peak) at 30 qubits; batched UCC energy evals/s + p99 vs plain"
 
 
@@ -56,8 +58,8 @@ def build_workload(qf, W, n, nlayers, nexp, nterms):
 
 def time_exp_stage(qf, qc, U):
     """Average launch duration of the passes of the exponential stage (the
-    dominant kernel: register-orbit passes, one read-write sweep of the state
-    each), HIP events on the engine stream around one application of U."""
+    dominant kernel: one read-write sweep of the state each), HIP events on the
+    engine stream around one application of U."""
     qf.synchronize()
     qf.reset_counters()
     t = qf.DeviceTimer()
@@ -741,8 +743,10 @@ def main():
     qc = qf.Computer(n)
 
     if args.roofline_only:
-        # short run for hardware-counter passes: the exponential stage once,
-        # then two plain read-write sweeps (k_scale) as the calibration kernel
+        # short run for hardware-counter passes: the gate layers and the
+        # exponential stage once, the stage again, then two plain read-write
+        # sweeps (k_scale) as the calibration kernel
+        qc.apply_circuit(layer_circ)
         qc.apply_circuit(U)
         avg_ms, passes = time_exp_stage(qf, qc, U)
         qc.apply_constant(1.0)
@@ -787,21 +791,23 @@ def main():
         gate_ms = time_single_gate_sweep(qf, qc, n)
         copy_ms = time_attainable_sweep(qf, qc)
         dims = qf.get_pass_tuning()
-        if dims > 4:
-            kname = (f"k_orbit_lanes<4, {dims - 4}> ({dims}-dimension register orbits over {1 << (dims - 4)} lanes "
-                     f"of 16 amplitudes")
+        if dims == 7 and tuple(qf.get_tuning()) == (-1, -1, -1):
+            kname, what = "k_wide", "LDS tiles of 11 dimensions, eight flips a pass"
+        elif dims > 4:
+            kname = f"k_orbit_lanes<4, {dims - 4}>"
+            what = f"{dims}-dimension register orbits over {1 << (dims - 4)} lanes of 16 amplitudes"
         else:
-            kname = f"k_orbit<{dims}> ({dims}-dimension register orbits in one lane"
+            kname, what = f"k_orbit<{dims}>", f"{dims}-dimension register orbits in one lane"
         roofline = {
-            "kernel": (kname + "; the exponential stage: %d passes for %d exponentials, 2S = %.2f GB per launch)"
-                       % (passes, len(strings), 2 * S / 1e9)),
+            "kernel": ("%s (%s; the exponential stage: %d passes for %d exponentials, 2S = %.2f GB per launch)"
+                       % (kname, what, passes, len(strings), 2 * S / 1e9)),
             "stage_ms": round(avg_ms * passes, 1),
             "bound": "hbm",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBPS, 4),
-            "traffic": TRAFFIC_PER_LAUNCH.get((n, dims)),
+            "traffic": TRAFFIC_PER_LAUNCH.get((n, kname)),
             "avg_launch_ms": round(avg_ms, 4),
             "single_exponential_sweep": {"kernel": "k_pexp", "avg_launch_ms": round(single_ms, 4),
                                          "achieved": round(2 * S / (single_ms * 1e-3) / 1e9, 1),
