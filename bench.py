@@ -367,7 +367,7 @@ def timed(fn, reps=3):
 def gradient_leg(qf, W, nqubit=20, seed=20, fd_components=6, full_pool_sample=128):
     """Full UCCSD gradient at 20 qubits through torch.autograd (adjoint
     backward), checked against central differences and the full-space
-    program, plus ADAPT GSD pool gradients in batches of 64."""
+    program, plus ADAPT GSD pool gradients."""
     import numpy as np
     import torch
 

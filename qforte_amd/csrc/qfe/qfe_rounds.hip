@@ -22,7 +22,7 @@
 // 1.7 us at 12-bit tiles), the phase tables and the rotations (0.5 us each, FP64
 // at one wave per SIMD).  500 random gates on 12 qubits are 28 rounds in one
 // launch of one workgroup, 55 us (15 launches of gate-by-gate 8-qubit tiles on
-// 16 workgroups: 374 us); 800 on 17 qubits seven launches of 18 us (27 of 30 us).
+// 16 workgroups: 374 us); 800 on 17 qubits six launches of 20 us (27 of 30 us).
 // On states beyond 22 qubits every tile pass is planned on its own and works in
 // place (a move's target lies in the tile, so its frame stays in the coset), with
 // 11-bit tiles, three flips a round and 8 amplitudes per thread: four waves per

@@ -1140,10 +1140,10 @@ constexpr uint32_t kTableLds = 1024;
 
 // Tile shape.  Larger tiles take fewer passes but longer chains of steps per
 // workgroup.  20-qubit residuals / 16-qubit gradient / 512 mixed energies / 128
-// mixed gradients (us): 64 threads and 512 amplitudes 3709 / 1526 / 16480 /
-// 18470, 64 and 1024 3590 / 1538 / 15680 / 17870, 128 and 1024 3475 / 1458 /
-// 15560 / 17610, 128 and 2048 3510 / 1514 / 15390 / 17330, 128 and 4096 3975 /
-// 1762 / 15990 / 18090, 256 and 4096 3518 / 1542 / 15020 / 17020.
+// mixed gradients (us): 64 threads and 512 amplitudes 1489 / 621 / 8867 / 6602,
+// 64 and 1024 1368 / 634 / 8165 / 5942, 128 and 1024 1247 / 556 / 7982 / 5620,
+// 256 and 1024 1213 / 540 / 8841 / 6355, 128 and 2048 1274 / 610 / 7595 / 5377,
+// 256 and 2048 1219 / 596 / 7531 / 5242: lone requests and batches differ.
 constexpr int kTileThreads = 128;
 constexpr uint64_t kTileAmps = 1024;  // amplitudes of a tile
 

@@ -4,8 +4,8 @@ A request is a ``SectorTemplate`` (one size class: ansatz and Hamiltonian
 structure), its amplitudes and its Hamiltonian inputs (integrals packed by
 ``HamiltonianMap.pack``).  The native engine (``qfe_batch``) queues requests
 on the host; every ``step``/``poll`` launches what can be admitted onto one of
-a few streams (one workgroup per request, requests of any size class in the
-same launch, bounded by the HBM budget), so work that arrives while other
+a few streams (the tiles and rows of all its requests in each launch, requests
+of one size tier together, bounded by the HBM budget), so work that arrives while other
 launches run is admitted into the next launch and launches overlap on the
 device.  A gradient request (``gradient=True``) returns the energy and the
 adjoint gradient of the amplitudes (``SectorTemplate.gradient``); it is
