@@ -30,6 +30,7 @@ int fail(int code, const std::string& msg) {
 }
 
 int hip_fail(hipError_t e, const char* what) {
+    (void)hipGetLastError();  // reported here: the next launch's check must not find it again
     g_last_error = std::string("HIP error in ") + what + ": " + hipGetErrorString(e);
     return e == hipErrorOutOfMemory ? QFE_ERR_NOMEM : QFE_ERR_DEVICE;
 }

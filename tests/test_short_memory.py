@@ -65,6 +65,18 @@ prog.gradient(t)
 prog.residuals(t, [0, 1])
 assert "k_program_tileILi1" in names() and "k_program_tileILi2" not in names(), names()
 """,
+    "error reported once": """
+qc = qf.Computer(12)
+qc.apply_circuit(circuit(12, 4))
+spare(0)
+for _ in range(2):
+    try: qf.Computer(24)
+    except RuntimeError as e: assert "out of memory" in str(e)
+    else: raise SystemExit("created")
+    qc.apply_circuit(circuit(12, 4))
+host.host_limit(2**63)
+qf.Computer(24)
+""",
     "given back": """
 qc = qf.Computer(20)
 qc.apply_circuit(circuit(20, 500))
