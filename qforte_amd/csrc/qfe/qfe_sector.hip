@@ -3124,6 +3124,8 @@ int grow_pinned(void*& p, size_t& cap, size_t need) {
 // Largest launch of gradient requests (the sigma kernel's grid y is the request).
 constexpr size_t kMaxGradLaunch = 65535;
 
+int lane_start(qfe_batch b, Lane& L, bool grad, const std::vector<Request>& take);
+
 int lane_launch(qfe_batch b, Lane& L) {
     // a launch holds one kind: the kind whose oldest queued request arrived first
     std::deque<Request>& qe = b->queue[L.tier];
@@ -3159,6 +3161,15 @@ int lane_launch(qfe_batch b, Lane& L) {
     if (take.empty()) return QFE_OK;
     // heaviest requests first, so their workgroups start first
     std::stable_sort(take.begin(), take.end(), [](const Request& x, const Request& y) { return x.t->cost > y.t->cost; });
+    const int rc = lane_start(b, L, grad, take);
+    if (rc) {  // no request is lost: they keep their places for a later step
+        for (Request& r : take) queue.push_front(std::move(r));
+        std::sort(queue.begin(), queue.end(), [](const Request& x, const Request& y) { return x.id < y.id; });
+    }
+    return rc;
+}
+
+int lane_start(qfe_batch b, Lane& L, bool grad, const std::vector<Request>& take) {
     const size_t k = take.size();
     size_t io_total = 0, work_total = 0, gtotal = 0;
     uint64_t items = 0;

@@ -37,6 +37,26 @@ print("ok")
     assert out.strip() == "ok"
 
 
+@pytest.mark.parametrize("gradient", [False, True])
+def test_a_launch_that_fails_keeps_its_requests(on_host, gradient):  # noqa: F811
+    out = on_host(SETUP + f"""
+eng = qf.BatchEngine(64 << 30, 1 << 20)
+ids = [eng.submit(tpl, t, inputs, {gradient}) for _ in range(5)]
+host.host_limit(host.host_used())
+for _ in range(2):
+    try: eng.step()
+    except RuntimeError as e: assert "out of memory" in str(e)
+    else: raise SystemExit("launched")
+    assert eng.pending() == (5, 0)
+host.host_limit(2**63)
+done = []
+while len(done) < 5: done += eng.step()
+assert sorted(i for i, _ in done) == ids and eng.pending() == (0, 0)
+print("ok")
+""")
+    assert out.strip() == "ok"
+
+
 @pytest.mark.gpu
 def test_many_small_requests_values(qf):
     ns = {"qf": qf}
